@@ -54,6 +54,7 @@
  *   lv_token_shift           mixes of every token's input with its predecessor's
  *   lv_gated_scan            S <- decay S + write k v^T, o = S^T q with the state in f32, decay and write from step sizes,
  *                            from log gates under a running maximum, or one decay per row of the state with a bonus
+ *   lv_chunk_scan            the recurrences with one decay per head and token, 32 tokens at a time on the matrix cores
  *   lv_scaled_head_norm_gate lv_head_norm_gate with a weight per head and a division of every head by its own number
  *   lv_grouped_gate_norm     o * silu(z), RMS norm in equal parts, weight
  *   lv_residual_pair_norm    single f32 residual: adds the scaled sum of two RMS-normed and weighted sublayer outputs, RMS norm
@@ -86,7 +87,7 @@
 extern "C" {
 #endif
 
-#define LV_MIX_ABI_VERSION 9
+#define LV_MIX_ABI_VERSION 10
 #define LV_MIX_BF16 0
 #define LV_MIX_F32 1
 #define LV_MIX_MAX_STREAMS 8
@@ -103,6 +104,9 @@ extern "C" {
 #define LV_MIX_SCAN_STEP 0        /* lv_gated_scan: how a state decays and what it takes, see there */
 #define LV_MIX_SCAN_LOG_GATES 1
 #define LV_MIX_SCAN_ROW_DECAY 2
+#define LV_MIX_CHUNK_STEP 0       /* lv_chunk_scan: lv_gated_scan's LV_MIX_SCAN_STEP */
+#define LV_MIX_CHUNK_CONST 1      /* lv_lightning_attn */
+#define LV_MIX_CHUNK_DELTA 2      /* lv_gated_delta_rule with one decay per head */
 #define LV_MIX_SCORE_SIGMOID 0
 #define LV_MIX_SCORE_SOFTMAX 1
 #define LV_MIX_GROUP_TOP2_SUM 0   /* a group of experts is ranked by the sum of its two highest selection scores */
@@ -400,6 +404,21 @@ int lv_gated_scan(int kind, const void* q, int64_t ldq, const void* k, int64_t l
                   const void* a2, int64_t lda, const void* p0, const void* p1, const void* p2, float q_scale, float cap,
                   void* state, void* norm_state, void* max_state, const int32_t* cu_q, const int32_t* ctx_lens,
                   const int32_t* slots, void* o, void* den, int B, int H, int G, int D, int Dv, int dtype, void* stream);
+
+/* The recurrences of lv_gated_scan (step sizes), lv_lightning_attn and lv_gated_delta_rule (one decay per head) over chunks of
+ * 32 tokens, for steps with long portions; the same f32 products and sums in another order. G query/key groups of D (64 or 128), H
+ * value heads of Dv (64 or a multiple of 128). kind:
+ *   LV_MIX_CHUNK_STEP   bf16 rows; a, lda, p0, p1, p2 as in lv_gated_scan
+ *   LV_MIX_CHUNK_CONST  bf16 rows, silu applied as they are read; decay f32 [H]; G == H
+ *   LV_MIX_CHUNK_DELTA  f32 rows q, k, v; a = beta f32 [T, H], decay f32 [T, H]
+ * q, k aligned to four entries, ldq and ldk multiples of 4. max_new >= every sequence's new tokens. seg_len > 0 (a multiple of
+ * 32, not for the delta rule): sequences are cut into segments of that many tokens whose contributions are formed side by
+ * side. workspace: lv_chunk_scan_workspace_bytes with the same numbers, aligned to 16 bytes. */
+int lv_chunk_scan(int kind, const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, const void* a,
+                  int64_t lda, const void* decay, const void* p0, const void* p1, const void* p2, void* state,
+                  const int32_t* cu_q, const int32_t* ctx_lens, const int32_t* slots, void* o, void* workspace,
+                  int64_t workspace_bytes, int64_t T, int B, int max_new, int H, int G, int D, int Dv, int seg_len, void* stream);
+int64_t lv_chunk_scan_workspace_bytes(int kind, int64_t T, int B, int max_new, int H, int D, int Dv, int seg_len);
 
 /* lv_head_norm_gate with o[t, h] divided by den[t, h] first (den f32 [T, H] or NULL) and the norm weight of head h at
  * norm_w + h * w_ld (w_ld 0: one weight for all heads; Dv: each its own). */

@@ -17,8 +17,8 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc", "mixers")
 LIB_PATH = os.path.join(_HERE, "lib", "liblvmix.so")
 SOURCES = ["mix_stream.hip", "mix_window_attn.hip", "mix_window_mfma.hip", "mix_latent.hip", "mix_moe_gemm.hip",
-           "mix_sandwich.hip", "mix_parallel.hip", "mix_recurrent.hip", "mix_prep.hip", "mix_lru.hip"]
-ABI_VERSION = 9
+           "mix_sandwich.hip", "mix_parallel.hip", "mix_recurrent.hip", "mix_prep.hip", "mix_lru.hip", "mix_chunk.hip"]
+ABI_VERSION = 10
 
 _P = c_void_p
 SIGNATURES = {
@@ -80,6 +80,9 @@ SIGNATURES = {
     "lv_token_shift": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, c_int64, c_int, c_int, c_int, _P]),
     "lv_gated_scan": (c_int, [c_int, _P, c_int64, _P, c_int64, _P, c_int64, _P, _P, c_int64, _P, _P, _P, c_float, c_float, _P, _P,
                               _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P]),
+    "lv_chunk_scan": (c_int, [c_int, _P, c_int64, _P, c_int64, _P, c_int64, _P, c_int64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, c_int64,
+                              c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P]),
+    "lv_chunk_scan_workspace_bytes": (c_int64, [c_int, c_int64, c_int, c_int, c_int, c_int, c_int, c_int]),
     "lv_scaled_head_norm_gate": (c_int, [_P, _P, _P, c_int64, _P, c_int, _P, c_int64, c_int, c_int, c_float, c_int, c_int, _P]),
     "lv_grouped_gate_norm": (c_int, [_P, _P, c_int64, _P, _P, c_int64, c_int, c_int, c_float, c_int, _P]),
     "lv_residual_pair_norm": (c_int, [_P, _P, _P, _P, _P, c_float, c_float, _P, c_float, _P, c_int64, c_int, c_float, c_int, _P]),

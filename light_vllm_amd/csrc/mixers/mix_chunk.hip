@@ -1,0 +1,541 @@
+// Recurrences with one decay per head and token, 32 tokens at a time on the f32 matrix instructions.
+//
+//   S_t = g_t S_(t-1) + k_t u_t^T,   o_t = S_t^T q_t,   u_t = w_t v_t                          (step sizes, constant decays)
+//                                                       u_t = beta_t (v_t - g_t S_(t-1)^T k_t)  (delta rule)
+//
+// With G_t the product of a chunk's decays up to t, E_t the product of those behind t, D_tj = g_(j+1) .. g_t and S the state
+// in front of the chunk:
+//
+//   U = V                       (delta rule: U = T (V - diag(G) K S),  T = (I + tril(diag(beta) (D o K K^T), -1))^-1 diag(beta))
+//   O = diag(G) Q S + P U,      P_tj = D_tj (q_t . k_j) w_j for j <= t   (w = 1 for the delta rule)
+//   S <- G_last S + K^T diag(E w) U
+//
+// chunk_prep_kernel      T, P, G and E w of every chunk, all of them side by side
+// chunk_scan_kernel      the chain over a sequence's chunks; a wave owns all D rows of 32 columns of the state
+// chunk_combine_kernel   starting states of a sequence's segments, where there are too few sequences for the chip
+//
+// Every product of decays is formed as one (no exponentials of differences of logarithms), so a ratio is as exact as in the
+// token loop and a decay of zero stays zero.
+//
+// All products run on v_mfma_f32_32x32x2_f32: f32 operands and sums, as in the token loop. Its result layout (16 registers, rows
+// 8 (i / 4) + 4 (lane / 32) + i % 4, column lane % 32) is its own right-hand operand layout if step i multiplies the left-hand
+// column of the same number: the state, U and V - G K S go from product to product in registers, and only q, k, T and P
+// pass through LDS.
+//
+// Bound by the f32 matrix rate: 4 D Dv + 64 (D + Dv) multiply-adds a token and head, 6 D Dv + 96 D + 128 Dv for the delta rule. The
+// token loop they replace did fewer, but on the vector ALU, one token behind the other. Layer kernels on one box, us:
+// 16 x 1024 tokens, delta rule (16 heads, 128 x 128) 993 -> 328; constant decays (16 heads, 128 x 128) 596 -> 280; step sizes (32
+// heads, 128 x 64; 7 prompts, the longest 3750) 1531 -> 445.
+#include "mix_common.h"
+
+namespace lvmix {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kCh = 32;               // tokens of a chunk
+constexpr int kPad = 4;               // floats behind every LDS row: 16-byte reads of 8 rows meet 8 different bank groups
+
+enum ChunkKind { kChunkStep = LV_MIX_CHUNK_STEP, kChunkConst = LV_MIX_CHUNK_CONST, kChunkDelta = LV_MIX_CHUNK_DELTA };
+
+struct ChunkParams {
+  const void *q, *k, *v;              // act rows of stride ldq, ldk, ldv: query/key group h / (H/G) of D, value head h of Dv
+  int64_t ldq, ldk, ldv;
+  const void* a;                      // step sizes: act rows of stride lda; delta rule: beta f32 [T, H]
+  int64_t lda;
+  const float* decay;                 // [H] (constant) or [T, H] (delta rule)
+  const float *p0, *p1, *p2;          // step sizes: bias, log rate, skip [H]
+  float* state;
+  const int32_t *cu_q, *ctx_lens, *slots;
+  float* o;
+  float *P, *Tm, *Gf, *Ef;            // workspace: [T, H, 32], [T, H, 32] (delta rule), [T, H], [T, H]
+  float *seg_state, *seg_decay;       // workspace: [B, segments, H, D, Dv], [B, segments, H]
+  int H, G, D, Dv, seg_len, segs;
+};
+
+__device__ __forceinline__ float chunk_lane(float x, int i) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), i));
+}
+__device__ __forceinline__ int acc_row(int i, int half) { return 8 * (i >> 2) + 4 * half + (i & 3); }
+
+// x / (1 + exp(-x)) in about half the instructions of siluf_, to the same two units in the last place: the exponent as a sum of
+// two floats in front of the hardware exp2, the hardware reciprocal with one Newton step behind it. Where exp(-x) would
+// overflow, x is multiplied by 1e-38.
+__device__ __forceinline__ float chunk_silu(float x) {
+  constexpr float kLog2e = 1.44269504f, kLog2eRest = 1.92596303e-8f, kLn2 = 0.69314718f;
+  const float c = __builtin_amdgcn_fmed3f(x, -87.0f, 87.0f);
+  const float t = -kLog2e * c, rest = fmaf(-kLog2e, c, -t) - kLog2eRest * c;
+  float e = __builtin_amdgcn_exp2f(t);
+  e = fmaf(e, kLn2 * rest, e);
+  const float d = 1.0f + e;
+  float q = __builtin_amdgcn_rcpf(d);
+  q = fmaf(q, fmaf(-d, q, 1.0f), q);
+  return x * q;
+}
+template <bool SILU>
+__device__ __forceinline__ float4 chunk_act(float4 x) {
+  if constexpr (SILU) return float4{chunk_silu(x.x), chunk_silu(x.y), chunk_silu(x.z), chunk_silu(x.w)};
+  return x;
+}
+
+// grid: (chunk, group, sequence), four waves. The products q k^T and k k^T do not depend on the head: the waves take a share of
+// the key dimension each, and every wave then takes heads of the group.
+template <typename T, int KIND>
+__global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
+  constexpr bool DELTA = KIND == kChunkDelta, SILU = KIND == kChunkConst;
+  constexpr int RS = kCh + 1;
+  __shared__ float prod[4][kCh * RS];                  // partial products; afterwards each wave's own scratch
+  __shared__ __attribute__((aligned(16))) float amat[DELTA ? 4 : 1][kCh * (kCh + kPad)];
+  __shared__ float powers[KIND == kChunkConst ? 4 : 1][kCh + 1];
+  const int b = blockIdx.z, g = blockIdx.y, c0 = blockIdx.x * kCh;
+  const int q0 = p.cu_q[b], n = p.cu_q[b + 1] - q0;
+  if (c0 >= n) return;
+  const int cn = min(kCh, n - c0);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, half = lane >> 5;
+  const int64_t t0 = static_cast<int64_t>(q0) + c0;
+  {
+    const bool kk = DELTA && w < 2;                    // delta rule: waves 0, 1 k k^T, waves 2, 3 q k^T; otherwise all q k^T
+    const int shares = DELTA ? 2 : 4, share = DELTA ? (w & 1) : w;
+    const T* left = static_cast<const T*>(kk ? p.k : p.q) + (t0 + r) * (kk ? p.ldk : p.ldq) + static_cast<int64_t>(g) * p.D;
+    const T* right = static_cast<const T*>(p.k) + (t0 + r) * p.ldk + static_cast<int64_t>(g) * p.D;
+    const bool in = r < cn;
+    f32x16 acc, acc2;                                  // two sums of half the length: half the roundings each
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = acc2[i] = 0.0f;
+    for (int d = share * 8; d < p.D; d += shares * 8) {
+      float4 x{0, 0, 0, 0}, y{0, 0, 0, 0};
+      if (in) {
+        x = chunk_act<SILU>(ld4(left + d + 4 * half));
+        y = chunk_act<SILU>(ld4(right + d + 4 * half));
+      }
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, y.x, acc, 0, 0, 0);
+      acc2 = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, y.y, acc2, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, y.z, acc, 0, 0, 0);
+      acc2 = __builtin_amdgcn_mfma_f32_32x32x2f32(x.w, y.w, acc2, 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) prod[w][acc_row(i, half) * RS + r] = acc[i] + acc2[i];
+  }
+  __syncthreads();
+  const int rep = p.H / p.G;
+  const uint32_t p_off = static_cast<uint32_t>(4 * half * p.H * kCh) + r;
+  int r_here = r, half_here = half, cn_here = cn;
+#pragma unroll 1
+  for (int hr = w; hr < rep; hr += 4) {
+    asm volatile("" : "+v"(r_here), "+v"(half_here), "+s"(cn_here) : : "memory");      // masks and reads stay in the loop: hoisted they spill
+    const int r = r_here, half = half_here, cn = cn_here;
+    const int h = g * rep + hr;
+    // lane = token (both halves alike): decay, factor of the written value
+    float dec = 1.0f, wr = 1.0f;
+    if (r < cn) {
+      const int64_t at = (t0 + r) * p.H + h;
+      if constexpr (KIND == kChunkStep) {
+        wr = softplusf_(ldf(static_cast<const T*>(p.a) + (t0 + r) * p.lda + h) + p.p0[h]);
+        dec = expf(-expf(p.p1[h]) * wr);
+      } else if constexpr (DELTA) {
+        wr = static_cast<const float*>(p.a)[at];       // beta
+        dec = p.decay[at];
+      }
+    } else {
+      wr = 0.0f;
+    }
+    // G_t and E_t, lane = t; D_tj, lane = j with t in the result layout's registers. The products are formed in 64 bits and
+    // rounded once: a constant decay rounds the same way at every step, and its error would grow with the tokens it spans.
+    float gt = 1.0f, et = 1.0f;
+    float dm[16];
+    if constexpr (KIND == kChunkConst) {
+      double pw = 1.0, sq = p.decay[h];
+      for (int e = lane; e > 0; e >>= 1, sq *= sq)
+        if (e & 1) pw *= sq;
+      if (lane <= kCh) powers[w][lane] = static_cast<float>(pw);
+      __builtin_amdgcn_wave_barrier();
+      gt = powers[w][r + 1];
+      et = powers[w][max(cn - 1 - r, 0)];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int e = acc_row(i, half) - r;
+        dm[i] = e >= 0 ? powers[w][max(e, 0)] : 0.0f;
+      }
+      __builtin_amdgcn_wave_barrier();
+    } else {
+      double run = 1.0, back = 1.0, col = 0.0;
+#pragma unroll
+      for (int t = 0; t < kCh; ++t) {
+        const double gd = chunk_lane(dec, t);
+        run *= gd;
+        gt = r == t ? static_cast<float>(run) : gt;
+        col = r == t ? 1.0 : col * gd;                 // zero above the diagonal
+        const float colf = static_cast<float>(col);
+        if (((t >> 2) & 1) == 0) dm[4 * (t >> 3) + (t & 3)] = colf;   // rows of the lower half of the lanes
+        else dm[4 * (t >> 3) + (t & 3)] = half ? colf : dm[4 * (t >> 3) + (t & 3)];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = kCh - 1; t >= 0; --t) {
+        et = r == t ? static_cast<float>(back) : et;
+        back *= chunk_lane(dec, t);
+      }
+    }
+    if (half == 0 && r < cn) {
+      p.Gf[(t0 + r) * p.H + h] = gt;
+      p.Ef[(t0 + r) * p.H + h] = DELTA ? et : et * wr;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int t = acc_row(i, half);
+      float x;
+      if constexpr (DELTA) x = prod[2][t * RS + r] + prod[3][t * RS + r];
+      else x = (prod[0][t * RS + r] + prod[1][t * RS + r]) + (prod[2][t * RS + r] + prod[3][t * RS + r]);
+      x *= dm[i];
+      if constexpr (!DELTA) x *= wr;
+      if (t < cn) p.P[((t0 + 8 * (i >> 2) + (i & 3)) * p.H + h) * kCh + p_off] = x;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (DELTA) {
+      constexpr int AS = kCh + kPad;
+      float* am = amat[w];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int t = acc_row(i, half);
+        const float x = prod[0][t * RS + r] + prod[1][t * RS + r];
+        // lanes hold beta of token r: the row's own beta is another lane's
+        am[t * AS + r] = r < t ? x * dm[i] : 0.0f;
+      }
+      __builtin_amdgcn_wave_barrier();
+      // column r of (I + diag(beta) A)^-1 by forward substitution, times beta_r (the row of diag(beta) on the right)
+      float x[kCh];
+#pragma unroll
+      for (int t = 0; t < kCh; ++t) {
+        float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < t; i += 4) {
+          const float4 av = *reinterpret_cast<const float4*>(am + t * AS + i);
+          s[0] += av.x * x[i];
+          if (i + 1 < t) s[1] += av.y * x[i + 1];
+          if (i + 2 < t) s[2] += av.z * x[i + 2];
+          if (i + 3 < t) s[3] += av.w * x[i + 3];
+        }
+        x[t] = (r == t ? 1.0f : 0.0f) - chunk_lane(wr, t) * ((s[0] + s[1]) + (s[2] + s[3]));
+        asm volatile("" : "+v"(x[t]) : : "memory");    // a row's reads at a time: hoisted ones spill
+      }
+#pragma unroll
+      for (int t = 0; t < kCh; ++t)
+        if (t < cn && (t & 1) == half) p.Tm[((t0 + t) * p.H + h) * kCh + r] = x[t] * wr;
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+}
+
+// MODE 0: the whole sequence; 1: what a segment adds to the state, and its decay; 2: a segment from its starting state.
+// grid: (heads / HPW * column parts, segments, sequences), NW waves on 16 columns of the state each: the columns of one head,
+// or of HPW heads of one group (they share q and k). Sixteen columns and not 32: a compute unit that gets one workgroup then
+// holds two waves a SIMD, and one's LDS reads, staging and row factors run beside the other's products.
+template <typename T, int KIND, int DT, int NW, int HPW, int MODE>
+__global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
+  constexpr bool DELTA = KIND == kChunkDelta, SILU = KIND == kChunkConst, FULL = MODE != 1;
+  constexpr int D = DT * 16, RS = D + kPad, PS = kCh + kPad, NT = NW * 64, WPW = NW / HPW;
+  constexpr int MATS = FULL ? HPW * (DELTA ? 2 : 1) : 0;       // P of every head, then T of every head
+  __shared__ __attribute__((aligned(16))) float k_all[2][kCh * RS];
+  __shared__ __attribute__((aligned(16))) float q_all[2][FULL ? kCh * RS : 4];
+  __shared__ __attribute__((aligned(16))) float pt_all[2][MATS > 0 ? MATS : 1][MATS > 0 ? kCh * PS : 4];
+  __shared__ __attribute__((aligned(16))) float ge_all[2][HPW][2 * kCh];      // G, then E
+  const int b = blockIdx.z;
+  const int q0 = p.cu_q[b], n_all = p.cu_q[b + 1] - q0;
+  const int s0 = MODE == 0 ? 0 : blockIdx.y * p.seg_len;
+  const int s1 = MODE == 0 ? n_all : min(n_all, s0 + p.seg_len);
+  if (s0 >= n_all || (MODE == 1 && s1 == n_all)) return;       // what the last segment adds is nobody's start
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, quad = lane >> 4;
+  const int parts = p.Dv / 16 / WPW;                           // 1 where several heads share the workgroup
+  const int h0 = static_cast<int>(blockIdx.x) / parts * HPW, hw = w / WPW, h = h0 + hw;         // (uniform over a wave)
+  const int col = ((static_cast<int>(blockIdx.x) % parts) * WPW + w % WPW) * 16 + r;
+  const int g = h0 / (p.H / p.G);
+  const T* kp = static_cast<const T*>(p.k) + static_cast<int64_t>(q0) * p.ldk + static_cast<int64_t>(g) * D;
+  const T* qp = static_cast<const T*>(p.q) + static_cast<int64_t>(q0) * p.ldq + static_cast<int64_t>(g) * D;
+  const T* vp = static_cast<const T*>(p.v) + static_cast<int64_t>(q0) * p.ldv + static_cast<int64_t>(h) * p.Dv;
+  const int64_t row0 = static_cast<int64_t>(q0) * p.H;
+  float* sbase = p.state + (static_cast<int64_t>(p.slots[b]) * p.H + h) * D * p.Dv;
+  float* gbase = MODE == 0 ? nullptr : p.seg_state + ((static_cast<int64_t>(b) * p.segs + blockIdx.y) * p.H + h) * D * p.Dv;
+
+  // addresses are a uniform row plus a lane's 32-bit offset inside it
+  const uint32_t st_off = static_cast<uint32_t>(4 * quad * p.Dv) + col;
+  f32x4 S[DT];
+  {
+    const bool carry = MODE == 2 ? p.segs > 0 : MODE == 0 && p.ctx_lens[b] > 0;
+    const float* from = MODE == 2 ? gbase : sbase;
+#pragma unroll
+    for (int j = 0; j < DT; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[j][i] = carry ? from[(16 * j + i) * p.Dv + st_off] : 0.0f;
+  }
+  float skip = 0.0f;
+  if (KIND == kChunkStep && FULL) skip = p.p2[h];
+  float seg_dec = 1.0f;
+
+  // the next chunk's rows on their way: q and k four entries a thread, P and T too, a value for each of the wave's 32 x 16
+  constexpr int KQ = kCh * D / 4 / NT, PN = (MATS * kCh * kCh / 4 + NT - 1) / NT, PX = PN > 0 ? PN : 1;
+  static_assert(kCh * D / 4 % NT == 0, "whole rows of q and k a step");
+  float4 kreg[KQ], qreg[FULL ? KQ : 1], preg[PX];
+  float vreg[8], gereg;
+  const uint32_t kq_off = static_cast<uint32_t>(threadIdx.x % (D / 4) * 4);
+  const int kq_tok = threadIdx.x / (D / 4);
+  const uint32_t k_off = kq_tok * static_cast<uint32_t>(p.ldk) + kq_off, q_off = kq_tok * static_cast<uint32_t>(p.ldq) + kq_off;
+  const uint32_t v_off = 4 * quad * static_cast<uint32_t>(p.ldv) + col;
+  const uint32_t o_off = static_cast<uint32_t>(4 * quad * p.H * p.Dv) + col;
+  const uint32_t ge_off = static_cast<uint32_t>((lane & 31) * p.H + hw);
+  const int p_tok = (threadIdx.x >> 3) & 31;
+  const uint32_t p_off = static_cast<uint32_t>(p_tok * p.H * kCh + (threadIdx.x & 7) * 4);
+  auto fetch_rows = [&](int c0, auto whole) __attribute__((always_inline)) {
+    constexpr bool WHOLE = decltype(whole)::value;     // all 32 tokens are there: loads without conditions
+    const int cn = s1 - c0;
+#pragma unroll
+    for (int it = 0; it < KQ; ++it) {
+      constexpr int per = NT / (D / 4);
+      const bool in = WHOLE || kq_tok + it * per < cn;
+      kreg[it] = in ? ld4(kp + static_cast<int64_t>(c0 + it * per) * p.ldk + k_off) : float4{0, 0, 0, 0};
+      if constexpr (FULL) qreg[it] = in ? ld4(qp + static_cast<int64_t>(c0 + it * per) * p.ldq + q_off) : float4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int it = 0; it < PN; ++it) {
+      const int m = (it * NT + (w << 6)) >> 8;         // matrix of this wave's pieces
+      const bool in = m < MATS && (WHOLE || p_tok < cn);
+      const float* from = DELTA && m >= HPW ? p.Tm : p.P;
+      const int64_t at = (row0 + static_cast<int64_t>(c0) * p.H + h0 + (DELTA && m >= HPW ? m - HPW : m)) * kCh;
+      preg[it] = in ? ld4(from + at + p_off) : float4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int lo = 16 * (i >> 2) + (i & 3);
+      vreg[i] = WHOLE || lo + 4 * quad < cn ? ldf(vp + static_cast<int64_t>(c0 + lo) * p.ldv + v_off) : 0.0f;
+    }
+    const bool in = WHOLE || (lane & 31) < cn;         // lane = token, G in the lower half of the lanes, E in the upper
+    const int64_t at = row0 + static_cast<int64_t>(c0) * p.H + h0;
+    gereg = in ? (lane >= 32 ? p.Ef : p.Gf)[at + ge_off] : 0.0f;
+  };
+  auto fetch = [&](int c0) __attribute__((always_inline)) {
+    if (s1 - c0 >= kCh) fetch_rows(c0, std::true_type{});
+    else fetch_rows(c0, std::false_type{});
+  };
+  // rows 16 x + 4 quad .. + 3 of a vector, a row of a left-hand matrix from column 16 j on
+  auto rows4 = [&](const float* from, int x) __attribute__((always_inline)) {
+    return *reinterpret_cast<const float4*>(from + 16 * x + 4 * quad);
+  };
+  auto left = [&](const float* m, int stride, int x, int j) __attribute__((always_inline)) {
+    return *reinterpret_cast<const float4*>(m + (16 * x + r) * stride + 16 * j + 4 * quad);
+  };
+  auto mul4 = [&](f32x4 acc, float4 a, f32x4 bb) __attribute__((always_inline)) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, bb[0], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, bb[1], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, bb[2], acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, bb[3], acc, 0, 0, 0);
+  };
+  auto scale4 = [&](f32x4 x, float4 f) __attribute__((always_inline)) { return f32x4{x[0] * f.x, x[1] * f.y, x[2] * f.z, x[3] * f.w}; };
+  const f32x4 zero{0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 U_next[2];
+  auto stage = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int it = 0; it < KQ; ++it) {
+      const int at = (kq_tok + it * (NT / (D / 4))) * RS + kq_off;
+      st4(k_all[buf] + at, chunk_act<SILU>(kreg[it]));
+      if constexpr (FULL) st4(q_all[buf] + at, chunk_act<SILU>(qreg[it]));
+    }
+#pragma unroll
+    for (int it = 0; it < PN; ++it) {
+      const int m = (it * NT + (w << 6)) >> 8;
+      if (m < MATS) st4(pt_all[buf][m] + p_tok * PS + (threadIdx.x & 7) * 4, preg[it]);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) U_next[i >> 2][i & 3] = SILU ? chunk_silu(vreg[i]) : vreg[i];
+    if (w % WPW == 0) ge_all[buf][hw][lane] = gereg;
+  };
+  // Two buffers: a chunk is staged while the one before it is computed, each wave at its own time, and two chunks ahead are on
+  // their way in registers. One barrier a chunk.
+  fetch(s0);
+  stage(0);
+  if (s0 + kCh < s1) fetch(s0 + kCh);
+  __syncthreads();
+  int buf = 0;
+  for (int c0 = s0; c0 < s1; c0 += kCh, buf ^= 1) {
+    const int cn = min(kCh, s1 - c0);
+    const float *k_lds = k_all[buf], *q_lds = q_all[buf];
+    const auto& pt_lds = pt_all[buf];
+    const auto& ge_lds = ge_all[buf];
+    f32x4 U[2] = {U_next[0], U_next[1]};
+    f32x4 o[2], u2[2];
+    if constexpr (FULL) {
+      f32x4 ks[2][2], qs[4][2];                        // [sum][rows]: several sums each, shorter and with fewer roundings
+#pragma unroll
+      for (int x = 0; x < 2; ++x) qs[0][x] = qs[1][x] = qs[2][x] = qs[3][x] = ks[0][x] = ks[1][x] = zero;
+#pragma unroll
+      for (int j = 0; j < DT; ++j) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          if constexpr (DELTA) ks[j & 1][x] = mul4(ks[j & 1][x], left(k_lds, RS, x, j), S[j]);
+          qs[j & 3][x] = mul4(qs[j & 3][x], left(q_lds, RS, x, j), S[j]);
+        }
+      }
+      if constexpr (DELTA) {
+        f32x4 rest[2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) rest[x] = U[x] - scale4(ks[0][x] + ks[1][x], rows4(ge_lds[hw], x));
+        U[0] = mul4(zero, left(pt_lds[HPW + hw], PS, 0, 0), rest[0]);               // T is lower triangular
+        U[1] = mul4(mul4(zero, left(pt_lds[HPW + hw], PS, 1, 0), rest[0]), left(pt_lds[HPW + hw], PS, 1, 1), rest[1]);
+      }
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        o[x] = scale4((qs[0][x] + qs[1][x]) + (qs[2][x] + qs[3][x]), rows4(ge_lds[hw], x));
+        if constexpr (KIND == kChunkStep) o[x] += skip * U[x];
+      }
+      o[0] += mul4(zero, left(pt_lds[hw], PS, 0, 0), U[0]);
+      o[1] += mul4(mul4(zero, left(pt_lds[hw], PS, 1, 0), U[0]), left(pt_lds[hw], PS, 1, 1), U[1]);
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x) u2[x] = scale4(U[x], rows4(ge_lds[hw] + kCh, x));
+    const float g_last = ge_lds[hw][cn - 1];
+    if (c0 + kCh < s1) {
+      stage(buf ^ 1);
+      if (c0 + 2 * kCh < s1) fetch(c0 + 2 * kCh);
+    }
+#pragma unroll
+    for (int j = 0; j < DT; ++j) {
+      S[j] *= g_last;
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(k_lds[(16 * (i >> 2) + 4 * quad + (i & 3)) * RS + 16 * j + r], u2[i >> 2][i & 3], S[j], 0, 0, 0);
+    }
+    if constexpr (FULL) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int lo = 16 * (i >> 2) + (i & 3);
+        if (lo + 4 * quad < cn) p.o[(row0 + static_cast<int64_t>(c0 + lo) * p.H + h) * p.Dv + o_off] = o[i >> 2][i & 3];
+      }
+    }
+    seg_dec *= g_last;
+    __syncthreads();                                   // the next chunk is complete, and nobody reads this one any more
+  }
+  if (MODE == 1 || s1 == n_all) {
+    float* to = MODE == 1 ? gbase : sbase;
+#pragma unroll
+    for (int j = 0; j < DT; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) to[(16 * j + i) * p.Dv + st_off] = S[j][i];
+  }
+  if (MODE == 1 && lane == 0) p.seg_decay[(static_cast<int64_t>(b) * p.segs + blockIdx.y) * p.H + h] = seg_dec;
+}
+
+// seg_state: what each segment adds -> the state that each segment starts from. A thread owns four entries of a head's state.
+__global__ __launch_bounds__(256) void chunk_combine_kernel(ChunkParams p) {
+  const int b = blockIdx.z, h = blockIdx.y;
+  const int n = p.cu_q[b + 1] - p.cu_q[b];
+  const int segs = (n + p.seg_len - 1) / p.seg_len;
+  const int64_t size = static_cast<int64_t>(p.D) * p.Dv;
+  const int64_t x = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 4;
+  if (x >= size) return;
+  float4 s{0, 0, 0, 0};
+  if (p.ctx_lens[b] > 0) s = ld4(p.state + (static_cast<int64_t>(p.slots[b]) * p.H + h) * size + x);
+  for (int i = 0; i < segs; ++i) {
+    float* at = p.seg_state + ((static_cast<int64_t>(b) * p.segs + i) * p.H + h) * size + x;
+    const bool last = i + 1 == segs;
+    const float4 add = last ? float4{0, 0, 0, 0} : ld4(at);
+    const float d = last ? 0.0f : p.seg_decay[(static_cast<int64_t>(b) * p.segs + i) * p.H + h];
+    st4(at, s);
+    s = float4{d * s.x + add.x, d * s.y + add.y, d * s.z + add.z, d * s.w + add.w};
+  }
+}
+
+template <typename T, int KIND, int DT, int NW, int HPW>
+static void chunk_launch(const ChunkParams& p, int B, hipStream_t s) {
+  dim3 grid(p.H / HPW * (p.Dv / 16 / (NW / HPW)), 1, B), block(NW * 64);
+  if (p.segs <= 1) {
+    chunk_scan_kernel<T, KIND, DT, NW, HPW, 0><<<grid, block, 0, s>>>(p);
+    return;
+  }
+  if constexpr (KIND != kChunkDelta) {
+    grid.y = p.segs;
+    chunk_scan_kernel<T, KIND, DT, NW, HPW, 1><<<grid, block, 0, s>>>(p);
+    chunk_combine_kernel<<<dim3((p.D * p.Dv / 4 + 255) / 256, p.H, B), dim3(256), 0, s>>>(p);
+    chunk_scan_kernel<T, KIND, DT, NW, HPW, 2><<<grid, block, 0, s>>>(p);
+  }
+}
+
+template <typename T, int KIND, int DT>
+static void chunk_waves(const ChunkParams& p, int B, hipStream_t s) {
+  if (p.Dv % 128 == 0) chunk_launch<T, KIND, DT, 8, 1>(p, B, s);
+  else if (p.H / p.G % 2 == 0) chunk_launch<T, KIND, DT, 8, 2>(p, B, s);     // Dv == 64: two heads of a group
+  else chunk_launch<T, KIND, DT, 4, 1>(p, B, s);
+}
+
+template <typename T, int KIND>
+static void chunk_dispatch(const ChunkParams& p, int B, int max_new, hipStream_t s) {
+  chunk_prep_kernel<T, KIND><<<dim3((max_new + kCh - 1) / kCh, p.G, B), dim3(256), 0, s>>>(p);
+  if (p.D == 64) chunk_waves<T, KIND, 4>(p, B, s);
+  else chunk_waves<T, KIND, 8>(p, B, s);
+}
+
+static int chunk_segments(int kind, int max_new, int seg_len) {
+  return kind == kChunkDelta || seg_len <= 0 || max_new <= seg_len ? 1 : (max_new + seg_len - 1) / seg_len;
+}
+
+static bool chunk_sizes_ok(int H, int G, int D, int Dv) {
+  return H > 0 && G > 0 && H % G == 0 && (D == 64 || D == 128) && (Dv == 64 || (Dv > 0 && Dv % 128 == 0));
+}
+
+}  // namespace lvmix
+
+using namespace lvmix;
+
+extern "C" {
+
+int64_t lv_chunk_scan_workspace_bytes(int kind, int64_t T, int B, int max_new, int H, int D, int Dv, int seg_len) {
+  if (T < 0 || B < 0 || H <= 0 || D <= 0 || Dv <= 0 || max_new < 0) return fail(-1, "lv_chunk_scan_workspace_bytes: bad sizes");
+  const int64_t rows = T * H;
+  int64_t floats = rows * kCh * (kind == kChunkDelta ? 2 : 1) + 2 * ((rows + 3) / 4 * 4);
+  const int segs = chunk_segments(kind, max_new, seg_len);
+  if (segs > 1) floats += static_cast<int64_t>(B) * segs * H * (static_cast<int64_t>(D) * Dv + 1);
+  return floats * static_cast<int64_t>(sizeof(float));
+}
+
+int lv_chunk_scan(int kind, const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, const void* a,
+                  int64_t lda, const void* decay, const void* p0, const void* p1, const void* p2, void* state,
+                  const int32_t* cu_q, const int32_t* ctx_lens, const int32_t* slots, void* o, void* workspace,
+                  int64_t workspace_bytes, int64_t T, int B, int max_new, int H, int G, int D, int Dv, int seg_len,
+                  void* stream) {
+  if (B == 0 || T == 0) return 0;
+  if (!q || !k || !v || !state || !cu_q || !ctx_lens || !slots || !o || !workspace) return fail(-1, "lv_chunk_scan: null pointer");
+  if (kind != kChunkStep && kind != kChunkConst && kind != kChunkDelta) return fail(-1, "lv_chunk_scan: kind %d", kind);
+  if (kind == kChunkStep && (!a || !p0 || !p1 || !p2)) return fail(-1, "lv_chunk_scan: step sizes without their parameters");
+  if (kind != kChunkStep && (!decay || (kind == kChunkDelta && !a))) return fail(-1, "lv_chunk_scan: no decays");
+  if (B < 0 || T < 0 || max_new <= 0 || max_new > T || seg_len < 0 || seg_len % kCh != 0 || !chunk_sizes_ok(H, G, D, Dv))
+    return fail(-1, "lv_chunk_scan: bad sizes");
+  const uintptr_t piece = kind == kChunkDelta ? 16 : 8;      // four entries of a row: f32 for the delta rule, bf16 otherwise
+  if (ldq < static_cast<int64_t>(G) * D || ldk < static_cast<int64_t>(G) * D || ldv < static_cast<int64_t>(H) * Dv || ldq % 4 != 0 ||
+      ldk % 4 != 0 || reinterpret_cast<uintptr_t>(q) % piece != 0 || reinterpret_cast<uintptr_t>(k) % piece != 0 ||
+      reinterpret_cast<uintptr_t>(state) % 16 != 0 || reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
+    return fail(-1, "lv_chunk_scan: strides or alignment");
+  if (workspace_bytes < lv_chunk_scan_workspace_bytes(kind, T, B, max_new, H, D, Dv, seg_len))
+    return fail(-3, "lv_chunk_scan: workspace of %lld bytes", static_cast<long long>(workspace_bytes));
+  const int64_t rows = T * H, rows4 = (rows + 3) / 4 * 4;
+  float* ws = static_cast<float*>(workspace);
+  ChunkParams p{q, k, v, ldq, ldk, ldv, a, lda, static_cast<const float*>(decay), static_cast<const float*>(p0),
+                static_cast<const float*>(p1), static_cast<const float*>(p2), static_cast<float*>(state), cu_q, ctx_lens, slots,
+                static_cast<float*>(o), nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, H, G, D, Dv, seg_len,
+                chunk_segments(kind, max_new, seg_len)};
+  p.P = ws;
+  ws += rows * kCh;
+  if (kind == kChunkDelta) {
+    p.Tm = ws;
+    ws += rows * kCh;
+  }
+  p.Gf = ws;
+  p.Ef = ws + rows4;
+  ws += 2 * rows4;
+  if (p.segs > 1) {
+    p.seg_state = ws;
+    p.seg_decay = ws + static_cast<int64_t>(B) * p.segs * H * D * Dv;
+  }
+  hipStream_t s = as_stream(stream);
+  if (kind == kChunkDelta) chunk_dispatch<float, kChunkDelta>(p, B, max_new, s);
+  else if (kind == kChunkStep) chunk_dispatch<bf16_t, kChunkStep>(p, B, max_new, s);
+  else chunk_dispatch<bf16_t, kChunkConst>(p, B, max_new, s);
+  return launched("lv_chunk_scan");
+}
+
+}  // extern "C"

@@ -25,6 +25,16 @@ WINDOW_ATTN_KERNEL = "auto"
 SPLIT_WORKGROUPS = 256     # decode-shaped attention: key tiles are cut until a launch has about this many workgroups
 
 
+# recurrences with one decay per head: "auto" takes the chunked kernel for steps that bring a long portion, "token" the token loop
+SCAN_KERNEL = "auto"
+CHUNK_STEP, CHUNK_CONST, CHUNK_DELTA = 0, 1, 2
+# New tokens of a sequence from which a step takes the chunked kernel: where its two launches meet the token loop's time. Token
+# loop / chunks in us, 1 sequence and 32: delta rule (16 heads of 128) 28.6 / 24.4 and 69 / 44 at 32 tokens, 17.5 / 25.2 at 16;
+# constant decays (16 heads) 24.6 / 24.0 and 76 / 52 at 64 tokens of 128 x 128, but 15.7 / 20.2 of 64 x 64, which are level at 90;
+# step sizes (32 heads, 128 x 64) 24.7 / 22.4 and 57 / 47 at 64.
+CHUNK_FROM = {CHUNK_STEP: 80, CHUNK_CONST: 80, CHUNK_DELTA: 32}
+
+
 def _stream(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
@@ -191,6 +201,48 @@ def clamped_glu(x, limit: float, alpha: float):
     return out
 
 
+# ------------------------------------------------------------------------------- recurrences in chunks
+def _chunk_ok(kind, step, D, Dv, *rows) -> bool:
+    """Whether lv_chunk_scan takes this step: sizes and alignment it knows and a sequence with CHUNK_FROM[kind] new tokens or more.
+    rows: the query and key rows (four entries at a time)."""
+    return (SCAN_KERNEL == "auto" and not step.static and D in (64, 128) and (Dv == 64 or Dv % 128 == 0)
+            and all(x.stride(0) % 4 == 0 and x.data_ptr() % (4 * x.element_size()) == 0 for x in rows)
+            and max(step.host_lens_q) >= CHUNK_FROM[kind])
+
+
+def _segment_length(lens, wgs, state_bytes) -> int:
+    """Tokens of the segments that sequences are cut into, 0: none. A workgroup (one of `wgs` a sequence or segment) fills a
+    compute unit, so a launch takes rounds of 256 of them, as long as their segment; segments cost 1.45 times the products (their
+    contributions are formed first). 7 prompts of 900 to 3750 tokens, 32 heads of 128 x 64: 741 us whole, 445 / 463 / 615 us
+    in segments of 256 / 512 / 1024; one of 4096: 713, 119 / 173 / 303 us; 8 of 2048, 16 heads of 128 x 128: 471 us whole, 440 / 404 /
+    409 us. Segments whose states would take more than 256 MB are not considered."""
+    longest = max(lens)
+    whole = len(lens) * wgs
+    best, cost = 0, longest if whole <= 256 else max(longest, sum(lens) * wgs // 256 + longest // 2)
+    for seg in (2048, 1024, 512, 256):
+        if seg >= longest or len(lens) * -(-longest // seg) * state_bytes > 1 << 28:
+            continue
+        c = 1.45 * seg * -(-sum(-(-n // seg) for n in lens) * wgs // 256)
+        if c < cost:
+            best, cost = seg, c
+    return best
+
+
+def _chunk_scan(kind, q, k, v, a, decay, p0, p1, p2, state, step, H, G, D, Dv):
+    """o f32 [T, H, Dv] of lv_chunk_scan; q, k, v 2-d rows."""
+    T, B, longest = q.size(0), len(step.host_lens_q), max(step.host_lens_q)
+    seg = _segment_length(step.host_lens_q, max(1, H * Dv // 128), H * D * Dv * 4) if kind != CHUNK_DELTA else 0
+    lib = _mixlib.load()
+    nbytes = lib.lv_chunk_scan_workspace_bytes(kind, T, B, longest, H, D, Dv, seg)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+    o = torch.empty(T, H, Dv, dtype=torch.float32, device=q.device)
+    _mixlib.check(lib.lv_chunk_scan(kind, _p(q), q.stride(0), _p(k), k.stride(0), _p(v), v.stride(0), _p(a),
+                                    a.stride(0) if a is not None else 0, _p(decay), _p(p0), _p(p1), _p(p2), _p(state), _p(step.cu_q),
+                                    _p(step.ctx_lens), _p(step.slots), _p(o), _p(ws), nbytes, T, B, longest, H, G, D, Dv, seg,
+                                    _stream(q)), "lv_chunk_scan")
+    return o
+
+
 # ------------------------------------------------------------------------------------- delta rule
 def delta_prep(proj, conv_w, conv_state, A_log, dt_bias, step, G, H, D, Dv, taps, off_b, a, unit_eps,
                decay_per_channel=False):
@@ -279,6 +331,9 @@ def gated_delta_rule(qn, kn, v, beta, decay, state, step):
     assert state.shape[1:] == (H, D, Dv)
     per_channel = decay.dim() == 3
     assert decay.shape == ((T, H, D) if per_channel else (T, H))
+    if qn.is_cuda and not per_channel and T > 0 and _chunk_ok(CHUNK_DELTA, step, D, Dv, qn, kn):
+        return _chunk_scan(CHUNK_DELTA, qn.view(T, G * D), kn.view(T, G * D), v.view(T, H * Dv), beta, decay, None, None, None, state,
+                           step, H, G, D, Dv)
     o = torch.empty(T, H, Dv, dtype=torch.float32, device=qn.device)
     if qn.is_cuda:
         lib = _mixlib.load()
@@ -1123,6 +1178,11 @@ def lightning_attention(proj, off_q, off_k, off_v, decay, state, step, H, D, Dv)
     T = proj.size(0)
     _f32(decay, state)
     assert state.shape[1:] == (H, D, Dv) and decay.numel() == H
+    if proj.is_cuda and T > 0 and proj.dtype == torch.bfloat16:
+        assert proj.stride(1) == 1
+        q, k, v = (proj[:, at:at + H * n] for at, n in ((off_q, D), (off_k, D), (off_v, Dv)))
+        if _chunk_ok(CHUNK_CONST, step, D, Dv, q, k):
+            return _chunk_scan(CHUNK_CONST, q, k, v, None, decay, None, None, None, state, step, H, H, D, Dv)
     o = torch.empty(T, H, Dv, dtype=torch.float32, device=proj.device)
     if proj.is_cuda:
         assert proj.stride(1) == 1
@@ -1278,6 +1338,9 @@ def gated_scan(kind, q, k, v, a, p0, p1, step, state, H, G, D, Dv, a2=None, p2=N
     _f32(state, p0, p1, p2, norm_state, max_state)
     assert state.shape[1:] == (H, D, Dv) and q.size(1) == G * D and k.size(1) == G * D and v.size(1) == H * Dv
     assert a.size(1) == (H * D if kind == SCAN_ROW_DECAY else H) and a.dtype == q.dtype == k.dtype == v.dtype
+    if (kind == SCAN_STEP and q.is_cuda and T > 0 and q.dtype == torch.bfloat16 and q_scale == 1.0
+            and all(x.stride(1) == 1 for x in (q, k, v, a)) and _chunk_ok(CHUNK_STEP, step, D, Dv, q, k)):
+        return _chunk_scan(CHUNK_STEP, q, k, v, a, None, p0, p1, p2, state, step, H, G, D, Dv)
     o = torch.empty(T, H, Dv, dtype=torch.float32, device=q.device)
     den = None
     if kind == SCAN_LOG_GATES:

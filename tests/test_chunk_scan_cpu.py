@@ -1,0 +1,26 @@
+"""lv_chunk_scan rejects bad arguments on the host, before any launch."""
+import ctypes
+
+
+def test_argument_validation():
+    from light_vllm_amd import _mixlib
+    lib = _mixlib.load()
+    buf = ctypes.create_string_buffer(256)
+    p = (ctypes.addressof(buf) + 15) & ~15
+
+    def call(kind=1, q=p, ldq=256, ldk=256, ldv=256, a=p, decay=p, p0=p, ws=p, nbytes=1 << 40, T=64, B=1, longest=64, H=2, G=2, D=64, Dv=64,
+             seg=0):
+        return lib.lv_chunk_scan(kind, q, ldq, p, ldk, p, ldv, a, 2, decay, p0, p, p, p, p, p, p, p, ws, nbytes, T, B, longest, H, G, D, Dv,
+                                 seg, None)
+
+    assert call(B=0) == 0 and call(T=0) == 0                        # nothing to do
+    for bad in (dict(q=None), dict(ws=None), dict(kind=3), dict(kind=0, p0=None), dict(decay=None), dict(kind=2, a=None), dict(D=96),
+                dict(Dv=96), dict(H=3), dict(ldq=100), dict(ldk=130), dict(q=p + 4), dict(kind=2, q=p + 8), dict(ws=p + 4), dict(seg=48),
+                dict(longest=65), dict(longest=0)):
+        assert call(**bad) == -1, bad
+    assert call(nbytes=64) == -3
+    need = lib.lv_chunk_scan_workspace_bytes
+    assert need(1, 64, 1, 64, 2, 64, 64, 0) >= 64 * 2 * 34 * 4
+    assert need(2, 64, 1, 64, 2, 64, 64, 32) >= 64 * 2 * 66 * 4      # the delta rule is never cut
+    assert need(1, 64, 1, 64, 2, 64, 64, 32) > need(1, 64, 1, 64, 2, 64, 64, 64)
+    assert need(1, -1, 1, 64, 2, 64, 64, 0) < 0

@@ -1,0 +1,145 @@
+"""The chunked recurrences (lv_chunk_scan) against the recurrence in float64, at the edges of their chunks and segments, and the
+rule that takes a step to them against the token loop."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from light_vllm_amd import mix_ops
+from light_vllm_amd.utils.context import RaggedStep
+
+pytestmark = pytest.mark.gpu
+F64 = torch.float64
+# f32 products and sums: a read-out is a sum over at most 128 rows of the state and 32 tokens of the chunk, each addition off
+# by half a unit in the last place at most, and the state carries the errors of as many additions
+REL = (128 + 2 * 32) * 2.0 ** -24
+
+
+def make_step(new, ctx, static=False):
+    cu, tok = [0], []
+    for b, n in enumerate(new):
+        cu.append(cu[-1] + n)
+        tok += [b] * n
+    i32 = dict(dtype=torch.int32, device="cuda")
+    B = len(new)
+    slots = list(reversed(range(B)))
+    return RaggedStep(torch.tensor(cu, **i32), torch.tensor(ctx, **i32), torch.tensor(slots, **i32), torch.tensor(tok, **i32),
+                      torch.zeros(B, 1, **i32), new, ctx, slots, [[0]] * B, static=static)
+
+
+def recurrence(q, k, v, g, beta, state, step):
+    """q, k [T, H, D], v [T, H, Dv], g [T, H] in float64; beta [T, H]: delta rule. -> (o, state)."""
+    S_all, o = state.to(F64).clone(), torch.empty_like(v)
+    at = 0
+    for b, n in enumerate(step.host_lens_q):
+        slot = step.host_slots[b]
+        S = S_all[slot] if step.host_ctx_lens[b] > 0 else torch.zeros_like(S_all[slot])
+        for t in range(at, at + n):
+            S = S * g[t][:, None, None]
+            u = v[t] if beta is None else beta[t][:, None] * (v[t] - torch.einsum("hdv,hd->hv", S, k[t]))
+            S = S + k[t][:, :, None] * u[:, None, :]
+            o[t] = torch.einsum("hdv,hd->hv", S, q[t])
+        if n > 0:
+            S_all[slot] = S
+        at += n
+    return o, S_all
+
+
+def case(kind, new, H, G, D, Dv, seed, pad=4, zeros=False):
+    """(call(state, step), float64 arguments of recurrence, skip) on seeded inputs; rows are views of a wider tensor."""
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    T, rep = sum(new), H // G
+
+    def rn(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen)
+
+    def heads(x):
+        return x.to(F64).view(T, G, D).repeat_interleave(rep, 1)
+
+    if kind == "delta":
+        q, k, v = F.normalize(rn(T, G, D), dim=-1) * D ** -0.5, F.normalize(rn(T, G, D), dim=-1), rn(T, H, Dv)
+        beta, g = torch.sigmoid(rn(T, H)), torch.exp(-torch.exp(0.5 * rn(H)) * F.softplus(rn(T, H)))
+        if zeros:
+            g[::5] = 0.0
+        return (lambda st, step: mix_ops.gated_delta_rule(q, k, v, beta, g, st, step),
+                (heads(q), heads(k), v.to(F64), g.to(F64), beta.to(F64)), 0.0)
+    if kind == "step":
+        u = (0.6 * rn(T, 2 * G * D + H * Dv + pad)).bfloat16()[:, pad:]
+        a, p0, p1, p2 = rn(T, H).bfloat16(), 0.5 * rn(H), 0.5 * rn(H), rn(H)
+        q, k, v = u[:, :G * D], u[:, G * D:2 * G * D], u[:, 2 * G * D:]
+        dt = F.softplus(a.to(F64) + p0.to(F64))
+        v64 = v.to(F64).view(T, H, Dv)
+        return (lambda st, step: mix_ops.gated_scan(mix_ops.SCAN_STEP, q, k, v, a, p0, p1, step, st, H, G, D, Dv, p2=p2),
+                (heads(q), heads(k) * dt[..., None], v64, torch.exp(-torch.exp(p1.to(F64)) * dt), None), p2.to(F64)[:, None] * v64)
+    proj = rn(T, 2 * H * D + H * Dv + pad).bfloat16()
+    decay = torch.tensor([0.0 if zeros and h == 0 else 1.0 - 2.0 ** (-5.0 - 5.0 * h / H) for h in range(H)], device="cuda")
+    x = F.silu(proj[:, pad:].to(F64))
+    return (lambda st, step: mix_ops.lightning_attention(proj, pad, pad + H * D, pad + 2 * H * D, decay, st, step, H, D, Dv),
+            (x[:, :H * D].view(T, H, D), x[:, H * D:2 * H * D].view(T, H, D), x[:, 2 * H * D:].reshape(T, H, Dv),
+             decay.to(F64).expand(T, H), None), 0.0)
+
+
+def rel(x, y):
+    return ((x.to(F64) - y).norm() / y.norm()).item()
+
+
+@pytest.mark.parametrize("kind,H,G,D,Dv", [("delta", 4, 2, 64, 64), ("delta", 3, 1, 128, 64), ("delta", 4, 1, 128, 128), ("delta", 2, 2, 64, 256),
+                                           ("step", 6, 3, 128, 64), ("step", 3, 3, 64, 64), ("step", 2, 1, 64, 128),
+                                           ("const", 2, 2, 64, 64), ("const", 3, 3, 128, 128), ("const", 2, 2, 64, 256)])
+@pytest.mark.parametrize("new,ctx", [([96], [0]), ([97, 1, 31, 32, 33], [0, 7, 0, 1, 0]), ([128, 0, 64, 65], [3, 0, 0, 2])])
+def test_chunks_match_the_recurrence(kind, H, G, D, Dv, new, ctx):
+    call, args, skip = case(kind, new, H, G, D, Dv, seed=D + Dv + len(new))
+    step = make_step(new, ctx)
+    state = 0.3 * torch.randn(len(new), H, D, Dv, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    want_o, want_s = recurrence(*args, state, step)
+    o = call(state, step)
+    assert rel(o, want_o + skip) < REL and rel(state, want_s) < REL
+
+
+@pytest.mark.parametrize("kind", ["step", "const"])
+@pytest.mark.parametrize("new", [[1024], [1500, 40, 1057]])
+def test_segments_match_the_recurrence(kind, new):
+    """Long portions on few sequences are cut into segments."""
+    H, D, Dv = 2, 64, 64
+    call, args, skip = case(kind, new, H, H, D, Dv, seed=sum(new))
+    step = make_step(new, [5] * len(new))
+    state = 0.3 * torch.randn(len(new), H, D, Dv, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    want_o, want_s = recurrence(*args, state, step)
+    o = call(state, step)
+    # decays of 1 - 2^-7.5: the state of `const` sums about 200 tokens, whose additions add their errors
+    assert rel(o, want_o + skip) < 2 * REL and rel(state, want_s) < 2 * REL
+
+
+@pytest.mark.parametrize("kind", ["delta", "const"])
+def test_decays_of_zero(kind):
+    new = [85, 40]
+    call, args, _ = case(kind, new, 2, 2, 64, 64, seed=5, zeros=True)
+    step = make_step(new, [0, 3])
+    state = torch.randn(2, 2, 64, 64, device="cuda")
+    want_o, want_s = recurrence(*args, state, step)
+    o = call(state, step)
+    assert rel(o, want_o) < REL and rel(state, want_s) < REL
+
+
+@pytest.mark.parametrize("kind", ["step", "const"])
+@pytest.mark.parametrize("pad", [1, 2, 3])
+def test_misaligned_rows_and_captured_steps_take_the_token_loop(kind, pad, monkeypatch):
+    """Rows that do not lie on four entries, and steps that are captured, run where they ran before."""
+    new = [96, 5]
+    state = torch.randn(2, 2, 64, 64, device="cuda")
+    monkeypatch.setattr(mix_ops, "SCAN_KERNEL", "token")
+    call, args, skip = case(kind, new, 2, 2, 64, 64, seed=pad, pad=pad)
+    s_token = state.clone()
+    o_token = call(s_token, make_step(new, [0, 2]))
+    monkeypatch.setattr(mix_ops, "SCAN_KERNEL", "auto")
+    s_auto = state.clone()
+    o_auto = call(s_auto, make_step(new, [0, 2]))
+    assert torch.equal(o_auto, o_token) and torch.equal(s_auto, s_token)
+    call, args, skip = case(kind, new, 2, 2, 64, 64, seed=pad, pad=4)
+    s_token, s_static, s_auto = state.clone(), state.clone(), state.clone()
+    monkeypatch.setattr(mix_ops, "SCAN_KERNEL", "token")
+    o_token = call(s_token, make_step(new, [0, 2]))
+    monkeypatch.setattr(mix_ops, "SCAN_KERNEL", "auto")
+    o_static = call(s_static, make_step(new, [0, 2], static=True))
+    assert torch.equal(o_static, o_token) and torch.equal(s_static, s_token)
+    o_auto = call(s_auto, make_step(new, [0, 2]))        # aligned and not captured: the same numbers in another order
+    assert rel(o_auto, o_token.to(F64)) < REL and rel(s_auto, s_token.to(F64)) < REL
