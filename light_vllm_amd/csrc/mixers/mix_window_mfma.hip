@@ -406,6 +406,334 @@ __global__ __launch_bounds__(256) void window_pool_merge_kernel(const float* __r
   }
 }
 
+// ---------------------------------------------------------------------------------------------------- prompts
+// Steps that bring more than a tile of queries, on the head sizes that the models use. A wave owns 32 consecutive queries of one
+// head and walks 64 keys a tile on v_mfma_f32_32x32x16_bf16: S^T = K Q^T leaves a query in each lane (its keys in 16 registers and the
+// lane 32 further), and the rounded probabilities are the right-hand operand of O^T += V^T P^T as they lie. The four waves take
+// up to four heads of one kv head (fewer heads: further queries), and share the K and V tile in LDS: bytes in flight per product
+// are a quarter of the 16-query form above, whose waves fetch every key row for themselves.
+// Tiles of tokens start at multiples of 64, so that a tile lies in one page and a thread's address is the page's plus a constant;
+// pooled entries and kept first tokens are looked up row by row. SAME: the values are the first DV entries of the key rows, one tile
+// serves both. Two buffers: a tile is computed while the next one's rows are on their way in registers.
+// The running maximum is held in the domain of exp2 and moves when a query outgrows it by 2^6 (the sums and outputs are f32, the
+// probabilities keep their relative precision at any magnitude).
+// Bound by the matrix pipe and the LDS reads that feed it, about level at 32 queries a wave. Against the 16-query form on one box: 11
+// prompts of 1500 tokens on average, window 1024, 16 heads over 4 of 128: 478 -> 220 us; 16 x 1024 tokens, 16 heads on latent rows of 256
+// (values 192): 978 -> 342 us; 1 x 4000 full causal, 16 over 4: 391 -> 122 us; 17 tokens behind 4000: 67 -> 43 us; never slower
+// from 17 new tokens on.
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+typedef __attribute__((address_space(3))) unsigned char lds_u8;
+constexpr int kPromptQ = 32;
+
+// byte of 16-byte chunk ch of row `row`: rows of 256 bytes and more turn their 16 lowest chunks by the row so that 16 rows read at
+// one chunk, and 4 rows x 4 chunks read transposed, meet different banks; rows of 128 bytes do so in pairs
+template <int ROW_BYTES>
+__device__ __forceinline__ int prompt_off(int row, int ch) {
+  if constexpr (ROW_BYTES == 128) return 128 * row + 16 * (ch ^ ((((row >> 1) & 1) << 2) | ((row >> 2) & 3)));
+  else return ROW_BYTES * row + 16 * (ch ^ (((row & 3) << 2) | ((row >> 2) & 3)));
+}
+
+__device__ __forceinline__ float half_max(float x) {
+  const unsigned xb = __builtin_bit_cast(unsigned, x);
+  const auto sw = __builtin_amdgcn_permlane32_swap(xb, xb, false, false);
+  const unsigned lo = sw[0], hi = sw[1];
+  return fmaxf(__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi));
+}
+
+template <int DK, int DV, bool SAME, int FORM>
+__global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WindowMfmaParams p, int hpw, int tiles, int by_count) {
+  constexpr int KB = DK * 2, VB = SAME ? KB : DV * 2;                       // bytes of a staged row
+  constexpr int KT = kTileK * KB, VT = SAME ? 0 : kTileK * VB;
+  constexpr int KCH = DK / 8, VCH = DV / 8, KN = kTileK * KCH / 256, VN = SAME ? 0 : kTileK * VCH / 256;
+  constexpr int NS = DK / 16, ND = DV / 32;
+  constexpr bool FIRST = DK <= 128;                                         // latent rows come without pooled blocks and kept tokens
+  constexpr float kLog2e = 1.44269504088896f;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * (KT + VT)];
+  __shared__ __attribute__((aligned(16))) float ks_lds[FORM == kExtended ? 2 * kTileK : 4];
+  __shared__ float bias_lds[FORM == kExtended ? 4 * kBiasLds : 1];
+  lds_u8* const base3 = (lds_u8*)lds;
+  // sequences and kv heads fastest: with a multiple of 8 of them all tiles of one run on one XCD; last queries (most keys) first
+  const int by = blockIdx.x % by_count, xt = tiles - 1 - blockIdx.x / by_count;
+  const int groups = p.G * p.ngroups, b = by / groups, gy = by % groups;
+  const int g = gy / p.ngroups, hg = gy % p.ngroups;
+  const int q0 = p.cu_q[b], n = p.cu_q[b + 1] - q0;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane & 31, half = lane >> 5;
+  const int r0 = xt * kPromptQ * (4 / hpw);
+  if (r0 >= n) return;
+  const int ctx = p.ctx_lens[b];
+  const int h = g * (p.H / p.G) + hg * hpw + wave % hpw;
+  const int rw = r0 + kPromptQ * (wave / hpw);                              // first query row of this wave
+  const int i0 = ctx + r0, i1 = ctx + min(n, r0 + kPromptQ * (4 / hpw)) - 1;
+  const bool live = rw < n;
+  const int w0 = ctx + rw, w1 = ctx + min(n, rw + kPromptQ) - 1;            // positions of this wave's first and last query
+  const int row = min(rw + c, n - 1), pos = ctx + row;
+  const int64_t t = q0 + row;
+  const int page = p.page, P = p.P, W = p.window, chunk = p.chunk, keep = p.keep_first;
+  const int cstart = chunk > 0 ? (pos / chunk) * chunk : 0;
+  const int32_t* bt = p.block_tables + static_cast<int64_t>(b) * p.bt_stride;
+  const int64_t GD = static_cast<int64_t>(p.G) * DK, GDv = static_cast<int64_t>(p.G) * DV;
+
+  bf16x8_t qf[NS];
+  {
+    const uint16_t* qrow = p.q + (t * p.H + h) * DK + 8 * half;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) qf[s] = *reinterpret_cast<const bf16x8_t*>(qrow + 16 * s);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) asm volatile("" ::"v"(qf[s]));            // the loads end here, not at a wait inside the tile loop
+  }
+  const int jlo = (chunk > 0 ? (i0 / chunk) * chunk : max(0, i0 - W + 1)) & ~(kTileK - 1);
+  const int nbmax = P > 0 ? ((chunk == 0 && i1 - W + 1 > 0) ? (i1 - W + 1) / P : 0) : min(keep, jlo);
+  const int npt = FIRST ? (nbmax + kTileK - 1) / kTileK : 0, ntiles = npt + (i1 - jlo) / kTileK + 1;
+
+  // staging: chunk tid % KCH of rows tid / KCH + (256 / KCH) i
+  const int k_ch = threadIdx.x % KCH, k_r = threadIdx.x / KCH, v_ch = threadIdx.x % VCH, v_r = threadIdx.x / VCH;
+  u32x4_t kreg[KN], vreg[SAME ? 1 : VN];
+  float ksreg = 1.0f;
+  const bool keyed = FORM == kExtended && p.key_scale != nullptr && threadIdx.x < kTileK;
+  auto slot_of = [&](int e) __attribute__((always_inline)) {                // row of an entry of the first phase
+    const int ec = min(e, nbmax - 1);
+    if (P > 0) {
+      const int pj = fdiv(ec * P + P - 1, page, p.m_page);
+      return static_cast<int64_t>(bt[pj]) * p.PP + (ec - fdiv(page * pj, P, p.m_P));
+    }
+    const int pj = fdiv(ec, page, p.m_page);
+    return static_cast<int64_t>(bt[pj]) * page + (ec - pj * page);
+  };
+  auto load = [&](int tile) __attribute__((always_inline)) {
+    if (FIRST && tile < npt) {
+      const uint16_t* kb = (P > 0 ? p.kp : p.k_cache) + g * DK + 8 * k_ch;
+      const uint16_t* vb = (P > 0 ? p.vp : p.v_cache) + g * DV + 8 * v_ch;
+      const int64_t kld = P > 0 ? GD : p.k_ld, vld = P > 0 ? GDv : p.v_ld;
+#pragma unroll
+      for (int x = 0; x < KN; ++x)
+        kreg[x] = *reinterpret_cast<const u32x4_t*>(kb + slot_of(tile * kTileK + k_r + 256 / KCH * x) * kld);
+#pragma unroll
+      for (int x = 0; x < VN; ++x)
+        vreg[x] = *reinterpret_cast<const u32x4_t*>(vb + slot_of(tile * kTileK + v_r + 256 / VCH * x) * vld);
+      if (keyed) ksreg = p.key_scale[slot_of(tile * kTileK + threadIdx.x) * p.G + g];
+    } else {
+      const int e0 = jlo + (tile - npt) * kTileK, pj = fdiv(e0, page, p.m_page), last = i1 - e0;
+      const int64_t slot = static_cast<int64_t>(bt[pj]) * page + (e0 - pj * page);
+      const uint16_t* kb = p.k_cache + slot * p.k_ld + g * DK;
+      const uint16_t* vb = p.v_cache + slot * p.v_ld + g * DV;
+#pragma unroll
+      for (int x = 0; x < KN; ++x)                                          // rows past the last query's repeat its row: finite values
+        kreg[x] = *reinterpret_cast<const u32x4_t*>(kb + static_cast<uint32_t>(min(k_r + 256 / KCH * x, last)) * static_cast<uint32_t>(p.k_ld) + 8 * k_ch);
+#pragma unroll
+      for (int x = 0; x < VN; ++x)
+        vreg[x] = *reinterpret_cast<const u32x4_t*>(vb + static_cast<uint32_t>(min(v_r + 256 / VCH * x, last)) * static_cast<uint32_t>(p.v_ld) + 8 * v_ch);
+      if (keyed) ksreg = p.key_scale[(slot + min(static_cast<int>(threadIdx.x), last)) * p.G + g];
+    }
+  };
+  auto store = [&](int buf) __attribute__((always_inline)) {
+    unsigned char* kt = lds + buf * (KT + VT);
+#pragma unroll
+    for (int x = 0; x < KN; ++x) *reinterpret_cast<u32x4_t*>(kt + prompt_off<KB>(k_r + 256 / KCH * x, k_ch)) = kreg[x];
+#pragma unroll
+    for (int x = 0; x < VN; ++x) *reinterpret_cast<u32x4_t*>(kt + KT + prompt_off<VB>(v_r + 256 / VCH * x, v_ch)) = vreg[x];
+    if (FORM == kExtended && threadIdx.x < kTileK) ks_lds[buf * kTileK + threadIdx.x] = ksreg;
+  };
+  const float* bias_h = nullptr;
+  bool bias_cached = false;
+  if constexpr (FORM == kExtended) {
+    if (p.dist_bias != nullptr) {
+      bias_h = p.dist_bias + static_cast<int64_t>(h) * p.bias_len;
+      bias_cached = p.bias_len <= kBiasLds;
+      if (bias_cached)
+        for (int x = lane; x < p.bias_len; x += kWave) bias_lds[wave * kBiasLds + x] = bias_h[x];     // read by this wave alone
+    }
+  }
+
+  // LDS addresses inside a buffer: rows of K (lane = key), V transposed (16 lanes read 4 keys x 16 columns)
+  const int tq = (lane & 15) >> 2, tp = lane & 3, gi = lane >> 4;
+  // (chunks 16 further lie 256 bytes further: a turn touches the four lowest bits)
+  constexpr int NKA = NS < 8 ? NS : 8, NVA = ND < 4 ? ND : 4;
+  int kaddr[NKA], vaddr[2][NVA];
+#pragma unroll
+  for (int x = 0; x < NKA; ++x) kaddr[x] = prompt_off<KB>(c, 2 * x + half);
+#pragma unroll
+  for (int second = 0; second < 2; ++second)
+#pragma unroll
+    for (int d = 0; d < NVA; ++d)
+      vaddr[second][d] = (SAME ? 0 : KT) + prompt_off<VB>(8 * second + 4 * (gi >> 1) + tq, 4 * d + 2 * (gi & 1) + (tp >> 1)) + 8 * (tp & 1);
+
+  f32x16_t o[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[d][i] = 0.0f;
+  const float cs = FORM == kPlain ? p.scale * kLog2e : kLog2e;              // from what the products leave to the exponent of 2
+  float m = (p.sinks != nullptr ? p.sinks[h] : p.m0) * kLog2e, l = half == 0 ? p.sink : 0.0f;
+
+  auto compute = [&](int tile, int buf) __attribute__((always_inline)) {
+    const int phase = FIRST && tile < npt ? 0 : 1;
+    const int e0 = phase == 0 ? tile * kTileK : jlo + (tile - npt) * kTileK;
+    const int e_end = phase == 0 ? nbmax : i1 + 1;
+    if (!live) return;
+    if (phase == 1) {                                                       // nothing here for this wave's queries
+      if (e0 > w1) return;
+      if (e0 >= keep && (chunk > 0 ? e0 + kTileK - 1 < (w0 / chunk) * chunk : w0 - (e0 + kTileK - 1) >= W)) return;
+    } else if (P > 0 && e0 * P + P - 1 > w1 - W) {
+      return;
+    }
+    const bool whole = phase == 1 && e0 + kTileK - 1 <= w0 && (chunk > 0 ? e0 >= w1 - w1 % chunk : w1 - e0 < W);
+    lds_u8* const kt = base3 + buf * (KT + VT);
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub) {
+      f32x16_t s;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+#pragma unroll
+      for (int x = 0; x < NS; ++x) {
+        const bf16x8_t ka = *reinterpret_cast<const __attribute__((address_space(3))) bf16x8_t*>(kt + kaddr[x % NKA] + (KB * 32 * sub + 256 * (x / NKA)));
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka, qf[x], s, 0, 0, 0);
+        if (DK == 256 && x % 4 == 3) __builtin_amdgcn_sched_barrier(0);     // fragments of four steps at a time: more of them spill
+      }
+      const int ks0 = e0 + 32 * sub;
+      if constexpr (FORM == kCapped) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = p.cap * fast_tanh(s[i] * p.cap_in);
+      }
+      if constexpr (FORM == kExtended) {
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const f32x4_t ks = *reinterpret_cast<const f32x4_t*>(ks_lds + buf * kTileK + 32 * sub + 8 * x + 4 * half);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[4 * x + i] *= ks[i] * p.scale;
+        }
+        if (bias_h != nullptr) {
+          const float* table = bias_cached ? bias_lds + wave * kBiasLds : bias_h;
+          const int top = p.bias_len - 1;
+          if (w0 - (ks0 + 31) >= top) {                                     // all of the tile at the last bias
+            const float far = table[top];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] += far;
+          } else {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const int dist = min(max(pos - (ks0 + (i & 3) + 8 * (i >> 2) + 4 * half), 0), top);
+              s[i] += table[dist];
+            }
+          }
+        }
+      }
+      if (!whole) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int ke = ks0 + (i & 3) + 8 * (i >> 2) + 4 * half;
+          bool vis = ke < e_end;
+          if (phase == 0) vis = vis && (P == 0 || ke * P + P - 1 <= pos - W);
+          else vis = vis && ke <= pos && ((chunk > 0 ? ke >= cstart : pos - ke < W) || ke < keep);
+          s[i] = vis ? s[i] : -INFINITY;
+        }
+      }
+      float mx = s[0];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+      mx = half_max(mx) * cs;
+      if (__builtin_amdgcn_ballot_w64(mx - m > 6.0f) != 0) {
+        const float nm = fmaxf(m, mx), f = __builtin_amdgcn_exp2f(m - nm);
+        m = nm;
+        l *= f;
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[d][i] *= f;
+      }
+      bf16x8_t pf[2];
+      float sum = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float e = __builtin_amdgcn_exp2f(fmaf(s[i], cs, -m));
+        sum += e;
+        pf[i >> 3][i & 7] = static_cast<__bf16>(e);
+      }
+      l += sum;
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        if (DK == 256) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+          const lds_u8* v = kt + VB * (32 * sub + 16 * x);
+          const bf16x4v_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(v + vaddr[0][d % NVA] + 256 * (d / NVA)));
+          const bf16x4v_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(v + vaddr[1][d % NVA] + 256 * (d / NVA)));
+          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), pf[x], o[d], 0, 0, 0);
+          if (DK == 256 && d % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+  };
+
+  load(0);
+  store(0);
+  __syncthreads();
+  if (ntiles > 1) load(1);
+  for (int tile = 0; tile < ntiles; ++tile) {
+    compute(tile, tile & 1);
+    if (tile + 1 < ntiles) store((tile + 1) & 1);
+    if (tile + 2 < ntiles) load(tile + 2);
+    __syncthreads();
+  }
+  if (!live) return;
+  const float total = l + __shfl_xor(l, 32, kWave);
+  const float inv = total > 0.0f ? 1.0f / total : 0.0f;
+  if (rw + c >= n) return;
+  uint16_t* orow = p.out + t * p.out_ld + static_cast<int64_t>(h) * DV + 4 * half;
+  const uint16_t* grow = p.gate != nullptr ? p.gate + t * p.ld_gate + static_cast<int64_t>(h) * p.gate_dv : nullptr;
+  const float gate1 = grow != nullptr && p.gate_dv == 1 ? sigmoidf_(ldf(reinterpret_cast<const bf16_t*>(grow))) : 1.0f;
+#pragma unroll
+  for (int d = 0; d < ND; ++d)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      float4 y{o[d][4 * x] * inv, o[d][4 * x + 1] * inv, o[d][4 * x + 2] * inv, o[d][4 * x + 3] * inv};
+      if (grow != nullptr) {
+        if (p.gate_dv == 1) {
+          y = float4{y.x * gate1, y.y * gate1, y.z * gate1, y.w * gate1};
+        } else {
+          const float4 gv = ld4(reinterpret_cast<const bf16_t*>(grow) + 32 * d + 8 * x + 4 * half);
+          y = float4{y.x * sigmoidf_(gv.x), y.y * sigmoidf_(gv.y), y.z * sigmoidf_(gv.z), y.w * sigmoidf_(gv.w)};
+        }
+      }
+      st4(reinterpret_cast<bf16_t*>(orow) + 32 * d + 8 * x, y);
+    }
+}
+
+// The head sizes and forms that prompt_attn_kernel is built for; false: the launch belongs to window_pool_mfma_kernel. It also
+// needs pages of whole tiles, a positive scale (the maximum is taken before it is applied), and rows that allow 8-byte accesses of
+// gate and output.
+static bool prompt_launch(const WindowMfmaParams& p, int form, int B, int max_new, hipStream_t s) {
+  auto at = [](const void* q, uintptr_t a) { return reinterpret_cast<uintptr_t>(q) % a == 0; };
+  if (p.D > 128 && (p.P > 0 || p.keep_first > 0)) return false;
+  if (max_new <= kTileQ || p.page % kTileK != 0 || !(p.scale > 0.0f) || !at(p.q, 16) || !at(p.out, 8) || p.out_ld % 4 != 0 ||
+      (p.P > 0 && (!at(p.kp, 16) || !at(p.vp, 16))) ||
+      (p.gate != nullptr && p.gate_dv > 1 && (!at(p.gate, 8) || p.ld_gate % 4 != 0)))
+    return false;
+  const bool same = p.P == 0 && (p.G == 1 || p.D == p.Dv) && p.k_cache == p.v_cache && p.k_ld == p.v_ld;
+  const int rep = p.H / p.G, hpw = rep % 4 == 0 ? 4 : (rep % 2 == 0 ? 2 : 1);
+  WindowMfmaParams q = p;
+  q.ngroups = rep / hpw;
+  const int rows = kPromptQ * (4 / hpw), tiles = (max_new + rows - 1) / rows, by = B * p.G * q.ngroups;
+  if (static_cast<int64_t>(tiles) * by >= (1ll << 31)) return false;
+  const dim3 grid(static_cast<unsigned>(tiles) * by), block(256);
+#define LVMIX_PROMPT(DK, DV, SAME, FORM)                                                              \
+  if (p.D == DK && p.Dv == DV && same == SAME && form == FORM) {                                      \
+    prompt_attn_kernel<DK, DV, SAME, FORM><<<grid, block, 0, s>>>(q, hpw, tiles, by);                 \
+    return true;                                                                                      \
+  }
+  LVMIX_PROMPT(64, 64, false, kPlain)
+  LVMIX_PROMPT(64, 64, false, kCapped)
+  LVMIX_PROMPT(64, 64, false, kExtended)
+  LVMIX_PROMPT(128, 128, false, kPlain)
+  LVMIX_PROMPT(128, 128, false, kCapped)
+  LVMIX_PROMPT(128, 128, false, kExtended)
+  LVMIX_PROMPT(128, 128, true, kPlain)
+  LVMIX_PROMPT(128, 128, true, kExtended)
+  LVMIX_PROMPT(256, 192, true, kPlain)
+  LVMIX_PROMPT(256, 256, true, kPlain)
+#undef LVMIX_PROMPT
+  return false;
+}
+
 }  // namespace lvmix
 
 using namespace lvmix;
@@ -469,10 +797,12 @@ extern "C" int lv_masked_attn_mfma(const void* q, const void* k_cache, const voi
                      extended ? static_cast<const float*>(extras->dist_bias) : nullptr, extended ? extras->bias_len : 0, out_ld};
   if (nsplit > 1 && (max_new_tokens > kTileQ || workspace == nullptr || T <= 0 || nsplit > kWave))
     return fail(-1, "lv_window_pool_attn_mfma: key splits need one query tile per sequence and a workspace");
+  hipStream_t st = as_stream(stream);
+  if (nsplit <= 1 && prompt_launch(p, softcap > 0.0f ? kCapped : (extended ? kExtended : kPlain), B, max_new_tokens, st))
+    return launched("lv_masked_attn_mfma");
   size_t shm = static_cast<size_t>(kTileK) * v_row(Dv) * sizeof(uint16_t);
   if (extended) shm += sizeof(float) * (kTileK + (p.dist_bias != nullptr && p.bias_len <= kBiasLds ? 4 * static_cast<size_t>(p.bias_len) : 0));
   dim3 grid(nsplit > 1 ? nsplit : (max_new_tokens + kTileQ - 1) / kTileQ, G * ngroups, B), block(256);
-  hipStream_t st = as_stream(stream);
   const bool tiny = D <= 64 && Dv <= 64, small = D <= 128 && Dv <= 128;
 #define LVMIX_ATT_FORM(AHEAD, FORM)                                                               \
   do {                                                                                            \

@@ -1,0 +1,97 @@
+"""The 32-query form of the windowed attention (prompt_attn_kernel) at the edges of its tiles, windows, pages and head groups,
+against the vector kernel (f32 products of the same bf16 rows), and the rule that takes a launch to it."""
+import pytest
+import torch
+
+from light_vllm_amd import mix_ops
+from light_vllm_amd.utils.context import RaggedStep
+
+pytestmark = pytest.mark.gpu
+# probabilities and outputs are rounded to bf16 (2^-9 each); an output is an average of values of magnitude 1 to 4
+ATOL = 4 * 2.0 ** -8
+
+
+def make_step(new, ctx, page, seed):
+    cu, tok = [0], []
+    for b, n in enumerate(new):
+        cu.append(cu[-1] + n)
+        tok += [b] * n
+    need = [-(-(n + c) // page) for n, c in zip(new, ctx)]
+    perm = torch.randperm(sum(need), generator=torch.Generator().manual_seed(seed)).tolist()
+    tables, at = [], 0
+    for k in need:
+        tables.append(perm[at:at + k])
+        at += k
+    wide = max(need)
+    i32 = dict(dtype=torch.int32, device="cuda")
+    return RaggedStep(torch.tensor(cu, **i32), torch.tensor(ctx, **i32), torch.arange(len(new), **i32), torch.tensor(tok, **i32),
+                      torch.tensor([t + [-1] * (wide - len(t)) for t in tables], **i32), new, ctx, list(range(len(new))), tables), sum(need)
+
+
+def both(monkeypatch, new, ctx, H, G, D, Dv, page=256, same=False, gate=None, ext=False, pool=0, out_pad=0, seed=0, **kw):
+    step, pages = make_step(new, ctx, page, seed)
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    T = sum(new)
+
+    def rn(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen).bfloat16()
+
+    q, kc = rn(T, H * D), rn(pages, page, G, D)
+    vc = kc[..., :Dv] if same else rn(pages, page, G, Dv)
+    pp = max(mix_ops.pooled_slots(page, pool), 1)
+    kp, vp = (rn(pages, pp, G, D), rn(pages, pp, G, Dv)) if pool else (None, None)
+    g = None if gate is None else rn(T, H if gate == "head" else H * Dv)
+    if ext:
+        kw.update(key_scale=torch.rand(pages, page, G, device="cuda", generator=gen) + 0.5,
+                  dist_bias=torch.randn(H, ext, device="cuda", generator=gen))
+    got = []
+    for kernel in ("valu", "auto"):
+        monkeypatch.setattr(mix_ops, "WINDOW_ATTN_KERNEL", kernel)
+        wide = torch.full((T, H * Dv + out_pad), 7.0, device="cuda", dtype=torch.bfloat16)
+        out = wide[:, :H * Dv]
+        mix_ops.window_pool_attention(q, kc, vc, kp, vp, g, step, H, G, D, Dv, kw.get("window", 1 << 30), pool, D ** -0.5,
+                                      gate_per_head=gate == "head", out=out, **{k: v for k, v in kw.items() if k != "window"})
+        assert bool((wide[:, H * Dv:] == 7.0).all())
+        got.append(out.float())
+    assert bool(torch.isfinite(got[1]).all())
+    assert (got[0] - got[1]).abs().max().item() <= ATOL
+
+
+@pytest.mark.parametrize("n", [17, 31, 32, 33, 63, 64, 65, 129])
+@pytest.mark.parametrize("ctx", [0, 1, 63, 200])
+def test_tiles(monkeypatch, n, ctx):
+    both(monkeypatch, [n, 1, 40], [ctx, ctx, 0], 4, 1, 64, 64, has_sink=False, seed=n + ctx)
+
+
+@pytest.mark.parametrize("H,G", [(1, 1), (2, 1), (3, 1), (4, 1), (6, 2), (8, 1), (8, 4)])
+def test_head_groups(monkeypatch, H, G):
+    both(monkeypatch, [70, 150], [5, 0], H, G, 128, 128, window=100, gate="channel", has_sink=True, seed=H)
+
+
+@pytest.mark.parametrize("D,Dv", [(256, 192), (256, 256), (128, 128)])
+def test_values_inside_the_key_rows(monkeypatch, D, Dv):
+    both(monkeypatch, [65, 200], [130, 0], 8, 1, D, Dv, same=True, has_sink=False, out_pad=64, seed=D)
+    both(monkeypatch, [65, 200], [130, 0], 8, 1, D, Dv, same=True, window=90, sinks=torch.randn(8, device="cuda"), seed=D)
+
+
+@pytest.mark.parametrize("window", [1, 31, 64, 65, 100])
+@pytest.mark.parametrize("pool", [0, 16, 64])
+def test_windows_and_pooled_blocks(monkeypatch, window, pool):
+    both(monkeypatch, [300, 33], [0, 270], 4, 2, 64, 64, page=64, window=window, pool=pool, gate="head", seed=window)
+
+
+@pytest.mark.parametrize("kw", [dict(window=50, keep_first=3), dict(window=64, keep_first=130), dict(window=1, chunk=48),
+                                dict(window=1, chunk=128, keep_first=5), dict(window=70, softcap=5.0), dict(softcap=20.0),
+                                dict(window=90, ext=32), dict(ext=1500), dict(window=1, chunk=100, ext=7)])
+@pytest.mark.parametrize("D", [64, 128])
+def test_masks_and_scores(monkeypatch, kw, D):
+    kw = dict(kw)
+    both(monkeypatch, [210, 20, 64], [0, 140, 64], 4, 1, D, D, has_sink=kw.get("window", 0) % 2 == 0, seed=D, **kw)
+
+
+def test_other_pages_and_sizes_keep_their_kernel(monkeypatch):
+    """Pages that do not hold whole tiles, head sizes without an instance, latent rows with kept tokens, a scale of another sign."""
+    both(monkeypatch, [80, 20], [9, 0], 4, 2, 64, 64, page=48, window=60)
+    both(monkeypatch, [80, 20], [9, 0], 4, 2, 48, 80, window=60)
+    both(monkeypatch, [80, 20], [9, 0], 4, 1, 256, 192, same=True, window=60, keep_first=4)
+    both(monkeypatch, [80, 20], [9, 0], 4, 1, 256, 192, window=60)
