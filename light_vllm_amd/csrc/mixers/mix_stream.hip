@@ -18,6 +18,8 @@
 //   head_norm_gate_kernel     one wave per (token, head); optionally the head is divided by a number of its own first.
 #include "mix_common.h"
 
+#include <algorithm>
+
 namespace lvmix {
 
 static thread_local char g_err[512] = "";
@@ -307,6 +309,114 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(DeltaPrepParams p) {
   ss = wave_sum(ss);
   const float inv = post / sqrtf(ss + p.unit_eps);
   for (int e = lane; e < n; e += kWave) dst[e] *= inv;    // each lane rescales what it wrote itself
+}
+
+// The same for heads of 64, 128 or 256 entries (keys and values alike) and up to four taps: a thread owns four channels, their
+// filters and last inputs in registers, and walks a tile of packed tokens, so that a row is read once and written once. The
+// D / 4 lanes of a head add up its squares. One more column of workgroups forms the write strengths and decays of its tokens.
+// Bound by memory (the projection's rows in, f32 rows out). The wave-per-(token, head) form above reads every row once per tap,
+// two bytes a lane: 16 x 1024 tokens, 3072 channels, four taps 374 us, this form 109 us;
+// 64 decoded tokens 5.5 -> 4.2 us.
+template <typename T, int TAPS>
+__global__ __launch_bounds__(256) void delta_prep_tile_kernel(DeltaPrepParams p, int tile) {
+  const int64_t t0 = static_cast<int64_t>(blockIdx.y) * tile, t1 = min(t0 + tile, p.T);
+  const T* proj = static_cast<const T*>(p.proj);
+  const int GD = p.G * p.D, C = 2 * GD + p.H * p.Dv;
+  if (blockIdx.x == gridDim.x - 1) {
+    const T* a = static_cast<const T*>(p.a);
+    for (int x = threadIdx.x; x < static_cast<int>(t1 - t0) * p.H; x += blockDim.x) {
+      const int64_t t = t0 + x / p.H;
+      const int h = x % p.H;
+      p.beta[t * p.H + h] = sigmoidf_(ldf(proj + t * p.ld + p.off_b + h));
+      if (p.dec_dim == 1) p.decay[t * p.H + h] = expf(-expf(p.A_log[h]) * softplusf_(ldf(a + t * p.ld_a + h) + p.dt_bias[h]));
+    }
+    if (p.dec_dim > 1) {
+      const int wide = p.H * p.dec_dim;
+      for (int x = threadIdx.x; x < wide; x += blockDim.x) {
+        const float rate = expf(p.A_log[x / p.dec_dim]), bias = p.dt_bias[x];
+        for (int64_t t = t0; t < t1; ++t) p.decay[t * wide + x] = expf(-rate * softplusf_(ldf(a + t * p.ld_a + x) + bias));
+      }
+    }
+    return;
+  }
+  const int c = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  if (c >= C) return;                              // whole heads: the sums below stay among live lanes
+  constexpr int HIST = TAPS > 1 ? TAPS - 1 : 1;
+  float w[TAPS][4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) w[j][e] = p.conv_w[(c + e) * TAPS + j];
+  const bool unit = c < 2 * GD;
+  const float post = c < GD ? 1.0f / sqrtf(static_cast<float>(p.D)) : 1.0f;
+  float* dst = c < GD ? p.qn + c : (unit ? p.kn + (c - GD) : p.v + (c - 2 * GD));
+  const int64_t ldd = unit ? GD : static_cast<int64_t>(p.H) * p.Dv;
+  const int lanes = p.D / 4;
+  float4 hist[HIST];
+  auto history = [&](int64_t t, int b) {           // the inputs before token t of sequence b
+    const int r = static_cast<int>(t) - p.cu_q[b], ctx = p.ctx_lens[b];
+    const T* state = static_cast<const T*>(p.conv_state) + static_cast<int64_t>(p.slots[b]) * (TAPS - 1) * C + c;
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) {
+      const int rr = r - (TAPS - 1) + j;
+      if (rr >= 0) hist[j] = ld4(proj + (t - (TAPS - 1) + j) * p.ld + c);
+      else if (ctx + rr >= 0) hist[j] = ld4(state + static_cast<int64_t>(TAPS - 1 + rr) * C);
+      else hist[j] = float4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+  };
+  auto emit = [&](int64_t t, float4 u) __attribute__((always_inline)) {
+    float4 y{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) {
+      const float4 x = j < TAPS - 1 ? hist[j] : u;
+      y.x += w[j][0] * x.x; y.y += w[j][1] * x.y; y.z += w[j][2] * x.z; y.w += w[j][3] * x.w;
+    }
+#pragma unroll
+    for (int j = 0; j + 1 < TAPS - 1; ++j) hist[j] = hist[j + 1];
+    if (TAPS > 1) hist[HIST - 1] = u;
+    y = float4{siluf_(y.x), siluf_(y.y), siluf_(y.z), siluf_(y.w)};
+    if (unit) {                                    // the same for all lanes of a head
+      float ss = row16_sum((y.x * y.x + y.y * y.y) + (y.z * y.z + y.w * y.w));
+      if (lanes > 16) ss += __shfl_xor(ss, 16, kWave);
+      if (lanes > 32) ss += __shfl_xor(ss, 32, kWave);
+      const float f = post / sqrtf(ss + p.unit_eps);
+      y = float4{y.x * f, y.y * f, y.z * f, y.w * f};
+    }
+    st4(dst + t * ldd, y);
+  };
+  int b = p.tok_seq[t0];
+  history(t0, b);
+  if (p.tok_seq[t1 - 1] == b) {                    // one sequence: the next rows' loads need not wait for a look at its end
+#pragma unroll 4
+    for (int64_t t = t0; t < t1; ++t) emit(t, ld4(proj + t * p.ld + c));
+    return;
+  }
+  for (int64_t t = t0; t < t1; ++t) {
+    const int now = p.tok_seq[t];
+    if (now != b) history(t, b = now);
+    emit(t, ld4(proj + t * p.ld + c));
+  }
+}
+
+template <typename T>
+static bool delta_prep_tiles(const DeltaPrepParams& p, hipStream_t s) {
+  auto at = [](const void* q, uintptr_t a) { return reinterpret_cast<uintptr_t>(q) % a == 0; };
+  constexpr uintptr_t piece = 4 * sizeof(T);
+  if (p.D != p.Dv || (p.D != 64 && p.D != 128 && p.D != 256) || p.taps > 4 || p.ld % 4 != 0 || !at(p.proj, piece) ||
+      !at(p.conv_state, piece) || !at(p.qn, 16) || !at(p.kn, 16) || !at(p.v, 16))
+    return false;
+  const int cols = ((2 * p.G * p.D + p.H * p.Dv) / 4 + 255) / 256;
+  // tiles of up to 16 tokens, shorter ones where the launch would have fewer than four workgroups a compute unit
+  const int tile = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(16, p.T * (cols + 1) / 1024)));
+  dim3 grid(cols + 1, static_cast<unsigned>((p.T + tile - 1) / tile)), block(256);
+  if (grid.y > 65535) return false;
+  switch (p.taps) {
+    case 1: delta_prep_tile_kernel<T, 1><<<grid, block, 0, s>>>(p, tile); break;
+    case 2: delta_prep_tile_kernel<T, 2><<<grid, block, 0, s>>>(p, tile); break;
+    case 3: delta_prep_tile_kernel<T, 3><<<grid, block, 0, s>>>(p, tile); break;
+    default: delta_prep_tile_kernel<T, 4><<<grid, block, 0, s>>>(p, tile); break;
+  }
+  return true;
 }
 
 template <typename T>
@@ -636,6 +746,9 @@ int lv_delta_prep(const void* proj, int64_t ld, const void* conv_w, const void* 
                     static_cast<float*>(decay), T, G, H, D, Dv, taps, off_b, unit_eps, a, ld_a, dec_dim};
   const int units = 2 * G + H + 1 + (dec_dim > 1 ? H : 0);
   dim3 grid(static_cast<unsigned>(T), (units + 3) / 4), block(256);
+  if ((dtype == LV_MIX_BF16 && delta_prep_tiles<bf16_t>(p, as_stream(stream))) ||
+      (dtype == LV_MIX_F32 && delta_prep_tiles<float>(p, as_stream(stream))))
+    return launched("lv_delta_prep");
   if (dtype == LV_MIX_BF16) delta_prep_kernel<bf16_t><<<grid, block, 0, as_stream(stream)>>>(p);
   else if (dtype == LV_MIX_F32) delta_prep_kernel<float><<<grid, block, 0, as_stream(stream)>>>(p);
   else return fail(-1, "lv_delta_prep: dtype %d", dtype);
