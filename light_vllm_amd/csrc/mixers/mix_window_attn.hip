@@ -49,6 +49,123 @@ __global__ __launch_bounds__(256) void qk_fullnorm_store_kernel(
   for (int i = threadIdx.x; i < GDv; i += blockDim.x) v_cache[slot * GDv + i] = v[t * ld + i];
 }
 
+// Rows of at most 4096 queries' and 1024 keys' entries, four an access: every entry is read once and kept in registers between the
+// sum of squares and the scaling. Bound by memory: 15179 tokens of 2048 + 512 + 512 entries 101 us in the form above (two bytes a
+// lane, read twice), 49 us here.
+constexpr int kNormQ = 4;
+template <typename T>
+__global__ __launch_bounds__(256) void qk_fullnorm_store_vec_kernel(
+    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, int64_t ld, const float* __restrict__ q_w,
+    const float* __restrict__ k_w, T* __restrict__ q_out, T* __restrict__ k_cache, T* __restrict__ v_cache,
+    const int32_t* __restrict__ cu_q, const int32_t* __restrict__ ctx_lens, const int32_t* __restrict__ tok_seq,
+    const int32_t* __restrict__ block_tables, int bt_stride, int HD, int GD, int GDv, int page, float eps) {
+  __shared__ float red[2][4];
+  const int64_t t = blockIdx.x;
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, c = threadIdx.x * 4;
+  const float4 none{0.0f, 0.0f, 0.0f, 0.0f};
+  float4 x[kNormQ], y = c < GD ? ld4(k + t * ld + c) : none;
+  float sq = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kNormQ; ++i) {
+    x[i] = c + 1024 * i < HD ? ld4(q + t * ld + c + 1024 * i) : none;
+    sq += (x[i].x * x[i].x + x[i].y * x[i].y) + (x[i].z * x[i].z + x[i].w * x[i].w);
+  }
+  const int b = tok_seq[t];
+  const int pos = ctx_lens[b] + static_cast<int>(t) - cu_q[b];
+  const int64_t slot = static_cast<int64_t>(block_tables[static_cast<int64_t>(b) * bt_stride + pos / page]) * page + pos % page;
+  for (int i = c; i < GDv; i += 1024) st4(v_cache + slot * GDv + i, ld4(v + t * ld + i));
+  sq = wave_sum(sq);
+  const float sk = wave_sum((y.x * y.x + y.y * y.y) + (y.z * y.z + y.w * y.w));
+  if (lane == 0) {
+    red[0][wave] = sq;
+    red[1][wave] = sk;
+  }
+  __syncthreads();
+  const float inv_q = 1.0f / sqrtf((red[0][0] + red[0][1] + red[0][2] + red[0][3]) / static_cast<float>(HD) + eps);
+  const float inv_k = 1.0f / sqrtf((red[1][0] + red[1][1] + red[1][2] + red[1][3]) / static_cast<float>(GD) + eps);
+#pragma unroll
+  for (int i = 0; i < kNormQ; ++i)
+    if (c + 1024 * i < HD) {
+      const float4 w = ld4(q_w + c + 1024 * i);
+      st4(q_out + t * HD + c + 1024 * i, float4{x[i].x * inv_q * w.x, x[i].y * inv_q * w.y, x[i].z * inv_q * w.z, x[i].w * inv_q * w.w});
+    }
+  if (c < GD) {
+    const float4 w = ld4(k_w + c);
+    st4(k_cache + slot * GD + c, float4{y.x * inv_k * w.x, y.y * inv_k * w.y, y.z * inv_k * w.z, y.w * inv_k * w.w});
+  }
+}
+
+template <typename T>
+static bool qk_fullnorm_vec(const T* q, const T* k, const T* v, int64_t ld, const float* q_w, const float* k_w, T* q_out, T* k_cache,
+                            T* v_cache, const int32_t* cu_q, const int32_t* ctx_lens, const int32_t* tok_seq, const int32_t* block_tables,
+                            int bt_stride, int64_t Tn, int HD, int GD, int GDv, int page, float eps, hipStream_t s) {
+  auto at = [](const void* x, uintptr_t a) { return reinterpret_cast<uintptr_t>(x) % a == 0; };
+  constexpr uintptr_t piece = 4 * sizeof(T);
+  if (HD > 1024 * kNormQ || GD > 1024 || HD % 4 != 0 || GD % 4 != 0 || GDv % 4 != 0 || ld % 4 != 0 || !at(q, piece) || !at(k, piece) ||
+      !at(v, piece) || !at(q_w, 16) || !at(k_w, 16) || !at(q_out, piece) || !at(k_cache, piece) || !at(v_cache, piece))
+    return false;
+  qk_fullnorm_store_vec_kernel<T><<<dim3(static_cast<unsigned>(Tn)), dim3(256), 0, s>>>(
+      q, k, v, ld, q_w, k_w, q_out, k_cache, v_cache, cu_q, ctx_lens, tok_seq, block_tables, bt_stride, HD, GD, GDv, page, eps);
+  return true;
+}
+
+// Means of a block's rows, four entries an access: a thread sums every `parts`-th row of its entries, four rows in flight, and
+// the parts meet in LDS. (One thread per entry and one row after the other, the form below, is a chain of P memory latencies: 91 us
+// for 15179 tokens in blocks of 64; here 9.4.)
+template <typename T>
+__global__ __launch_bounds__(256) void pool_update_vec_kernel(const T* __restrict__ k_cache, const T* __restrict__ v_cache,
+                                                              T* __restrict__ kp, T* __restrict__ vp, const int32_t* __restrict__ cu_q,
+                                                              const int32_t* __restrict__ ctx_lens, const int32_t* __restrict__ block_tables,
+                                                              int bt_stride, int GD, int GDv, int page, int P, int PP, int cols) {
+  __shared__ __attribute__((aligned(16))) float4 part_sums[256];
+  const int b = blockIdx.y;
+  const int ctx = ctx_lens[b], n = cu_q[b + 1] - cu_q[b];
+  const int blk = ctx / P + blockIdx.x;                 // blocks complete before the step: floor(ctx / P)
+  if (blk >= (ctx + n) / P) return;
+  const int32_t* bt = block_tables + static_cast<int64_t>(b) * bt_stride;
+  const int first = blk * P, pj = (first + P - 1) / page;
+  const int64_t dst = static_cast<int64_t>(bt[pj]) * PP + (blk - (page * pj) / P);
+  const float invP = 1.0f / static_cast<float>(P);
+  const int parts = 256 / cols, part = threadIdx.x / cols;
+  const int i = (blockIdx.z * cols + threadIdx.x % cols) * 4;
+  const bool live = i < GD + GDv;
+  const T* src = i < GD ? k_cache + i : v_cache + (i - GD);
+  const int64_t lds = i < GD ? GD : GDv;
+  float4 acc{0.0f, 0.0f, 0.0f, 0.0f};
+  if (live) {
+#pragma unroll 4
+    for (int j = part; j < P; j += parts) {
+      const int at = first + j, pg = at / page;
+      const float4 x = ld4(src + (static_cast<int64_t>(bt[pg]) * page + (at - pg * page)) * lds);
+      acc.x += x.x; acc.y += x.y; acc.z += x.z; acc.w += x.w;
+    }
+  }
+  part_sums[threadIdx.x] = acc;
+  __syncthreads();
+  if (part != 0 || !live) return;
+  for (int x = 1; x < parts; ++x) {
+    const float4 y = part_sums[x * cols + threadIdx.x];
+    acc.x += y.x; acc.y += y.y; acc.z += y.z; acc.w += y.w;
+  }
+  acc = float4{acc.x * invP, acc.y * invP, acc.z * invP, acc.w * invP};
+  if (i < GD) st4(kp + dst * GD + i, acc);
+  else st4(vp + dst * GDv + (i - GD), acc);
+}
+
+template <typename T>
+static bool pool_update_vec(const T* k_cache, const T* v_cache, T* kp, T* vp, const int32_t* cu_q, const int32_t* ctx_lens,
+                            const int32_t* block_tables, int bt_stride, int B, int max_new_blocks, int GD, int GDv, int page, int P, int PP,
+                            hipStream_t s) {
+  auto at = [](const void* x, uintptr_t a) { return reinterpret_cast<uintptr_t>(x) % a == 0; };
+  constexpr uintptr_t piece = 4 * sizeof(T);
+  if (GD % 4 != 0 || GDv % 4 != 0 || !at(k_cache, piece) || !at(v_cache, piece) || !at(kp, piece) || !at(vp, piece)) return false;
+  constexpr int cols = 32;                             // eight parts of the rows, 128 entries a workgroup
+  dim3 grid(max_new_blocks, B, ((GD + GDv) / 4 + cols - 1) / cols);
+  pool_update_vec_kernel<T><<<grid, dim3(256), 0, s>>>(k_cache, v_cache, kp, vp, cu_q, ctx_lens, block_tables, bt_stride, GD, GDv, page,
+                                                      P, PP, cols);
+  return true;
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void pool_update_kernel(const T* __restrict__ k_cache, const T* __restrict__ v_cache,
                                                           T* __restrict__ kp, T* __restrict__ vp,
@@ -262,6 +379,13 @@ int lv_qk_fullnorm_store(const void* q, const void* k, const void* v, int64_t ld
   if (T < 0 || H <= 0 || G <= 0 || H % G != 0 || D <= 0 || Dv <= 0 || page <= 0 || bt_stride <= 0)
     return fail(-1, "lv_qk_fullnorm_store: bad sizes");
   dim3 grid(static_cast<unsigned>(T)), block(256);
+#define LVMIX_QKN(TT)                                                                                                          \
+  qk_fullnorm_vec<TT>(static_cast<const TT*>(q), static_cast<const TT*>(k), static_cast<const TT*>(v), ld,                     \
+                      static_cast<const float*>(q_w), static_cast<const float*>(k_w), static_cast<TT*>(q_out),                 \
+                      static_cast<TT*>(k_cache), static_cast<TT*>(v_cache), cu_q, ctx_lens, tok_seq, block_tables, bt_stride, T, \
+                      H * D, G * D, G * Dv, page, eps, as_stream(stream))
+  if ((dtype == LV_MIX_BF16 && LVMIX_QKN(bf16_t)) || (dtype == LV_MIX_F32 && LVMIX_QKN(float))) return launched("lv_qk_fullnorm_store");
+#undef LVMIX_QKN
   if (dtype == LV_MIX_BF16)
     qk_fullnorm_store_kernel<bf16_t><<<grid, block, 0, as_stream(stream)>>>(
         static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k), static_cast<const bf16_t*>(v), ld,
@@ -288,6 +412,12 @@ int lv_pool_update(const void* k_cache, const void* v_cache, void* kp, void* vp,
   if (B < 0 || G <= 0 || D <= 0 || Dv <= 0 || page <= 0 || bt_stride <= 0) return fail(-1, "lv_pool_update: bad sizes");
   const int PP = (page + P - 1) / P;
   dim3 grid(max_new_blocks, B), block(256);
+#define LVMIX_POOL(TT)                                                                                                        \
+  pool_update_vec<TT>(static_cast<const TT*>(k_cache), static_cast<const TT*>(v_cache), static_cast<TT*>(kp),                 \
+                      static_cast<TT*>(vp), cu_q, ctx_lens, block_tables, bt_stride, B, max_new_blocks, G * D, G * Dv, page, P, \
+                      PP, as_stream(stream))
+  if ((dtype == LV_MIX_BF16 && LVMIX_POOL(bf16_t)) || (dtype == LV_MIX_F32 && LVMIX_POOL(float))) return launched("lv_pool_update");
+#undef LVMIX_POOL
   if (dtype == LV_MIX_BF16)
     pool_update_kernel<bf16_t><<<grid, block, 0, as_stream(stream)>>>(
         static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache), static_cast<bf16_t*>(kp),
