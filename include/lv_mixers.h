@@ -207,7 +207,8 @@ int lv_latent_prep(const void* proj, int64_t ld, int off_q, int off_kv, const vo
                    int rot_dims, int page, float eps, int dtype, void* stream);
 
 /* Latent attention, step 2. q act [T, H, Dn + Dr] (the rotated part last), q_lat act [H, T, R] (the unrotated part
- * already multiplied into the latent space).  q_out act [T, H, R + Dr] = q_lat | rotate(q[.., Dn:], position). */
+ * already multiplied into the latent space).  q_out act [T, H, R + Dr] = q_lat | rotate(q[.., Dn:], position). q_lat NULL: the
+ * first R entries are in q_out already, the rotated ones are put behind them. */
 int lv_latent_q_finish(const void* q, const void* q_lat, const void* inv_freq, void* q_out, const int32_t* cu_q,
                        const int32_t* ctx_lens, const int32_t* tok_seq, int64_t T, int H, int Dn, int Dr, int R,
                        int rot_dims, int dtype, void* stream);

@@ -100,9 +100,50 @@ __global__ __launch_bounds__(256) void latent_q_finish_kernel(const T* __restric
   for (int i = threadIdx.x; i < H * Dk; i += blockDim.x) {
     const int h = i / Dk, c = i - h * Dk;
     T* dst = q_out + (t * H + h) * Dk + c;
+    if (c < R && q_lat == nullptr) continue;      // already there
     if (c < R) *dst = q_lat[(static_cast<int64_t>(h) * Tn + t) * R + c];
     else stf(dst, rotated(q + (t * H + h) * (Dn + Dr) + Dn, c - R, half, cs));
   }
+}
+
+// The rotated parts alone, where the absorbed parts already lie in q_out (q_lat NULL): four entries a lane. 16 x 1024 tokens, 16
+// heads of 192 + 64: 142 us for the join above, two bytes a lane, 27 us for this with the product written in place.
+template <typename T>
+__global__ __launch_bounds__(256) void latent_q_rotate_kernel(const T* __restrict__ q, const float* __restrict__ inv_freq,
+                                                              T* __restrict__ q_out, const int32_t* __restrict__ cu_q,
+                                                              const int32_t* __restrict__ ctx_lens,
+                                                              const int32_t* __restrict__ tok_seq, int H, int Dn, int Dr, int R,
+                                                              int rot_dims) {
+  extern __shared__ __attribute__((aligned(16))) float cs[];
+  const int64_t t = blockIdx.x;
+  const int half = rot_dims / 2, b = tok_seq[t], per = Dr / 4;
+  fill_angles(cs, inv_freq, half, ctx_lens[b] + static_cast<int>(t) - cu_q[b]);
+  __syncthreads();
+  for (int x = threadIdx.x; x < H * per; x += blockDim.x) {
+    const int h = x / per, j = 4 * (x - h * per);
+    const T* src = q + (t * H + h) * (Dn + Dr) + Dn;
+    float4 v = ld4(src + j);
+    if (j < rot_dims) {                            // (half is a multiple of four: the partners lie side by side too)
+      const bool lead = j < half;
+      const int i = lead ? j : j - half;
+      const float4 u = ld4(src + (lead ? j + half : j - half)), c = ld4(cs + i), s = ld4(cs + half + i);
+      v = lead ? float4{v.x * c.x - u.x * s.x, v.y * c.y - u.y * s.y, v.z * c.z - u.z * s.z, v.w * c.w - u.w * s.w}
+               : float4{v.x * c.x + u.x * s.x, v.y * c.y + u.y * s.y, v.z * c.z + u.z * s.z, v.w * c.w + u.w * s.w};
+    }
+    st4(q_out + (t * H + h) * (R + Dr) + R + j, v);
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void latent_out_gate_vec_kernel(const T* __restrict__ o, const T* __restrict__ gate,
+                                                                  int64_t ld_gate, T* __restrict__ out, int64_t Tn, int H, int Dv) {
+  const int per = H * Dv / 4;
+  const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (idx >= Tn * per) return;
+  const int64_t t = idx / per;
+  const int c = static_cast<int>(idx - t * per) * 4, h = c / Dv;
+  const float4 g = ld4(gate + t * ld_gate + c), x = ld4(o + (static_cast<int64_t>(h) * Tn + t) * Dv + (c - h * Dv));
+  st4(out + t * (H * Dv) + c, float4{x.x * sigmoidf_(g.x), x.y * sigmoidf_(g.y), x.z * sigmoidf_(g.z), x.w * sigmoidf_(g.w)});
 }
 
 template <typename T>
@@ -308,12 +349,26 @@ int lv_latent_q_finish(const void* q, const void* q_lat, const void* inv_freq, v
                        const int32_t* ctx_lens, const int32_t* tok_seq, int64_t T, int H, int Dn, int Dr, int R,
                        int rot_dims, int dtype, void* stream) {
   if (T == 0) return 0;
-  if (!q || !q_lat || !q_out || !cu_q || !ctx_lens || !tok_seq) return fail(-1, "lv_latent_q_finish: null pointer");
+  if (!q || !q_out || !cu_q || !ctx_lens || !tok_seq) return fail(-1, "lv_latent_q_finish: null pointer");
   if (T < 0 || H <= 0 || Dn <= 0 || Dr < 0 || R <= 0 || rot_dims < 0 || rot_dims > Dr || rot_dims % 2 != 0 ||
       (rot_dims > 0 && !inv_freq))
     return fail(-1, "lv_latent_q_finish: bad sizes");
+  if (q_lat == nullptr && Dr == 0) return 0;
   const size_t shm = sizeof(float) * static_cast<size_t>(rot_dims > 0 ? rot_dims : 1);
   dim3 grid(static_cast<unsigned>(T)), block(256);
+  const uintptr_t piece = dtype == LV_MIX_BF16 ? 8 : 16;
+  if (q_lat == nullptr && Dn % 4 == 0 && Dr % 4 == 0 && R % 4 == 0 && rot_dims % 8 == 0 && reinterpret_cast<uintptr_t>(q) % piece == 0 &&
+      reinterpret_cast<uintptr_t>(q_out) % piece == 0 && (dtype == LV_MIX_BF16 || dtype == LV_MIX_F32)) {
+    if (dtype == LV_MIX_BF16)
+      latent_q_rotate_kernel<bf16_t><<<grid, block, shm, as_stream(stream)>>>(
+          static_cast<const bf16_t*>(q), static_cast<const float*>(inv_freq), static_cast<bf16_t*>(q_out), cu_q, ctx_lens, tok_seq, H, Dn,
+          Dr, R, rot_dims);
+    else
+      latent_q_rotate_kernel<float><<<grid, block, shm, as_stream(stream)>>>(
+          static_cast<const float*>(q), static_cast<const float*>(inv_freq), static_cast<float*>(q_out), cu_q, ctx_lens, tok_seq, H, Dn,
+          Dr, R, rot_dims);
+    return launched("lv_latent_q_finish");
+  }
   if (dtype == LV_MIX_BF16)
     latent_q_finish_kernel<bf16_t><<<grid, block, shm, as_stream(stream)>>>(
         static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(q_lat), static_cast<const float*>(inv_freq),
@@ -336,6 +391,18 @@ int lv_latent_out_gate(const void* o, const void* gate, int64_t ld_gate, int gat
     return fail(-1, "lv_latent_out_gate: bad arguments");
   const int64_t n = T * H * Dv;
   dim3 grid(static_cast<unsigned>((n + 255) / 256)), block(256);
+  const uintptr_t piece = dtype == LV_MIX_BF16 ? 8 : 16;
+  auto at = [piece](const void* x) { return reinterpret_cast<uintptr_t>(x) % piece == 0; };
+  if (per_channel && Dv % 4 == 0 && ld_gate % 4 == 0 && at(o) && at(gate) && at(out) && (dtype == LV_MIX_BF16 || dtype == LV_MIX_F32)) {
+    dim3 vgrid(static_cast<unsigned>((n / 4 + 255) / 256));
+    if (dtype == LV_MIX_BF16)
+      latent_out_gate_vec_kernel<bf16_t><<<vgrid, block, 0, as_stream(stream)>>>(
+          static_cast<const bf16_t*>(o), static_cast<const bf16_t*>(gate), ld_gate, static_cast<bf16_t*>(out), T, H, Dv);
+    else
+      latent_out_gate_vec_kernel<float><<<vgrid, block, 0, as_stream(stream)>>>(
+          static_cast<const float*>(o), static_cast<const float*>(gate), ld_gate, static_cast<float*>(out), T, H, Dv);
+    return launched("lv_latent_out_gate");
+  }
   if (dtype == LV_MIX_BF16)
     latent_out_gate_kernel<bf16_t><<<grid, block, 0, as_stream(stream)>>>(
         static_cast<const bf16_t*>(o), static_cast<const bf16_t*>(gate), ld_gate, per_channel, static_cast<bf16_t*>(out), T, H, Dv);

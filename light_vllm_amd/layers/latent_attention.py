@@ -89,11 +89,11 @@ class LatentAttention(nn.Module):
         self.inv_freq = mix_ops.rotary_inv_freq(max(self.rot_dims, 2), self.rot_base, device, self.rot_scaling)
         self.magnitude = mix_ops.rotary_magnitude(self.rot_scaling)
 
-    def _attend(self, q_abs: torch.Tensor, step) -> torch.Tensor:
-        """Per-head weighted sums of the cached latents, [T, H * R]."""
+    def _attend(self, q_abs: torch.Tensor, step, gate: torch.Tensor | None = None) -> torch.Tensor:
+        """Per-head weighted sums of the cached latents, [T, H * R], times the sigmoid of one gate per head."""
         rows = self.cache.unsqueeze(2)                                                              # [pages, page, 1, R + Dr]
-        return mix_ops.window_pool_attention(q_abs, rows, rows[..., :self.R], None, None, None, step, self.H, 1, self.R + self.Dr,
-                                             self.R, self.window, 0, self.scale, has_sink=False, sinks=self.sink)
+        return mix_ops.window_pool_attention(q_abs, rows, rows[..., :self.R], None, None, gate, step, self.H, 1, self.R + self.Dr,
+                                             self.R, self.window, 0, self.scale, has_sink=False, gate_per_head=True, sinks=self.sink)
 
     def forward(self, h: torch.Tensor, proj: torch.Tensor | None = None, col0: int = 0, out: torch.Tensor | None = None) -> torch.Tensor:
         """proj, col0: a projection of h computed by the caller whose columns from col0 on are this mixer's. A fused module writes
@@ -106,12 +106,22 @@ class LatentAttention(nn.Module):
         cq = mix_ops.latent_prep(proj, 0, self.Rq, self.q_norm_weight, self.kv_norm_weight, self.inv_freq, self.cache,
                                  step, self.Rq, R, Dr, self.rot_dims, self.norm_eps)
         q = self.uq(cq)
-        q_lat = torch.bmm(q.view(T, H, Dn + Dr)[:, :, :Dn].transpose(0, 1), self.uk)              # [H, T, R]
-        q_abs = mix_ops.latent_q_finish(q, q_lat, self.inv_freq, step, H, Dn, Dr, R, self.rot_dims)
-        o_lat = self._attend(q_abs, step)
-        o = torch.bmm(o_lat.view(T, H, R).transpose(0, 1), self.uv)                                 # [H, T, Dv]
         gate = proj[:, self.sizes[0] + self.sizes[1]:]
-        return self.o_proj(mix_ops.latent_out_gate(o, gate, self.gate_per_channel))
+        with torch.no_grad():           # the kernels between them carry no gradient, and `out` may not ask for one
+            # both batched products write where the next step reads; a gate per head goes on the sum that the value matrix
+            # multiplies (the same product), in the attention kernel
+            q_abs = torch.empty(T, H, R + Dr, dtype=h.dtype, device=h.device)
+            torch.bmm(q.view(T, H, Dn + Dr)[:, :, :Dn].transpose(0, 1), self.uk, out=q_abs[:, :, :R].transpose(0, 1))
+            if Dr > 0:
+                mix_ops.latent_q_finish(q, None, self.inv_freq, step, H, Dn, Dr, R, self.rot_dims, out=q_abs.view(T, H * (R + Dr)))
+            if self.gate_per_channel:
+                o = torch.bmm(self._attend(q_abs.view(T, H * (R + Dr)), step).view(T, H, R).transpose(0, 1), self.uv)   # [H, T, Dv]
+                o = mix_ops.latent_out_gate(o, gate, True)
+            else:
+                o_lat = self._attend(q_abs.view(T, H * (R + Dr)), step, gate)
+                o = torch.empty(T, H * self.Dv, dtype=h.dtype, device=h.device)
+                torch.bmm(o_lat.view(T, H, R).transpose(0, 1), self.uv, out=o.view(T, H, self.Dv).transpose(0, 1))
+        return self.o_proj(o)
 
     def _forward_direct(self, h, step, proj, col0, out):
         T, H, R, Dn, Dr = h.size(0), self.H, self.R, self.Dn, self.Dr

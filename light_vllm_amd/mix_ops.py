@@ -793,12 +793,14 @@ def head_norm_store(proj, off_q, off_k, q_w, cache, key_scale, step, H, G, D, ep
     return q_out
 
 
-def latent_q_finish(q, q_lat, inv_freq, step, H, Dn, Dr, R, rot_dims):
+def latent_q_finish(q, q_lat, inv_freq, step, H, Dn, Dr, R, rot_dims, out=None):
     """q [T, H*(Dn+Dr)] (per head: Dn unrotated entries, then Dr to rotate), q_lat [H, T, R] (the unrotated
-    part multiplied into the latent space) -> [T, H*(R+Dr)] = per head [q_lat | rotated part]."""
+    part multiplied into the latent space) -> [T, H*(R+Dr)] = per head [q_lat | rotated part]. q_lat None: the product is in
+    `out` already, the rotated parts are put beside it."""
     T = q.size(0)
-    out = torch.empty(T, H * (R + Dr), dtype=q.dtype, device=q.device)
-    assert q.is_contiguous() and q_lat.is_contiguous() and q_lat.shape == (H, T, R)
+    if out is None:
+        out = torch.empty(T, H * (R + Dr), dtype=q.dtype, device=q.device)
+    assert q.is_contiguous() and out.is_contiguous() and (q_lat is None or (q_lat.is_contiguous() and q_lat.shape == (H, T, R)))
     if q.is_cuda:
         _f32(inv_freq)
         lib = _mixlib.load()
@@ -807,7 +809,8 @@ def latent_q_finish(q, q_lat, inv_freq, step, H, Dn, Dr, R, rot_dims):
                       "lv_latent_q_finish")
         return out
     o = out.view(T, H, R + Dr)
-    o[:, :, :R] = q_lat.transpose(0, 1)
+    if q_lat is not None:
+        o[:, :, :R] = q_lat.transpose(0, 1)
     if Dr:
         qr = q.view(T, H, Dn + Dr)[:, :, Dn:].float()
         o[:, :, R:] = _rotate(qr, _positions(step, q.device), inv_freq, rot_dims).to(q.dtype)
