@@ -60,6 +60,13 @@ SIGNATURES = {
     "lv_comm_destroy": (c_int, [c_void_p]),
 }
 
+# include/lv_decode_store.h
+STORE_SIGNATURES = {
+    "lv_decode_attn_store": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p,
+                                     c_int64, c_int64, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float,
+                                     c_void_p, c_size_t, c_int, c_void_p, c_int, c_void_p]),
+}
+
 _lib = None
 
 
@@ -74,7 +81,7 @@ def load() -> ctypes.CDLL:
             f"{LIB_PATH} not found: build it with `python -c 'import __graft_entry__ as g; g.build()'` "
             "or `make -C light_vllm_amd/csrc` (hipcc --offload-arch=gfx950). There is no fallback path.")
     lib = ctypes.CDLL(LIB_PATH)
-    for name, (res, args) in SIGNATURES.items():
+    for name, (res, args) in {**SIGNATURES, **STORE_SIGNATURES}.items():
         fn = getattr(lib, name)  # AttributeError if the symbol is missing
         fn.restype = res
         fn.argtypes = args

@@ -7,6 +7,7 @@
 #include <mutex>
 
 #include "lv_kernels.h"
+#include "lv_decode_store.h"
 
 namespace lv {
 
@@ -41,6 +42,17 @@ constexpr int kSaturatedUnits = 1024;     // (sequence, kv head) pairs that fill
 //            sequences never gain from a cut (-3 ... -8 %) - but no such split under 512 tokens.
 // The larger of the two, never below the kernel's 64-token split unit. Within 4 % of the best
 // count on every shape of the sweeps (the first rule, 1024 workgroups always: up to 30 % off).
+// Where the caller leaves the choice to the library, one pass on eight waves a workgroup takes the place of a
+// cut that would fill the chip, because the cut costs a merge launch: contexts of one block, and shapes that already give most
+// compute units a workgroup and short ones. A compute unit streams about 30 GB/s from memory, so longer contexts on few
+// workgroups stay cut. A layer's store and attention from a replayed graph, us, cut against one pass (16q/8kv): 1 x 64 tokens
+// 7.9 / 5.2; 24 x 1000 25.6 / 22.0; 31 x 900 28.6 / 25.4; but 1 x 1000 8.3 / 16.9 and 16 x 500 17.1 / 18.1, which stay cut.
+constexpr int64_t kWideTokens = 256, kWideFullTokens = 1024, kWideFullUnits = 160, kWideBelow = 256;
+static bool decode_wide(int batch, int num_kv_heads, int max_blocks_per_seq, int block_size) {
+  const int64_t units = static_cast<int64_t>(batch) * num_kv_heads, tokens = static_cast<int64_t>(max_blocks_per_seq) * block_size;
+  return units < kWideBelow && (tokens <= kWideTokens || (tokens <= kWideFullTokens && units >= kWideFullUnits));
+}
+
 static int heuristic_splits(int batch, int num_kv_heads, int max_blocks_per_seq, int block_size) {
   const int64_t units = static_cast<int64_t>(batch) * num_kv_heads;
   if (units <= 0 || max_blocks_per_seq <= 0) return 1;
@@ -406,6 +418,12 @@ size_t lv_decode_workspace_bytes(int batch, int num_heads, int head_dim, int num
 
 // Shared body of lv_decode_attn and lv_decode_attn_static. `static_scratch`: the workspace is the
 // library's own device array, resolved (once per device) only when the call needs splits.
+struct NewRows {
+  const void *key = nullptr, *value = nullptr;
+  int64_t key_stride0 = 0, value_stride0 = 0;
+  const int32_t* slot_mapping = nullptr;
+  int64_t num_slots = 0;
+};
 static int decode_entry(const void* q, const void* k_cache, const void* v_cache, void* o,
                         int64_t q_stride0, int64_t o_stride0, const int32_t* context_lens,
                         const int32_t* block_table, int block_table_stride, int batch,
@@ -413,7 +431,7 @@ static int decode_entry(const void* q, const void* k_cache, const void* v_cache,
                         int head_dim, float scale, void* workspace, size_t workspace_bytes,
                         bool static_scratch, int num_splits, const int32_t* seq_order,
                         const int32_t* work_items, int num_work_items, const int32_t* seq_splits,
-                        int kernel_hint, lv_stream_t stream) {
+                        int kernel_hint, lv_stream_t stream, const NewRows& fresh = NewRows{}) {
   if (batch < 0 || max_blocks_per_seq < 0 || num_heads <= 0 || num_kv_heads <= 0 || num_splits < 0)
     return fail(LV_ERR_INVALID_ARGUMENT, "decode: negative size");
   if (head_dim != kHeadDim) return fail(LV_ERR_UNSUPPORTED, "decode: head_dim %d != 128", head_dim);
@@ -442,7 +460,8 @@ static int decode_entry(const void* q, const void* k_cache, const void* v_cache,
   if (q_stride0 % 8 != 0 || o_stride0 % 8 != 0 || !aligned16(q) || !aligned16(o) ||
       !aligned16(k_cache) || !aligned16(v_cache))
     return fail(LV_ERR_UNSUPPORTED, "decode: q/o/caches must be 16-byte aligned with strides %% 8 == 0");
-  int nsplit = num_splits == 0 ? heuristic_splits(batch, num_kv_heads, max_blocks_per_seq, block_size) : num_splits;
+  const bool wide = num_splits == 0 && decode_wide(batch, num_kv_heads, max_blocks_per_seq, block_size);
+  int nsplit = num_splits != 0 ? num_splits : (wide ? 1 : heuristic_splits(batch, num_kv_heads, max_blocks_per_seq, block_size));
   if (nsplit > kMaxSplits) return fail(LV_ERR_INVALID_ARGUMENT, "decode: num_splits %d > %d", nsplit, kMaxSplits);
   if (work_items) {
     // a work list: num_splits is the split capacity of a workspace row, the grid is the list's capacity
@@ -495,10 +514,37 @@ static int decode_entry(const void* q, const void* k_cache, const void* v_cache,
   p.nsplit = nsplit;
   p.kernel_hint = kernel_hint;
   p.scale_log2e = scale * kLog2e;
+  p.wide = wide;
+  p.k_new = static_cast<const uint16_t*>(fresh.key);
+  p.v_new = static_cast<const uint16_t*>(fresh.value);
+  p.k_new_stride0 = fresh.key_stride0;
+  p.v_new_stride0 = fresh.value_stride0;
+  p.slot_mapping = fresh.slot_mapping;
+  p.num_slots = fresh.num_slots;
   return launch_decode_attn(p, static_cast<hipStream_t>(stream));
 }
 
 extern "C" {
+
+int lv_decode_attn_store(const void* q, const void* key, const void* value, int64_t key_stride0, int64_t value_stride0,
+                         void* k_cache, void* v_cache, const int32_t* slot_mapping, int64_t num_slots, void* o, int64_t q_stride0,
+                         int64_t o_stride0, const int32_t* context_lens, const int32_t* block_table, int block_table_stride, int batch,
+                         int max_blocks_per_seq, int block_size, int num_heads, int num_kv_heads, int head_dim, float scale,
+                         void* workspace, size_t workspace_bytes, int num_splits, const int32_t* seq_order, int kernel_hint,
+                         lv_stream_t stream) {
+  if (batch == 0) return LV_OK;
+  if (num_slots < 0 || num_kv_heads <= 0 || head_dim <= 0) return fail(LV_ERR_INVALID_ARGUMENT, "decode_store: negative size");
+  if (!key || !value || !slot_mapping) return fail(LV_ERR_INVALID_ARGUMENT, "decode_store: null pointer");
+  const int64_t row = static_cast<int64_t>(num_kv_heads) * head_dim;
+  if (key_stride0 < row || value_stride0 < row)
+    return fail(LV_ERR_INVALID_ARGUMENT, "decode_store: row stride smaller than num_kv_heads*head_dim");
+  if (key_stride0 % 8 != 0 || value_stride0 % 8 != 0 || !aligned16(key) || !aligned16(value))
+    return fail(LV_ERR_UNSUPPORTED, "decode_store: key and value must be 16-byte aligned with strides %% 8 == 0");
+  return decode_entry(q, k_cache, v_cache, o, q_stride0, o_stride0, context_lens, block_table, block_table_stride, batch,
+                      max_blocks_per_seq, block_size, num_heads, num_kv_heads, head_dim, scale, workspace, workspace_bytes, false,
+                      num_splits, seq_order, nullptr, 0, nullptr, kernel_hint, stream,
+                      NewRows{key, value, key_stride0, value_stride0, slot_mapping, num_slots});
+}
 
 int lv_decode_attn(const void* q, const void* k_cache, const void* v_cache, void* o,
                    int64_t q_stride0, int64_t o_stride0, const int32_t* context_lens,

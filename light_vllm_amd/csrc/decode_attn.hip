@@ -105,8 +105,44 @@ __device__ __forceinline__ bool decode_work(const DecodeParams& p, DecodeWork& w
          w.nsplit <= p.nsplit && w.split < w.nsplit;
 }
 
-template <int G, int U, bool NT>
-__global__ __launch_bounds__(256) void decode_attn_kernel(const DecodeParams p) {
+// STORE launches bring this step's key and value rows along. The workgroup that owns a sequence's last token writes its kv head's
+// two rows (256 bytes each) to the caches at slot_mapping[b], as store_kvcache does, and where that slot is the last token's own
+// place takes the rows from the inputs instead of reading back what it has just written. A slot elsewhere, or none
+// (negative, out of range), changes nothing about what is read.
+// The slot and the last token's place are requested with the kernel's first loads and compared where the last chunk is loaded;
+// the rows are written behind the loop: nothing at the start waits for them. (With the comparison up front the 256 x 1024 launch at
+// 32q/8kv took 182 us instead of 171.) What it saves is the store's launch, about 1.5 us in a replayed graph: with the rule on
+// splits (api.hip) a layer's step at 4 x 512 ragged tokens, 16q/8kv, went from 11.3 to 9.7 us, 1 x 64 from 9.1 to 5.2,
+// 128 x 100 at 8q/1kv from 12.3 to 8.3; 256 x 1024 stays at 171.
+struct NewRow {
+  int64_t slot = -1, place = -2;
+  bool write = false;
+  __device__ __forceinline__ bool own() const { return slot == place; }
+};
+__device__ __forceinline__ NewRow new_row(const DecodeParams& p, const DecodeWork& w, int ctx, int t1) {
+  NewRow r;
+  if (t1 != ctx || (ctx == 0 && w.split + 1 != w.nsplit)) return r;
+  r.slot = p.slot_mapping[w.b];
+  r.write = true;
+  if (ctx > 0) {
+    const int last = ctx - 1;
+    r.place = static_cast<int64_t>(p.block_table[static_cast<int64_t>(w.b) * p.bt_stride + last / p.block_size]) * p.block_size +
+              last % p.block_size;
+  }
+  return r;
+}
+__device__ __forceinline__ void write_row(const DecodeParams& p, const DecodeWork& w, const NewRow& r) {
+  constexpr int c = kHeadDim / 8;
+  const int tid = threadIdx.x, at = w.kvh * kHeadDim + 8 * (tid % c);
+  if (!r.write || r.slot < 0 || r.slot >= p.num_slots || tid >= 2 * c) return;
+  const uint16_t* src = tid >= c ? p.v_new + w.b * p.v_new_stride0 : p.k_new + w.b * p.k_new_stride0;
+  uint16_t* cache = const_cast<uint16_t*>(tid >= c ? p.v_cache : p.k_cache);
+  *reinterpret_cast<u32x4*>(cache + r.slot * p.num_kv_heads * kHeadDim + at) = *reinterpret_cast<const u32x4*>(src + at);
+}
+
+// NW waves: 4, or 8 (see launch_group).
+template <int G, int U, bool NT, int NW, bool STORE>
+__global__ __launch_bounds__(64 * NW) void decode_attn_kernel(const DecodeParams p) {
   constexpr int TOK = 4 * U;  // tokens per wave chunk
   const int Hkv = p.num_kv_heads;
   // Workgroup order: split fastest, then sequence, kv head slowest, so the 8 heads of one token
@@ -137,6 +173,13 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(const DecodeParams p) 
 
   const int64_t row_elems = static_cast<int64_t>(Hkv) * kHeadDim;
   const int32_t* bt_row = p.block_table + static_cast<int64_t>(b) * p.bt_stride;
+  NewRow fresh;
+  const uint16_t *k_own = nullptr, *v_own = nullptr;
+  if constexpr (STORE) {
+    fresh = new_row(p, dw, ctx, t1);
+    k_own = p.k_new + b * p.k_new_stride0 + kvh * kHeadDim + 8 * i;
+    v_own = p.v_new + b * p.v_new_stride0 + kvh * kHeadDim + 8 * i;
+  }
 
   // q fragments: 8 dims of each of the G heads, kept packed as bf16 pairs.
   u32x4 qv[G];
@@ -168,19 +211,28 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(const DecodeParams p) 
     const int last = ntok - 1 - c * TOK;
     return min(4 * u + g, last);
   };
+  // The U rows of chunk c; in the split's last chunk the lanes at its last token look at the step's own row.
+  auto load_rows = [&](u32x4 (&to)[U], const uint16_t* cache, const uint16_t* own_row, int c, int64_t base) __attribute__((always_inline)) {
+    if (STORE && c == nchunks - 1 && fresh.own()) {
+      const int last = ntok - 1 - c * TOK;
+#pragma unroll
+      for (int u = 0; u < U; ++u) to[u] = load16<NT>(4 * u + g >= last ? own_row : cache + base + tok_off(c, u) * row_elems);
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) to[u] = load16<NT>(cache + base + tok_off(c, u) * row_elems);
+    }
+  };
 
   int c = wave;
   if (c < nchunks) {
     u32x4 kb[U], vb[U];
     {
       const int64_t base = chunk_base(c);
-#pragma unroll
-      for (int u = 0; u < U; ++u) kb[u] = load16<NT>(p.k_cache + base + tok_off(c, u) * row_elems);
-#pragma unroll
-      for (int u = 0; u < U; ++u) vb[u] = load16<NT>(p.v_cache + base + tok_off(c, u) * row_elems);
+      load_rows(kb, p.k_cache, k_own, c, base);
+      load_rows(vb, p.v_cache, v_own, c, base);
     }
-    for (; c < nchunks; c += 4) {
-      const int cn = c + 4;
+    for (; c < nchunks; c += NW) {
+      const int cn = c + NW;
       const bool has_next = cn < nchunks;
       int64_t base_n = 0;
       if (has_next) base_n = chunk_base(cn);
@@ -203,11 +255,7 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(const DecodeParams p) 
           s[u][h] = d;
         }
       }
-      if (has_next) {
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-          kb[u] = load16<NT>(p.k_cache + base_n + tok_off(cn, u) * row_elems);
-      }
+      if (has_next) load_rows(kb, p.k_cache, k_own, cn, base_n);
       const int valid = ntok - c * TOK;  // tokens of this chunk inside the split
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -260,13 +308,11 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(const DecodeParams p) 
           for (int h = 0; h < G; ++h) acc[h][u & 7] = fmaf(s[u][h], vx, acc[h][u & 7]);
         }
       }
-      if (has_next) {
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-          vb[u] = load16<NT>(p.v_cache + base_n + tok_off(cn, u) * row_elems);
-      }
+      if (has_next) load_rows(vb, p.v_cache, v_own, cn, base_n);
     }
   }
+
+  if constexpr (STORE) write_row(p, dw, fresh);
 
   // ---- merge the 4 token groups of the wave (lanes ^16, ^32)
 #pragma unroll
@@ -289,9 +335,9 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(const DecodeParams p) 
     }
   }
 
-  // ---- merge the 4 waves through LDS
-  __shared__ float sm_acc[4][G][kHeadDim];
-  __shared__ float sm_ml[4][G][2];
+  // ---- merge the waves through LDS
+  __shared__ float sm_acc[NW][G][kHeadDim];
+  __shared__ float sm_ml[NW][G][2];
   if (g == 0) {
 #pragma unroll
     for (int h = 0; h < G; ++h) {
@@ -306,16 +352,16 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(const DecodeParams p) 
   }
   __syncthreads();
 
-  for (int e = tid; e < G * kHeadDim; e += 256) {
+  for (int e = tid; e < G * kHeadDim; e += 64 * NW) {
     const int h = e / kHeadDim;
     const int d = e % kHeadDim;
     float M = sm_ml[0][h][0];
 #pragma unroll
-    for (int w = 1; w < 4; ++w) M = fmaxf(M, sm_ml[w][h][0]);
+    for (int w = 1; w < NW; ++w) M = fmaxf(M, sm_ml[w][h][0]);
     const float Mu = (M == -INFINITY) ? 0.f : M;
     float val = 0.f, L = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < NW; ++w) {
       const float sc = fast_exp2(sm_ml[w][h][0] - Mu);
       val += sc * sm_acc[w][h][d];
       L += sc * sm_ml[w][h][1];
@@ -359,12 +405,12 @@ __device__ __forceinline__ int v_lds_off(int row, int ch) {  // [rows][128 x bf1
   return 256 * row + 16 * (ch ^ (((row & 3) << 2) | ((row >> 2) & 3)));
 }
 
-template <int G>
-__global__ __launch_bounds__(256, 2) void decode_mfma_kernel(const DecodeParams p) {
+template <int G, int NW, bool STORE>
+__global__ __launch_bounds__(64 * NW, 2) void decode_mfma_kernel(const DecodeParams p) {
   constexpr int CH = 32;  // keys per wave chunk
   constexpr float kDefer = 6.0f;  // running max moves only when a row outgrows it by 2^6
   // per wave: 8 KiB V image during the sweep; afterwards per wave G x (128 + 2) floats of partials
-  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * 8192];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[NW * 8192];
   lds_byte_t* const lds3 = (lds_byte_t*)lds;
 
   const int Hkv = p.num_kv_heads;
@@ -389,6 +435,13 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(const DecodeParams 
   const int nchunks = ntok > 0 ? (ntok + CH - 1) / CH : 0;
   const int64_t row_bytes = static_cast<int64_t>(Hkv) * kHeadDim * 2;
   const int32_t* bt_row = p.block_table + static_cast<int64_t>(b) * p.bt_stride;
+  NewRow fresh;
+  const char *k_own = nullptr, *v_own = nullptr;
+  if constexpr (STORE) {
+    fresh = new_row(p, dw, ctx, t1);
+    k_own = reinterpret_cast<const char*>(p.k_new + b * p.k_new_stride0 + kvh * kHeadDim) + 16 * q;
+    v_own = reinterpret_cast<const char*>(p.v_new + b * p.v_new_stride0 + kvh * kHeadDim) + 16 * c16;
+  }
 
   // Q^T fragments (B operand), k-step s covers d = 32s .. 32s+31; heads >= G are zero columns
   bf16x8_t qf[4];
@@ -433,9 +486,11 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(const DecodeParams 
   auto issue_k = [&](int c) {
     const char* base = reinterpret_cast<const char*>(p.k_cache) + chunk_row(c) * row_bytes + kvh * (kHeadDim * 2);
     const int last = ntok - 1 - c * CH;  // rows past the split's end re-read its last row (masked below)
+    const bool own = STORE && c == nchunks - 1 && fresh.own();
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const char* rp = base + static_cast<int64_t>(min(16 * t + a_key, last)) * row_bytes + 16 * q;
+      if (STORE && own && 16 * t + a_key >= last) rp = k_own;
 #pragma unroll
       for (int s = 0; s < 4; ++s) kreg[t][s] = load16<true>(reinterpret_cast<const uint16_t*>(rp + 64 * s));
     }
@@ -443,9 +498,13 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(const DecodeParams 
   auto issue_v = [&](int c) {
     const char* base = reinterpret_cast<const char*>(p.v_cache) + chunk_row(c) * row_bytes + kvh * (kHeadDim * 2) + 16 * c16;
     const int last = ntok - 1 - c * CH;
+    const bool own = STORE && c == nchunks - 1 && fresh.own();
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-      vreg[u] = load16<true>(reinterpret_cast<const uint16_t*>(base + static_cast<int64_t>(min(4 * u + q, last)) * row_bytes));
+    for (int u = 0; u < 8; ++u) {
+      const char* rp = base + static_cast<int64_t>(min(4 * u + q, last)) * row_bytes;
+      if (STORE && own && 4 * u + q >= last) rp = v_own;
+      vreg[u] = load16<true>(reinterpret_cast<const uint16_t*>(rp));
+    }
   };
 
   int c = wave;
@@ -453,8 +512,8 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(const DecodeParams 
     issue_k(c);
     issue_v(c);
   }
-  for (; c < nchunks; c += 4) {
-    const int cn = c + 4;
+  for (; c < nchunks; c += NW) {
+    const int cn = c + NW;
     // ---- S^T = K Q^T for the two 16-key tiles
     f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -517,11 +576,13 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(const DecodeParams 
     }
   }
 
+  if constexpr (STORE) write_row(p, dw, fresh);
+
   // ---- row sums: every 16-lane group holds a share
   l_run += __shfl_xor(l_run, 16);
   l_run += __shfl_xor(l_run, 32);
 
-  // ---- merge the 4 waves through LDS: per wave [G][128] partial outputs + (m, l)
+  // ---- merge the waves through LDS: per wave [G][128] partial outputs + (m, l)
   __syncthreads();   // all waves are done with their V images
   float* const part = reinterpret_cast<float*>(lds);
   constexpr int kPartStride = G * kHeadDim + 2 * G;  // floats per wave
@@ -536,16 +597,16 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(const DecodeParams 
     }
   }
   __syncthreads();
-  for (int e = tid; e < G * kHeadDim; e += 256) {
+  for (int e = tid; e < G * kHeadDim; e += 64 * NW) {
     const int h = e / kHeadDim;
     const int d = e % kHeadDim;
     float M = part[G * kHeadDim + 2 * h];
 #pragma unroll
-    for (int w = 1; w < 4; ++w) M = fmaxf(M, part[w * kPartStride + G * kHeadDim + 2 * h]);
+    for (int w = 1; w < NW; ++w) M = fmaxf(M, part[w * kPartStride + G * kHeadDim + 2 * h]);
     const float Mu = (M == -INFINITY) ? 0.f : M;
     float val = 0.f, L = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < NW; ++w) {
       const float f = fast_exp2(part[w * kPartStride + G * kHeadDim + 2 * h] - Mu);
       val += f * part[w * kPartStride + h * kHeadDim + d];
       L += f * part[w * kPartStride + G * kHeadDim + 2 * h + 1];
@@ -665,36 +726,45 @@ static unsigned decode_grid(const DecodeParams& p) {
   return static_cast<unsigned>(p.batch) * p.num_kv_heads * p.nsplit;
 }
 
-template <int G, int U>
-static void launch_g(const DecodeParams& p, hipStream_t stream) {
-  hipLaunchKernelGGL((decode_attn_kernel<G, U, true>), dim3(decode_grid(p)), dim3(256), 0, stream, p);
+// wide: eight waves a workgroup instead of four, for launches in one pass on fewer workgroups than the chip has compute units: more
+// bytes in flight from each, and no second launch to merge splits (decode_wide in api.hip).
+template <int G, int U, bool STORE>
+static void launch_valu(const DecodeParams& p, bool wide, hipStream_t stream) {
+  if (wide) hipLaunchKernelGGL((decode_attn_kernel<G, U, true, 8, STORE>), dim3(decode_grid(p)), dim3(512), 0, stream, p);
+  else hipLaunchKernelGGL((decode_attn_kernel<G, U, true, 4, STORE>), dim3(decode_grid(p)), dim3(256), 0, stream, p);
 }
 
-template <int G>
-static void launch_mfma(const DecodeParams& p, hipStream_t stream) {
-  hipLaunchKernelGGL((decode_mfma_kernel<G>), dim3(decode_grid(p)), dim3(256), 0, stream, p);
+template <int G, bool STORE>
+static void launch_mfma(const DecodeParams& p, bool wide, hipStream_t stream) {
+  if (wide) hipLaunchKernelGGL((decode_mfma_kernel<G, 8, STORE>), dim3(decode_grid(p)), dim3(512), 0, stream, p);
+  else hipLaunchKernelGGL((decode_mfma_kernel<G, 4, STORE>), dim3(decode_grid(p)), dim3(256), 0, stream, p);
+}
+
+// Kernel choice: the matrix-core kernel for 4 and 8 query heads per kv head, the vector-ALU kernel for 1 and 2, unless the
+// caller's kernel_hint names one of them. Other group sizes (Qwen3-14B has 40 q / 8 kv heads = 5): the matrix-core kernel only,
+// its head dimension is a 16-column tile of which G columns are live.
+template <bool STORE>
+static bool launch_group(const DecodeParams& p, hipStream_t stream) {
+  const int G = p.num_heads / p.num_kv_heads;
+  const bool mfma = p.kernel_hint == LV_DECODE_KERNEL_MFMA || (p.kernel_hint == LV_DECODE_KERNEL_AUTO && G >= 4);
+  const bool wide = p.wide;
+  switch (G) {
+    case 1: if (mfma) launch_mfma<1, STORE>(p, wide, stream); else launch_valu<1, 8, STORE>(p, wide, stream); break;
+    case 2: if (mfma) launch_mfma<2, STORE>(p, wide, stream); else launch_valu<2, 8, STORE>(p, wide, stream); break;
+    case 4: if (mfma) launch_mfma<4, STORE>(p, wide, stream); else launch_valu<4, 4, STORE>(p, wide, stream); break;
+    case 8: if (mfma) launch_mfma<8, STORE>(p, wide, stream); else launch_valu<8, 4, STORE>(p, wide, stream); break;
+    case 3: launch_mfma<3, STORE>(p, wide, stream); break;
+    case 5: launch_mfma<5, STORE>(p, wide, stream); break;
+    case 6: launch_mfma<6, STORE>(p, wide, stream); break;
+    case 7: launch_mfma<7, STORE>(p, wide, stream); break;
+    default: return false;
+  }
+  return true;
 }
 
 int launch_decode_attn(const DecodeParams& p, hipStream_t stream) {
-  const int G = p.num_heads / p.num_kv_heads;
-  // Kernel choice: the matrix-core kernel for 4 and 8 query heads per kv head, the vector-ALU
-  // kernel for 1 and 2, unless the caller's kernel_hint names one of them.
-  const bool mfma = p.kernel_hint == LV_DECODE_KERNEL_MFMA ||
-                    (p.kernel_hint == LV_DECODE_KERNEL_AUTO && G >= 4);
-  switch (G) {
-    case 1: if (mfma) launch_mfma<1>(p, stream); else launch_g<1, 8>(p, stream); break;
-    case 2: if (mfma) launch_mfma<2>(p, stream); else launch_g<2, 8>(p, stream); break;
-    case 4: if (mfma) launch_mfma<4>(p, stream); else launch_g<4, 4>(p, stream); break;
-    case 8: if (mfma) launch_mfma<8>(p, stream); else launch_g<8, 4>(p, stream); break;
-    // other group sizes (Qwen3-14B has 40 q / 8 kv heads = 5): the matrix-core kernel only, its
-    // head dimension is a 16-column tile of which G columns are live
-    case 3: launch_mfma<3>(p, stream); break;
-    case 5: launch_mfma<5>(p, stream); break;
-    case 6: launch_mfma<6>(p, stream); break;
-    case 7: launch_mfma<7>(p, stream); break;
-    default:
-      return fail(LV_ERR_UNSUPPORTED, "decode: num_heads/num_kv_heads = %d not in 1..8", G);
-  }
+  if (!(p.k_new != nullptr ? launch_group<true>(p, stream) : launch_group<false>(p, stream)))
+    return fail(LV_ERR_UNSUPPORTED, "decode: num_heads/num_kv_heads = %d not in 1..8", p.num_heads / p.num_kv_heads);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(LV_ERR_LAUNCH, "decode_attn launch: %s", hipGetErrorString(e));
   if (p.nsplit > 1) {

@@ -22,6 +22,12 @@ struct DecodeParams {
   int bt_stride, batch, block_size, num_heads, num_kv_heads, nsplit;
   int kernel_hint;           // LV_DECODE_KERNEL_*
   float scale_log2e;
+  bool wide;                 // eight waves a workgroup (one pass, no work list)
+  // with k_new: this step's key and value rows, written to the caches at slot_mapping on the way
+  const uint16_t *k_new, *v_new;
+  int64_t k_new_stride0, v_new_stride0;
+  const int32_t* slot_mapping;
+  int64_t num_slots;
 };
 
 struct PrefillParams {

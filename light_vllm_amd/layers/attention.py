@@ -38,9 +38,10 @@ class Attention(nn.Module):
         context = get_context()
         k_cache, v_cache = self.k_cache, self.v_cache
 
-        # The store is stream-ordered before the attention launch below, so a prefix-cached
-        # prefill and every decode step read the rows written here (reference :149-150).
-        if not kv_stored and k_cache.numel() and v_cache.numel():
+        # A prefix-cached prefill and every decode step read the rows written here (reference :149-150): the store is
+        # stream-ordered before a prefill's attention launch, and rides in a decode step's.
+        store = not kv_stored and k_cache.numel() and v_cache.numel()
+        if store and context.is_prefill:
             store_kvcache(k, v, k_cache, v_cache, context.slot_mapping)
 
         if context.is_prefill:
@@ -52,5 +53,6 @@ class Attention(nn.Module):
         else:
             o = ops.decode_attention(q, k_cache, v_cache, context.context_lens,
                                      context.block_tables, self.scale, seq_order=context.seq_order,
-                                     plan=context.decode_plan)
+                                     plan=context.decode_plan,
+                                     new_kv=(k, v, context.slot_mapping) if store else None)
         return o.view(-1, self.num_heads * self.head_dim)

@@ -99,6 +99,18 @@ def _require_gpu(*tensors: torch.Tensor) -> torch.device:
     return dev
 
 
+def _check_store(key, value, k_cache, v_cache, slot_mapping) -> None:
+    N, num_heads, head_dim = key.shape
+    assert value.shape == key.shape
+    assert key.dtype == _BF16 and value.dtype == _BF16 and k_cache.dtype == _BF16 and v_cache.dtype == _BF16
+    assert key.stride(-1) == 1 and value.stride(-1) == 1
+    assert key.stride(1) == head_dim and value.stride(1) == head_dim
+    assert k_cache.is_contiguous() and v_cache.is_contiguous()
+    assert k_cache.shape == v_cache.shape and k_cache.numel() % (num_heads * head_dim) == 0
+    assert slot_mapping.dtype == torch.int32 and slot_mapping.is_contiguous()
+    assert slot_mapping.numel() == N
+
+
 def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
                   v_cache: torch.Tensor, slot_mapping: torch.Tensor) -> None:
     """k_cache.view(-1, Hkv*D)[slot_mapping[i]] = key[i]; same for value. Slots < 0 are skipped.
@@ -109,14 +121,7 @@ def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
     dev = _require_gpu(key, value, k_cache, v_cache, slot_mapping)
     N, num_heads, head_dim = key.shape
     D = num_heads * head_dim
-    assert value.shape == key.shape
-    assert key.dtype == _BF16 and value.dtype == _BF16 and k_cache.dtype == _BF16 and v_cache.dtype == _BF16
-    assert key.stride(-1) == 1 and value.stride(-1) == 1
-    assert key.stride(1) == head_dim and value.stride(1) == head_dim
-    assert k_cache.is_contiguous() and v_cache.is_contiguous()
-    assert k_cache.shape == v_cache.shape and k_cache.numel() % D == 0
-    assert slot_mapping.dtype == torch.int32 and slot_mapping.is_contiguous()
-    assert slot_mapping.numel() == N
+    _check_store(key, value, k_cache, v_cache, slot_mapping)
     if N == 0:
         return
     lib = _lib.load()
@@ -261,7 +266,7 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
                      num_splits: int = 0, out: Optional[torch.Tensor] = None,
                      seq_order: Optional[torch.Tensor] = None, kernel: Optional[str] = None,
                      workspace: Optional[torch.Tensor] = None,
-                     static_scratch: bool = False, plan=None) -> torch.Tensor:
+                     static_scratch: bool = False, plan=None, new_kv=None) -> torch.Tensor:
     """One query token per sequence over the paged cache.
 
     q: [B, Hq, D]; caches [num_blocks, block_size, Hkv, D] contiguous; context_lens int32 [B]
@@ -278,6 +283,9 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     from the host's lengths that cuts long sequences into more pieces than short ones; num_splits
     and seq_order are then ignored. With plan_max_splits (a captured graph's fixed workspace row
     capacity) attribute absent the plan's own max_splits sizes the workspace.
+    new_kv: optional (key, value, slot_mapping) of store_kvcache, one row per sequence: the rows of the tokens that
+    context_lens counts last. They are stored as store_kvcache would before the attention, in one launch with it (in two with a
+    plan or static_scratch).
     """
     dev = _require_gpu(q, k_cache, v_cache, context_lens, block_table)
     B, Hq, D = q.shape
@@ -298,6 +306,16 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         out = torch.empty((B, Hq, D), dtype=_BF16, device=dev)
     else:
         assert out.shape == (B, Hq, D) and out.dtype == _BF16 and out.stride(-1) == 1 and out.stride(1) == D
+    if new_kv is not None:
+        key, value, slots = new_kv
+        _require_gpu(q, key, value, slots)
+        one_launch = (plan is None and not static_scratch and B > 0 and key.size(0) == B and key.shape[1:] == (Hkv, D)
+                      and all(x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 for x in (key, value)))
+        if not one_launch:
+            store_kvcache(key, value, k_cache, v_cache, slots)
+            new_kv = None
+        else:
+            _check_store(key, value, k_cache, v_cache, slots)
     if B == 0:
         return out
     lib = _lib.load()
@@ -342,13 +360,21 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     else:
         ws_ptr, ws_bytes, keep = _workspace(dev, need)
     with torch.cuda.device(dev):
-        rc = lib.lv_decode_attn(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
-                                q.stride(0), out.stride(0), context_lens.data_ptr(),
-                                block_table.data_ptr(), block_table.stride(0), B, max_blocks, block_size,
-                                Hq, Hkv, D, float(softmax_scale), ws_ptr, ws_bytes, nsplit,
-                                seq_order.data_ptr() if seq_order is not None else None,
-                                _decode_hint(kernel, Hq // Hkv), _stream_ptr(dev))
-    _lib.check(rc, "lv_decode_attn")
+        order = seq_order.data_ptr() if seq_order is not None else None
+        # num_splits 0 goes down as it is: the library may prefer one pass on wider workgroups to the splits that `need` covers
+        if new_kv is not None:
+            rc = lib.lv_decode_attn_store(q.data_ptr(), key.data_ptr(), value.data_ptr(), key.stride(0), value.stride(0),
+                                          k_cache.data_ptr(), v_cache.data_ptr(), slots.data_ptr(), k_cache.numel() // (Hkv * D),
+                                          out.data_ptr(), q.stride(0), out.stride(0), context_lens.data_ptr(), block_table.data_ptr(),
+                                          block_table.stride(0), B, max_blocks, block_size, Hq, Hkv, D, float(softmax_scale), ws_ptr,
+                                          ws_bytes, num_splits, order, _decode_hint(kernel, Hq // Hkv), _stream_ptr(dev))
+        else:
+            rc = lib.lv_decode_attn(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
+                                    q.stride(0), out.stride(0), context_lens.data_ptr(),
+                                    block_table.data_ptr(), block_table.stride(0), B, max_blocks, block_size,
+                                    Hq, Hkv, D, float(softmax_scale), ws_ptr, ws_bytes, num_splits, order,
+                                    _decode_hint(kernel, Hq // Hkv), _stream_ptr(dev))
+    _lib.check(rc, "lv_decode_attn" if new_kv is None else "lv_decode_attn_store")
     del keep
     return out
 
