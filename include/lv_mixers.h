@@ -25,6 +25,7 @@
  *   lv_router_logits         f32 router logits of steps of few tokens, straight from the activations
  *   lv_relu2_scale           squared relu of the experts' up projections times the routing weight
  *   lv_moe_grouped_ff        the experts' feed-forward on rows sorted by expert (grouped GEMMs on the matrix cores)
+ *   lv_moe_tiled_ff          the same for prompt steps, on LDS tiles
  *   lv_moe_sort, lv_moe_combine   its first and last step alone, for callers that multiply the sorted rows themselves
  *   lv_sandwich_add_norm     single f32 residual of layers that norm both sides of a sublayer: adds the RMS-normed
  *                            sublayer output, a row of activations and a vector, RMS norm with weight (offset + w)
@@ -87,7 +88,7 @@
 extern "C" {
 #endif
 
-#define LV_MIX_ABI_VERSION 10
+#define LV_MIX_ABI_VERSION 11
 #define LV_MIX_BF16 0
 #define LV_MIX_F32 1
 #define LV_MIX_MAX_STREAMS 8
@@ -126,6 +127,15 @@ int lv_hc_update_norm(void* x, const void* y, const void* mix, const void* out_w
  * out act [T, W] = x / sqrt(mean(x^2) + eps) * (w_offset + w), w f32 [W]. */
 int lv_residual_add_norm(void* x, const void* y1, const void* y2, const void* w, float w_offset, void* out, int64_t T,
                          int W, float eps, int dtype, void* stream);
+
+/* The experts' feed-forward for prompt steps: both products on LDS tiles over rows sorted by expert, nothing read back to the
+ * host. glu 0: lv_moe_grouped_act_ff (act LV_MIX_ACT_RELU2 or one of the two gelus, which read the product rounded to bf16);
+ * glu 1: lv_moe_grouped_glu_ff (n_through 0). down_ld: row stride of down_w in elements, 0 for E_real * F. h, up_w, down_w and
+ * workspace are 16-byte aligned. workspace: lv_moe_tiled_workspace_bytes(T, W, F, E_real + n_through, top) bytes. */
+int lv_moe_tiled_ff(const void* h, const void* ids, const void* weights, const void* up_w, const void* down_w, int64_t down_ld,
+                    void* out, void* workspace, int64_t T, int W, int F, int E_real, int n_through, int top, int act, int glu,
+                    float limit, float alpha, void* stream);
+int64_t lv_moe_tiled_workspace_bytes(int64_t T, int W, int F, int E, int top);
 
 /* in act [T, 2F] (row stride ld_in) = [gate | up];  out act [T, F]. */
 int lv_clamped_glu(const void* in, int64_t ld_in, void* out, int64_t T, int F, float limit, float alpha,

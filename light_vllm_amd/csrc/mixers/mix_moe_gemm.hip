@@ -16,8 +16,8 @@
 //   moe_combine_kernel   one workgroup per token: sum over its choices of weight * expert output row, in f32.
 // A row's result does not depend on where the sort put it or on what else is in the tile: every output element is
 // its own chain of MFMA accumulations over k.
-// lv_moe_sort and lv_moe_combine are also exported alone: large eager steps run the experts' products as vendor GEMMs
-// on the sorted rows in between (mix_ops.moe_sorted_ff).
+// lv_moe_sort and lv_moe_combine are also exported alone, for callers that multiply the sorted rows themselves. Prompt steps
+// take the LDS tiles of mix_moe_tiles.hip.
 #include "mix_common.h"
 
 namespace lvmix {

@@ -15,10 +15,10 @@ matrices one [width, experts * ff] weight. Two forms compute the same sum:
   * gathered (bf16, width and ff in multiples of 32, at least GATHER_FROM experts per choice): the (token,
     choice) pairs are sorted by expert on the device and every expert multiplies only its own rows
     (mix_ops.moe_grouped_ff: sort, two grouped GEMMs on the matrix cores, weighted sum; four launches);
-  * sorted (bf16, eager steps with at least SORTED_FROM rows per expert): the same device-side sort, then every
-    expert's two products as vendor GEMMs on its slice of the sorted rows, after reading the experts' row counts
-    back once (mix_ops.moe_sorted_ff); large prompt steps, where the vendor GEMM's rate outweighs the one host
-    synchronisation. Steps captured into a hipGraph never take it;
+  * sorted (bf16, eager steps with at least TILED_FROM rows per expert): the same sum with both products on LDS tiles of
+    128 or 256 rows (mix_ops.moe_sorted_ff). Weights whose layout those do not take go, from SORTED_FROM rows per expert,
+    through vendor GEMMs on the sorted rows, after reading the experts' row counts back once. Steps captured into a
+    hipGraph never take this form;
   * masked (f32, other sizes, few experts per choice): the up projection of every expert in one vendor
     GEMM, one kernel applies the activation times the token's weight for the column's expert (zero for
     experts the token did not choose), and the down GEMM sums over experts by itself. It spends
@@ -34,8 +34,7 @@ projections are linear, s * h enters as a factor on the pre-activations (mix_ops
 expert's token gate as a factor on its activations, so all of it is GEMMs on h plus one elementwise kernel.
 Forms: masked (everything in one up GEMM and one down GEMM; any dtype and size), gathered (bf16: sort, two
 grouped GEMMs on the matrix cores with the gated unit in the first one's epilogue, sum; the shared expert as
-vendor GEMMs beside it) and sorted (bf16, eager steps with at least SORTED_FROM rows per expert: the same sort, then
-every expert's products as vendor GEMMs on its slice of the sorted rows).
+vendor GEMMs beside it) and sorted (bf16, eager steps with at least TILED_FROM rows per expert: the same on LDS tiles).
 """
 from __future__ import annotations
 
@@ -49,7 +48,11 @@ from .tp import tp_size
 
 
 GATHER_FROM = 2.0     # experts / top from which the gathered form is taken
-SORTED_FROM = 256     # rows per expert from which an eager step runs the experts as vendor GEMMs on sorted rows
+# Rows per expert from which an eager step multiplies on LDS tiles. 32 experts of 2048 x 1536: 118 against 160 us for the
+# gathered form at 16 rows, 129 / 254 at 64, 246 / 539 at 256, 1006 / 3412 at 2048; below 16 the gathered form's tiles of 16
+# rows read each weight once and pad little.
+TILED_FROM = 16
+SORTED_FROM = 256     # the same for weights that the tiles do not take: vendor GEMMs on sorted rows
 MOE_KERNEL = "auto"   # "auto" | "masked" | "gathered" | "sorted" (tests force one or the other)
 
 
@@ -89,7 +92,8 @@ class SparseMoE(nn.Module):
             return "masked"
         step = get_context().ragged
         captured = step is not None and step.static
-        return "sorted" if not captured and h.size(0) * self.top >= SORTED_FROM * self.E else "gathered"
+        tiles = mix_ops.moe_tiles_ok(h, self.up_weight, self.down_weight, self.E, self.ff, 1, self.act, self.identity)
+        return "sorted" if not captured and h.size(0) * self.top >= (TILED_FROM if tiles else SORTED_FROM) * self.E else "gathered"
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         ids, weights, dense = self.route(h)
@@ -133,7 +137,8 @@ class GLUSparseMoE(nn.Module):
             return "masked"
         step = get_context().ragged
         captured = step is not None and step.static
-        return "sorted" if not captured and h.size(0) * self.top >= SORTED_FROM * self.E else "gathered"
+        tiles = mix_ops.moe_tiles_ok(h, self.up_weight, self.down_weight, self.E, self.ff, 2)
+        return "sorted" if not captured and h.size(0) * self.top >= (TILED_FROM if tiles else SORTED_FROM) * self.E else "gathered"
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         ids, weights, dense = self.route(h)

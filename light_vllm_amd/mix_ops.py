@@ -1077,15 +1077,47 @@ def moe_combine(rows, inv, weights=None, ids=None, n_real=0, h=None):
     return out
 
 
+def moe_tiles_ok(h, up_w, down_w, E, Fe, ups=1, act="relu2", n_through=0) -> bool:
+    """Whether lv_moe_tiled_ff takes these operands (ups: 2 for gate and up rows): bf16 on the device, widths in multiples of
+    32, rows of 16-byte pieces, and offsets inside an operand tile in 32 bits."""
+    T, W = h.shape
+    ld = down_w.stride(0)
+    return (h.is_cuda and moe_grouped_ok(h, Fe) and act in ("relu2", "gelu", "gelu_tanh") and E + n_through <= 4096
+            and up_w.dtype == down_w.dtype == h.dtype and up_w.size(0) >= E * ups * Fe and up_w.size(1) == W
+            and down_w.size(0) == W and down_w.size(1) >= E * Fe
+            and h.is_contiguous() and up_w.is_contiguous() and down_w.stride(1) == 1 and ld >= E * Fe and ld % 8 == 0
+            and all(x.data_ptr() % 16 == 0 for x in (h, up_w, down_w))
+            and max(T * W, (Fe + 256) * W, 256 * ld, 256 * Fe) < 1 << 31)
+
+
+def _choices_ok(ids, weights) -> bool:
+    return (ids.dtype == torch.int32 and ids.is_contiguous() and weights.dtype == torch.float32 and weights.is_contiguous()
+            and weights.shape == ids.shape and ids.numel() <= 1 << 30)
+
+
+def _moe_tiled(h, ids, weights, up_w, down_w, E, Fe, act, n_through, glu, limit, alpha):
+    T, W = h.shape
+    top = ids.size(1)
+    out = torch.empty(T, W, dtype=h.dtype, device=h.device)
+    lib = _mixlib.load()
+    ws = torch.empty(lib.lv_moe_tiled_workspace_bytes(T, W, Fe, E + n_through, top), dtype=torch.uint8, device=h.device)
+    _mixlib.check(lib.lv_moe_tiled_ff(_p(h), _p(ids), _p(weights), _p(up_w), _p(down_w), down_w.stride(0), _p(out), _p(ws), T, W, Fe,
+                                      E, n_through, top, ACTS[act], glu, limit, alpha, _stream(h)), "lv_moe_tiled_ff")
+    return out
+
+
 SORTED_ALIGN = 128
 
 
 def moe_sorted_ff(h, ids, weights, up_w, down_w, E, Fe, act="relu2", n_through=0):
-    """The same sum as moe_grouped_ff for large eager steps: rows sorted by expert on the device, the experts' row
-    counts read back once, and each expert's two products run as vendor GEMMs on its slice of the sorted rows. One host
+    """The same sum as moe_grouped_ff for prompt steps. Where moe_tiles_ok holds, both products run as grouped GEMMs on LDS
+    tiles (lv_moe_tiled_ff) and nothing is read back. Otherwise: rows sorted by expert on the device, the experts' row
+    counts read back once, and each expert's two products run as vendor GEMMs on its slice of the sorted rows, with one host
     synchronisation per call, so not for steps that are captured into a graph. Every expert's slice is padded to a
     multiple of SORTED_ALIGN rows (copies of token 0 that no one reads back): the GEMM library then sees a handful of
     shapes instead of a new one per expert and step, each of which would cost it a kernel selection on the host."""
+    if moe_tiles_ok(h, up_w, down_w, E, Fe, 1, act, n_through) and _choices_ok(ids, weights):
+        return _moe_tiled(h, ids, weights, up_w, down_w, E, Fe, act, n_through, 0, 0.0, 0.0)
     T, W = h.shape
     top = ids.size(1)
     sorted_pair, inv, offsets = moe_sort(ids, E + n_through, SORTED_ALIGN)
@@ -1109,10 +1141,12 @@ def moe_sorted_ff(h, ids, weights, up_w, down_w, E, Fe, act="relu2", n_through=0
 
 
 def moe_sorted_glu_ff(h, ids, weights, up_w, down_w, E, Fe, limit, alpha):
-    """The same sum as moe_grouped_glu_ff for large eager steps, the way moe_sorted_ff does it: rows sorted by expert on
-    the device, the experts' row counts read back once, each expert's gate|up product and down product as vendor GEMMs on
+    """The same sum as moe_grouped_glu_ff for prompt steps, the way moe_sorted_ff does it: on LDS tiles with the gated unit in
+    the first product's epilogue, or, for operands that lv_moe_tiled_ff does not take, rows sorted by expert on the device, the experts' row counts read back once, each expert's gate|up product and down product as vendor GEMMs on
     its slice of the sorted rows (slices padded to SORTED_ALIGN rows), the gated unit over all sorted rows in one launch
     with every row's routing weight as the factor on its pre-activations, and the plain sum of every token's rows."""
+    if moe_tiles_ok(h, up_w, down_w, E, Fe, 2) and _choices_ok(ids, weights):
+        return _moe_tiled(h, ids, weights, up_w, down_w, E, Fe, "relu2", 0, 1, limit, alpha)
     T, W = h.shape
     top = ids.size(1)
     sorted_pair, inv, offsets = moe_sort(ids, E, SORTED_ALIGN)
