@@ -419,7 +419,7 @@ __global__ __launch_bounds__(256) void window_pool_merge_kernel(const float* __r
 // probabilities keep their relative precision at any magnitude).
 // Bound by the matrix pipe and the LDS reads that feed it, about level at 32 queries a wave. Against the 16-query form on one box: 11
 // prompts of 1500 tokens on average, window 1024, 16 heads over 4 of 128: 478 -> 220 us; 16 x 1024 tokens, 16 heads on latent rows of 256
-// (values 192): 978 -> 342 us; 1 x 4000 full causal, 16 over 4: 391 -> 122 us; 17 tokens behind 4000: 67 -> 43 us; never slower
+// (values 192): 978 -> 195 us (342 while their rows passed through registers and 54 of them spilled); 1 x 4000 full causal, 16 over 4: 391 -> 122 us; 17 tokens behind 4000: 67 -> 43 us; never slower
 // from 17 new tokens on.
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 typedef __attribute__((address_space(3))) unsigned char lds_u8;
@@ -448,7 +448,11 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WindowMfmaParams p,
   constexpr int NS = DK / 16, ND = DV / 32;
   constexpr bool FIRST = DK <= 128;                                         // latent rows come without pooled blocks and kept tokens
   constexpr float kLog2e = 1.44269504088896f;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * (KT + VT)];
+  constexpr bool DMA = !FIRST;
+  static_assert(!DMA || (SAME && KB == 512 && FORM == kPlain), "rows of 512 bytes, two of them a load instruction");
+  __shared__ __attribute__((aligned(16))) unsigned char lds[DMA ? 16 : 2 * (KT + VT)];
+  __shared__ __attribute__((aligned(1024))) unsigned char tile0[DMA ? KT : 16];
+  __shared__ __attribute__((aligned(1024))) unsigned char tile1[DMA ? KT : 16];
   __shared__ __attribute__((aligned(16))) float ks_lds[FORM == kExtended ? 2 * kTileK : 4];
   __shared__ float bias_lds[FORM == kExtended ? 4 * kBiasLds : 1];
   lds_u8* const base3 = (lds_u8*)lds;
@@ -565,7 +569,7 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WindowMfmaParams p,
   const float cs = FORM == kPlain ? p.scale * kLog2e : kLog2e;              // from what the products leave to the exponent of 2
   float m = (p.sinks != nullptr ? p.sinks[h] : p.m0) * kLog2e, l = half == 0 ? p.sink : 0.0f;
 
-  auto compute = [&](int tile, int buf) __attribute__((always_inline)) {
+  auto compute = [&](int tile, int buf, lds_u8* kt) __attribute__((always_inline)) {
     const int phase = FIRST && tile < npt ? 0 : 1;
     const int e0 = phase == 0 ? tile * kTileK : jlo + (tile - npt) * kTileK;
     const int e_end = phase == 0 ? nbmax : i1 + 1;
@@ -577,7 +581,6 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WindowMfmaParams p,
       return;
     }
     const bool whole = phase == 1 && e0 + kTileK - 1 <= w0 && (chunk > 0 ? e0 >= w1 - w1 % chunk : w1 - e0 < W);
-    lds_u8* const kt = base3 + buf * (KT + VT);
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) {
       f32x16_t s;
@@ -664,15 +667,49 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WindowMfmaParams p,
     }
   };
 
-  load(0);
-  store(0);
-  __syncthreads();
-  if (ntiles > 1) load(1);
-  for (int tile = 0; tile < ntiles; ++tile) {
-    compute(tile, tile & 1);
-    if (tile + 1 < ntiles) store((tile + 1) & 1);
-    if (tile + 2 < ntiles) load(tile + 2);
+  if constexpr (DMA) {
+    // Latent rows go straight from memory into the tile, whose buffers are arrays of their own so that the compiler sees which of
+    // them a read has to wait for; held in registers on the way they cost 32 of the wave's 256, and accumulators spilled.
+    const int d_r = 2 * wave + half;                                        // row of piece `wave`; piece wave + 4 i: 8 i further
+    auto request = [&](int tile, lds_u8* at) __attribute__((always_inline)) {
+      const int e0 = jlo + tile * kTileK, pj = fdiv(e0, page, p.m_page), last = i1 - e0;
+      const int64_t slot = static_cast<int64_t>(bt[pj]) * page + (e0 - pj * page);
+      const char* kb = reinterpret_cast<const char*>(p.k_cache + slot * p.k_ld + g * DK);
+#pragma unroll
+      for (int i = 0; i < KT / 4096; ++i) {
+        const int r = 8 * i + d_r, ch = (lane & 31) ^ (((r & 3) << 2) | ((r >> 2) & 3));
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void*)(kb + static_cast<uint32_t>(min(r, last)) * static_cast<uint32_t>(2 * p.k_ld) + 16 * ch),
+            (__attribute__((address_space(3))) void*)(at + 1024 * (wave + 4 * i)), 16, 0, 0);
+      }
+    };
+    auto turn = [&]() __attribute__((always_inline)) {
+      __builtin_amdgcn_s_waitcnt(0x0070);                                   // own pieces landed, own reads done; then everyone's
+      asm volatile("s_barrier" ::: "memory");
+    };
+    request(0, (lds_u8*)tile0);
+    turn();
+    for (int tile = 0;;) {
+      if (tile + 1 < ntiles) request(tile + 1, (lds_u8*)tile1);
+      compute(tile, 0, (lds_u8*)tile0);
+      turn();
+      if (++tile >= ntiles) break;
+      if (tile + 1 < ntiles) request(tile + 1, (lds_u8*)tile0);
+      compute(tile, 1, (lds_u8*)tile1);
+      turn();
+      if (++tile >= ntiles) break;
+    }
+  } else {
+    load(0);
+    store(0);
     __syncthreads();
+    if (ntiles > 1) load(1);
+    for (int tile = 0; tile < ntiles; ++tile) {
+      compute(tile, tile & 1, base3 + (tile & 1) * (KT + VT));
+      if (tile + 1 < ntiles) store((tile + 1) & 1);
+      if (tile + 2 < ntiles) load(tile + 2);
+      __syncthreads();
+    }
   }
   if (!live) return;
   const float total = l + __shfl_xor(l, 32, kWave);
