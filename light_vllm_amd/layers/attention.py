@@ -39,9 +39,10 @@ class Attention(nn.Module):
         k_cache, v_cache = self.k_cache, self.v_cache
 
         # A prefix-cached prefill and every decode step read the rows written here (reference :149-150): the store is
-        # stream-ordered before a prefill's attention launch, and rides in a decode step's.
+        # stream-ordered before the attention launch; on the device a decode step's rides in that launch.
         store = not kv_stored and k_cache.numel() and v_cache.numel()
-        if store and context.is_prefill:
+        rides = store and not context.is_prefill and q.is_cuda
+        if store and not rides:
             store_kvcache(k, v, k_cache, v_cache, context.slot_mapping)
 
         if context.is_prefill:
@@ -51,8 +52,8 @@ class Attention(nn.Module):
                                       context.max_seqlen_q, context.max_seqlen_k, self.scale,
                                       block_table=context.block_tables, tile_order=context.tile_order)
         else:
+            new = dict(new_kv=(k, v, context.slot_mapping)) if rides else {}
             o = ops.decode_attention(q, k_cache, v_cache, context.context_lens,
                                      context.block_tables, self.scale, seq_order=context.seq_order,
-                                     plan=context.decode_plan,
-                                     new_kv=(k, v, context.slot_mapping) if store else None)
+                                     plan=context.decode_plan, **new)
         return o.view(-1, self.num_heads * self.head_dim)
