@@ -1217,8 +1217,10 @@ def lightning_attention(proj, off_q, off_k, off_v, decay, state, step, H, D, Dv)
     assert state.shape[1:] == (H, D, Dv) and decay.numel() == H
     if proj.is_cuda and T > 0 and proj.dtype == torch.bfloat16:
         assert proj.stride(1) == 1
-        q, k, v = (proj[:, at:at + H * n] for at, n in ((off_q, D), (off_k, D), (off_v, Dv)))
-        if _chunk_ok(CHUNK_CONST, step, D, Dv, q, k):
+        columns = ((off_q, H * D), (off_k, H * D), (off_v, H * Dv))
+        q, k, v = (proj[:, at:at + n] for at, n in columns)
+        # columns outside the rows go to the entry below, which refuses them
+        if all(0 <= at <= proj.size(1) - n for at, n in columns) and _chunk_ok(CHUNK_CONST, step, D, Dv, q, k):
             return _chunk_scan(CHUNK_CONST, q, k, v, None, decay, None, None, None, state, step, H, H, D, Dv)
     o = torch.empty(T, H, Dv, dtype=torch.float32, device=proj.device)
     if proj.is_cuda:

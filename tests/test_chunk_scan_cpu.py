@@ -1,5 +1,12 @@
-"""lv_chunk_scan rejects bad arguments on the host, before any launch."""
+"""lv_chunk_scan rejects bad arguments on the host, before any launch, and which calls of the recurrences take it."""
 import ctypes
+
+import pytest
+import torch
+
+from light_vllm_amd import mix_ops
+from tests._ragged import ragged_step
+from tests._route import device, record
 
 
 def test_argument_validation():
@@ -24,3 +31,21 @@ def test_argument_validation():
     assert need(2, 64, 1, 64, 2, 64, 64, 32) >= 64 * 2 * 66 * 4      # the delta rule is never cut
     assert need(1, 64, 1, 64, 2, 64, 64, 32) > need(1, 64, 1, 64, 2, 64, 64, 64)
     assert need(1, -1, 1, 64, 2, 64, 64, 0) < 0
+
+
+def lightning(off_q, off_k, off_v, width, H=2, D=64, Dv=64):
+    step, _ = ragged_step([96, 3], [0, 0], 16, "cpu")
+    proj = device(torch.zeros(99, width, dtype=torch.bfloat16))
+    state = torch.zeros(2, H, D, Dv)
+    return mix_ops.lightning_attention(proj, off_q, off_k, off_v, torch.full((H,), 0.9), state, step, H, D, Dv)
+
+
+def test_columns_outside_the_row_are_refused(monkeypatch):
+    """A head's columns that do not lie in the row of the projection are an argument error on long steps as on short ones."""
+    calls = record(monkeypatch, real=("lv_lightning_attn",))
+    lightning(0, 128, 256, 384)
+    assert calls == ["lv_chunk_scan"]
+    for bad in ((0, 128, 260, 384), (260, 0, 128, 384), (0, 400, 128, 384), (-4, 128, 256, 384), (0, 128, 256, 256)):
+        with pytest.raises(RuntimeError):
+            lightning(*bad)
+    assert calls == ["lv_chunk_scan"]
