@@ -202,10 +202,10 @@ def clamped_glu(x, limit: float, alpha: float):
 
 
 # ------------------------------------------------------------------------------- recurrences in chunks
-def _chunk_ok(kind, step, D, Dv, *rows) -> bool:
+def _chunk_ok(kind, step, D, Dv, state, *rows) -> bool:
     """Whether lv_chunk_scan takes this step: sizes and alignment it knows and a sequence with CHUNK_FROM[kind] new tokens or more.
-    rows: the query and key rows (four entries at a time)."""
-    return (SCAN_KERNEL == "auto" and not step.static and D in (64, 128) and (Dv == 64 or Dv % 128 == 0)
+    rows: the query and key rows (four entries at a time, as the state)."""
+    return (SCAN_KERNEL == "auto" and not step.static and D in (64, 128) and (Dv == 64 or Dv % 128 == 0) and state.data_ptr() % 16 == 0
             and all(x.stride(0) % 4 == 0 and x.data_ptr() % (4 * x.element_size()) == 0 for x in rows)
             and max(step.host_lens_q) >= CHUNK_FROM[kind])
 
@@ -331,7 +331,7 @@ def gated_delta_rule(qn, kn, v, beta, decay, state, step):
     assert state.shape[1:] == (H, D, Dv)
     per_channel = decay.dim() == 3
     assert decay.shape == ((T, H, D) if per_channel else (T, H))
-    if qn.is_cuda and not per_channel and T > 0 and _chunk_ok(CHUNK_DELTA, step, D, Dv, qn, kn):
+    if qn.is_cuda and not per_channel and T > 0 and _chunk_ok(CHUNK_DELTA, step, D, Dv, state, qn, kn):
         return _chunk_scan(CHUNK_DELTA, qn.view(T, G * D), kn.view(T, G * D), v.view(T, H * Dv), beta, decay, None, None, None, state,
                            step, H, G, D, Dv)
     o = torch.empty(T, H, Dv, dtype=torch.float32, device=qn.device)
@@ -1220,7 +1220,7 @@ def lightning_attention(proj, off_q, off_k, off_v, decay, state, step, H, D, Dv)
         columns = ((off_q, H * D), (off_k, H * D), (off_v, H * Dv))
         q, k, v = (proj[:, at:at + n] for at, n in columns)
         # columns outside the rows go to the entry below, which refuses them
-        if all(0 <= at <= proj.size(1) - n for at, n in columns) and _chunk_ok(CHUNK_CONST, step, D, Dv, q, k):
+        if all(0 <= at <= proj.size(1) - n for at, n in columns) and _chunk_ok(CHUNK_CONST, step, D, Dv, state, q, k):
             return _chunk_scan(CHUNK_CONST, q, k, v, None, decay, None, None, None, state, step, H, H, D, Dv)
     o = torch.empty(T, H, Dv, dtype=torch.float32, device=proj.device)
     if proj.is_cuda:
@@ -1378,7 +1378,7 @@ def gated_scan(kind, q, k, v, a, p0, p1, step, state, H, G, D, Dv, a2=None, p2=N
     assert state.shape[1:] == (H, D, Dv) and q.size(1) == G * D and k.size(1) == G * D and v.size(1) == H * Dv
     assert a.size(1) == (H * D if kind == SCAN_ROW_DECAY else H) and a.dtype == q.dtype == k.dtype == v.dtype
     if (kind == SCAN_STEP and q.is_cuda and T > 0 and q.dtype == torch.bfloat16 and q_scale == 1.0
-            and all(x.stride(1) == 1 for x in (q, k, v, a)) and _chunk_ok(CHUNK_STEP, step, D, Dv, q, k)):
+            and all(x.stride(1) == 1 for x in (q, k, v, a)) and _chunk_ok(CHUNK_STEP, step, D, Dv, state, q, k)):
         return _chunk_scan(CHUNK_STEP, q, k, v, a, None, p0, p1, p2, state, step, H, G, D, Dv)
     o = torch.empty(T, H, Dv, dtype=torch.float32, device=q.device)
     den = None

@@ -49,3 +49,17 @@ def test_columns_outside_the_row_are_refused(monkeypatch):
         with pytest.raises(RuntimeError):
             lightning(*bad)
     assert calls == ["lv_chunk_scan"]
+
+
+def delta_call(state, D=64, Dv=64, H=2):
+    step, _ = ragged_step([96, 3], [0, 0], 16, "cpu")
+    rows = [device(torch.zeros(99, H, n)) for n in (D, D, Dv)]
+    return mix_ops.gated_delta_rule(*rows, torch.zeros(99, H), torch.ones(99, H), state, step)
+
+
+def test_state_off_a_16_byte_boundary_takes_the_token_loop(monkeypatch):
+    """The chunked kernel's combine step reads states four entries at a time; a state that lies elsewhere is still served."""
+    calls = record(monkeypatch, real=("lv_chunk_scan",))
+    flat = torch.zeros(2 * 2 * 64 * 64 + 1)
+    delta_call(flat[1:].view(2, 2, 64, 64))
+    assert calls == ["lv_gated_delta_rule"]
