@@ -506,8 +506,9 @@ int lv_chunk_scan(int kind, const void* q, int64_t ldq, const void* k, int64_t l
   if (B < 0 || T < 0 || max_new <= 0 || max_new > T || seg_len < 0 || seg_len % kCh != 0 || !chunk_sizes_ok(H, G, D, Dv))
     return fail(-1, "lv_chunk_scan: bad sizes");
   const uintptr_t piece = kind == kChunkDelta ? 16 : 8;      // four entries of a row: f32 for the delta rule, bf16 otherwise
-  if (ldq < static_cast<int64_t>(G) * D || ldk < static_cast<int64_t>(G) * D || ldv < static_cast<int64_t>(H) * Dv || ldq % 4 != 0 ||
-      ldk % 4 != 0 || reinterpret_cast<uintptr_t>(q) % piece != 0 || reinterpret_cast<uintptr_t>(k) % piece != 0 ||
+  if (ldq < static_cast<int64_t>(G) * D || ldk < static_cast<int64_t>(G) * D || ldv < static_cast<int64_t>(H) * Dv ||
+      (kind == kChunkStep && lda < H) || ldq % 4 != 0 || ldk % 4 != 0 ||
+      reinterpret_cast<uintptr_t>(q) % piece != 0 || reinterpret_cast<uintptr_t>(k) % piece != 0 ||
       reinterpret_cast<uintptr_t>(state) % 16 != 0 || reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
     return fail(-1, "lv_chunk_scan: strides or alignment");
   if (workspace_bytes < lv_chunk_scan_workspace_bytes(kind, T, B, max_new, H, D, Dv, seg_len))

@@ -4,6 +4,8 @@ import torch
 
 from light_vllm_amd import _mixlib, mix_ops
 
+_load = _mixlib.load          # before a test puts a recorder in its place
+
 
 class Device(torch.Tensor):
     is_cuda = property(lambda self: True)
@@ -15,7 +17,7 @@ def device(x):
 
 class Recorder:
     def __init__(self, real=()):
-        self.calls, self._real, self._lib = [], real, _mixlib.load()
+        self.calls, self._real, self._lib = [], real, _load()
 
     def __getattr__(self, name):
         if name in self._real or name.endswith(("_bytes", "_error")):

@@ -63,3 +63,21 @@ def test_state_off_a_16_byte_boundary_takes_the_token_loop(monkeypatch):
     flat = torch.zeros(2 * 2 * 64 * 64 + 1)
     delta_call(flat[1:].view(2, 2, 64, 64))
     assert calls == ["lv_gated_delta_rule"]
+
+
+def step_call(a_ld, H=2, D=64, Dv=64):
+    step, _ = ragged_step([96, 3], [0, 0], 16, "cpu")
+    q, k, v = (device(torch.zeros(99, H * n, dtype=torch.bfloat16)) for n in (D, D, Dv))
+    a = torch.zeros(99, a_ld, dtype=torch.bfloat16)[:, :H] if a_ld >= H else torch.zeros(1, H, dtype=torch.bfloat16).expand(99, H)
+    one = torch.zeros(H)
+    return mix_ops.gated_scan(mix_ops.SCAN_STEP, q, k, v, a, one, one, step, torch.zeros(2, H, D, Dv), H, H, D, Dv, p2=one)
+
+
+def test_step_sizes_that_share_a_row_are_refused(monkeypatch):
+    """Row strides below the heads' count are an argument error on long steps as on short ones."""
+    calls = record(monkeypatch, real=("lv_gated_scan",))
+    step_call(4)
+    assert calls == ["lv_chunk_scan"]
+    record(monkeypatch, real=("lv_gated_scan", "lv_chunk_scan"))
+    with pytest.raises(RuntimeError, match="bad sizes|strides"):
+        step_call(0)
