@@ -107,6 +107,11 @@ class LatentAttention(nn.Module):
                                  step, self.Rq, R, Dr, self.rot_dims, self.norm_eps)
         q = self.uq(cq)
         gate = proj[:, self.sizes[0] + self.sizes[1]:]
+        if not h.is_cuda:               # torch ops throughout: gradients pass
+            q_lat = torch.bmm(q.view(T, H, Dn + Dr)[:, :, :Dn].transpose(0, 1), self.uk)          # [H, T, R]
+            q_abs = mix_ops.latent_q_finish(q, q_lat, self.inv_freq, step, H, Dn, Dr, R, self.rot_dims)
+            o = torch.bmm(self._attend(q_abs, step).view(T, H, R).transpose(0, 1), self.uv)         # [H, T, Dv]
+            return self.o_proj(mix_ops.latent_out_gate(o, gate, self.gate_per_channel))
         with torch.no_grad():           # the kernels between them carry no gradient, and `out` may not ask for one
             # both batched products write where the next step reads; a gate per head goes on the sum that the value matrix
             # multiplies (the same product), in the attention kernel
