@@ -1,4 +1,4 @@
-/* A layer's decode step in one call: lv_store_kvcache and lv_decode_attn (lv_attention.h) with one launch for both. */
+/* A layer's decode step in one call: lv_store_kvcache and lv_decode_attn (lv_attention.h). */
 #ifndef LV_DECODE_STORE_H
 #define LV_DECODE_STORE_H
 
@@ -12,10 +12,10 @@ extern "C" {
  *   lv_store_kvcache(key, value, key_stride0, value_stride0, k_cache, v_cache, slot_mapping, batch, num_kv_heads, head_dim,
  *                    num_slots, stream);
  *   lv_decode_attn(q, k_cache, v_cache, o, ..., stream);
- * for decode steps, in which row b of key and value belongs to the last token of sequence b: the attention kernel writes the rows on
- * its way and reads that token's from them. A slot that is not the last token's place (or is skipped: negative, past num_slots)
- * is written, or not, all the same; such a slot must not lie among the tokens that another sequence of the batch reads. seq_order must
- * be a permutation. num_splits 0 leaves the choice to the library; a workspace for lv_decode_num_splits splits always serves. */
+ * for any slots: one elsewhere among the tokens that this or another sequence reads (tokens of one sequence as several rows of the
+ * batch) is read as it was stored. Two rows with one slot leave either. Up to 64 sequences take one launch: the attention kernel
+ * reads the step's rows from key and value and writes them to the caches on its way. num_splits 0 leaves the choice to the
+ * library; a workspace for lv_decode_num_splits splits always serves. */
 int lv_decode_attn_store(const void* q, const void* key, const void* value, int64_t key_stride0, int64_t value_stride0,
                          void* k_cache, void* v_cache, const int32_t* slot_mapping, int64_t num_slots, void* o, int64_t q_stride0,
                          int64_t o_stride0, const int32_t* context_lens, const int32_t* block_table, int block_table_stride, int batch,

@@ -540,10 +540,17 @@ int lv_decode_attn_store(const void* q, const void* key, const void* value, int6
     return fail(LV_ERR_INVALID_ARGUMENT, "decode_store: row stride smaller than num_kv_heads*head_dim");
   if (key_stride0 % 8 != 0 || value_stride0 % 8 != 0 || !aligned16(key) || !aligned16(value))
     return fail(LV_ERR_UNSUPPORTED, "decode_store: key and value must be 16-byte aligned with strides %% 8 == 0");
+  // more rows than a wave has lanes to look them up with: two launches (256 x 1024 tokens: 168.2 us against 167.2)
+  NewRows rows{key, value, key_stride0, value_stride0, slot_mapping, num_slots};
+  if (batch > kRowLanes) {
+    const int code = lv_store_kvcache(key, value, key_stride0, value_stride0, k_cache, v_cache, slot_mapping, batch, num_kv_heads, head_dim,
+                                      num_slots, stream);
+    if (code != LV_OK) return code;
+    rows = NewRows{};
+  }
   return decode_entry(q, k_cache, v_cache, o, q_stride0, o_stride0, context_lens, block_table, block_table_stride, batch,
                       max_blocks_per_seq, block_size, num_heads, num_kv_heads, head_dim, scale, workspace, workspace_bytes, false,
-                      num_splits, seq_order, nullptr, 0, nullptr, kernel_hint, stream,
-                      NewRows{key, value, key_stride0, value_stride0, slot_mapping, num_slots});
+                      num_splits, seq_order, nullptr, 0, nullptr, kernel_hint, stream, rows);
 }
 
 int lv_decode_attn(const void* q, const void* k_cache, const void* v_cache, void* o,

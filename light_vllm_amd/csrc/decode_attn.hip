@@ -105,39 +105,37 @@ __device__ __forceinline__ bool decode_work(const DecodeParams& p, DecodeWork& w
          w.nsplit <= p.nsplit && w.split < w.nsplit;
 }
 
-// STORE launches bring this step's key and value rows along. The workgroup that owns a sequence's last token writes its kv head's
-// two rows (256 bytes each) to the caches at slot_mapping[b], as store_kvcache does, and where that slot is the last token's own
-// place takes the rows from the inputs instead of reading back what it has just written. A slot elsewhere, or none
-// (negative, out of range), changes nothing about what is read.
-// The slot and the last token's place are requested with the kernel's first loads and compared where the last chunk is loaded;
-// the rows are written behind the loop: nothing at the start waits for them. (With the comparison up front the 256 x 1024 launch at
-// 32q/8kv took 182 us instead of 171.) What it saves is the store's launch, about 1.5 us in a replayed graph: with the rule on
-// splits (api.hip) a layer's step at 4 x 512 ragged tokens, 16q/8kv, went from 11.3 to 9.7 us, 1 x 64 from 9.1 to 5.2,
-// 128 x 100 at 8q/1kv from 12.3 to 8.3; 256 x 1024 stays at 171.
-struct NewRow {
-  int64_t slot = -1, place = -2;
-  bool write = false;
-  __device__ __forceinline__ bool own() const { return slot == place; }
-};
-__device__ __forceinline__ NewRow new_row(const DecodeParams& p, const DecodeWork& w, int ctx, int t1) {
-  NewRow r;
-  if (t1 != ctx || (ctx == 0 && w.split + 1 != w.nsplit)) return r;
-  r.slot = p.slot_mapping[w.b];
-  r.write = true;
-  if (ctx > 0) {
-    const int last = ctx - 1;
-    r.place = static_cast<int64_t>(p.block_table[static_cast<int64_t>(w.b) * p.bt_stride + last / p.block_size]) * p.block_size +
-              last % p.block_size;
-  }
-  return r;
+// STORE launches (no work list, at most kRowLanes sequences) bring this step's key and value rows along and give what store_kvcache
+// in front of the launch would give: no cache row that the step writes is read from the cache. Every lane holds one row's slot; a
+// wave finds the slots among the tokens of a chunk with one vote, whichever sequence's table names them, and takes those tokens
+// from the inputs. Each row is written once, by a workgroup that the workgroup index alone names, and nobody waits for it.
+// The slots are requested with the kernel's first loads, the rows are written behind the loop. It saves the store's launch: a layer's
+// step at 4 x 512 ragged tokens, 16q/8kv, takes 10.0 us in a replayed graph, 11.4 in two launches; at 32 x 32768, 32q/8kv, 653
+// against 654. Models that store in lv_qk_norm_rope_store (the fused default) have no such launch to save.
+__device__ __forceinline__ int row_slot(const DecodeParams& p) {
+  const int lane = threadIdx.x & 63;
+  const int slot = lane < p.batch ? p.slot_mapping[lane] : -1;
+  return slot < p.num_slots ? slot : -1;
 }
-__device__ __forceinline__ void write_row(const DecodeParams& p, const DecodeWork& w, const NewRow& r) {
+__device__ __forceinline__ void write_row(const DecodeParams& p) {
   constexpr int c = kHeadDim / 8;
-  const int tid = threadIdx.x, at = w.kvh * kHeadDim + 8 * (tid % c);
-  if (!r.write || r.slot < 0 || r.slot >= p.num_slots || tid >= 2 * c) return;
-  const uint16_t* src = tid >= c ? p.v_new + w.b * p.v_new_stride0 : p.k_new + w.b * p.k_new_stride0;
+  const int tid = threadIdx.x, bk = blockIdx.x / p.nsplit;
+  if (blockIdx.x % p.nsplit != 0 || tid >= 2 * c) return;
+  const int row = bk % p.batch, at = bk / p.batch * kHeadDim + 8 * (tid % c);
+  const int64_t slot = p.slot_mapping[row];
+  if (slot < 0 || slot >= p.num_slots) return;
+  const uint16_t* src = tid >= c ? p.v_new + row * p.v_new_stride0 : p.k_new + row * p.k_new_stride0;
   uint16_t* cache = const_cast<uint16_t*>(tid >= c ? p.v_cache : p.k_cache);
-  *reinterpret_cast<u32x4*>(cache + r.slot * p.num_kv_heads * kHeadDim + at) = *reinterpret_cast<const u32x4*>(src + at);
+  *reinterpret_cast<u32x4*>(cache + slot * p.num_kv_heads * kHeadDim + at) = *reinterpret_cast<const u32x4*>(src + at);
+}
+// This step's rows among `count` tokens from cache row `row0` on: a bit for each; off: the token of this lane's row.
+struct FreshRows {
+  uint64_t hit = 0;
+  int off = 0;
+};
+__device__ __forceinline__ FreshRows fresh_rows(int slot, int64_t row0, int count) {
+  const int64_t d = slot - row0;
+  return {__builtin_amdgcn_ballot_w64(slot >= 0 && d >= 0 && d < count), static_cast<int>(d)};
 }
 
 // NW waves: 4, or 8 (see launch_group).
@@ -151,7 +149,10 @@ __global__ __launch_bounds__(64 * NW) void decode_attn_kernel(const DecodeParams
   // the heads of a sequence are read concurrently (kv head fastest, or 8 sequences x 8 rotated
   // heads in adjacent workgroups).
   DecodeWork dw;
-  if (!decode_work(p, dw)) return;
+  if (!decode_work(p, dw)) {
+    if constexpr (STORE) write_row(p);
+    return;
+  }
   const int nsplit = dw.nsplit, split = dw.split, b = dw.b, kvh = dw.kvh;
 
   const int tid = threadIdx.x;
@@ -173,13 +174,8 @@ __global__ __launch_bounds__(64 * NW) void decode_attn_kernel(const DecodeParams
 
   const int64_t row_elems = static_cast<int64_t>(Hkv) * kHeadDim;
   const int32_t* bt_row = p.block_table + static_cast<int64_t>(b) * p.bt_stride;
-  NewRow fresh;
-  const uint16_t *k_own = nullptr, *v_own = nullptr;
-  if constexpr (STORE) {
-    fresh = new_row(p, dw, ctx, t1);
-    k_own = p.k_new + b * p.k_new_stride0 + kvh * kHeadDim + 8 * i;
-    v_own = p.v_new + b * p.v_new_stride0 + kvh * kHeadDim + 8 * i;
-  }
+  int slot = -1;
+  if constexpr (STORE) slot = row_slot(p);
 
   // q fragments: 8 dims of each of the G heads, kept packed as bf16 pairs.
   u32x4 qv[G];
@@ -198,12 +194,10 @@ __global__ __launch_bounds__(64 * NW) void decode_attn_kernel(const DecodeParams
     for (int d = 0; d < 8; ++d) acc[h][d] = 0.f;
   }
 
-  // Element offset of (first token of chunk c, this kv head, this lane's 16-byte chunk).
-  auto chunk_base = [&](int c) -> int64_t {
+  // Cache row of the first token of chunk c; a chunk lies in one block.
+  auto chunk_row = [&](int c) -> int64_t {
     const int t = t0 + c * TOK;
-    const int blk = bt_row[t / BS];
-    const int64_t row = static_cast<int64_t>(blk) * BS + (t % BS);
-    return (row * Hkv + kvh) * kHeadDim + 8 * i;
+    return static_cast<int64_t>(bt_row[t / BS]) * BS + (t % BS);
   };
   // Token offset inside chunk c for load slot u; rows past the split's end are redirected
   // to its last valid row (their scores are masked below), so no out-of-range row is read.
@@ -211,31 +205,46 @@ __global__ __launch_bounds__(64 * NW) void decode_attn_kernel(const DecodeParams
     const int last = ntok - 1 - c * TOK;
     return min(4 * u + g, last);
   };
-  // The U rows of chunk c; in the split's last chunk the lanes at its last token look at the step's own row.
-  auto load_rows = [&](u32x4 (&to)[U], const uint16_t* cache, const uint16_t* own_row, int c, int64_t base) __attribute__((always_inline)) {
-    if (STORE && c == nchunks - 1 && fresh.own()) {
-      const int last = ntok - 1 - c * TOK;
+  // This lane's pieces of the U rows of chunk c, which starts at cache row `row`.
+  auto load_rows = [&](u32x4 (&to)[U], const uint16_t* cache, const uint16_t* fresh, int64_t fresh_stride, int c, int64_t row,
+                       const FreshRows& f) __attribute__((always_inline)) {
+    const int64_t base = (row * Hkv + kvh) * kHeadDim + 8 * i;
+    if (STORE && f.hit != 0) {
+      const uint16_t* at[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) to[u] = load16<NT>(4 * u + g >= last ? own_row : cache + base + tok_off(c, u) * row_elems);
+      for (int u = 0; u < U; ++u) at[u] = cache + base + tok_off(c, u) * row_elems;
+      for (uint64_t left = f.hit; left != 0; left &= left - 1) {
+        const int j = __builtin_ctzll(left), off = __builtin_amdgcn_readlane(f.off, j);
+        const uint16_t* own = fresh + j * fresh_stride + kvh * kHeadDim + 8 * i;
+#pragma unroll
+        for (int u = 0; u < U; ++u) at[u] = tok_off(c, u) == off ? own : at[u];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) to[u] = load16<NT>(at[u]);
     } else {
 #pragma unroll
       for (int u = 0; u < U; ++u) to[u] = load16<NT>(cache + base + tok_off(c, u) * row_elems);
     }
+  };
+  auto fresh_of = [&](int c, int64_t row) __attribute__((always_inline)) {
+    return STORE ? fresh_rows(slot, row, min(TOK, ntok - c * TOK)) : FreshRows{};
   };
 
   int c = wave;
   if (c < nchunks) {
     u32x4 kb[U], vb[U];
     {
-      const int64_t base = chunk_base(c);
-      load_rows(kb, p.k_cache, k_own, c, base);
-      load_rows(vb, p.v_cache, v_own, c, base);
+      const int64_t row = chunk_row(c);
+      const FreshRows f = fresh_of(c, row);
+      load_rows(kb, p.k_cache, p.k_new, p.k_new_stride0, c, row, f);
+      load_rows(vb, p.v_cache, p.v_new, p.v_new_stride0, c, row, f);
     }
     for (; c < nchunks; c += NW) {
       const int cn = c + NW;
       const bool has_next = cn < nchunks;
-      int64_t base_n = 0;
-      if (has_next) base_n = chunk_base(cn);
+      int64_t row_n = 0;
+      if (has_next) row_n = chunk_row(cn);
+      const FreshRows fresh_n = has_next ? fresh_of(cn, row_n) : FreshRows{};
 
       // ---- scores: s[u][h] = log2(e) * scale * <q_h, k_u>
       float s[U][G];
@@ -255,7 +264,7 @@ __global__ __launch_bounds__(64 * NW) void decode_attn_kernel(const DecodeParams
           s[u][h] = d;
         }
       }
-      if (has_next) load_rows(kb, p.k_cache, k_own, cn, base_n);
+      if (has_next) load_rows(kb, p.k_cache, p.k_new, p.k_new_stride0, cn, row_n, fresh_n);
       const int valid = ntok - c * TOK;  // tokens of this chunk inside the split
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -308,11 +317,11 @@ __global__ __launch_bounds__(64 * NW) void decode_attn_kernel(const DecodeParams
           for (int h = 0; h < G; ++h) acc[h][u & 7] = fmaf(s[u][h], vx, acc[h][u & 7]);
         }
       }
-      if (has_next) load_rows(vb, p.v_cache, v_own, cn, base_n);
+      if (has_next) load_rows(vb, p.v_cache, p.v_new, p.v_new_stride0, cn, row_n, fresh_n);
     }
   }
 
-  if constexpr (STORE) write_row(p, dw, fresh);
+  if constexpr (STORE) write_row(p);
 
   // ---- merge the 4 token groups of the wave (lanes ^16, ^32)
 #pragma unroll
@@ -415,7 +424,10 @@ __global__ __launch_bounds__(64 * NW, 2) void decode_mfma_kernel(const DecodePar
 
   const int Hkv = p.num_kv_heads;
   DecodeWork dw;
-  if (!decode_work(p, dw)) return;
+  if (!decode_work(p, dw)) {
+    if constexpr (STORE) write_row(p);
+    return;
+  }
   const int nsplit = dw.nsplit, split = dw.split, b = dw.b, kvh = dw.kvh;
 
   const int tid = threadIdx.x;
@@ -435,13 +447,8 @@ __global__ __launch_bounds__(64 * NW, 2) void decode_mfma_kernel(const DecodePar
   const int nchunks = ntok > 0 ? (ntok + CH - 1) / CH : 0;
   const int64_t row_bytes = static_cast<int64_t>(Hkv) * kHeadDim * 2;
   const int32_t* bt_row = p.block_table + static_cast<int64_t>(b) * p.bt_stride;
-  NewRow fresh;
-  const char *k_own = nullptr, *v_own = nullptr;
-  if constexpr (STORE) {
-    fresh = new_row(p, dw, ctx, t1);
-    k_own = reinterpret_cast<const char*>(p.k_new + b * p.k_new_stride0 + kvh * kHeadDim) + 16 * q;
-    v_own = reinterpret_cast<const char*>(p.v_new + b * p.v_new_stride0 + kvh * kHeadDim) + 16 * c16;
-  }
+  int slot = -1;
+  if constexpr (STORE) slot = row_slot(p);
 
   // Q^T fragments (B operand), k-step s covers d = 32s .. 32s+31; heads >= G are zero columns
   bf16x8_t qf[4];
@@ -483,34 +490,50 @@ __global__ __launch_bounds__(64 * NW, 2) void decode_mfma_kernel(const DecodePar
     return static_cast<int64_t>(blk) * BS + (t % BS);
   };
   u32x4 kreg[2][4], vreg[8];
-  auto issue_k = [&](int c) {
-    const char* base = reinterpret_cast<const char*>(p.k_cache) + chunk_row(c) * row_bytes + kvh * (kHeadDim * 2);
+  auto fresh_of = [&](int c, int64_t row) __attribute__((always_inline)) {
+    return STORE ? fresh_rows(slot, row, min(CH, ntok - c * CH)) : FreshRows{};
+  };
+  // the address of token `tok` of a chunk among the step's rows, if it is one of them
+  auto redirect = [&](const char* rp, int tok, const uint16_t* fresh, int64_t stride, int byte, const FreshRows& f)
+                      __attribute__((always_inline)) {
+    for (uint64_t left = f.hit; left != 0; left &= left - 1) {
+      const int j = __builtin_ctzll(left), off = __builtin_amdgcn_readlane(f.off, j);
+      rp = tok == off ? reinterpret_cast<const char*>(fresh + j * stride + kvh * kHeadDim) + byte : rp;
+    }
+    return rp;
+  };
+  auto issue_k = [&](int c, int64_t row, const FreshRows& f) {
+    const char* base = reinterpret_cast<const char*>(p.k_cache) + row * row_bytes + kvh * (kHeadDim * 2);
     const int last = ntok - 1 - c * CH;  // rows past the split's end re-read its last row (masked below)
-    const bool own = STORE && c == nchunks - 1 && fresh.own();
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const char* rp = base + static_cast<int64_t>(min(16 * t + a_key, last)) * row_bytes + 16 * q;
-      if (STORE && own && 16 * t + a_key >= last) rp = k_own;
+      const int tok = min(16 * t + a_key, last);
+      const char* rp = base + static_cast<int64_t>(tok) * row_bytes + 16 * q;
+      if constexpr (STORE) rp = redirect(rp, tok, p.k_new, p.k_new_stride0, 16 * q, f);
 #pragma unroll
       for (int s = 0; s < 4; ++s) kreg[t][s] = load16<true>(reinterpret_cast<const uint16_t*>(rp + 64 * s));
     }
   };
-  auto issue_v = [&](int c) {
-    const char* base = reinterpret_cast<const char*>(p.v_cache) + chunk_row(c) * row_bytes + kvh * (kHeadDim * 2) + 16 * c16;
+  auto issue_v = [&](int c, int64_t row, const FreshRows& f) {
+    const char* base = reinterpret_cast<const char*>(p.v_cache) + row * row_bytes + kvh * (kHeadDim * 2) + 16 * c16;
     const int last = ntok - 1 - c * CH;
-    const bool own = STORE && c == nchunks - 1 && fresh.own();
+    const char* at[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const char* rp = base + static_cast<int64_t>(min(4 * u + q, last)) * row_bytes;
-      if (STORE && own && 4 * u + q >= last) rp = v_own;
-      vreg[u] = load16<true>(reinterpret_cast<const uint16_t*>(rp));
+    for (int u = 0; u < 8; ++u) at[u] = base + static_cast<int64_t>(min(4 * u + q, last)) * row_bytes;
+    if (STORE && f.hit != 0) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) at[u] = redirect(at[u], min(4 * u + q, last), p.v_new, p.v_new_stride0, 16 * c16, f);
     }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) vreg[u] = load16<true>(reinterpret_cast<const uint16_t*>(at[u]));
   };
 
   int c = wave;
   if (c < nchunks) {
-    issue_k(c);
-    issue_v(c);
+    const int64_t row = chunk_row(c);
+    const FreshRows f = fresh_of(c, row);
+    issue_k(c, row, f);
+    issue_v(c, row, f);
   }
   for (; c < nchunks; c += NW) {
     const int cn = c + NW;
@@ -521,7 +544,13 @@ __global__ __launch_bounds__(64 * NW, 2) void decode_mfma_kernel(const DecodePar
       s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kreg[0][s]), qf[s], s0, 0, 0, 0);
       s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kreg[1][s]), qf[s], s1, 0, 0, 0);
     }
-    if (cn < nchunks) issue_k(cn);
+    int64_t row_n = 0;
+    FreshRows fresh_n;
+    if (cn < nchunks) {
+      row_n = chunk_row(cn);
+      fresh_n = fresh_of(cn, row_n);
+      issue_k(cn, row_n, fresh_n);
+    }
     // ---- scale, mask keys past the split's end, row maximum over the chunk's 32 keys
     const int valid = ntok - c * CH;
     float sv[8];
@@ -558,7 +587,7 @@ __global__ __launch_bounds__(64 * NW, 2) void decode_mfma_kernel(const DecodePar
 #pragma unroll
     for (int u = 0; u < 8; ++u)
       *reinterpret_cast<__attribute__((address_space(3))) u32x4*>(vimg + ((vw_off ^ (16 * (u & 3))) + 1024 * u)) = vreg[u];
-    if (cn < nchunks) issue_v(cn);
+    if (cn < nchunks) issue_v(cn, row_n, fresh_n);
     // ---- O^T += V^T P^T, one 16-column block of d per MFMA
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) {
@@ -576,7 +605,7 @@ __global__ __launch_bounds__(64 * NW, 2) void decode_mfma_kernel(const DecodePar
     }
   }
 
-  if constexpr (STORE) write_row(p, dw, fresh);
+  if constexpr (STORE) write_row(p);
 
   // ---- row sums: every 16-lane group holds a share
   l_run += __shfl_xor(l_run, 16);

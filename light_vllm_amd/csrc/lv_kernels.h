@@ -5,6 +5,8 @@
 
 namespace lv {
 
+constexpr int kRowLanes = 64;   // sequences of a decode launch that stores their rows: a lane each
+
 struct DecodeParams {
   const uint16_t* q;
   const uint16_t* k_cache;

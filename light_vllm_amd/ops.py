@@ -283,9 +283,8 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     from the host's lengths that cuts long sequences into more pieces than short ones; num_splits
     and seq_order are then ignored. With plan_max_splits (a captured graph's fixed workspace row
     capacity) attribute absent the plan's own max_splits sizes the workspace.
-    new_kv: optional (key, value, slot_mapping) of store_kvcache, one row per sequence: the rows of the tokens that
-    context_lens counts last. They are stored as store_kvcache would before the attention, in one launch with it (in two with a
-    plan or static_scratch).
+    new_kv: optional (key, value, slot_mapping) of store_kvcache, one row per sequence. They are stored as store_kvcache would
+    before the attention; batches of up to 64 sequences store them in the attention's launch (not with a plan or static_scratch).
     """
     dev = _require_gpu(q, k_cache, v_cache, context_lens, block_table)
     B, Hq, D = q.shape

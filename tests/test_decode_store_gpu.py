@@ -112,3 +112,57 @@ def test_attention_module_replays_in_a_graph():
         torch.cuda.synchronize()
         assert torch.equal(attn.k_cache, kc) and torch.equal(attn.v_cache, vc)
         assert (out.view(4, 16, D).float() - want.float()).abs().max().item() <= ATOL
+
+
+def several_rows(ctx, rows, Hq, Hkv, seed=0):
+    """`rows` tokens of one sequence behind `ctx` tokens, each a row of the batch with the same pages, and a sequence of its own."""
+    c = case([ctx + rows, 70], Hq, Hkv, seed=seed)
+    gen = torch.Generator(device="cuda").manual_seed(seed + 1)
+    B = rows + 1
+
+    def rn(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen).bfloat16()
+
+    table = c["table"].tolist()
+    slots = [table[0][j // BS] * BS + j % BS for j in range(ctx, ctx + rows)] + [table[1][0] * BS + 69]
+    c.update(q=rn(B, Hq, D), k=rn(B, Hkv, D), v=rn(B, Hkv, D), table=torch.tensor([table[0]] * rows + [table[1]], dtype=torch.int32, device="cuda"),
+             ctx=torch.tensor([ctx + i + 1 for i in range(rows)] + [70], dtype=torch.int32, device="cuda"), slots=slots)
+    return c
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(16, 8), (32, 8), (8, 1), (40, 8)])
+@pytest.mark.parametrize("kernel", ["auto", "mfma"])
+@pytest.mark.parametrize("ctx,rows", [(0, 5), (30, 4), (250, 16), (500, 63), (500, 64)])
+def test_rows_that_read_each_others_tokens(Hq, Hkv, kernel, ctx, rows):
+    """Tokens of one sequence as rows of the batch: every row sees the tokens of the rows before it, as after a store."""
+    c = several_rows(ctx, rows, Hq, Hkv, seed=ctx + rows)
+    for splits in (0, 1, 3, 16):
+        both(c, c["slots"], num_splits=splits, kernel=kernel)
+    both(c, c["slots"], num_splits=2, kernel=kernel, seq_order=torch.arange(rows, -1, -1, dtype=torch.int32, device="cuda"))
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(16, 8), (32, 8), (8, 1)])
+def test_slots_inside_contexts(Hq, Hkv):
+    """A row stored over an earlier token of its own sequence, or over another sequence's token, is what that token reads as."""
+    c = case([300, 700, 40, 513], Hq, Hkv, seed=Hq)
+    table = c["table"].tolist()
+
+    def at(b, j):
+        return table[b][j // BS] * BS + j % BS
+
+    for splits in (0, 1, 4, 16):
+        both(c, [at(0, 17), at(1, 699), at(2, 0), at(3, 256)], num_splits=splits)
+        both(c, [at(1, 3), at(1, 2), at(3, 512), at(1, 640)], num_splits=splits)
+
+
+def test_an_order_that_leaves_rows_out_still_stores_them():
+    c = case([300, 40, 700], 16, 8)
+    order = torch.tensor([2, 2, 9], dtype=torch.int32, device="cuda")
+    slots = torch.tensor(c["slots"], dtype=torch.int32, device="cuda")
+    kc, vc = c["kc"].clone(), c["vc"].clone()
+    ops.store_kvcache(c["k"], c["v"], kc, vc, slots)
+    want = ops.decode_attention(c["q"], kc, vc, c["ctx"], c["table"], D ** -0.5)
+    kc2, vc2 = c["kc"].clone(), c["vc"].clone()
+    got = ops.decode_attention(c["q"], kc2, vc2, c["ctx"], c["table"], D ** -0.5, new_kv=(c["k"], c["v"], slots), seq_order=order)
+    assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
+    assert (got[2].float() - want[2].float()).abs().max().item() <= ATOL
