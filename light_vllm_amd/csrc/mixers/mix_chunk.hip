@@ -58,8 +58,8 @@ __device__ __forceinline__ float chunk_lane(float x, int i) {
 __device__ __forceinline__ int acc_row(int i, int half) { return 8 * (i >> 2) + 4 * half + (i & 3); }
 
 // x / (1 + exp(-x)) in about half the instructions of siluf_, to the same two units in the last place: the exponent as a sum of
-// two floats in front of the hardware exp2, the hardware reciprocal with one Newton step behind it. Where exp(-x) would
-// overflow, x is multiplied by 1e-38.
+// two floats in front of the hardware exp2, the hardware reciprocal with one Newton step behind it. Below -87, where the
+// function is within 1.5e-36 of zero and exp(-x) would overflow, zero (a NaN for -infinity, as siluf_).
 __device__ __forceinline__ float chunk_silu(float x) {
   constexpr float kLog2e = 1.44269504f, kLog2eRest = 1.92596303e-8f, kLn2 = 0.69314718f;
   const float c = __builtin_amdgcn_fmed3f(x, -87.0f, 87.0f);
@@ -69,7 +69,7 @@ __device__ __forceinline__ float chunk_silu(float x) {
   const float d = 1.0f + e;
   float q = __builtin_amdgcn_rcpf(d);
   q = fmaf(q, fmaf(-d, q, 1.0f), q);
-  return x * q;
+  return x * (x < -87.0f ? 0.0f : q);
 }
 template <bool SILU>
 __device__ __forceinline__ float4 chunk_act(float4 x) {

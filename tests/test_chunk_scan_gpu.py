@@ -143,3 +143,23 @@ def test_misaligned_rows_and_captured_steps_take_the_token_loop(kind, pad, monke
     assert torch.equal(o_static, o_token) and torch.equal(s_static, s_token)
     o_auto = call(s_auto, make_step(new, [0, 2]))        # aligned and not captured: the same numbers in another order
     assert rel(o_auto, o_token.to(F64)) < REL and rel(s_auto, s_token.to(F64)) < REL
+
+
+def test_silu_of_large_arguments():
+    """Constant decays read their rows through silu: zero far below zero (not a small multiple of the argument), the argument far
+    above. Values of 1e-36 and less are taken as zero."""
+    H, D, Dv, new = 2, 64, 64, [96]
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    proj = torch.randn(96, 2 * H * D + H * Dv, device="cuda", generator=gen).bfloat16()
+    proj[3, ::3] = -3e38
+    proj[7, 1::2] = -1e30
+    proj[11, ::5] = -88.5
+    proj[13, ::4] = -86.0
+    proj[17, ::7] = 200.0
+    decay = torch.full((H,), 0.9, device="cuda")
+    x = F.silu(proj.to(F64))
+    q, k, v = x[:, :H * D].view(96, H, D), x[:, H * D:2 * H * D].view(96, H, D), x[:, 2 * H * D:].reshape(96, H, Dv)
+    step, state = make_step(new, [0]), torch.zeros(1, H, D, Dv, device="cuda")
+    want_o, want_s = recurrence(q, k, v, decay.to(F64).expand(96, H), None, state, step)
+    o = mix_ops.lightning_attention(proj, 0, H * D, 2 * H * D, decay, state, step, H, D, Dv)
+    assert rel(o, want_o) < REL and rel(state, want_s) < REL
