@@ -187,6 +187,7 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
       else x = (prod[0][t * RS + r] + prod[1][t * RS + r]) + (prod[2][t * RS + r] + prod[3][t * RS + r]);
       x *= dm[i];
       if constexpr (!DELTA) x *= wr;
+      x = r <= t ? x : 0.0f;                           // selected: what a later token brings may not be finite
       if (t < cn) p.P[((t0 + 8 * (i >> 2) + (i & 3)) * p.H + h) * kCh + p_off] = x;
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -219,7 +220,7 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
       }
 #pragma unroll
       for (int t = 0; t < kCh; ++t)
-        if (t < cn && (t & 1) == half) p.Tm[((t0 + t) * p.H + h) * kCh + r] = x[t] * wr;
+        if (t < cn && (t & 1) == half) p.Tm[((t0 + t) * p.H + h) * kCh + r] = r <= t ? x[t] * wr : 0.0f;
       __builtin_amdgcn_wave_barrier();
     }
   }
@@ -329,6 +330,30 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
   };
   auto scale4 = [&](f32x4 x, float4 f) __attribute__((always_inline)) { return f32x4{x[0] * f.x, x[1] * f.y, x[2] * f.z, x[3] * f.w}; };
   const f32x4 zero{0.0f, 0.0f, 0.0f, 0.0f};
+  // y += m x for a lower triangular m. The products run over whole 16 x 16 blocks, in which a token's value meets the zeros of the
+  // tokens before it: one that is not finite would reach them, so a wave that sees one goes token by token.
+  auto triangle = [&](f32x4 (&y)[2], const float* m, const f32x4 (&x)[2]) __attribute__((always_inline)) {
+    float z = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) z = fmaf(x[i >> 2][i & 3], 0.0f, z);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(z != 0.0f) == 0, 1)) {
+      y[0] += mul4(zero, left(m, PS, 0, 0), x[0]);
+      y[1] += mul4(mul4(zero, left(m, PS, 1, 0), x[0]), left(m, PS, 1, 1), x[1]);
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll 1
+      for (int from = 0; from < 4; ++from) {
+        const int j = 16 * (i >> 2) + 4 * from + (i & 3);
+        const float v = __shfl(x[i >> 2][i & 3], 16 * from + r, kWave);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const int t = 16 * (k >> 2) + 4 * quad + (k & 3);
+          y[k >> 2][k & 3] = j <= t ? fmaf(m[t * PS + j], v, y[k >> 2][k & 3]) : y[k >> 2][k & 3];
+        }
+      }
+  };
   f32x4 U_next[2];
   auto stage = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
@@ -376,16 +401,15 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
         f32x4 rest[2];
 #pragma unroll
         for (int x = 0; x < 2; ++x) rest[x] = U[x] - scale4(ks[0][x] + ks[1][x], rows4(ge_lds[hw], x));
-        U[0] = mul4(zero, left(pt_lds[HPW + hw], PS, 0, 0), rest[0]);               // T is lower triangular
-        U[1] = mul4(mul4(zero, left(pt_lds[HPW + hw], PS, 1, 0), rest[0]), left(pt_lds[HPW + hw], PS, 1, 1), rest[1]);
+        U[0] = U[1] = zero;
+        triangle(U, pt_lds[HPW + hw], rest);
       }
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
         o[x] = scale4((qs[0][x] + qs[1][x]) + (qs[2][x] + qs[3][x]), rows4(ge_lds[hw], x));
         if constexpr (KIND == kChunkStep) o[x] += skip * U[x];
       }
-      o[0] += mul4(zero, left(pt_lds[hw], PS, 0, 0), U[0]);
-      o[1] += mul4(mul4(zero, left(pt_lds[hw], PS, 1, 0), U[0]), left(pt_lds[hw], PS, 1, 1), U[1]);
+      triangle(o, pt_lds[hw], U);
     }
 #pragma unroll
     for (int x = 0; x < 2; ++x) u2[x] = scale4(U[x], rows4(ge_lds[hw] + kCh, x));

@@ -163,3 +163,57 @@ def test_silu_of_large_arguments():
     want_o, want_s = recurrence(q, k, v, decay.to(F64).expand(96, H), None, state, step)
     o = mix_ops.lightning_attention(proj, 0, H * D, 2 * H * D, decay, state, step, H, D, Dv)
     assert rel(o, want_o) < REL and rel(state, want_s) < REL
+
+
+def test_a_bad_token_reaches_no_earlier_one():
+    """An infinity or a NaN in a token's query, key, value, write strength or decay leaves the outputs of every token before it and of
+    every other sequence and head as they were (bit for bit before its chunk; inside, sums in another order); outputs behind a bad
+    key or value are not finite."""
+    G, H, D, Dv, new = 2, 4, 128, 128, [100, 70]
+    gen = torch.Generator(device="cuda").manual_seed(4)
+
+    def rn(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen)
+
+    T, step = sum(new), make_step(new, [3, 0])
+    delta = dict(q=F.normalize(rn(T, G, D), dim=-1), k=F.normalize(rn(T, G, D), dim=-1), v=rn(T, H, Dv), beta=torch.sigmoid(rn(T, H)),
+                 decay=torch.sigmoid(rn(T, H) + 2))
+    steps = {n: rn(T, c).bfloat16() for n, c in (("q", G * D), ("k", G * D), ("v", H * Dv), ("a", H))}
+    const = rn(T, 2 * H * D + H * Dv).bfloat16()
+    small = [0.5 * rn(H) for _ in range(3)]
+    rate = torch.full((H,), 0.95, device="cuda")
+
+    def run_delta(x, st):
+        return mix_ops.gated_delta_rule(x["q"], x["k"], x["v"], x["beta"], x["decay"], st, step)
+
+    def run_step(x, st):
+        return mix_ops.gated_scan(mix_ops.SCAN_STEP, x["q"], x["k"], x["v"], x["a"], small[0], small[1], step, st, H, G, D, Dv, p2=small[2])
+
+    def run_const(x, st):
+        return mix_ops.lightning_attention(x["p"], 0, H * D, 2 * H * D, rate, st, step, H, D, Dv)
+
+    for run, inputs, carried in ((run_delta, delta, ("k", "v", "beta", "decay")), (run_step, steps, ("k", "v", "a")), (run_const, dict(p=const), ("p",))):
+        state = rn(2, H, D, Dv)
+        clean = run(inputs, state.clone())
+        for name, x in inputs.items():
+            for at in (0, 5, 15, 16, 31, 32, 50, 99):
+                for bad in (float("nan"), float("inf")):
+                    y = x.clone()
+                    y[at] = bad                        # (silu leaves +inf, softplus too)
+                    st = state.clone()
+                    o = run({**inputs, name: y}, st)
+                    chunk = at // 32 * 32
+                    assert torch.equal(o[:chunk], clean[:chunk]) and torch.equal(o[100:], clean[100:]), (name, at, bad)
+                    assert at == chunk or rel(o[chunk:at], clean[chunk:at].to(F64)) < REL, (name, at, bad)
+                    if name in carried and name != "beta" and not (bad > 0 and name in ("a", "decay")):
+                        assert not bool(torch.isfinite(o[at]).any()) and not bool(torch.isfinite(st[1]).any()), (name, at, bad)
+    # one value column of one head: the others stay clean, bit for bit
+    y = {**delta, "v": delta["v"].clone()}
+    y["v"][40, 1, 17] = float("inf")
+    st = torch.zeros(2, H, D, Dv, device="cuda")
+    clean = run_delta(delta, st.clone())
+    o = run_delta(y, st)
+    keep = torch.ones(H, Dv, dtype=torch.bool, device="cuda")
+    keep[1, 17] = False
+    assert torch.equal(o[:32], clean[:32]) and rel(o[:40], clean[:40].to(F64)) < REL and rel(o[:, keep], clean[:, keep].to(F64)) < REL
+    assert not bool(torch.isfinite(o[40:100, 1, 17]).any())
