@@ -32,6 +32,7 @@ namespace lvmix {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 constexpr int kCh = 32;               // tokens of a chunk
 constexpr int kPad = 4;               // floats behind every LDS row: 16-byte reads of 8 rows meet 8 different bank groups
 
@@ -97,23 +98,56 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
     const int shares = DELTA ? 2 : 4, share = DELTA ? (w & 1) : w;
     const T* left = static_cast<const T*>(kk ? p.k : p.q) + (t0 + r) * (kk ? p.ldk : p.ldq) + static_cast<int64_t>(g) * p.D;
     const T* right = static_cast<const T*>(p.k) + (t0 + r) * p.ldk + static_cast<int64_t>(g) * p.D;
-    const bool in = r < cn;
-    f32x16 acc, acc2;                                  // two sums of half the length: half the roundings each
+    if (DELTA && !kk) {
+      // q k^T in 64 bits: read-outs are sums of few of these products, each a small difference of large terms. Summed in f32 they
+      // were most of an output's error (1.33e-7 at heads of 128 x 128; 0.86e-7 with these, 0.95e-7 in the token loop).
+      const int r16 = lane & 15, quad = lane >> 4;
+      f64x4 acc[2][2];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = acc2[i] = 0.0f;
-    for (int d = share * 8; d < p.D; d += shares * 8) {
-      float4 x{0, 0, 0, 0}, y{0, 0, 0, 0};
-      if (in) {
-        x = chunk_act<SILU>(ld4(left + d + 4 * half));
-        y = chunk_act<SILU>(ld4(right + d + 4 * half));
+      for (int x = 0; x < 4; ++x) acc[x >> 1][x & 1] = f64x4{0.0, 0.0, 0.0, 0.0};
+      const T* q16 = static_cast<const T*>(p.q) + (t0 + r16) * p.ldq + static_cast<int64_t>(g) * p.D + 4 * quad;
+      const T* k16 = static_cast<const T*>(p.k) + (t0 + r16) * p.ldk + static_cast<int64_t>(g) * p.D + 4 * quad;
+      for (int d = share * 16; d < p.D; d += 32) {
+        float4 x[2], y[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const bool in = 16 * e + r16 < cn;
+          x[e] = in ? ld4(q16 + 16 * e * p.ldq + d) : float4{0, 0, 0, 0};
+          y[e] = in ? ld4(k16 + 16 * e * p.ldk + d) : float4{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          f64x4& to = acc[e >> 1][e & 1];
+          const float4 a = x[e >> 1], b = y[e & 1];
+          to = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, to, 0, 0, 0);
+          to = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.y, to, 0, 0, 0);
+          to = __builtin_amdgcn_mfma_f64_16x16x4f64(a.z, b.z, to, 0, 0, 0);
+          to = __builtin_amdgcn_mfma_f64_16x16x4f64(a.w, b.w, to, 0, 0, 0);
+        }
       }
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, y.x, acc, 0, 0, 0);
-      acc2 = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, y.y, acc2, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, y.z, acc, 0, 0, 0);
-      acc2 = __builtin_amdgcn_mfma_f32_32x32x2f32(x.w, y.w, acc2, 0, 0, 0);
-    }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) prod[w][acc_row(i, half) * RS + r] = acc[i] + acc2[i];
+      for (int e = 0; e < 4; ++e)                      // (its result rows are lane / 16 + 4 i)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) prod[w][(16 * (e >> 1) + quad + 4 * i) * RS + 16 * (e & 1) + r16] = static_cast<float>(acc[e >> 1][e & 1][i]);
+    } else {
+      const bool in = r < cn;
+      f32x16 acc, acc2;                                  // two sums of half the length: half the roundings each
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[i] = acc2[i] = 0.0f;
+      for (int d = share * 8; d < p.D; d += shares * 8) {
+        float4 x{0, 0, 0, 0}, y{0, 0, 0, 0};
+        if (in) {
+          x = chunk_act<SILU>(ld4(left + d + 4 * half));
+          y = chunk_act<SILU>(ld4(right + d + 4 * half));
+        }
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, y.x, acc, 0, 0, 0);
+        acc2 = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, y.y, acc2, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, y.z, acc, 0, 0, 0);
+        acc2 = __builtin_amdgcn_mfma_f32_32x32x2f32(x.w, y.w, acc2, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) prod[w][acc_row(i, half) * RS + r] = acc[i] + acc2[i];
+    }
   }
   __syncthreads();
   const int rep = p.H / p.G;
@@ -138,7 +172,7 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
     } else {
       wr = 0.0f;
     }
-    // G_t and E_t, lane = t; D_tj, lane = j with t in the result layout's registers. The products are formed in 64 bits and
+    // G_t and E_t w_t, lane = t; D_tj w_j, lane = j with t in the result layout's registers (w = 1 but for step sizes). The products are formed in 64 bits and
     // rounded once: a constant decay rounds the same way at every step, and its error would grow with the tokens it spans.
     float gt = 1.0f, et = 1.0f;
     float dm[16];
@@ -163,7 +197,7 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
         const double gd = chunk_lane(dec, t);
         run *= gd;
         gt = r == t ? static_cast<float>(run) : gt;
-        col = r == t ? 1.0 : col * gd;                 // zero above the diagonal
+        col = r == t ? (DELTA ? 1.0 : static_cast<double>(wr)) : col * gd;       // zero above the diagonal
         const float colf = static_cast<float>(col);
         if (((t >> 2) & 1) == 0) dm[4 * (t >> 3) + (t & 3)] = colf;   // rows of the lower half of the lanes
         else dm[4 * (t >> 3) + (t & 3)] = half ? colf : dm[4 * (t >> 3) + (t & 3)];
@@ -171,13 +205,13 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int t = kCh - 1; t >= 0; --t) {
-        et = r == t ? static_cast<float>(back) : et;
+        et = r == t ? static_cast<float>(back * (DELTA ? 1.0 : static_cast<double>(wr))) : et;
         back *= chunk_lane(dec, t);
       }
     }
     if (half == 0 && r < cn) {
       p.Gf[(t0 + r) * p.H + h] = gt;
-      p.Ef[(t0 + r) * p.H + h] = DELTA ? et : et * wr;
+      p.Ef[(t0 + r) * p.H + h] = et;
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -186,7 +220,6 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
       if constexpr (DELTA) x = prod[2][t * RS + r] + prod[3][t * RS + r];
       else x = (prod[0][t * RS + r] + prod[1][t * RS + r]) + (prod[2][t * RS + r] + prod[3][t * RS + r]);
       x *= dm[i];
-      if constexpr (!DELTA) x *= wr;
       x = r <= t ? x : 0.0f;                           // selected: what a later token brings may not be finite
       if (t < cn) p.P[((t0 + 8 * (i >> 2) + (i & 3)) * p.H + h) * kCh + p_off] = x;
     }
@@ -269,7 +302,15 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
   }
   float skip = 0.0f;
   if (KIND == kChunkStep && FULL) skip = p.p2[h];
-  float seg_dec = 1.0f;
+  // a whole chunk's decay in two parts: a constant one, rounded, would be off the same way in every chunk
+  double g_chunk = 1.0, seg_dec = 1.0;
+  float g_rest = 0.0f;
+  if constexpr (KIND == kChunkConst) {
+    g_chunk = p.decay[h];
+#pragma unroll
+    for (int i = 1; i < kCh; i *= 2) g_chunk *= g_chunk;
+    g_rest = static_cast<float>(g_chunk - static_cast<double>(static_cast<float>(g_chunk)));
+  }
 
   // the next chunk's rows on their way: q and k four entries a thread, P and T too, a value for each of the wave's 32 x 16
   constexpr int KQ = kCh * D / 4 / NT, PN = (MATS * kCh * kCh / 4 + NT - 1) / NT, PX = PN > 0 ? PN : 1;
@@ -420,10 +461,17 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
     }
 #pragma unroll
     for (int j = 0; j < DT; ++j) {
-      S[j] *= g_last;
+      // constant decays, slow as a rule: what the chunk adds in two sums of its own, for fewer roundings at the state's magnitude
+      constexpr bool APART = KIND == kChunkConst;
+      f32x4 add[2] = {APART ? zero : S[j] * g_last, zero};
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(k_lds[(16 * (i >> 2) + 4 * quad + (i & 3)) * RS + 16 * j + r], u2[i >> 2][i & 3], S[j], 0, 0, 0);
+      for (int i = 0; i < 8; ++i) {
+        f32x4& to = add[APART ? i >> 2 : 0];
+        to = __builtin_amdgcn_mfma_f32_16x16x4f32(k_lds[(16 * (i >> 2) + 4 * quad + (i & 3)) * RS + 16 * j + r], u2[i >> 2][i & 3], to, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        S[j][i] = APART ? fmaf(S[j][i], g_last, fmaf(S[j][i], cn == kCh ? g_rest : 0.0f, add[0][i] + add[1][i])) : add[0][i];
     }
     if constexpr (FULL) {
 #pragma unroll
@@ -432,7 +480,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
         if (lo + 4 * quad < cn) p.o[(row0 + static_cast<int64_t>(c0 + lo) * p.H + h) * p.Dv + o_off] = o[i >> 2][i & 3];
       }
     }
-    seg_dec *= g_last;
+    if constexpr (MODE == 1) seg_dec *= KIND == kChunkConst ? g_chunk : static_cast<double>(g_last);      // (only whole chunks)
     __syncthreads();                                   // the next chunk is complete, and nobody reads this one any more
   }
   if (MODE == 1 || s1 == n_all) {
@@ -442,7 +490,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) to[(16 * j + i) * p.Dv + st_off] = S[j][i];
   }
-  if (MODE == 1 && lane == 0) p.seg_decay[(static_cast<int64_t>(b) * p.segs + blockIdx.y) * p.H + h] = seg_dec;
+  if (MODE == 1 && lane == 0) p.seg_decay[(static_cast<int64_t>(b) * p.segs + blockIdx.y) * p.H + h] = static_cast<float>(seg_dec);
 }
 
 // seg_state: what each segment adds -> the state that each segment starts from. A thread owns four entries of a head's state.
