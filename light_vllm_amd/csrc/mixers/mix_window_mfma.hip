@@ -567,7 +567,9 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WindowMfmaParams p,
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[d][i] = 0.0f;
   const float cs = FORM == kPlain ? p.scale * kLog2e : kLog2e;              // from what the products leave to the exponent of 2
-  float m = (p.sinks != nullptr ? p.sinks[h] : p.m0) * kLog2e, l = half == 0 ? p.sink : 0.0f;
+  // (a sink of -infinity counts nothing: a start far below any score, since a query may not see its first tiles)
+  const float sink = p.sinks != nullptr ? p.sinks[h] : p.m0;
+  float m = (sink < -1e30f ? -1e30f : sink) * kLog2e, l = half == 0 ? p.sink : 0.0f;
 
   auto compute = [&](int tile, int buf, lds_u8* kt) __attribute__((always_inline)) {
     const int phase = FIRST && tile < npt ? 0 : 1;

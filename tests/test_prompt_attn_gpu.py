@@ -95,3 +95,22 @@ def test_other_pages_and_sizes_keep_their_kernel(monkeypatch):
     both(monkeypatch, [80, 20], [9, 0], 4, 2, 48, 80, window=60)
     both(monkeypatch, [80, 20], [9, 0], 4, 1, 256, 192, same=True, window=60, keep_first=4)
     both(monkeypatch, [80, 20], [9, 0], 4, 1, 256, 192, window=60)
+
+
+@pytest.mark.parametrize("D,Dv,G", [(64, 64, 2), (128, 128, 1), (256, 192, 1)])
+@pytest.mark.parametrize("window", [1, 100, 1 << 30])
+def test_sinks_of_minus_infinity_count_nothing(monkeypatch, D, Dv, G, window):
+    step, pages = make_step([300, 33], [140, 0], 256, D)
+    gen = torch.Generator(device="cuda").manual_seed(D)
+    H, T = 4, 333
+    q, kc = (torch.randn(*s, device="cuda", generator=gen).bfloat16() for s in ((T, H * D), (pages, 256, G, D)))
+    vc = kc[..., :Dv]
+    if D != Dv:
+        args = (q, kc, vc, None, None, None, step, H, G, D, Dv, window, 0, D ** -0.5)
+    else:
+        args = (q, kc, torch.randn(pages, 256, G, Dv, device="cuda", generator=gen).bfloat16(), None, None, None, step, H, G, D, Dv, window, 0, D ** -0.5)
+    none = mix_ops.window_pool_attention(*args, has_sink=False)
+    some = mix_ops.window_pool_attention(*args, has_sink=True, sinks=torch.tensor([-float("inf"), -3e38, 0.5, 2.0], device="cuda"))
+    assert bool(torch.isfinite(some.float()).all())
+    assert torch.equal(some.view(T, H, Dv)[:, :2], none.view(T, H, Dv)[:, :2])
+    assert not torch.equal(some.view(T, H, Dv)[:, 2:], none.view(T, H, Dv)[:, 2:])
