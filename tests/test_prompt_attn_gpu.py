@@ -114,3 +114,37 @@ def test_sinks_of_minus_infinity_count_nothing(monkeypatch, D, Dv, G, window):
     assert bool(torch.isfinite(some.float()).all())
     assert torch.equal(some.view(T, H, Dv)[:, :2], none.view(T, H, Dv)[:, :2])
     assert not torch.equal(some.view(T, H, Dv)[:, 2:], none.view(T, H, Dv)[:, 2:])
+
+
+@pytest.mark.parametrize("D,Dv,same", [(64, 64, False), (128, 128, False), (256, 192, True)])
+@pytest.mark.parametrize("n,window,sink,sharp", [(200, 1 << 30, True, 1.0), (200, 1 << 30, False, 4.0), (1500, 1024, True, 1.0), (600, 100, False, 2.0)])
+def test_as_precise_as_the_16_query_form(D, Dv, same, n, window, sink, sharp):
+    """Against float64 on the same rows, which the 16-query form serves from pages that do not hold whole tiles. Both round every
+    probability to bf16; a query's largest one is exact where the running maximum follows it."""
+    H, G = 4, 1
+    gen = torch.Generator(device="cuda").manual_seed(D + n)
+
+    def rn(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen).bfloat16()
+
+    q, k = rn(n, H * D) * sharp, rn(n, G, D)
+    v = k[..., :Dv] if same else rn(n, G, Dv)
+    s = q.double().view(n, H, D).transpose(0, 1) @ k[:, 0].double().T.contiguous() * D ** -0.5
+    i = torch.arange(n, device="cuda")
+    s.masked_fill_((i[None] > i[:, None]) | (i[:, None] - i[None] >= window), -float("inf"))
+    top = s.amax(-1, keepdim=True).clamp_min(0.0)
+    e = torch.exp(s - top)
+    want = (e @ v[:, 0].double() / (e.sum(-1, keepdim=True) + (torch.exp(-top) if sink else 0.0))).transpose(0, 1).reshape(n, H * Dv)
+    err = []
+    for page in (48, 64):
+        step, pages = make_step([n], [0], page, 1)
+        rows = torch.tensor([step.host_block_tables[0][j // page] * page + j % page for j in range(n)], device="cuda")
+        kc = torch.zeros(pages * page, G, D, device="cuda", dtype=torch.bfloat16)
+        kc[rows] = k
+        vc = torch.zeros(pages * page, G, Dv, device="cuda", dtype=torch.bfloat16)
+        vc[rows] = v
+        kc, vc = kc.view(pages, page, G, D), vc.view(pages, page, G, Dv)
+        o = mix_ops.window_pool_attention(q, kc, kc[..., :Dv] if same else vc, None, None, None, step, H, G, D, Dv, window, 0, D ** -0.5,
+                                          has_sink=sink)
+        err.append(((o.double() - want).norm() / want.norm()).item())
+    assert err[1] <= 1.005 * err[0], err
