@@ -441,8 +441,86 @@ __device__ __forceinline__ float half_max(float x) {
   return fmaxf(__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi));
 }
 
+// The 32 queries from row rw of sequence b, head h, key by key, each on the keys that it sees: for waves whose products met an
+// infinity or a NaN behind a mask. Lanes c and c + 32 hold query c and half of its entries each. It starts from the kernel's arguments
+// again so that nothing of it stays in registers through the kernel that ends with it.
+template <int DK, int DV, int FORM>
+__device__ __forceinline__ void prompt_redo(int b, int h, int rw) {
+  typedef const __attribute__((address_space(4))) WindowMfmaParams* kernarg_t;
+  kernarg_t pp = (kernarg_t)__builtin_amdgcn_kernarg_segment_ptr();
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+s"(pp), "+s"(b), "+s"(h), "+s"(rw), "+v"(lane));
+  const auto& p = *pp;
+  constexpr float kLog2e = 1.44269504088896f;
+  const int c = lane & 31, half = lane >> 5, g = h / (p.H / p.G);
+  const int q0 = p.cu_q[b], n = p.cu_q[b + 1] - q0, ctx = p.ctx_lens[b], row = min(rw + c, n - 1), pos = ctx + row;
+  const int64_t t = q0 + row, GD = static_cast<int64_t>(p.G) * DK, GDv = static_cast<int64_t>(p.G) * DV;
+  const int32_t* bt = p.block_tables + static_cast<int64_t>(b) * p.bt_stride;
+  const int lo = p.chunk > 0 ? pos / p.chunk * p.chunk : max(0, pos - p.window + 1);      // first token of this query's window or chunk
+  const int from = __shfl(lo, 0, kWave), w1 = ctx + min(n, rw + kPromptQ) - 1;              // of the wave's first query; last query
+  const int early = p.P > 0 ? (p.chunk == 0 && w1 - p.window + 1 > 0 ? (w1 - p.window + 1) / p.P : 0) : min(p.keep_first, from);
+  const float sink = p.sinks != nullptr ? p.sinks[h] : p.m0;
+  constexpr int PARTS = DV > 128 ? DV / 64 : 1, ND = DV / 8 / PARTS;                      // wide rows in parts: registers
+  const bf16_t* q = reinterpret_cast<const bf16_t*>(p.q) + (t * p.H + h) * DK + 4 * half;
+#pragma unroll 1
+  for (int col = 0; col < DV; col += DV / PARTS) {
+    float m = (sink < -1e30f ? -1e30f : sink) * kLog2e, l = p.sink, o[ND][4];
+#pragma unroll
+    for (int d = 0; d < ND; ++d) o[d][0] = o[d][1] = o[d][2] = o[d][3] = 0.0f;
+#pragma unroll 1
+    for (int x = 0; x < early + w1 + 1 - from; ++x) {
+      const bool first = x < early, pooled = first && p.P > 0;
+      const int e = first ? x : from + x - early, at = pooled ? e * p.P + p.P - 1 : e, pj = at / p.page;
+      const int64_t slot = pooled ? static_cast<int64_t>(bt[pj]) * p.PP + (e - p.page * pj / p.P) : static_cast<int64_t>(bt[pj]) * p.page + at % p.page;
+      const bf16_t* k = reinterpret_cast<const bf16_t*>(pooled ? p.kp + slot * GD : p.k_cache + slot * p.k_ld) + g * DK + 4 * half;
+      const bf16_t* v = reinterpret_cast<const bf16_t*>(pooled ? p.vp + slot * GDv : p.v_cache + slot * p.v_ld) + g * DV + col + 4 * half;
+      float s = 0.0f;
+#pragma unroll 4
+      for (int y = 0; y < DK; y += 8) {
+        const float4 u = ld4(q + y), w = ld4(k + y);
+        s = fmaf(u.x, w.x, fmaf(u.y, w.y, fmaf(u.z, w.z, fmaf(u.w, w.w, s))));
+      }
+      s += __shfl_xor(s, 32, kWave);
+      if constexpr (FORM == kPlain) s *= p.scale;
+      if constexpr (FORM == kCapped) s = p.cap * fast_tanh(s * p.cap_in);
+      if constexpr (FORM == kExtended) {
+        s *= p.scale * (p.key_scale != nullptr ? p.key_scale[slot * p.G + g] : 1.0f);
+        if (p.dist_bias != nullptr) s += p.dist_bias[static_cast<int64_t>(h) * p.bias_len + min(max(pos - e, 0), p.bias_len - 1)];
+      }
+      s *= kLog2e;
+      if (pooled ? at <= pos - p.window : e <= pos && (e >= lo || e < p.keep_first)) {
+        const float nm = fmaxf(m, s), f = __builtin_amdgcn_exp2f(m - nm), pe = __builtin_amdgcn_exp2f(s - nm);
+        const float pr = static_cast<float>(static_cast<__bf16>(pe));
+        m = nm;
+        l = l * f + pe;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+          const float4 u = ld4(v + 8 * d);
+          o[d][0] = fmaf(pr, u.x, o[d][0] * f);
+          o[d][1] = fmaf(pr, u.y, o[d][1] * f);
+          o[d][2] = fmaf(pr, u.z, o[d][2] * f);
+          o[d][3] = fmaf(pr, u.w, o[d][3] * f);
+          if (d % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    if (rw + c >= n) continue;
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    bf16_t* orow = reinterpret_cast<bf16_t*>(p.out) + t * p.out_ld + static_cast<int64_t>(h) * DV + col + 4 * half;
+    const bf16_t* grow = p.gate != nullptr ? reinterpret_cast<const bf16_t*>(p.gate) + t * p.ld_gate + static_cast<int64_t>(h) * p.gate_dv : nullptr;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      float y[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        y[i] = o[d][i] * inv * (grow != nullptr ? sigmoidf_(ldf(grow + (p.gate_dv > 1 ? col + 8 * d + 4 * half + i : 0))) : 1.0f);
+      st4(orow + 8 * d, float4{y[0], y[1], y[2], y[3]});
+    }
+  }
+}
+
 template <int DK, int DV, bool SAME, int FORM>
-__global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WindowMfmaParams p, int hpw, int tiles, int by_count) {
+__global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(WindowMfmaParams p, int hpw, int tiles, int by_count) {
   constexpr int KB = DK * 2, VB = SAME ? KB : DV * 2;                       // bytes of a staged row
   constexpr int KT = kTileK * KB, VT = SAME ? 0 : kTileK * VB;
   constexpr int KCH = DK / 8, VCH = DV / 8, KN = kTileK * KCH / 256, VN = SAME ? 0 : kTileK * VCH / 256;
@@ -571,19 +649,21 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WindowMfmaParams p,
   // (a sink of -infinity counts nothing: a start far below any score, since a query may not see its first tiles)
   const float sink = p.sinks != nullptr ? p.sinks[h] : p.m0;
   float m = (sink < -1e30f ? -1e30f : sink) * kLog2e, l = half == 0 ? p.sink : 0.0f;
+  // tiles that hold nothing for this wave's queries, and tiles of tokens that all of them see whole
+  auto skipped = [&](int phase, int e0) __attribute__((always_inline)) {
+    if (phase == 0) return P > 0 && e0 * P + P - 1 > w1 - W;
+    return e0 > w1 || (e0 >= keep && (chunk > 0 ? e0 + kTileK - 1 < (w0 / chunk) * chunk : w0 - (e0 + kTileK - 1) >= W));
+  };
+  auto seen_whole = [&](int e0) __attribute__((always_inline)) {
+    return e0 + kTileK - 1 <= w0 && (chunk > 0 ? e0 >= w1 - w1 % chunk : w1 - e0 < W);
+  };
 
   auto compute = [&](int tile, int buf, lds_u8* kt) __attribute__((always_inline)) {
     const int phase = FIRST && tile < npt ? 0 : 1;
     const int e0 = phase == 0 ? tile * kTileK : jlo + (tile - npt) * kTileK;
     const int e_end = phase == 0 ? nbmax : i1 + 1;
-    if (!live) return;
-    if (phase == 1) {                                                       // nothing here for this wave's queries
-      if (e0 > w1) return;
-      if (e0 >= keep && (chunk > 0 ? e0 + kTileK - 1 < (w0 / chunk) * chunk : w0 - (e0 + kTileK - 1) >= W)) return;
-    } else if (P > 0 && e0 * P + P - 1 > w1 - W) {
-      return;
-    }
-    const bool whole = phase == 1 && e0 + kTileK - 1 <= w0 && (chunk > 0 ? e0 >= w1 - w1 % chunk : w1 - e0 < W);
+    if (!live || skipped(phase, e0)) return;
+    const bool whole = phase == 1 && seen_whole(e0);
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) {
       f32x16_t s;
@@ -715,6 +795,40 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WindowMfmaParams p,
     }
   }
   if (!live) return;
+  // A probability of zero does not keep an infinity or a NaN of a value row out of the products. Where an output is not finite, the value
+  // rows of the tiles that had a mask are looked at, and if one of them is the cause the wave's queries are done again (prompt_redo).
+  float odd = 0.0f;
+#pragma unroll
+  for (int d = 0; d < ND; ++d)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) odd = fmaf(o[d][i], 0.0f, odd);
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd != 0.0f) != 0, 0)) {
+    auto row_of = [&](int e, bool first) __attribute__((always_inline)) {
+      if (first) return slot_of(e);
+      const int pj = fdiv(e, page, p.m_page);
+      return static_cast<int64_t>(bt[pj]) * page + (e - pj * page);
+    };
+    const uint16_t *kp = P > 0 ? p.kp : p.k_cache, *vp = P > 0 ? p.vp : p.v_cache;
+    const int64_t kp_ld = P > 0 ? GD : p.k_ld, vp_ld = P > 0 ? GDv : p.v_ld;
+    bool bad = false;
+#pragma unroll 1
+    for (int tile = 0; tile < ntiles; ++tile) {
+      const bool first = tile < npt;
+      const int e0 = first ? tile * kTileK : jlo + (tile - npt) * kTileK;
+      if (skipped(first ? 0 : 1, e0) || (!first && seen_whole(e0))) continue;
+      const int e = min(e0 + lane, first ? nbmax - 1 : i1);
+      const uint16_t* v = first ? vp + row_of(e, true) * vp_ld + g * DV : p.v_cache + row_of(e, false) * p.v_ld + g * DV;
+#pragma unroll 1
+      for (int x = 0; x < DV; x += 2) {
+        const uint32_t u = *reinterpret_cast<const uint32_t*>(v + x);
+        bad = bad || (u & 0x7f80u) == 0x7f80u || (u & 0x7f800000u) == 0x7f800000u;
+      }
+    }
+    if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+      prompt_redo<DK, DV, FORM>(b, __builtin_amdgcn_readfirstlane(h), __builtin_amdgcn_readfirstlane(rw));
+      return;
+    }
+  }
   const float total = l + __shfl_xor(l, 32, kWave);
   const float inv = total > 0.0f ? 1.0f / total : 0.0f;
   if (rw + c >= n) return;

@@ -148,3 +148,48 @@ def test_as_precise_as_the_16_query_form(D, Dv, same, n, window, sink, sharp):
                                           has_sink=sink)
         err.append(((o.double() - want).norm() / want.norm()).item())
     assert err[1] <= 1.005 * err[0], err
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("D,Dv,same,kw", [(64, 64, False, dict(window=100)), (64, 64, False, dict(window=64, pool=16, page=64)), (128, 128, False, dict()),
+                                          (128, 128, False, dict(window=70, keep_first=3, softcap=20.0)), (64, 64, False, dict(window=1, chunk=96)),
+                                          (64, 64, False, dict(window=90, ext=32)), (256, 192, True, dict()), (256, 256, True, dict(window=120))])
+def test_a_bad_token_reaches_only_who_sees_it(D, Dv, same, kw, bad):
+    """An infinity or a NaN in the value row of one cached token makes the outputs of the queries that see it not finite and leaves
+    all others as they are: queries before it, behind its window or chunk, and other sequences."""
+    kw = dict(kw)
+    window, pool, page, ext = kw.pop("window", 1 << 30), kw.pop("pool", 0), kw.pop("page", 256), kw.pop("ext", 0)
+    H, G, new, ctx = 4, 1, [290, 40], [37, 5]
+    step, pages = make_step(new, ctx, page, 3)
+    gen = torch.Generator(device="cuda").manual_seed(D + Dv)
+
+    def rn(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen).bfloat16()
+
+    T = sum(new)
+    q, kc = rn(T, H * D), rn(pages, page, G, D)
+    vc = kc[..., :Dv] if same else rn(pages, page, G, Dv)
+    pp = max(mix_ops.pooled_slots(page, pool), 1)
+    kp, vp = (rn(pages, pp, G, D), rn(pages, pp, G, Dv)) if pool else (None, None)
+    if ext:
+        kw.update(key_scale=torch.rand(pages, page, G, device="cuda", generator=gen) + 0.5, dist_bias=torch.randn(H, ext, device="cuda", generator=gen))
+
+    def run(cache):
+        v = cache if not same else cache[..., :Dv]
+        return mix_ops.window_pool_attention(q, kc if not same else cache, v, kp, vp, None, step, H, G, D, Dv, window, pool, D ** -0.5, **kw).float()
+
+    base = kc if same else vc
+    clean = run(base)
+    pos = torch.cat([torch.arange(c, c + n) for n, c in zip(new, ctx)]).cuda()
+    first = torch.arange(T, device="cuda") < new[0]
+    for at in (1, 40, 63, 64, 100, 170, 255, 326):
+        cache = base.clone()
+        cache.view(-1, G, base.size(-1))[step.host_block_tables[0][at // page] * page + at % page] = bad
+        o = run(cache)
+        sees = first & (pos >= at)
+        if kw.get("chunk"):
+            sees &= pos // kw["chunk"] == at // kw["chunk"]
+        elif at >= kw.get("keep_first", 0):
+            sees &= pos - at < window
+        assert not bool(torch.isfinite(o[sees]).any()), at
+        assert (o[~sees] - clean[~sees]).abs().max().item() <= 2.0 ** -6, at      # sums in another order: a rounding of values up to 4
