@@ -236,3 +236,15 @@ def test_as_precise_as_the_token_loop(kind, H, G, D, Dv, new, monkeypatch):
         o = call(s, step)
         err.append((rel(o, want_o + skip), rel(s, want_s)))
     assert err[1][0] <= 1.1 * err[0][0] and err[1][1] <= 1.1 * err[0][1] + 2.0 ** -26
+
+
+@pytest.mark.parametrize("kind,H,G,D,Dv", [("delta", 2, 1, 64, 64), ("step", 2, 1, 64, 64), ("const", 2, 2, 64, 64)])
+@pytest.mark.parametrize("new", [[1] * 63 + [130], [200] + [1] * 63, [1] * 64 + [97], [0] * 70 + [33, 0, 64] + [1] * 60 + [0], [31, 32, 33] * 45])
+def test_many_sequences(kind, H, G, D, Dv, new):
+    """The places of chunks among those of all sequences, which a wave looks up 64 sequences at a time."""
+    call, args, skip = case(kind, new, H, G, D, Dv, seed=len(new))
+    step = make_step(new, [i % 3 for i in range(len(new))])
+    state = 0.3 * torch.randn(len(new), H, D, Dv, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    want_o, want_s = recurrence(*args, state, step)
+    o = call(state, step)
+    assert rel(o, want_o + skip) < REL and rel(state, want_s) < REL
