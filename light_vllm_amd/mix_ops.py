@@ -25,14 +25,20 @@ WINDOW_ATTN_KERNEL = "auto"
 SPLIT_WORKGROUPS = 256     # decode-shaped attention: key tiles are cut until a launch has about this many workgroups
 
 
-# recurrences with one decay per head: "auto" takes the chunked kernel for steps that bring a long portion, "token" the token loop
+# recurrences with one decay per head: "auto" takes the chunked kernel where it pays, "chunk" wherever it serves, "token" the token loop
 SCAN_KERNEL = "auto"
 CHUNK_STEP, CHUNK_CONST, CHUNK_DELTA = 0, 1, 2
-# New tokens of a sequence from which a step takes the chunked kernel: where its two launches meet the token loop's time. Token
-# loop / chunks in us, 1 sequence and 32: delta rule (16 heads of 128) 28.6 / 24.4 and 69 / 44 at 32 tokens, 17.5 / 25.2 at 16;
-# constant decays (16 heads) 24.6 / 24.0 and 76 / 52 at 64 tokens of 128 x 128, but 15.7 / 20.2 of 64 x 64, which are level at 90;
-# step sizes (32 heads, 128 x 64) 24.7 / 22.4 and 57 / 47 at 64.
+# New tokens of a sequence below which no step takes the chunked kernel. Token loop / chunks in us, 1 sequence and 32: delta rule (16
+# heads of 128) 28.6 / 24.4 and 69 / 44 at 32 tokens, 17.5 / 25.2 at 16; constant decays (16 heads) 24.6 / 24.0 and 76 / 52 at 64
+# tokens of 128 x 128, but 15.7 / 20.2 of 64 x 64, which are level at 90; step sizes (32 heads, 128 x 64) 24.7 / 22.4 and 57 / 47 at 64.
 CHUNK_FROM = {CHUNK_STEP: 80, CHUNK_CONST: 80, CHUNK_DELTA: 32}
+# What _chunk_pays weighs from there on, in us, by kind and rows of the state: a token of the longest sequence in the token loop
+# (launches of fewer than 1024 workgroups, of more), 256 x 128 columns by a token in it; a chunk behind another one, 256 x 128
+# columns by a chunk; what two launches cost more than one. Fitted to 258 steps of 1 to 256 sequences, one portion beside decoded
+# tokens, equal portions and mixtures: of those that CHUNK_FROM lets through, the choice is within 7 % of the better one.
+CHUNK_COSTS = {(CHUNK_STEP, 64): (0.29, 0.49, 0.28, 1.1, 5.6, 14.5), (CHUNK_STEP, 128): (0.34, 0.78, 0.47, 2.8, 7.2, 10.5),
+               (CHUNK_CONST, 64): (0.19, 0.40, 0.46, 1.8, 5.3, 12.5), (CHUNK_CONST, 128): (0.32, 0.80, 0.62, 4.0, 7.2, 14.5),
+               (CHUNK_DELTA, 64): (0.51, 0.59, 0.41, 5.3, 8.7, 11.0), (CHUNK_DELTA, 128): (0.76, 1.0, 0.83, 7.9, 8.2, 9.5)}
 
 
 def _stream(t: torch.Tensor) -> int:
@@ -202,12 +208,30 @@ def clamped_glu(x, limit: float, alpha: float):
 
 
 # ------------------------------------------------------------------------------- recurrences in chunks
+def _chunk_pays(kind, lens, H, D, Dv) -> bool:
+    """Whether chunks beat the token loop on sequences with these numbers of new tokens. Both read and write every state once, the token
+    loop beside its products and the chunks in front of and behind them, and a sequence with one new token costs the chunked kernel
+    a chunk: a step that decodes many sequences beside one portion of a prompt may be the token loop's. us, token loop / chunks,
+    with one sequence of the given length among others of one token: delta rule (16 heads of 128 x 128) 64 sequences, 32: 41 / 72,
+    256: 228 / 119; 256 sequences, 64: 123 / 239, 256: 269 / 237; step sizes (32 heads, 128 x 64) 256 sequences, 160: 159 / 209, 640:
+    476 / 284."""
+    longest = max(lens)
+    if longest < CHUNK_FROM[kind]:
+        return False
+    few, many, by_token, chunk, by_chunk, launches = CHUNK_COSTS[kind, D]
+    columns = max(1, H * Dv // 128) / 256
+    states = len(lens) * H * D * Dv * 8 / 5e6
+    serial = many if len(lens) * H * -(-Dv // 64) >= 1024 else few
+    token = max(serial * longest, by_token * sum(lens) * columns, states)
+    return max(chunk * -(-longest // 32), by_chunk * sum(-(-n // 32) for n in lens) * columns) + states + launches < token
+
+
 def _chunk_ok(kind, step, D, Dv, state, *rows) -> bool:
-    """Whether lv_chunk_scan takes this step: sizes and alignment it knows and a sequence with CHUNK_FROM[kind] new tokens or more.
-    rows: the query and key rows (four entries at a time, as the state)."""
-    return (SCAN_KERNEL == "auto" and not step.static and D in (64, 128) and (Dv == 64 or Dv % 128 == 0) and state.data_ptr() % 16 == 0
+    """Whether lv_chunk_scan takes this step: sizes and alignment it knows and sequences on which it pays. rows: the query and key rows
+    (four entries at a time, as the state)."""
+    return (SCAN_KERNEL != "token" and not step.static and D in (64, 128) and (Dv == 64 or Dv % 128 == 0) and state.data_ptr() % 16 == 0
             and all(x.stride(0) % 4 == 0 and x.data_ptr() % (4 * x.element_size()) == 0 for x in rows)
-            and max(step.host_lens_q) >= CHUNK_FROM[kind])
+            and (SCAN_KERNEL == "chunk" or _chunk_pays(kind, step.host_lens_q, state.size(1), D, Dv)))
 
 
 def _segment_length(lens, wgs, state_bytes) -> int:

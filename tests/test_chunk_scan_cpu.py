@@ -81,3 +81,34 @@ def test_step_sizes_that_share_a_row_are_refused(monkeypatch):
     record(monkeypatch, real=("lv_gated_scan", "lv_chunk_scan"))
     with pytest.raises(RuntimeError, match="bad sizes|strides"):
         step_call(0)
+
+
+@pytest.mark.parametrize("kind,H,D,Dv,lens,chunks", [
+    # measured, us, token loop / chunks: 30 / 25, 67 / 73, 228 / 119, 123 / 239, 61 / 74, 1030 / 328
+    (2, 16, 128, 128, [32], True), (2, 16, 128, 128, [64] + [1] * 63, False), (2, 16, 128, 128, [256] + [1] * 63, True),
+    (2, 16, 128, 128, [64] + [1] * 255, False), (2, 16, 64, 64, [32] + [1] * 255, False), (2, 16, 128, 128, [1024] * 16, True),
+    # 159 / 209, 476 / 284, 57 / 40, 105 / 217
+    (0, 32, 128, 64, [160] + [1] * 255, False), (0, 32, 128, 64, [640] + [1] * 255, True), (0, 32, 128, 64, [160], True),
+    (0, 32, 128, 64, [80] + [1] * 255, False),
+    # 19 / 21, 35 / 25, 104 / 149, 596 / 280; below every threshold
+    (1, 32, 64, 64, [80], False), (1, 32, 64, 64, [160], True), (1, 32, 64, 64, [160] + [1] * 255, False), (1, 16, 128, 128, [1024] * 16, True),
+    (1, 16, 128, 128, [1] * 64, False), (2, 16, 128, 128, [31], False)])
+def test_which_steps_take_chunks(kind, H, D, Dv, lens, chunks):
+    """A portion of a prompt beside many decoded tokens is the token loop's, where a chunk for every sequence would cost more."""
+    assert mix_ops._chunk_pays(kind, lens, H, D, Dv) == chunks
+
+
+@pytest.mark.parametrize("lens,wgs,seg", [([1024] * 16, 16, 0), ([4096], 16, 256), ([900, 3750, 2000, 1500, 2500, 1200, 2150], 16, 256), ([255], 16, 0),
+                                          ([1, 1, 1], 16, 0), ([2048] * 8, 16, 512), ([5000], 2, 256)])
+def test_segment_lengths(lens, wgs, seg):
+    """Few long sequences are cut into multiples of a chunk; what fills the chip by itself, and short portions, are not."""
+    got = mix_ops._segment_length(lens, wgs, wgs * 128 * 128 * 4)
+    assert got == seg or (seg and got % 32 == 0 and 256 <= got < max(lens)), got
+    assert (got > 0) == (seg > 0)
+
+
+def test_segments_keep_their_states_within_256_mb():
+    assert mix_ops._segment_length([4096] * 40, 1, 1 << 24) == 0
+    for n in (1, 3, 40):
+        seg = mix_ops._segment_length([4096] * n, 1, 1 << 20)
+        assert seg == 0 or n * -(-4096 // seg) * (1 << 20) <= 1 << 28

@@ -14,6 +14,12 @@ F64 = torch.float64
 REL = (128 + 2 * 32) * 2.0 ** -24
 
 
+@pytest.fixture(autouse=True)
+def chunks(monkeypatch):
+    """The chunked kernel wherever it serves; which steps it pays on is tested on the CPU."""
+    monkeypatch.setattr(mix_ops, "SCAN_KERNEL", "chunk")
+
+
 def make_step(new, ctx, static=False):
     cu, tok = [0], []
     for b, n in enumerate(new):
@@ -130,7 +136,7 @@ def test_misaligned_rows_and_captured_steps_take_the_token_loop(kind, pad, monke
     call, args, skip = case(kind, new, 2, 2, 64, 64, seed=pad, pad=pad)
     s_token = state.clone()
     o_token = call(s_token, make_step(new, [0, 2]))
-    monkeypatch.setattr(mix_ops, "SCAN_KERNEL", "auto")
+    monkeypatch.setattr(mix_ops, "SCAN_KERNEL", "chunk")
     s_auto = state.clone()
     o_auto = call(s_auto, make_step(new, [0, 2]))
     assert torch.equal(o_auto, o_token) and torch.equal(s_auto, s_token)
@@ -138,7 +144,7 @@ def test_misaligned_rows_and_captured_steps_take_the_token_loop(kind, pad, monke
     s_token, s_static, s_auto = state.clone(), state.clone(), state.clone()
     monkeypatch.setattr(mix_ops, "SCAN_KERNEL", "token")
     o_token = call(s_token, make_step(new, [0, 2]))
-    monkeypatch.setattr(mix_ops, "SCAN_KERNEL", "auto")
+    monkeypatch.setattr(mix_ops, "SCAN_KERNEL", "chunk")
     o_static = call(s_static, make_step(new, [0, 2], static=True))
     assert torch.equal(o_static, o_token) and torch.equal(s_static, s_token)
     o_auto = call(s_auto, make_step(new, [0, 2]))        # aligned and not captured: the same numbers in another order
@@ -230,7 +236,7 @@ def test_as_precise_as_the_token_loop(kind, H, G, D, Dv, new, monkeypatch):
     state = 0.3 * torch.randn(len(new), H, D, Dv, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
     want_o, want_s = recurrence(*args, state, step)
     err = []
-    for kernel in ("token", "auto"):
+    for kernel in ("token", "chunk"):
         monkeypatch.setattr(mix_ops, "SCAN_KERNEL", kernel)
         s = state.clone()
         o = call(s, step)
@@ -248,3 +254,24 @@ def test_many_sequences(kind, H, G, D, Dv, new):
     want_o, want_s = recurrence(*args, state, step)
     o = call(state, step)
     assert rel(o, want_o + skip) < REL and rel(state, want_s) < REL
+
+
+@pytest.mark.parametrize("kind,H,G,D,Dv", [("step", 4, 2, 128, 64), ("step", 8, 2, 64, 64), ("step", 3, 3, 128, 64), ("step", 2, 1, 128, 256), ("const", 2, 2, 128, 128),
+                                           ("const", 2, 2, 64, 128), ("const", 3, 3, 128, 64)])
+@pytest.mark.parametrize("new,seg", [([1000, 256, 513, 255, 1, 0, 512], 256), ([96, 33, 65, 31], 32), ([700, 1400], 512)])
+def test_segments_of_every_instance(kind, H, G, D, Dv, new, seg, monkeypatch):
+    """Sequences shorter than a segment, of whole segments, one token past them and empty, cut as asked for, on the workgroups of one
+    head, of two heads of a group and of four waves; and what the cut costs in precision against none: nothing but the draw."""
+    assert any(n > seg for n in new)
+    call, args, skip = case(kind, new, H, G, D, Dv, seed=D + H)
+    step = make_step(new, [i % 2 for i in range(len(new))])
+    state = 0.3 * torch.randn(len(new), H, D, Dv, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    want_o, want_s = recurrence(*args, state, step)
+    err, asked = [], []
+    for length in (0, seg):
+        monkeypatch.setattr(mix_ops, "_segment_length", lambda *a: asked.append(length) or length)
+        s = state.clone()
+        o = call(s, step)
+        assert rel(o, want_o + skip) < 2 * REL and rel(s, want_s) < 2 * REL
+        err.append(rel(o, want_o + skip))
+    assert asked == [0, seg] and err[1] <= 1.15 * err[0]
