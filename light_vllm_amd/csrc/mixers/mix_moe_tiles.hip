@@ -336,8 +336,13 @@ namespace {
 // Rows of a tile. Below about a hundred rows an expert the taller tile is mostly padding and the shorter one's smaller
 // staging wins (32 experts of 2048 x 1536: 109 against 118 us at 16 rows, 121 against 129 at 64); above, most experts need
 // two short tiles and the taller one reads each weight half as often (145 against 178 us at 128 rows, 259 / 289 at 384,
-// 1006 / 1168 at 2048; only right at 256, where half of the experts spill into a second tall tile, 246 against 214).
-int tile_rows(int64_t pairs, int E) { return pairs >= static_cast<int64_t>(E) * 96 ? 256 : 128; }
+// 1006 / 1168 at 2048; only right at 256, where half of the experts spill into a second tall tile, 246 against 214). Where all short
+// tiles run at once, one a compute unit, the taller ones only leave more of the chip idle (8 experts of 1024 x 512 at 128 rows 54
+// against 40 us, of 2048 x 1536 89 against 70); F in columns of 128, as gated units have them.
+int tile_rows(int64_t pairs, int E, int W, int F) {
+  const int64_t tiles = pairs / 128 + (pairs < E ? pairs : E);
+  return pairs >= static_cast<int64_t>(E) * 96 && tiles * (((W > 2 * F ? W : 2 * F) + 255) / 256) > 256 ? 256 : 128;
+}
 
 int64_t most_tiles(int64_t pairs, int E, int BM) {
   const int64_t hit = pairs < E ? pairs : E;
@@ -370,7 +375,7 @@ extern "C" {
 
 int64_t lv_moe_tiled_workspace_bytes(int64_t T, int W, int F, int E, int top) {
   const int64_t M = T * top;
-  return index_words(M, E, tile_rows(M, E)) * 4 + M * (static_cast<int64_t>(F) + W) * 2;
+  return index_words(M, E, tile_rows(M, E, W, F)) * 4 + M * (static_cast<int64_t>(F) + W) * 2;
 }
 
 int lv_moe_tiled_ff(const void* h, const void* ids, const void* weights, const void* up_w, const void* down_w, int64_t down_ld,
@@ -393,7 +398,7 @@ int lv_moe_tiled_ff(const void* h, const void* ids, const void* weights, const v
   if (M > (1 << 30) || T * W >= far || static_cast<int64_t>(F + 256) * W >= far || 256 * down_ld >= far ||
       256 * static_cast<int64_t>(F) >= far)
     return fail(-2, "lv_moe_tiled_ff: %lld rows of %d", (long long)T, W);
-  const int BM = tile_rows(M, static_cast<int>(E));
+  const int BM = tile_rows(M, static_cast<int>(E), W, F);
   const int64_t most = most_tiles(M, static_cast<int>(E), BM);
   if (most * ((W + 127) / 128 + (F + 127) / 128) >= (1 << 30)) return fail(-2, "lv_moe_tiled_ff: %lld tiles", (long long)most);
   const int runs = sort_runs(M);

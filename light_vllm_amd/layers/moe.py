@@ -15,7 +15,7 @@ matrices one [width, experts * ff] weight. Two forms compute the same sum:
   * gathered (bf16, width and ff in multiples of 32, at least GATHER_FROM experts per choice): the (token,
     choice) pairs are sorted by expert on the device and every expert multiplies only its own rows
     (mix_ops.moe_grouped_ff: sort, two grouped GEMMs on the matrix cores, weighted sum; four launches);
-  * sorted (bf16, eager steps with at least TILED_FROM rows per expert): the same sum with both products on LDS tiles of
+  * sorted (bf16, eager steps from TILED_FROM to TILED_SURELY rows per expert on): the same sum with both products on LDS tiles of
     128 or 256 rows (mix_ops.moe_sorted_ff). Weights whose layout those do not take go, from SORTED_FROM rows per expert,
     through vendor GEMMs on the sorted rows, after reading the experts' row counts back once. Steps captured into a
     hipGraph never take this form;
@@ -34,7 +34,7 @@ projections are linear, s * h enters as a factor on the pre-activations (mix_ops
 expert's token gate as a factor on its activations, so all of it is GEMMs on h plus one elementwise kernel.
 Forms: masked (everything in one up GEMM and one down GEMM; any dtype and size), gathered (bf16: sort, two
 grouped GEMMs on the matrix cores with the gated unit in the first one's epilogue, sum; the shared expert as
-vendor GEMMs beside it) and sorted (bf16, eager steps with at least TILED_FROM rows per expert: the same on LDS tiles).
+vendor GEMMs beside it) and sorted (bf16, eager steps from TILED_FROM to TILED_SURELY rows per expert on: the same on LDS tiles).
 """
 from __future__ import annotations
 
@@ -52,8 +52,20 @@ GATHER_FROM = 2.0     # experts / top from which the gathered form is taken
 # gathered form at 16 rows, 129 / 254 at 64, 246 / 539 at 256, 1006 / 3412 at 2048; below 16 the gathered form's tiles of 16
 # rows read each weight once and pad little.
 TILED_FROM = 16
-SORTED_FROM = 256     # the same for weights that the tiles do not take: vendor GEMMs on sorted rows
+TILED_SURELY = 48     # rows per expert from which they always do
+# In between, entries of the sorted activations (of width, or twice ff where that is less) from which the tiles' longer sort and fewer,
+# larger workgroups pay. Tiled / gathered, us: 4 experts of 2048 x 1536 57 / 39 at 16 rows, 60 / 50 at 32, 61 / 111 at 48; 16 of
+# 1024 x 512 36 / 29 at 16, level at 32; 64 of 512 x 256 31 / 35 at 16; 32 of 2048 x 256 51 / 43 at 16, level at 32.
+TILED_ENTRIES = 1 << 19
+SORTED_FROM = 256     # rows per expert for weights that the tiles do not take: vendor GEMMs on sorted rows
 MOE_KERNEL = "auto"   # "auto" | "masked" | "gathered" | "sorted" (tests force one or the other)
+
+
+def sorted_pays(tiles: bool, pairs: int, experts: int, width: int, ff: int) -> bool:
+    """Whether an eager step of so many (token, choice) pairs takes the sorted form."""
+    if not tiles or pairs >= SORTED_FROM * experts:
+        return pairs >= SORTED_FROM * experts
+    return pairs >= TILED_SURELY * experts or (pairs >= TILED_FROM * experts and pairs * min(width, 2 * ff) >= TILED_ENTRIES)
 
 
 class SparseMoE(nn.Module):
@@ -93,7 +105,7 @@ class SparseMoE(nn.Module):
         step = get_context().ragged
         captured = step is not None and step.static
         tiles = mix_ops.moe_tiles_ok(h, self.up_weight, self.down_weight, self.E, self.ff, 1, self.act, self.identity)
-        return "sorted" if not captured and h.size(0) * self.top >= (TILED_FROM if tiles else SORTED_FROM) * self.E else "gathered"
+        return "sorted" if not captured and sorted_pays(tiles, h.size(0) * self.top, self.E, self.width, self.ff) else "gathered"
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         ids, weights, dense = self.route(h)
@@ -138,7 +150,7 @@ class GLUSparseMoE(nn.Module):
         step = get_context().ragged
         captured = step is not None and step.static
         tiles = mix_ops.moe_tiles_ok(h, self.up_weight, self.down_weight, self.E, self.ff, 2)
-        return "sorted" if not captured and h.size(0) * self.top >= (TILED_FROM if tiles else SORTED_FROM) * self.E else "gathered"
+        return "sorted" if not captured and sorted_pays(tiles, h.size(0) * self.top, self.E, self.width, self.ff) else "gathered"
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         ids, weights, dense = self.route(h)

@@ -21,6 +21,10 @@ CASES = [(1, 32, 32, 4, 2, "relu2", 0),
          (333, 32, 32, 16, 5, "relu2", 3),
          (2500, 544, 224, 5, 3, "relu2", 1),       # tall tiles, several runs of the sort
          (9000, 128, 128, 70, 2, "relu2", 0)]      # more experts than a wave scans at once
+# tiles of 256 rows, which launches of more than 256 short tiles take from 96 rows an expert on: one row past the last tile, a part
+# tile, several experts with one that no one chose, handed through
+TALL = [(4097, 2080, 96, 1, 1, "relu2", 0), (4200, 2080, 224, 1, 1, "gelu", 0), (3000, 1568, 160, 4, 2, "relu2", 0),
+        (1500, 2336, 288, 5, 4, "gelu_tanh", 2)]
 
 
 def operands(T, W, F, E, top, through, ups, seed):
@@ -60,7 +64,7 @@ def exact(h, ids, w, up, down, E, F, act, glu=None):
     return y, S
 
 
-@pytest.mark.parametrize("T,W,F,E,top,act,through", CASES)
+@pytest.mark.parametrize("T,W,F,E,top,act,through", CASES + TALL)
 def test_tiles_match_the_exact_sum(gpu, T, W, F, E, top, act, through):
     h, ids, w, up, down = operands(T, W, F, E, top, through, 1, T + F)
     assert mix_ops.moe_tiles_ok(h, up, down, E, F, 1, act, through)
@@ -69,7 +73,8 @@ def test_tiles_match_the_exact_sum(gpu, T, W, F, E, top, act, through):
     assert ((y.double() - ref).abs() <= 3.5 * 2.0 ** -9 * S + 1e-6).all()
 
 
-@pytest.mark.parametrize("T,W,F,E,top", [(1, 32, 32, 4, 2), (257, 96, 160, 1, 1), (700, 256, 288, 4, 2), (3000, 160, 96, 5, 3)])
+@pytest.mark.parametrize("T,W,F,E,top", [(1, 32, 32, 4, 2), (257, 96, 160, 1, 1), (700, 256, 288, 4, 2), (3000, 160, 96, 5, 3),
+                                           (4097, 2080, 96, 1, 1), (2500, 1568, 224, 4, 2), (1100, 96, 2080, 5, 3)])
 def test_gated_tiles_match_the_exact_sum(gpu, T, W, F, E, top):
     h, ids, w, up, down = operands(T, W, F, E, top, 0, 2, T)
     wide = torch.zeros(W, E * F + 64, dtype=torch.bfloat16, device=h.device)        # the experts' columns of a wider weight
@@ -93,9 +98,10 @@ def test_operands_beside_the_rule_take_the_general_path(gpu):
         assert ((y.double() - ref).abs() <= 6.5 * 2.0 ** -9 * S + 1e-6).all()
 
 
-def test_a_bad_token_stays_alone(gpu):
+@pytest.mark.parametrize("T,W", [(600, 64), (9000, 1056)])
+def test_a_bad_token_stays_alone(gpu, T, W):
     """A NaN in one token's row reaches that token's result and no other's."""
-    T, W, F, E, top = 600, 64, 64, 2, 1
+    F, E, top = 64, 2, 1
     h, ids, w, up, down = operands(T, W, F, E, top, 0, 1, 3)
     clean = mix_ops.moe_sorted_ff(h, ids, w, up, down, E, F)
     h[123, 5] = float("nan")
