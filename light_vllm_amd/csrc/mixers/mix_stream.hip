@@ -313,7 +313,9 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(DeltaPrepParams p) {
 
 // The same for heads of 64, 128 or 256 entries (keys and values alike) and up to four taps: a thread owns four channels, their
 // filters and last inputs in registers, and walks a tile of packed tokens, so that a row is read once and written once. The
-// D / 4 lanes of a head add up its squares. One more column of workgroups forms the write strengths and decays of its tokens.
+// D / 4 lanes of a head add up its squares. One more column of workgroups forms the write strengths and decays of its tokens, and
+// where every channel has a decay of its own, 256 of them take a column each (2100 tokens, 16 heads of 128: 30 us; 76 with one column
+// for all of them, 57 in the form above).
 // Bound by memory (the projection's rows in, f32 rows out). The wave-per-(token, head) form above reads every row once per tap,
 // two bytes a lane: 16 x 1024 tokens, 3072 channels, four taps 374 us, this form 109 us;
 // 64 decoded tokens 5.5 -> 4.2 us.
@@ -321,21 +323,22 @@ template <typename T, int TAPS>
 __global__ __launch_bounds__(256) void delta_prep_tile_kernel(DeltaPrepParams p, int tile) {
   const int64_t t0 = static_cast<int64_t>(blockIdx.y) * tile, t1 = min(t0 + tile, p.T);
   const T* proj = static_cast<const T*>(p.proj);
-  const int GD = p.G * p.D, C = 2 * GD + p.H * p.Dv;
-  if (blockIdx.x == gridDim.x - 1) {
+  const int GD = p.G * p.D, C = 2 * GD + p.H * p.Dv, cols = (C / 4 + 255) / 256, col = blockIdx.x;
+  if (col >= cols) {
     const T* a = static_cast<const T*>(p.a);
+    if (col > cols) {                              // a decay per channel: a channel a thread, token after token
+      const int wide = p.H * p.dec_dim, x = (col - cols - 1) * 256 + threadIdx.x;
+      if (x >= wide) return;
+      const float rate = expf(p.A_log[x / p.dec_dim]), bias = p.dt_bias[x];
+#pragma unroll 4
+      for (int64_t t = t0; t < t1; ++t) p.decay[t * wide + x] = expf(-rate * softplusf_(ldf(a + t * p.ld_a + x) + bias));
+      return;
+    }
     for (int x = threadIdx.x; x < static_cast<int>(t1 - t0) * p.H; x += blockDim.x) {
       const int64_t t = t0 + x / p.H;
       const int h = x % p.H;
       p.beta[t * p.H + h] = sigmoidf_(ldf(proj + t * p.ld + p.off_b + h));
       if (p.dec_dim == 1) p.decay[t * p.H + h] = expf(-expf(p.A_log[h]) * softplusf_(ldf(a + t * p.ld_a + h) + p.dt_bias[h]));
-    }
-    if (p.dec_dim > 1) {
-      const int wide = p.H * p.dec_dim;
-      for (int x = threadIdx.x; x < wide; x += blockDim.x) {
-        const float rate = expf(p.A_log[x / p.dec_dim]), bias = p.dt_bias[x];
-        for (int64_t t = t0; t < t1; ++t) p.decay[t * wide + x] = expf(-rate * softplusf_(ldf(a + t * p.ld_a + x) + bias));
-      }
     }
     return;
   }
@@ -408,7 +411,7 @@ static bool delta_prep_tiles(const DeltaPrepParams& p, hipStream_t s) {
   const int cols = ((2 * p.G * p.D + p.H * p.Dv) / 4 + 255) / 256;
   // tiles of up to 16 tokens, shorter ones where the launch would have fewer than four workgroups a compute unit
   const int tile = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(16, p.T * (cols + 1) / 1024)));
-  dim3 grid(cols + 1, static_cast<unsigned>((p.T + tile - 1) / tile)), block(256);
+  dim3 grid(cols + 1 + (p.dec_dim > 1 ? (p.H * p.dec_dim + 255) / 256 : 0), static_cast<unsigned>((p.T + tile - 1) / tile)), block(256);
   if (grid.y > 65535) return false;
   switch (p.taps) {
     case 1: delta_prep_tile_kernel<T, 1><<<grid, block, 0, s>>>(p, tile); break;
