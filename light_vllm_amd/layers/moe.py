@@ -102,10 +102,11 @@ class SparseMoE(nn.Module):
             return MOE_KERNEL
         if not (mix_ops.moe_grouped_ok(h, self.ff) and self.E >= GATHER_FROM * self.top):
             return "masked"
-        step = get_context().ragged
-        captured = step is not None and step.static
+        step, pairs = get_context().ragged, h.size(0) * self.top
+        if pairs < TILED_FROM * self.E or (step is not None and step.static):
+            return "gathered"
         tiles = mix_ops.moe_tiles_ok(h, self.up_weight, self.down_weight, self.E, self.ff, 1, self.act, self.identity)
-        return "sorted" if not captured and sorted_pays(tiles, h.size(0) * self.top, self.E, self.width, self.ff) else "gathered"
+        return "sorted" if sorted_pays(tiles, pairs, self.E, self.width, self.ff) else "gathered"
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         ids, weights, dense = self.route(h)
@@ -147,10 +148,11 @@ class GLUSparseMoE(nn.Module):
         ok = mix_ops.moe_grouped_ok(h, self.ff) and (self.E * self.ff + self.Fs) % 8 == 0
         if not (ok and self.E >= GATHER_FROM * self.top):
             return "masked"
-        step = get_context().ragged
-        captured = step is not None and step.static
+        step, pairs = get_context().ragged, h.size(0) * self.top
+        if pairs < TILED_FROM * self.E or (step is not None and step.static):
+            return "gathered"
         tiles = mix_ops.moe_tiles_ok(h, self.up_weight, self.down_weight, self.E, self.ff, 2)
-        return "sorted" if not captured and sorted_pays(tiles, h.size(0) * self.top, self.E, self.width, self.ff) else "gathered"
+        return "sorted" if sorted_pays(tiles, pairs, self.E, self.width, self.ff) else "gathered"
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         ids, weights, dense = self.route(h)

@@ -229,9 +229,9 @@ def _chunk_pays(kind, lens, H, D, Dv) -> bool:
 def _chunk_ok(kind, step, D, Dv, state, *rows) -> bool:
     """Whether lv_chunk_scan takes this step: sizes and alignment it knows and sequences on which it pays. rows: the query and key rows
     (four entries at a time, as the state)."""
-    return (SCAN_KERNEL != "token" and not step.static and D in (64, 128) and (Dv == 64 or Dv % 128 == 0) and state.data_ptr() % 16 == 0
-            and all(x.stride(0) % 4 == 0 and x.data_ptr() % (4 * x.element_size()) == 0 for x in rows)
-            and (SCAN_KERNEL == "chunk" or _chunk_pays(kind, step.host_lens_q, state.size(1), D, Dv)))
+    return (SCAN_KERNEL != "token" and not step.static and D in (64, 128) and (Dv == 64 or Dv % 128 == 0)
+            and (SCAN_KERNEL == "chunk" or _chunk_pays(kind, step.host_lens_q, state.size(1), D, Dv)) and state.data_ptr() % 16 == 0
+            and all(x.stride(0) % 4 == 0 and x.data_ptr() % (4 * x.element_size()) == 0 for x in rows))
 
 
 def _segment_length(lens, wgs, state_bytes) -> int:
@@ -1239,13 +1239,13 @@ def lightning_attention(proj, off_q, off_k, off_v, decay, state, step, H, D, Dv)
     T = proj.size(0)
     _f32(decay, state)
     assert state.shape[1:] == (H, D, Dv) and decay.numel() == H
-    if proj.is_cuda and T > 0 and proj.dtype == torch.bfloat16:
+    columns = ((off_q, H * D), (off_k, H * D), (off_v, H * Dv))
+    # columns outside the rows go to the entry below, which refuses them
+    if (proj.is_cuda and T > 0 and proj.dtype == torch.bfloat16 and off_q % 4 == off_k % 4 == 0 and _chunk_ok(CHUNK_CONST, step, D, Dv, state, proj)
+            and all(0 <= at <= proj.size(1) - n for at, n in columns)):
         assert proj.stride(1) == 1
-        columns = ((off_q, H * D), (off_k, H * D), (off_v, H * Dv))
         q, k, v = (proj[:, at:at + n] for at, n in columns)
-        # columns outside the rows go to the entry below, which refuses them
-        if all(0 <= at <= proj.size(1) - n for at, n in columns) and _chunk_ok(CHUNK_CONST, step, D, Dv, state, q, k):
-            return _chunk_scan(CHUNK_CONST, q, k, v, None, decay, None, None, None, state, step, H, H, D, Dv)
+        return _chunk_scan(CHUNK_CONST, q, k, v, None, decay, None, None, None, state, step, H, H, D, Dv)
     o = torch.empty(T, H, Dv, dtype=torch.float32, device=proj.device)
     if proj.is_cuda:
         assert proj.stride(1) == 1
