@@ -46,7 +46,9 @@ constexpr int kSaturatedUnits = 1024;     // (sequence, kv head) pairs that fill
 // cut that would fill the chip, because the cut costs a merge launch: contexts of one block, and shapes that already give most
 // compute units a workgroup and short ones. A compute unit streams about 30 GB/s from memory, so longer contexts on few
 // workgroups stay cut. A layer's store and attention from a replayed graph, us, cut against one pass (16q/8kv): 1 x 64 tokens
-// 7.9 / 5.2; 24 x 1000 25.6 / 22.0; 31 x 900 28.6 / 25.4; but 1 x 1000 8.3 / 16.9 and 16 x 500 17.1 / 18.1, which stay cut.
+// 7.7 / 5.2; 24 x 1000 24.2 / 21.2; 31 x 900 25.2 / 24.3; but 1 x 1000 8.3 / 16.9 and 16 x 500 17.1 / 18.1, which stay cut.
+// The rule sees the table's capacity, not the lengths: a captured step whose table holds the longest sequence a server admits (16
+// blocks of 256 at 4096 tokens) is beyond it. It is for eager steps and for servers of short contexts.
 constexpr int64_t kWideTokens = 256, kWideFullTokens = 1024, kWideFullUnits = 160, kWideBelow = 256;
 static bool decode_wide(int batch, int num_kv_heads, int max_blocks_per_seq, int block_size) {
   const int64_t units = static_cast<int64_t>(batch) * num_kv_heads, tokens = static_cast<int64_t>(max_blocks_per_seq) * block_size;

@@ -11,21 +11,21 @@
 //   S <- G_last S + K^T diag(E w) U
 //
 // chunk_prep_kernel      T, P, G and E w of every chunk, all of them side by side
-// chunk_scan_kernel      the chain over a sequence's chunks; a wave owns all D rows of 32 columns of the state
+// chunk_scan_kernel      the chain over a sequence's chunks; a wave owns all D rows of 16 columns of the state
 // chunk_combine_kernel   starting states of a sequence's segments, where there are too few sequences for the chip
 //
 // Every product of decays is formed as one (no exponentials of differences of logarithms), so a ratio is as exact as in the
 // token loop and a decay of zero stays zero.
 //
-// All products run on v_mfma_f32_32x32x2_f32: f32 operands and sums, as in the token loop. Its result layout (16 registers, rows
-// 8 (i / 4) + 4 (lane / 32) + i % 4, column lane % 32) is its own right-hand operand layout if step i multiplies the left-hand
-// column of the same number: the state, U and V - G K S go from product to product in registers, and only q, k, T and P
-// pass through LDS.
+// Products are f32 with f32 sums, as in the token loop: v_mfma_f32_16x16x4_f32 in the scan, v_mfma_f32_32x32x2_f32 in front of it (the
+// delta rule's q k^T in 64 bits). The 16 x 16 result layout (4 registers, rows 4 (lane / 16) + i, column lane % 16) is its own
+// right-hand operand layout if step i multiplies the left-hand column of the same number: the state, U and V - G K S go from product
+// to product in registers, and only q, k, T and P pass through LDS.
 //
-// Bound by the f32 matrix rate: 4 D Dv + 64 (D + Dv) multiply-adds a token and head, 6 D Dv + 96 D + 128 Dv for the delta rule. The
-// token loop they replace did fewer, but on the vector ALU, one token behind the other. Layer kernels on one box, us:
-// 16 x 1024 tokens, delta rule (16 heads, 128 x 128) 993 -> 328; constant decays (16 heads, 128 x 128) 596 -> 280; step sizes (32
-// heads, 128 x 64; 7 prompts, the longest 3750) 1531 -> 445.
+// Bound by the f32 matrix rate: 2 D Dv + 24 Dv multiply-adds a token and head in the scan and 32 D a token and group in front of it;
+// 3 D Dv + 48 Dv and 64 D for the delta rule, half of the latter in 64 bits. The token loop they replace did fewer, but on the vector
+// ALU, one token behind the other. Kernels of a layer, token loop -> chunks, us: 16 x 1024 tokens, delta rule (16 heads, 128 x 128) 993 ->
+// 373; constant decays (16 heads, 128 x 128) 596 -> 331; step sizes (32 heads, 128 x 64; 7 prompts, the longest 3750) 1531 -> 470.
 #include "mix_common.h"
 
 namespace lvmix {
@@ -80,13 +80,13 @@ __device__ __forceinline__ float4 chunk_act(float4 x) {
 
 // grid: (chunks, groups), four waves. The chunks of all sequences lie side by side: those of sequence b start at place
 // cu_q[b] / 32 + b, which leaves at most one place a sequence empty. (A grid over sequences and the longest one's chunks
-// spent 1.57 ms on empty workgroups where two portions of 1000 tokens ran beside 250 decoded ones.) The products q k^T and k k^T do not depend on the head: the waves take a share of
-// the key dimension each, and every wave then takes heads of the group.
+// spent 1.57 ms on empty workgroups where two portions of 1000 tokens ran beside 250 decoded ones.) The products q k^T and k k^T do
+// not depend on the head: the waves take a share of the key dimension each, and every wave then takes heads of the group.
 template <typename T, int KIND>
 __global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
   constexpr bool DELTA = KIND == kChunkDelta, SILU = KIND == kChunkConst;
   constexpr int RS = kCh + 1;
-  __shared__ float prod[4][kCh * RS];                  // partial products; afterwards each wave's own scratch
+  __shared__ float prod[4][kCh * RS];                  // partial products of the waves
   __shared__ __attribute__((aligned(16))) float amat[DELTA ? 4 : 1][kCh * (kCh + kPad)];
   __shared__ float powers[KIND == kChunkConst ? 4 : 1][kCh + 1];
   const int g = blockIdx.y, place = blockIdx.x, cu0 = p.cu_q[0];
@@ -182,8 +182,9 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
     } else {
       wr = 0.0f;
     }
-    // G_t and E_t w_t, lane = t; D_tj w_j, lane = j with t in the result layout's registers (w = 1 but for step sizes). The products are formed in 64 bits and
-    // rounded once: a constant decay rounds the same way at every step, and its error would grow with the tokens it spans.
+    // G_t and E_t w_t, lane = t; D_tj w_j, lane = j with t in the result layout's registers (w = 1 but for step sizes). The products
+    // are formed in 64 bits and rounded once: a constant decay rounds the same way at every step, and its error would grow with the
+    // tokens it spans.
     float gt = 1.0f, et = 1.0f;
     float dm[16];
     if constexpr (KIND == kChunkConst) {
