@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from light_vllm_amd import mix_ops
-from tests._ragged import close, ragged_step
+from tests._ragged import ragged_step
 
 pytestmark = pytest.mark.gpu
 
