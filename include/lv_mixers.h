@@ -199,7 +199,9 @@ int lv_window_pool_attn(const void* q, const void* k_cache, const void* v_cache,
 /* The same attention on the matrix cores: bf16 only, D and Dv multiples of 16 up to 256. Tiles of 16 new
  * tokens per sequence; max_new_tokens = the largest cu_q[b+1] - cu_q[b] of the step.
  * nsplit > 1 (only with max_new_tokens <= 16, i.e. decode-shaped steps): the key tiles of a sequence are cut over nsplit
- * workgroups whose partials a second kernel merges; workspace: f32 [T, H, nsplit, Dv + 4] (read-out, maximum, sum, padding), T = total new tokens. */
+ * workgroups whose partials a second kernel merges; workspace: f32 [T, H, nsplit, Dv + 4] (read-out, maximum, sum, padding), T = total new tokens.
+ * nsplit < 0: one pass, and steps with more than 16 new tokens take 32 queries a wave wherever sizes and alignment allow, not only where
+ * that is the faster form. */
 int lv_window_pool_attn_mfma(const void* q, const void* k_cache, const void* v_cache, const void* kp, const void* vp,
                              const void* gate, int64_t ld_gate, void* out, const int32_t* cu_q, const int32_t* ctx_lens,
                              const int32_t* block_tables, int bt_stride, int B, int max_new_tokens, int H, int G, int D,

@@ -21,6 +21,8 @@
 // product * scale * factor + bias before the softmax.
 #include "mix_common.h"
 
+#include <algorithm>
+
 namespace lvmix {
 
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4v_t;
@@ -420,8 +422,9 @@ __global__ __launch_bounds__(256) void window_pool_merge_kernel(const float* __r
 // 64-wide heads; the 16-query form has 2.0e-3.)
 // Bound by the matrix pipe and the LDS reads that feed it, about level at 32 queries a wave. Against the 16-query form on one box: 11
 // prompts of 1500 tokens on average, window 1024, 16 heads over 4 of 128: 478 -> 220 us; 16 x 1024 tokens, 16 heads on latent rows of 256
-// (values 192): 978 -> 195 us (342 while their rows passed through registers and 54 of them spilled); 1 x 4000 full causal, 16 over 4: 391 -> 122 us; 17 tokens behind 4000: 67 -> 43 us; never slower
-// from 17 new tokens on.
+// (values 192): 978 -> 195 us (342 while their rows passed through registers and 54 of them spilled); 1 x 4000 full causal, 16 over 4:
+// 391 -> 122 us; 17 tokens behind 4000: 67 -> 43 us. With four query heads a kv head never slower from 17 new tokens on; with fewer see
+// prompt_pays.
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 typedef __attribute__((address_space(3))) unsigned char lds_u8;
 constexpr int kPromptQ = 32;
@@ -852,16 +855,37 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(Wind
     }
 }
 
+// Whether 32 queries a wave pay. A workgroup takes fewer than four heads of a kv head as so many more queries of each, so a launch
+// that leaves most of the chip idle has fewer workgroups, with a longer chain of tiles each, than one with 16 queries a wave, whose
+// spare waves cost nothing there. With a multiple of four heads both have waves to fill. us, 16 / 32 queries: 100 tokens, 8 heads of 64
+// over 8 8.4 / 13.2, of 128 10.0 / 15.6, behind 1000 tokens 31.4 / 37.3; 16 over 8 9.1 / 10.0, but behind 1000 36.0 / 34.2; 6 over 2
+// 9.8 / 13.2; 16 x 500 tokens, 8 over 8 82.7 / 23.8. `keys`: what a workgroup of 16 queries passes, from the table's width. The lines
+// lie where the two cross in 1450 launches of 1 to 16 sequences of 17 to 1000 tokens behind 0 to 3000: the choice is within 14 % of
+// the better one, 0.6 % off it on average.
+static bool prompt_pays(const WindowMfmaParams& p, int64_t T, int B, int max_new) {
+  const int rep = p.H / p.G;
+  if (rep % 4 == 0 || rep == 6 || p.D > 128) return true;
+  int64_t keys = static_cast<int64_t>(p.bt_stride) * p.page, units = static_cast<int64_t>(B) * ((max_new + kTileQ - 1) / kTileQ);
+  if (T > 0) units = std::min<int64_t>(units, (T + static_cast<int64_t>(B) * (kTileQ - 1)) / kTileQ);
+  const int64_t pooled = p.P > 0 ? keys / p.P : 0;
+  keys = std::min<int64_t>(keys, (p.chunk > 0 ? p.chunk : p.window) + static_cast<int64_t>(kTileQ) + p.keep_first) + pooled;
+  const bool few = max_new <= 2 * kPromptQ;                                 // at most two of the four waves have queries
+  const int64_t most = rep == 1 ? (few ? 768 : 2048) : rep == 2 ? (few ? 512 : 768) : (few ? 0 : 256);
+  const int64_t volume = rep == 1 ? (few ? 8 : 24) : (few ? 4 : 8);
+  return keys > most || units * p.G * keys * p.D > volume << 20;
+}
+
 // The head sizes and forms that prompt_attn_kernel is built for; false: the launch belongs to window_pool_mfma_kernel. It also
 // needs pages of whole tiles, a positive scale (the maximum is taken before it is applied), and rows that allow 8-byte accesses of
 // gate and output.
-static bool prompt_launch(const WindowMfmaParams& p, int form, int B, int max_new, hipStream_t s) {
+static bool prompt_launch(const WindowMfmaParams& p, int form, int64_t T, int B, int max_new, bool forced, hipStream_t s) {
   auto at = [](const void* q, uintptr_t a) { return reinterpret_cast<uintptr_t>(q) % a == 0; };
   if (p.D > 128 && (p.P > 0 || p.keep_first > 0)) return false;
   if (max_new <= kTileQ || p.page % kTileK != 0 || !(p.scale > 0.0f) || !at(p.q, 16) || !at(p.out, 8) || p.out_ld % 4 != 0 ||
       (p.P > 0 && (!at(p.kp, 16) || !at(p.vp, 16))) ||
       (p.gate != nullptr && p.gate_dv > 1 && (!at(p.gate, 8) || p.ld_gate % 4 != 0)))
     return false;
+  if (!forced && !prompt_pays(p, T, B, max_new)) return false;
   const bool same = p.P == 0 && (p.G == 1 || p.D == p.Dv) && p.k_cache == p.v_cache && p.k_ld == p.v_ld;
   const int rep = p.H / p.G, hpw = rep % 4 == 0 ? 4 : (rep % 2 == 0 ? 2 : 1);
   WindowMfmaParams q = p;
@@ -952,7 +976,7 @@ extern "C" int lv_masked_attn_mfma(const void* q, const void* k_cache, const voi
   if (nsplit > 1 && (max_new_tokens > kTileQ || workspace == nullptr || T <= 0 || nsplit > kWave))
     return fail(-1, "lv_window_pool_attn_mfma: key splits need one query tile per sequence and a workspace");
   hipStream_t st = as_stream(stream);
-  if (nsplit <= 1 && prompt_launch(p, softcap > 0.0f ? kCapped : (extended ? kExtended : kPlain), B, max_new_tokens, st))
+  if (nsplit <= 1 && prompt_launch(p, softcap > 0.0f ? kCapped : (extended ? kExtended : kPlain), T, B, max_new_tokens, nsplit < 0, st))
     return launched("lv_masked_attn_mfma");
   size_t shm = static_cast<size_t>(kTileK) * v_row(Dv) * sizeof(uint16_t);
   if (extended) shm += sizeof(float) * (kTileK + (p.dist_bias != nullptr && p.bias_len <= kBiasLds ? 4 * static_cast<size_t>(p.bias_len) : 0));

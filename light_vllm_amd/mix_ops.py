@@ -20,7 +20,8 @@ from . import _mixlib
 
 _DT = {torch.bfloat16: 0, torch.float32: 1}
 # windowed pooled attention: "auto" takes the matrix-core kernel where it applies (bf16, head sizes that
-# are multiples of 16 up to 256) and the vector kernel elsewhere (f32, other head sizes); "valu" forces the latter
+# are multiples of 16 up to 256) and the vector kernel elsewhere (f32, other head sizes); "valu" forces the latter; "prompt" is "auto"
+# with 32 queries a wave on every prompt step that they serve, not only where they pay
 WINDOW_ATTN_KERNEL = "auto"
 SPLIT_WORKGROUPS = 256     # decode-shaped attention: key tiles are cut until a launch has about this many workgroups
 
@@ -516,12 +517,12 @@ def window_pool_attention(q, k_cache, v_cache, kp, vp, gate, step, H, G, D, Dv, 
             assert c.stride(3) == 1 and (G == 1 or c.stride(2) == d) and c.stride(0) == page * ld and ld >= G * d
         lib = _mixlib.load()
         extras = _mixlib.AttnExtras(_p(key_scale), _p(dist_bias), dist_bias.size(1) if dist_bias is not None else 0, out.stride(0))
-        if (WINDOW_ATTN_KERNEL == "auto" and q.dtype == torch.bfloat16 and D % 16 == 0 and Dv % 16 == 0
+        if (WINDOW_ATTN_KERNEL in ("auto", "prompt") and q.dtype == torch.bfloat16 and D % 16 == 0 and Dv % 16 == 0
                 and D <= 256 and Dv <= 256 and k_ld % 8 == 0 and v_ld % 8 == 0 and k_cache.data_ptr() % 16 == 0
                 and v_cache.data_ptr() % 16 == 0):
             # decode-shaped steps put one workgroup per (sequence, kv head) on the chip: cut each sequence's key
             # tiles over enough workgroups to fill it (partials merged by a second kernel)
-            nsplit, ws = 1, None
+            nsplit, ws = -1 if WINDOW_ATTN_KERNEL == "prompt" else 1, None
             B = len(step.host_lens_q)
             if max(step.host_lens_q) <= 16:
                 most = max(c + n for c, n in zip(step.host_ctx_lens, step.host_lens_q))

@@ -47,7 +47,7 @@ def both(monkeypatch, new, ctx, H, G, D, Dv, page=256, same=False, gate=None, ex
         kw.update(key_scale=torch.rand(pages, page, G, device="cuda", generator=gen) + 0.5,
                   dist_bias=torch.randn(H, ext, device="cuda", generator=gen))
     got = []
-    for kernel in ("valu", "auto"):
+    for kernel in ("valu", "prompt"):
         monkeypatch.setattr(mix_ops, "WINDOW_ATTN_KERNEL", kernel)
         wide = torch.full((T, H * Dv + out_pad), 7.0, device="cuda", dtype=torch.bfloat16)
         out = wide[:, :H * Dv]
@@ -103,6 +103,7 @@ def test_other_pages_and_sizes_keep_their_kernel(monkeypatch):
 @pytest.mark.parametrize("D,Dv,G", [(64, 64, 2), (128, 128, 1), (256, 192, 1)])
 @pytest.mark.parametrize("window", [1, 100, 1 << 30])
 def test_sinks_of_minus_infinity_count_nothing(monkeypatch, D, Dv, G, window):
+    monkeypatch.setattr(mix_ops, "WINDOW_ATTN_KERNEL", "prompt")
     step, pages = make_step([300, 33], [140, 0], 256, D)
     gen = torch.Generator(device="cuda").manual_seed(D)
     H, T = 4, 333
@@ -196,3 +197,27 @@ def test_a_bad_token_reaches_only_who_sees_it(D, Dv, same, kw, bad):
             sees &= pos - at < window
         assert not bool(torch.isfinite(o[sees]).any()), at
         assert (o[~sees] - clean[~sees]).abs().max().item() <= 2.0 ** -6, at      # sums in another order: a rounding of values up to 4
+
+
+@pytest.mark.parametrize("H,G,D,new,ctx,wide", [
+    # us, 16 / 32 queries a wave: 8.4 / 13.2, 10.0 / 15.6, 31 / 37, 9.1 / 10.0, 9.8 / 13.2, 7.4 / 8.9
+    (8, 8, 64, [100], [0], False), (8, 8, 128, [100], [0], False), (8, 8, 64, [100], [1000], False), (16, 8, 64, [100], [0], False),
+    (6, 2, 64, [100], [0], False), (8, 8, 64, [60], [0], False),
+    # 82.7 / 23.8, 36 / 34, 43.1 / 33.4, level; four heads a kv head
+    (8, 8, 64, [500] * 16, [0] * 16, True), (16, 8, 64, [100], [1000], True), (8, 8, 64, [64] * 16, [1000] * 16, True), (6, 2, 64, [60], [0], True),
+    (8, 2, 64, [100], [0], True), (8, 2, 64, [60], [0], True)])
+def test_which_launches_take_32_queries_a_wave(monkeypatch, H, G, D, new, ctx, wide):
+    """Small launches with fewer than four query heads a kv head keep the 16-query form: bit for bit what it gives on pages that do not
+    hold whole tiles, and not what the other form gives."""
+    gen = torch.Generator(device="cuda").manual_seed(H + len(new))
+    T, total = sum(new), sum(new) + sum(ctx)
+    q, k, v = (torch.randn(n, h * D, device="cuda", generator=gen).bfloat16() for n, h in ((T, H), (total, G), (total, G)))
+    got = {}
+    for page, kernel in ((256, "auto"), (256, "prompt"), (272, "auto")):
+        step, pages = make_step(new, ctx, page, 1)
+        at = torch.tensor([step.host_block_tables[b][j // page] * page + j % page for b in range(len(new)) for j in range(new[b] + ctx[b])], device="cuda")
+        kc, vc = (torch.zeros(pages * page, G * D, device="cuda", dtype=torch.bfloat16).index_copy(0, at, x).view(pages, page, G, D) for x in (k, v))
+        monkeypatch.setattr(mix_ops, "WINDOW_ATTN_KERNEL", kernel)
+        got[page, kernel] = mix_ops.window_pool_attention(q, kc, vc, None, None, None, step, H, G, D, D, 1 << 30, 0, D ** -0.5)
+    assert not torch.equal(got[256, "prompt"], got[272, "auto"])
+    assert torch.equal(got[256, "auto"], got[256, "prompt"] if wide else got[272, "auto"])
