@@ -5,8 +5,8 @@
 // aligned to the bottom-right corner (query row r sees keys t <= r + Lk - Lq).
 //
 // Structure (flash-attention forward, one pass over K/V with online softmax):
-//   * workgroup = 4 waves = one 128-row query tile of one (sequence, query head); wave w owns rows
-//     32w..32w+31. Query tiles are launched heaviest (latest rows) first.
+//   * workgroup = 4 waves = one 128-row query tile of one (sequence, query head), or 64 rows of two heads of a group (launch_w4);
+//     a wave owns 32 rows. Query tiles are launched heaviest (latest rows) first.
 //   * K/V tiles of 64 keys are staged HBM -> VGPR -> LDS by all 256 lanes in whole 256-byte rows
 //     (16 B per lane); the next tile's global loads are issued before the current tile's math so
 //     their latency hides under it. The LDS image XOR-swizzles the 16-byte chunk index with the row
@@ -219,10 +219,13 @@ __device__ __forceinline__ void acc_scale(float alpha) {
 // it from HBM for itself; a table that keeps a sequence inside one or two columns lets an XCD's L2
 // serve its stream once. Rows are taken in table order (heaviest first as the caller sorts them),
 // and every row is followed by all query heads of its group.
+// HPW: query heads of a workgroup (hq: the first of them). BY_TILE: the natural mapping takes every sequence's last tile first, then the
+// ones before them, with q0 the rows between a tile and its sequence's last one: all the heavy tiles start early, and what is left for a
+// launch's end is the short work of all sequences.
 struct TileWork { int kvh, split, hq, b, q0; };
-template <int BM>
+template <int BM, int HPW = 1, bool BY_TILE = false>
 __device__ __forceinline__ bool tile_of_block(const PrefillParams& p, TileWork& w) {
-  const int G = p.num_heads / p.num_kv_heads;
+  const int G = p.num_heads / p.num_kv_heads / HPW;
   const int qtiles = (p.max_seqlen_q + BM - 1) / BM;
   int wg = blockIdx.x;
   w.kvh = wg % p.num_kv_heads;
@@ -230,8 +233,13 @@ __device__ __forceinline__ bool tile_of_block(const PrefillParams& p, TileWork& 
   if (p.tile_order == nullptr) {
     w.split = wg % p.nsplit;
     wg /= p.nsplit;
-    w.hq = w.kvh * G + wg % G;
+    w.hq = (w.kvh * G + wg % G) * HPW;
     wg /= G;
+    if constexpr (BY_TILE) {
+      w.q0 = wg / p.batch * BM;
+      w.b = wg % p.batch;
+      return true;
+    }
     w.q0 = (qtiles - 1 - wg % qtiles) * BM;
     w.b = wg / qtiles;
     return true;
@@ -240,7 +248,7 @@ __device__ __forceinline__ bool tile_of_block(const PrefillParams& p, TileWork& 
   wg /= p.order_cols;
   w.split = wg % p.nsplit;
   wg /= p.nsplit;
-  w.hq = w.kvh * G + wg % G;
+  w.hq = (w.kvh * G + wg % G) * HPW;
   wg /= G;
   const int item = p.tile_order[static_cast<int64_t>(wg) * p.order_cols + col];
   if (item < 0) return false;
@@ -252,11 +260,14 @@ __device__ __forceinline__ bool tile_of_block(const PrefillParams& p, TileWork& 
 // NW = waves per workgroup, RB = 32-row query blocks per wave (1); the workgroup's query tile is
 // 32*RB*NW rows, two waves per SIMD on compiler-allocated registers.
 // DMA = true stages K/V tiles HBM -> LDS directly (global_load_lds, no VGPRs, no ds_write).
-template <bool PAGED, int NW, int RB, bool DMA>
+// HPW > 1 (natural mapping only): the waves share HPW query heads of one group, 32 NW / HPW rows of each, instead of one head's
+// rows: the same work on the same K/V tiles, with fewer rows past a prompt's end and past the causal limit.
+template <bool PAGED, int NW, int RB, bool DMA, int HPW>
 __global__ __launch_bounds__(64 * NW, (RB == 2 ? 1 : 2))
 void prefill_attn_kernel(const PrefillParams p) {
   static_assert(RB == 1, "one 32-row block per wave (64 rows per wave: prefill_w64_kernel)");
-  constexpr int BM = 32 * RB * NW;  // query rows per workgroup
+  constexpr int WPH = NW / HPW;      // waves of one head
+  constexpr int BM = 32 * RB * WPH;  // query rows per workgroup
   constexpr int NST = 16 / NW;      // 16-byte chunks of K (and of V) each thread stages per tile
   constexpr int RSTEP = 4 * NW;     // tile rows between two chunks of one thread
   // two buffers x (K tile | V tile)
@@ -267,13 +278,14 @@ void prefill_attn_kernel(const PrefillParams p) {
   // (few query tiles against a long context: a prefix-cached prompt, a short batch); the runs'
   // unnormalised outputs and (max, sum) go to the workspace and prefill_merge_kernel combines them.
   TileWork tw;
-  if (!tile_of_block<BM>(p, tw)) return;
-  const int kvh = tw.kvh, split = tw.split, hq = tw.hq, q0 = tw.q0, b = tw.b;
+  if (!tile_of_block<BM, HPW, true>(p, tw)) return;
+  const int kvh = tw.kvh, split = tw.split, b = tw.b;
   const int q_start = p.cu_q[b];
   const int Lq = p.cu_q[b + 1] - q_start;
   const int k_start = p.cu_k[b];
   const int Lk = p.cu_k[b + 1] - k_start;
-  if (q0 >= Lq) return;
+  const int q0 = p.tile_order ? tw.q0 : ((Lq + BM - 1) / BM - 1) * BM - tw.q0;
+  if (q0 >= Lq || q0 < 0) return;
   const int coff = Lk - Lq;  // causal offset: row r sees keys <= r + coff
 
   const int tid = threadIdx.x;
@@ -282,7 +294,8 @@ void prefill_attn_kernel(const PrefillParams p) {
   const int h = lane >> 5;  // which 8-wide half of an MFMA k-step this lane feeds
   const int c = lane & 31;  // MFMA column = query row inside a 32-row block
 
-  const int wrow0 = q0 + wave * (32 * RB);  // first row of the wave; block rb starts 32*rb later
+  const int hq = tw.hq + wave / WPH;
+  const int wrow0 = q0 + wave % WPH * (32 * RB);  // first row of the wave; block rb starts 32*rb later
   int my_lim[RB];                           // last visible key of this lane's row in block rb
 
   // Q^T fragments (B operand of S^T = K Q^T): per row block 8 k-steps x 8 bf16.
@@ -548,8 +561,8 @@ void prefill_attn_kernel(const PrefillParams p) {
     constexpr int BUF = decltype(buf_c)::value;
     constexpr int kBufOff = BUF * 2 * kTileBytes;
     const int kt0 = tile * BN;
-    // waves whose rows all lie above this tile have nothing to add
-    if (kt0 > wrow0 + 31 + coff) return;
+    // waves whose rows all lie above this tile, or past the prompt's end, have nothing to add
+    if (kt0 > wrow0 + 31 + coff || wrow0 >= Lq) return;
     LV_STAMP_COUNT
 
     bf16x8 kx[8];       // K fragments of A, then of B
@@ -2033,12 +2046,31 @@ static void launch_pp(const PrefillParams& p, hipStream_t stream) {
   hipLaunchKernelGGL((prefill_pp_kernel<PAGED, false>), dim3(static_cast<unsigned>(total)), dim3(512), 0, stream, p);
 }
 
-template <bool PAGED, int NW, int RB, bool DMA>
+template <bool PAGED, int NW, int RB, bool DMA, int HPW = 1>
 static void launch_cfg(const PrefillParams& p, hipStream_t stream) {
-  constexpr int BM = 32 * RB * NW;
-  const int64_t total = grid_items(p, BM) * p.num_heads * p.nsplit;
-  hipLaunchKernelGGL((prefill_attn_kernel<PAGED, NW, RB, DMA>), dim3(static_cast<unsigned>(total)), dim3(64 * NW), 0,
+  constexpr int BM = 32 * RB * NW / HPW;
+  const int64_t total = grid_items(p, BM) * (p.num_heads / HPW) * p.nsplit;
+  hipLaunchKernelGGL((prefill_attn_kernel<PAGED, NW, RB, DMA, HPW>), dim3(static_cast<unsigned>(total)), dim3(64 * NW), 0,
                      stream, p);
+}
+
+// Without a caller's order two query heads of a group share a workgroup of 4 waves, 64 rows of each: prompts end on tiles of 64 rows
+// instead of 128. us, 128 rows of one head / 64 of two: 13 ragged prompts of about 350 behind 1024 cached tokens, 16 heads over 8 102 / 92,
+// 32 over 8 154 / 137; 16 x 1024, 16 over 8 123 / 97 (by the order of the tiles, mostly); 32 ragged prompts of about 100, 32 over 8 31 / 26.
+// Four heads of 32 rows each gain nothing more (143, 142 and 26 at these), but for many prompts of at most 32 rows, where they
+// halve the workgroups: 32 x 16, 64 over 8 12.7 / 9.0. Splits cut a tile's keys, and where they cut must not depend on whether a caller
+// brought an order: with them, tiles of 128 rows either way.
+template <bool PAGED>
+static void launch_w4(const PrefillParams& p, bool dma, hipStream_t stream) {
+  const int G = p.num_heads / p.num_kv_heads;
+  if (dma || p.tile_order != nullptr || p.nsplit > 1 || G % 2 != 0) {
+    if (dma) launch_cfg<PAGED, 4, 1, true>(p, stream);
+    else launch_cfg<PAGED, 4, 1, false>(p, stream);
+  } else if (G % 4 == 0 && p.max_seqlen_q <= 32 && static_cast<int64_t>(p.batch) * (p.num_heads / 2) > 256) {
+    launch_cfg<PAGED, 4, 1, false, 4>(p, stream);
+  } else {
+    launch_cfg<PAGED, 4, 1, false, 2>(p, stream);
+  }
 }
 
 // Kernel configuration of a launch: 0 = W4 (128-row tiles), 1 = W8, 2 = PP, 4 = W64 (256-row tiles);
@@ -2096,10 +2128,10 @@ int launch_prefill_attn(const PrefillParams& p, hipStream_t stream) {
     if (p.block_table) launch_pp<true>(p, stream); else launch_pp<false>(p, stream);
   } else if (p.block_table) {
     if (cfg == 1) { if (dma) launch_cfg<true, 8, 1, true>(p, stream); else launch_cfg<true, 8, 1, false>(p, stream); }
-    else { if (dma) launch_cfg<true, 4, 1, true>(p, stream); else launch_cfg<true, 4, 1, false>(p, stream); }
+    else launch_w4<true>(p, dma, stream);
   } else {
     if (cfg == 1) { if (dma) launch_cfg<false, 8, 1, true>(p, stream); else launch_cfg<false, 8, 1, false>(p, stream); }
-    else { if (dma) launch_cfg<false, 4, 1, true>(p, stream); else launch_cfg<false, 4, 1, false>(p, stream); }
+    else launch_w4<false>(p, dma, stream);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(LV_ERR_LAUNCH, "prefill_attn launch: %s", hipGetErrorString(e));
