@@ -66,6 +66,7 @@
  *   lv_head_norm_store       per-head RMS norm of the queries, keys stored as they are with the factor of their norm beside them
  *   lv_gated_linear_recurrence   Griffin's RG-LRU: block-diagonal gates, S <- a S + sqrt(1 - a^2) i u per channel, gelu branch
  *   lv_scaled_embedding      token rows times a constant as the f32 residual
+ *   lv_rows_gemm             projections of up to 64 rows
  *   lv_residual_split        residual update, and the residual as the sum of two bf16 numbers for a matrix product
  *
  * A "ragged step" is a batch of B sequences; sequence b brings cu_q[b+1]-cu_q[b] new tokens that
@@ -88,7 +89,7 @@
 extern "C" {
 #endif
 
-#define LV_MIX_ABI_VERSION 11
+#define LV_MIX_ABI_VERSION 12
 #define LV_MIX_BF16 0
 #define LV_MIX_F32 1
 #define LV_MIX_MAX_STREAMS 8
@@ -497,6 +498,10 @@ int lv_scaled_embedding(const void* ids, const void* table, int vocab, float sca
 
 /* x f32 [T, W] += y (bf16 [T, W], may be NULL);  out bf16 [T, 2W] = x rounded | (x - x rounded) rounded. */
 int lv_residual_split(void* x, const void* y, void* out, int64_t T, int W, void* stream);
+
+/* y bf16 [M, N] = x bf16 [M, K] w^T, w bf16 [N, K], sums in f32. M <= 64, K a multiple of 32; row strides ldx, ldw (multiples of 8)
+ * and ldy in entries; x and w 16-byte, y 8-byte aligned. */
+int lv_rows_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, int64_t ldy, int M, int N, int K, void* stream);
 
 #ifdef __cplusplus
 }

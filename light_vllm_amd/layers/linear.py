@@ -1,6 +1,6 @@
 """Tensor-parallel linear layers (reference: lightvllm/layers/linear.py).
 
-The GEMMs are plain F.linear (hipBLASLt on MI355X). What matters to the attention path is the
+The GEMMs are mix_ops.linear: hipBLASLt, and a kernel of our own for the few rows of a decode step. What matters to the attention path is the
 sharding: QKVParallelLinear gives rank r the query heads [r*Hq/tp, (r+1)*Hq/tp) and kv heads
 [r*Hkv/tp, (r+1)*Hkv/tp) in a fused [q | k | v] output (linear.py:240-310), so attention needs no
 communication, and RowParallelLinear sums the per-rank partial outputs with one in-place
@@ -13,8 +13,13 @@ import torch.distributed as dist
 import torch.nn.functional as F
 from torch import nn
 
+from .. import mix_ops
 from . import tp
 from .tp import divide, tp_rank, tp_size
+
+
+def _linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
+    return mix_ops.linear(x, weight) if bias is None else F.linear(x, weight, bias)
 
 
 class LinearBase(nn.Module):
@@ -47,7 +52,7 @@ class ReplicatedLinear(LinearBase):
         param.data.copy_(loaded_weight)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x, self.weight, self.bias)
+        return _linear(x, self.weight, self.bias)
 
 
 class ColumnParallelLinear(LinearBase):
@@ -64,7 +69,7 @@ class ColumnParallelLinear(LinearBase):
         param.data.copy_(loaded_weight.narrow(self.tp_dim, self.tp_rank * shard, shard))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x, self.weight, self.bias)
+        return _linear(x, self.weight, self.bias)
 
 
 class MergedColumnParallelLinear(ColumnParallelLinear):
@@ -130,7 +135,7 @@ class RowParallelLinear(LinearBase):
         after the sum."""
         if self.tp_size == 1 and self.bias is not None:
             return F.linear(x, self.weight, self.bias)      # one rank: the bias rides in the GEMM, one rounding
-        y = F.linear(x, self.weight)
+        y = mix_ops.linear(x, self.weight)
         if not reduce:
             assert self.bias is None
             return y

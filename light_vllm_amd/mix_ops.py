@@ -14,7 +14,9 @@ import ctypes
 import math
 
 import torch
+import torch.autograd.forward_ad as forward_ad
 import torch.nn.functional as F
+from torch.utils._device import DeviceContext
 
 from . import _mixlib
 
@@ -1690,3 +1692,62 @@ def mm_f32(a, b_t, add=None):
         return torch.mm(a, b_t, out_dtype=torch.float32) if add is None else torch.addmm(add, a, b_t, out_dtype=torch.float32)
     y = torch.mm(a.float(), b_t.float())
     return y if add is None else y + add
+
+
+ROWS_GEMM_MAX = 64           # rows of x that lv_rows_gemm takes
+
+
+def _transformed(*ts) -> bool:
+    """Whether something is to see or rewrite torch's own operators on these tensors: forward-mode gradients, function transforms,
+    tracing, autocast, modes (a default device is none: the engine sets one) and subclasses. A launch of our own is invisible to all of
+    them."""
+    return (any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in ts) or forward_ad._current_level >= 0
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0
+            or any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
+            or torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing())
+
+
+def rows_gemm_ok(x, w) -> bool:
+    """Whether linear(x, w) takes lv_rows_gemm: bf16 matrices on one device with rows of whole 16-byte pieces, k a multiple of 32, at
+    most 64 rows of x. Above 32 rows the rows of x that every compute unit reads weigh as much as the weights, and large products
+    are the vendor's: us, vendor / own, 33, 48 and 64 rows: 10304 x 4096 29 / 26, 29 / 27, 29 / 30; 20480 x 4096 42 / 43, 44 / 45, 45 / 48;
+    8192 x 2048 14.7 / 12.0, 14.8 / 12.3, 14.7 / 12.0."""
+    if x.dim() != 2 or not 0 < x.size(0) <= ROWS_GEMM_MAX or not x.is_cuda or x.dtype != torch.bfloat16 or _transformed(x, w):
+        return False
+    M, K = x.shape
+    N = w.size(0)
+    return (w.dim() == 2 and w.dtype == torch.bfloat16 and w.device == x.device and w.size(1) == K and K > 0 and K % 32 == 0 and N > 0
+            and (M <= 32 or M * N * K <= 1 << 31) and x.stride(1) == 1 and w.stride(1) == 1 and x.stride(0) % 8 == 0
+            and w.stride(0) % 8 == 0 and w.stride(0) >= K and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and x.device.index == torch.cuda.current_device())
+
+
+def _rows_gemm(x, w):
+    M, K = x.shape
+    y = torch.empty(M, w.size(0), dtype=x.dtype, device=x.device)
+    lib = _mixlib.load()
+    _mixlib.check(lib.lv_rows_gemm(_p(x), x.stride(0), _p(w), w.stride(0), _p(y), y.stride(0), M, w.size(0), K, _stream(x)), "lv_rows_gemm")
+    return y
+
+
+class _RowsLinear(torch.autograd.Function):
+    """lv_rows_gemm where gradients are recorded: the same output, torch's products behind it."""
+
+    @staticmethod
+    def forward(ctx, x, w):
+        ctx.save_for_backward(x, w)
+        return _rows_gemm(x, w)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, w = ctx.saved_tensors
+        return (dy.mm(w) if ctx.needs_input_grad[0] else None), (dy.t().mm(x) if ctx.needs_input_grad[1] else None)
+
+
+def linear(x, w):
+    """x [..., K] w [N, K]^T. Few rows of bf16 (decode steps) take lv_rows_gemm, everything else torch's linear."""
+    if not rows_gemm_ok(x, w):
+        return F.linear(x, w)
+    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
+        return _RowsLinear.apply(x, w)
+    return _rows_gemm(x, w)
