@@ -12,6 +12,7 @@
 //
 // chunk_prep_kernel      T, P, G and E w of every chunk, all of them side by side
 // chunk_scan_kernel      the chain over a sequence's chunks; a wave owns all D rows of 16 columns of the state
+// chunk_step_kernel      the same for step sizes, on the bf16 matrix instructions
 // chunk_combine_kernel   starting states of a sequence's segments, where there are too few sequences for the chip
 //
 // Every product of decays is formed as one (no exponentials of differences of logarithms), so a ratio is as exact as in the
@@ -22,10 +23,13 @@
 // right-hand operand layout if step i multiplies the left-hand column of the same number: the state, U and V - G K S go from product
 // to product in registers, and only q, k, T and P pass through LDS.
 //
-// Bound by the f32 matrix rate: 2 D Dv + 24 Dv multiply-adds a token and head in the scan and 32 D a token and group in front of it;
-// 3 D Dv + 48 Dv and 64 D for the delta rule, half of the latter in 64 bits. The token loop they replace did fewer, but on the vector
-// ALU, one token behind the other. Kernels of a layer, token loop -> chunks, us: 16 x 1024 tokens, delta rule (16 heads, 128 x 128) 993 ->
-// 373; constant decays (16 heads, 128 x 128) 596 -> 331; step sizes (32 heads, 128 x 64; 7 prompts, the longest 3750) 1531 -> 470.
+// Bound by the chain of a chunk, two waves a SIMD: 2 D Dv + 24 Dv multiply-adds a token and head at the f32 matrix rate (3 D Dv + 48 Dv
+// for the delta rule), and beside them the vector ALU's work of staging the next chunk, which stands among the last products without a
+// branch between. The token loop they replace did fewer operations, but on the vector ALU, one token behind the other. Kernels of a
+// layer, us, token loop -> f32 chunks -> staged among the products / on bf16 instructions: 16 x 1024 tokens, delta rule (16 heads, 128 x
+// 128) 993 -> 377 -> 343; constant decays (16 heads, 128 x 128) 596 -> 295 -> 281; step sizes (32 heads, 128 x 64; 7 prompts, the longest
+// 3750) 1531 -> 456 -> 323. Pieces for the other two kinds, whose q, k and v are f32, were built and gained nothing: six to eight
+// products for one, and every row to cut.
 #include "mix_common.h"
 
 namespace lvmix {
@@ -33,6 +37,8 @@ namespace lvmix {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 chunk_bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 chunk_bf16x4 __attribute__((ext_vector_type(4)));
 constexpr int kCh = 32;               // tokens of a chunk
 constexpr int kPad = 4;               // floats behind every LDS row: 16-byte reads of 8 rows meet 8 different bank groups
 
@@ -323,11 +329,16 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
     g_rest = static_cast<float>(g_chunk - static_cast<double>(static_cast<float>(g_chunk)));
   }
 
-  // the next chunk's rows on their way: q and k four entries a thread, P and T too, a value for each of the wave's 32 x 16
+  // the next chunk's rows on their way, as they lie in memory (a conversion here would wait for them): q and k four entries a thread, P
+  // and T too, a value for each of the wave's 32 x 16
   constexpr int KQ = kCh * D / 4 / NT, PN = (MATS * kCh * kCh / 4 + NT - 1) / NT, PX = PN > 0 ? PN : 1;
   static_assert(kCh * D / 4 % NT == 0, "whole rows of q and k a step");
-  float4 kreg[KQ], qreg[FULL ? KQ : 1], preg[PX];
-  float vreg[8], gereg;
+  using Row4 = std::conditional_t<SILU, uint2, float4>;
+  using Entry = std::conditional_t<SILU, uint32_t, float>;
+  Row4 kreg[KQ], qreg[FULL ? KQ : 1];
+  float4 preg[PX];
+  Entry vreg[8];
+  float gereg;
   const uint32_t kq_off = static_cast<uint32_t>(threadIdx.x % (D / 4) * 4);
   const int kq_tok = threadIdx.x / (D / 4);
   const uint32_t k_off = kq_tok * static_cast<uint32_t>(p.ldk) + kq_off, q_off = kq_tok * static_cast<uint32_t>(p.ldq) + kq_off;
@@ -336,6 +347,14 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
   const uint32_t ge_off = static_cast<uint32_t>((lane & 31) * p.H + hw);
   const int p_tok = (threadIdx.x >> 3) & 31;
   const uint32_t p_off = static_cast<uint32_t>(p_tok * p.H * kCh + (threadIdx.x & 7) * 4);
+  auto entry = [](const T* at) __attribute__((always_inline)) {
+    if constexpr (SILU) return static_cast<uint32_t>(at->bits);
+    else return *at;
+  };
+  auto four = [](Row4 x) __attribute__((always_inline)) {
+    if constexpr (SILU) return chunk_act<true>(ld4(reinterpret_cast<const bf16_t*>(&x)));
+    else return x;
+  };
   auto fetch_rows = [&](int c0, auto whole) __attribute__((always_inline)) {
     constexpr bool WHOLE = decltype(whole)::value;     // all 32 tokens are there: loads without conditions
     const int cn = s1 - c0;
@@ -343,8 +362,8 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
     for (int it = 0; it < KQ; ++it) {
       constexpr int per = NT / (D / 4);
       const bool in = WHOLE || kq_tok + it * per < cn;
-      kreg[it] = in ? ld4(kp + static_cast<int64_t>(c0 + it * per) * p.ldk + k_off) : float4{0, 0, 0, 0};
-      if constexpr (FULL) qreg[it] = in ? ld4(qp + static_cast<int64_t>(c0 + it * per) * p.ldq + q_off) : float4{0, 0, 0, 0};
+      kreg[it] = in ? *reinterpret_cast<const Row4*>(kp + static_cast<int64_t>(c0 + it * per) * p.ldk + k_off) : Row4{};
+      if constexpr (FULL) qreg[it] = in ? *reinterpret_cast<const Row4*>(qp + static_cast<int64_t>(c0 + it * per) * p.ldq + q_off) : Row4{};
     }
 #pragma unroll
     for (int it = 0; it < PN; ++it) {
@@ -357,7 +376,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int lo = 16 * (i >> 2) + (i & 3);
-      vreg[i] = WHOLE || lo + 4 * quad < cn ? ldf(vp + static_cast<int64_t>(c0 + lo) * p.ldv + v_off) : 0.0f;
+      vreg[i] = WHOLE || lo + 4 * quad < cn ? entry(vp + static_cast<int64_t>(c0 + lo) * p.ldv + v_off) : Entry{};
     }
     const bool in = WHOLE || (lane & 31) < cn;         // lane = token, G in the lower half of the lanes, E in the upper
     const int64_t at = row0 + static_cast<int64_t>(c0) * p.H + h0;
@@ -411,8 +430,8 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
 #pragma unroll
     for (int it = 0; it < KQ; ++it) {
       const int at = (kq_tok + it * (NT / (D / 4))) * RS + kq_off;
-      st4(k_all[buf] + at, chunk_act<SILU>(kreg[it]));
-      if constexpr (FULL) st4(q_all[buf] + at, chunk_act<SILU>(qreg[it]));
+      st4(k_all[buf] + at, four(kreg[it]));
+      if constexpr (FULL) st4(q_all[buf] + at, four(qreg[it]));
     }
 #pragma unroll
     for (int it = 0; it < PN; ++it) {
@@ -420,7 +439,10 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
       if (m < MATS) st4(pt_all[buf][m] + p_tok * PS + (threadIdx.x & 7) * 4, preg[it]);
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) U_next[i >> 2][i & 3] = SILU ? chunk_silu(vreg[i]) : vreg[i];
+    for (int i = 0; i < 8; ++i) {
+      if constexpr (SILU) U_next[i >> 2][i & 3] = chunk_silu(__builtin_bit_cast(float, vreg[i] << 16));
+      else U_next[i >> 2][i & 3] = vreg[i];
+    }
     if (w % WPW == 0) ge_all[buf][hw][lane] = gereg;
   };
   // Two buffers: a chunk is staged while the one before it is computed, each wave at its own time, and two chunks ahead are on
@@ -466,10 +488,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
 #pragma unroll
     for (int x = 0; x < 2; ++x) u2[x] = scale4(U[x], rows4(ge_lds[hw] + kCh, x));
     const float g_last = ge_lds[hw][cn - 1];
-    if (c0 + kCh < s1) {
-      stage(buf ^ 1);
-      if (c0 + 2 * kCh < s1) fetch(c0 + 2 * kCh);
-    }
+    stage(buf ^ 1);                                    // (behind the last chunk for nobody: without a branch, among the products)
 #pragma unroll
     for (int j = 0; j < DT; ++j) {
       // constant decays, slow as a rule: what the chunk adds in two sums of its own, for fewer roundings at the state's magnitude
@@ -484,6 +503,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
       for (int i = 0; i < 4; ++i)
         S[j][i] = APART ? fmaf(S[j][i], g_last, fmaf(S[j][i], cn == kCh ? g_rest : 0.0f, add[0][i] + add[1][i])) : add[0][i];
     }
+    if (c0 + 2 * kCh < s1) fetch(c0 + 2 * kCh);
     if constexpr (FULL) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -492,6 +512,325 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
       }
     }
     if constexpr (MODE == 1) seg_dec *= KIND == kChunkConst ? g_chunk : static_cast<double>(g_last);      // (only whole chunks)
+    __syncthreads();                                   // the next chunk is complete, and nobody reads this one any more
+  }
+  if (MODE == 1 || s1 == n_all) {
+    float* to = MODE == 1 ? gbase : sbase;
+#pragma unroll
+    for (int j = 0; j < DT; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) to[(16 * j + i) * p.Dv + st_off] = S[j][i];
+  }
+  if (MODE == 1 && lane == 0) p.seg_decay[(static_cast<int64_t>(b) * p.segs + blockIdx.y) * p.H + h] = static_cast<float>(seg_dec);
+}
+
+// Three bf16 numbers whose sum is a finite f32 value: its 24 bits cut into eights, so that nothing is rounded. As operands of the bf16
+// matrix instructions (exact products, f32 sums) they give f32 products at four to eight times the f32 instructions' rate. An
+// infinity has no such pieces: a wave that meets one computes its chunk on the f32 instructions.
+struct Pieces4 { uint2 p[3]; };
+__device__ __forceinline__ uint32_t high_halves(float a, float b) {
+  return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
+}
+__device__ __forceinline__ float below_high(float a) { return a - __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, a) & 0xffff0000u); }
+__device__ __forceinline__ Pieces4 cut4(float x, float y, float z, float w) {
+  Pieces4 r;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    r.p[i] = uint2{high_halves(x, y), high_halves(z, w)};
+    if (i < 2) { x = below_high(x); y = below_high(y); z = below_high(z); w = below_high(w); }
+  }
+  return r;
+}
+__device__ __forceinline__ chunk_bf16x8 join8(uint2 lo, uint2 hi) {
+  return __builtin_bit_cast(chunk_bf16x8, uint4{lo.x, lo.y, hi.x, hi.y});
+}
+
+// The same scan for step sizes, whose q, k and v rows are bf16: an f32 value on the other side of a product is cut into its pieces, and
+// three products on the bf16 instructions (exact, summed in f32) do for an f32 one, at three sixteenths of its time. The state is cut
+// anew in every chunk. A chunk's read-out, its addition to the state and the staging of the next one stand in one block of code, so that
+// each one's products run beside the others' cutting and reads. us, f32 products -> this, with the kernel in front: 32 x 512 tokens, 32
+// heads of 128 x 64, 273 -> 190; 16 x 512 of 64 x 64 98 -> 77; one of 4096 in segments of 256 121 -> 94. It stays far from the matrix
+// rate (two waves a SIMD, some 3 us a chunk); more waves did not fit: at 128 registers it spills (315 us for the first).
+// Against 64 bits outputs are 0.77e-7 off, 0.83e-7 before, states 0.53 to 0.69e-7, as before.
+template <int DT, int NW, int HPW, int MODE>
+__global__ __launch_bounds__(NW * 64, 2) void chunk_step_kernel(ChunkParams p) {
+  constexpr bool FULL = MODE != 1;
+  constexpr int D = DT * 16, RB = D * 2 + 16, PB = kCh * 2 + 16, NT = NW * 64, WPW = NW / HPW;      // RB, PB: bytes of an LDS row
+  constexpr int MATS = FULL ? HPW : 0, kMatImg = kCh * PB;
+  __shared__ __attribute__((aligned(16))) unsigned char k_all[2][kCh * RB];
+  __shared__ __attribute__((aligned(16))) unsigned char q_all[2][FULL ? kCh * RB : 16];
+  __shared__ __attribute__((aligned(16))) unsigned char p_all[2][MATS > 0 ? MATS : 1][MATS > 0 ? 3 * kMatImg : 16];
+  __shared__ __attribute__((aligned(16))) float ge_all[2][HPW][2 * kCh];      // G, then E
+  __shared__ int odd_all[2][NW];                       // whether a wave staged a q, k or P that is not finite
+  const int b = blockIdx.z;
+  const int q0 = p.cu_q[b], n_all = p.cu_q[b + 1] - q0;
+  const int s0 = MODE == 0 ? 0 : blockIdx.y * p.seg_len;
+  const int s1 = MODE == 0 ? n_all : min(n_all, s0 + p.seg_len);
+  if (s0 >= n_all || (MODE == 1 && s1 == n_all)) return;       // what the last segment adds is nobody's start
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, quad = lane >> 4;
+  const int parts = p.Dv / 16 / WPW;                           // 1 where several heads share the workgroup
+  const int h0 = static_cast<int>(blockIdx.x) / parts * HPW, hw = w / WPW, h = h0 + hw;         // (uniform over a wave)
+  const int col = ((static_cast<int>(blockIdx.x) % parts) * WPW + w % WPW) * 16 + r;
+  const int g = h0 / (p.H / p.G);
+  const uint16_t* kp = static_cast<const uint16_t*>(p.k) + static_cast<int64_t>(q0) * p.ldk + static_cast<int64_t>(g) * D;
+  const uint16_t* qp = static_cast<const uint16_t*>(p.q) + static_cast<int64_t>(q0) * p.ldq + static_cast<int64_t>(g) * D;
+  const uint16_t* vp = static_cast<const uint16_t*>(p.v) + static_cast<int64_t>(q0) * p.ldv + static_cast<int64_t>(h) * p.Dv;
+  const int64_t row0 = static_cast<int64_t>(q0) * p.H;
+  float* sbase = p.state + (static_cast<int64_t>(p.slots[b]) * p.H + h) * D * p.Dv;
+  float* gbase = MODE == 0 ? nullptr : p.seg_state + ((static_cast<int64_t>(b) * p.segs + blockIdx.y) * p.H + h) * D * p.Dv;
+
+  // addresses are a uniform row plus a lane's 32-bit offset inside it
+  const uint32_t st_off = static_cast<uint32_t>(4 * quad * p.Dv) + col;
+  f32x4 S[DT];
+  {
+    const bool carry = MODE == 2 ? p.segs > 0 : MODE == 0 && p.ctx_lens[b] > 0;
+    const float* from = MODE == 2 ? gbase : sbase;
+#pragma unroll
+    for (int j = 0; j < DT; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[j][i] = carry ? from[(16 * j + i) * p.Dv + st_off] : 0.0f;
+  }
+  const float skip = FULL ? p.p2[h] : 0.0f;
+  double seg_dec = 1.0;
+
+  // the next chunk's rows on their way, as they lie in memory (a conversion here would wait for them): q and k four entries a thread, P
+  // too, a value for each of the wave's 32 x 16
+  constexpr int KQ = kCh * D / 4 / NT, PN = (MATS * kCh * kCh / 4 + NT - 1) / NT, PX = PN > 0 ? PN : 1;
+  static_assert(kCh * D / 4 % NT == 0, "whole rows of q and k a step");
+  uint2 kreg[KQ], qreg[FULL ? KQ : 1];
+  float4 preg[PX];
+  uint32_t vreg[8];
+  float gereg;
+  const int kq_d = threadIdx.x % (D / 4) * 4, kq_tok = threadIdx.x / (D / 4);
+  const uint32_t k_off = kq_tok * static_cast<uint32_t>(p.ldk) + kq_d, q_off = kq_tok * static_cast<uint32_t>(p.ldq) + kq_d;
+  const uint32_t v_off = 8 * quad * static_cast<uint32_t>(p.ldv) + col;
+  const uint32_t o_off = static_cast<uint32_t>(8 * quad * p.H * p.Dv) + col;
+  const uint32_t ge_off = static_cast<uint32_t>((lane & 31) * p.H + hw);
+  const int p_tok = (threadIdx.x >> 3) & 31;
+  const uint32_t p_off = static_cast<uint32_t>(p_tok * p.H * kCh + (threadIdx.x & 7) * 4);
+  auto fetch_rows = [&](int c0, auto whole) __attribute__((always_inline)) {
+    constexpr bool WHOLE = decltype(whole)::value;     // all 32 tokens are there: loads without conditions
+    const int cn = s1 - c0;
+#pragma unroll
+    for (int it = 0; it < KQ; ++it) {
+      constexpr int per = NT / (D / 4);
+      const bool in = WHOLE || kq_tok + it * per < cn;
+      kreg[it] = in ? *reinterpret_cast<const uint2*>(kp + static_cast<int64_t>(c0 + it * per) * p.ldk + k_off) : uint2{0, 0};
+      if constexpr (FULL) qreg[it] = in ? *reinterpret_cast<const uint2*>(qp + static_cast<int64_t>(c0 + it * per) * p.ldq + q_off) : uint2{0, 0};
+    }
+#pragma unroll
+    for (int it = 0; it < PN; ++it) {
+      const int m = (it * NT + (w << 6)) >> 8;         // matrix of this wave's pieces
+      const bool in = m < MATS && (WHOLE || p_tok < cn);
+      preg[it] = in ? ld4(p.P + (row0 + static_cast<int64_t>(c0) * p.H + h0 + m) * kCh + p_off) : float4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      vreg[i] = WHOLE || i + 8 * quad < cn ? vp[static_cast<int64_t>(c0 + i) * p.ldv + v_off] : 0u;
+    const bool in = WHOLE || (lane & 31) < cn;         // lane = token, G in the lower half of the lanes, E in the upper
+    const int64_t at = row0 + static_cast<int64_t>(c0) * p.H + h0;
+    gereg = in ? (lane >= 32 ? p.Ef : p.Gf)[at + ge_off] : 0.0f;
+  };
+  auto fetch = [&](int c0) __attribute__((always_inline)) {
+    if (s1 - c0 >= kCh) fetch_rows(c0, std::true_type{});
+    else fetch_rows(c0, std::false_type{});
+  };
+  // Rows 16 j + 4 quad + i of the state are those of a 16 x 16 result, and a lane's of two of them make its eight k slots of a product:
+  // rows of q and k lie in LDS in that order, four entries at a time. Result rows over tokens, 16 x + 4 quad + i, stand for token
+  // 8 quad + 4 x + i: a lane's are eight in a row, and sums over tokens run in their order, from the most decayed on.
+  auto place = [](int c) { return c < 4 ? 8 * c : 8 * (c - 4) + 4; };           // of the c-th four of 32
+  const int kq_byte = 2 * (kq_d / 32 * 32 + place(kq_d % 32 / 4)), p_byte = p_tok * PB + 8 * (threadIdx.x & 7);
+  const int r_tok = 8 * (r >> 2) + (r & 3), a_off = r_tok * RB + 16 * quad, m_off = r_tok * PB + 16 * quad;       // a lane's 16 bytes of a left-hand row
+  // K^T comes transposed out of LDS: a lane names four entries of one token and gets one entry of four tokens
+  const int t_off = (8 * quad + (r >> 2)) * RB + 16 * (r & 3);
+  auto frag = [&](const unsigned char* at) __attribute__((always_inline)) {
+    return __builtin_bit_cast(chunk_bf16x8, *reinterpret_cast<const uint4*>(at));
+  };
+  auto frag_t = [&](const unsigned char* img, int j) __attribute__((always_inline)) {
+    using lds_bf16x4 = __attribute__((address_space(3))) chunk_bf16x4;
+    const unsigned char* at = img + t_off + 64 * (j >> 1) + 8 * (j & 1);
+    const chunk_bf16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)at);
+    const chunk_bf16x4 y = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(at + 4 * RB));
+    return chunk_bf16x8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+  };
+  auto mm = [](chunk_bf16x8 a, chunk_bf16x8 bb, f32x4 c) __attribute__((always_inline)) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bb, c, 0, 0, 0);
+  };
+  auto rows4 = [&](const float* from, int x) __attribute__((always_inline)) {   // of a vector over tokens
+    return *reinterpret_cast<const float4*>(from + 8 * quad + 4 * x);
+  };
+  auto scale4 = [&](f32x4 x, float4 f) __attribute__((always_inline)) { return f32x4{x[0] * f.x, x[1] * f.y, x[2] * f.z, x[3] * f.w}; };
+  const f32x4 zero{0.0f, 0.0f, 0.0f, 0.0f};
+  auto cut8 = [](f32x4 a, f32x4 c, chunk_bf16x8 (&to)[3]) __attribute__((always_inline)) {
+    const Pieces4 x = cut4(a[0], a[1], a[2], a[3]), y = cut4(c[0], c[1], c[2], c[3]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) to[i] = join8(x.p[i], y.p[i]);
+  };
+  auto all_finite = [](const f32x4 (&x)[2]) __attribute__((always_inline)) {
+    float z = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) z = fmaf(x[i >> 2][i & 3], 0.0f, z);
+    return __builtin_amdgcn_ballot_w64(z != 0.0f) == 0;
+  };
+  // four entries from the place `at` on, put together from their pieces (an infinity's others are no numbers)
+  auto matrix4 = [&](const unsigned char* at) {
+    float4 x = ld4(reinterpret_cast<const bf16_t*>(at));
+#pragma unroll
+    for (int i = 1; i < 3; ++i) {
+      const float4 y = ld4(reinterpret_cast<const bf16_t*>(at + i * kMatImg));
+      auto add = [](float a, float c) { return __builtin_amdgcn_classf(a, 0x207) ? a : a + c; };
+      x = float4{add(x.x, y.x), add(x.y, y.y), add(x.z, y.z), add(x.w, y.w)};
+    }
+    return x;
+  };
+  f32x4 U_next[2];
+  auto stage = [&](int buf) __attribute__((always_inline)) {
+    float z = 0.0f;                                    // NaN if a value is not finite
+    auto put = [&](unsigned char* img, int at, uint2 v) __attribute__((always_inline)) {
+      *reinterpret_cast<uint2*>(img + at) = v;
+      auto hi = [](uint32_t x) { return __builtin_bit_cast(float, x & 0xffff0000u); };
+      auto lo = [](uint32_t x) { return __builtin_bit_cast(float, x << 16); };
+      z = fmaf(lo(v.x), 0.0f, fmaf(hi(v.x), 0.0f, fmaf(lo(v.y), 0.0f, fmaf(hi(v.y), 0.0f, z))));
+    };
+#pragma unroll
+    for (int it = 0; it < KQ; ++it) {
+      const int at = (kq_tok + it * (NT / (D / 4))) * RB + kq_byte;
+      put(k_all[buf], at, kreg[it]);
+      if constexpr (FULL) put(q_all[buf], at, qreg[it]);
+    }
+#pragma unroll
+    for (int it = 0; it < PN; ++it) {
+      const int m = (it * NT + (w << 6)) >> 8;
+      if (m < MATS) {
+        const float4 x = preg[it];
+        z = fmaf(x.x, 0.0f, fmaf(x.y, 0.0f, fmaf(x.z, 0.0f, fmaf(x.w, 0.0f, z))));
+        const Pieces4 c = cut4(x.x, x.y, x.z, x.w);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) *reinterpret_cast<uint2*>(p_all[buf][m] + i * kMatImg + p_byte) = c.p[i];
+      }
+    }
+    const bool odd = __builtin_amdgcn_ballot_w64(z != 0.0f) != 0;
+    if (lane == 0) odd_all[buf][w] = odd;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) U_next[i >> 2][i & 3] = __builtin_bit_cast(float, vreg[i] << 16);
+    if (w % WPW == 0) ge_all[buf][hw][lane] = gereg;
+  };
+  // Two buffers: a chunk is staged while the one before it is computed, each wave at its own time, and two chunks ahead are on
+  // their way in registers. One barrier a chunk.
+  fetch(s0);
+  stage(0);
+  if (s0 + kCh < s1) fetch(s0 + kCh);
+  __syncthreads();
+  int buf = 0;
+  for (int c0 = s0; c0 < s1; c0 += kCh, buf ^= 1) {
+    const int cn = min(kCh, s1 - c0);
+    const unsigned char *k_lds = k_all[buf], *q_lds = q_all[buf], *p_lds = p_all[buf][MATS > 0 ? hw : 0];
+    const float* ge_lds = ge_all[buf][hw];
+    const f32x4 U[2] = {U_next[0], U_next[1]};
+    f32x4 o[2], u2[2], next[DT];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) u2[x] = scale4(U[x], rows4(ge_lds + kCh, x));
+    const float g_last = ge_lds[cn - 1];
+    bool odd = __builtin_amdgcn_ballot_w64(odd_all[buf][lane & (NW - 1)] != 0) != 0 || !all_finite(u2) || (FULL && !all_finite(U));
+    if (__builtin_expect(!odd, 1)) {
+      f32x4 qs[2][2], pu[2];                           // [sum][rows]: the largest pieces' products apart from the others'
+#pragma unroll
+      for (int x = 0; x < 2; ++x) qs[0][x] = qs[1][x] = pu[x] = zero;
+      chunk_bf16x8 uc[3];
+      cut8(u2[0], u2[1], uc);
+      stage(buf ^ 1);
+#pragma unroll
+      for (int jj = 0; jj < DT / 2; ++jj) {
+        if constexpr (FULL) {
+          chunk_bf16x8 sc[3];
+          cut8(S[2 * jj], S[2 * jj + 1], sc);
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            const chunk_bf16x8 qf = frag(q_lds + 4 * x * RB + 64 * jj + a_off);
+            qs[1][x] = mm(qf, sc[2], qs[1][x]);
+            qs[1][x] = mm(qf, sc[1], qs[1][x]);
+            qs[0][x] = mm(qf, sc[0], qs[0][x]);
+          }
+        }
+#pragma unroll
+        for (int j = 2 * jj; j < 2 * jj + 2; ++j) {
+          const chunk_bf16x8 kf = frag_t(k_lds, j);
+          f32x4 rest = mm(kf, uc[1], mm(kf, uc[2], zero));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) rest[i] = fmaf(S[j][i], g_last, rest[i]);
+          next[j] = mm(kf, uc[0], rest);
+        }
+      }
+      if constexpr (FULL) {
+        // U as it came: bf16
+        const chunk_bf16x8 ub = join8(uint2{high_halves(U[0][0], U[0][1]), high_halves(U[0][2], U[0][3])},
+                                      uint2{high_halves(U[1][0], U[1][1]), high_halves(U[1][2], U[1][3])});
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+#pragma unroll
+          for (int i = 2; i >= 0; --i) pu[x] = mm(frag(p_lds + i * kMatImg + 4 * x * PB + m_off), ub, pu[x]);
+          o[x] = scale4(qs[0][x] + qs[1][x], rows4(ge_lds, x)) + skip * U[x] + pu[x];
+        }
+        odd = !all_finite(o);                          // the state itself may hold an infinity
+      }
+    } else {
+      stage(buf ^ 1);
+    }
+    if (c0 + 2 * kCh < s1) fetch(c0 + 2 * kCh);
+    if (__builtin_expect(odd, 0)) {
+      // the chunk in f32, the lower triangle token by token: a value that is not finite would reach the tokens before it through zeros
+      auto row4 = [&](const unsigned char* img, int tok, int d) {
+        return ld4(reinterpret_cast<const bf16_t*>(img + tok * RB + 64 * (d / 32) + 2 * place(d % 32 / 4)));
+      };
+      if constexpr (FULL) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          f32x4 acc = zero;
+#pragma unroll
+          for (int j = 0; j < DT; ++j) {
+            const float4 a = row4(q_lds, r_tok + 4 * x, 16 * j + 4 * quad);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, S[j][0], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, S[j][1], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, S[j][2], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, S[j][3], acc, 0, 0, 0);
+          }
+          o[x] = scale4(acc, rows4(ge_lds, x)) + skip * U[x];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll 1
+          for (int from = 0; from < 4; ++from) {
+            const int j = 8 * from + i;
+            const float v = __shfl(U[i >> 2][i & 3], 16 * from + r, kWave);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+              const int t = 8 * quad + k;
+              const float4 row = matrix4(p_lds + t * PB + 8 * (j / 4));
+              const float e = (j & 2) ? ((j & 1) ? row.w : row.z) : ((j & 1) ? row.y : row.x);
+              o[k >> 2][k & 3] = j <= t ? fmaf(e, v, o[k >> 2][k & 3]) : o[k >> 2][k & 3];
+            }
+          }
+      }
+#pragma unroll
+      for (int j = 0; j < DT; ++j) {
+        f32x4 add = S[j] * g_last;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float4 row = row4(k_lds, 8 * quad + i, 16 * j + (r & 12));
+          const float e = (r & 2) ? ((r & 1) ? row.w : row.z) : ((r & 1) ? row.y : row.x);
+          add = __builtin_amdgcn_mfma_f32_16x16x4f32(e, u2[i >> 2][i & 3], add, 0, 0, 0);
+        }
+        next[j] = add;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < DT; ++j) S[j] = next[j];
+    if constexpr (FULL) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (i + 8 * quad < cn) p.o[(row0 + static_cast<int64_t>(c0 + i) * p.H + h) * p.Dv + o_off] = o[i >> 2][i & 3];
+    }
+    if constexpr (MODE == 1) seg_dec *= static_cast<double>(g_last);      // (only whole chunks)
     __syncthreads();                                   // the next chunk is complete, and nobody reads this one any more
   }
   if (MODE == 1 || s1 == n_all) {
@@ -526,16 +865,19 @@ __global__ __launch_bounds__(256) void chunk_combine_kernel(ChunkParams p) {
 
 template <typename T, int KIND, int DT, int NW, int HPW>
 static void chunk_launch(const ChunkParams& p, int B, hipStream_t s) {
-  dim3 grid(p.H / HPW * (p.Dv / 16 / (NW / HPW)), 1, B), block(NW * 64);
+  dim3 grid(p.H / HPW * (p.Dv / 16 / (NW / HPW)), p.segs, B), block(NW * 64);
+  auto scan = [&](auto mode) {
+    if constexpr (KIND == kChunkStep) chunk_step_kernel<DT, NW, HPW, decltype(mode)::value><<<grid, block, 0, s>>>(p);
+    else chunk_scan_kernel<T, KIND, DT, NW, HPW, decltype(mode)::value><<<grid, block, 0, s>>>(p);
+  };
   if (p.segs <= 1) {
-    chunk_scan_kernel<T, KIND, DT, NW, HPW, 0><<<grid, block, 0, s>>>(p);
+    scan(std::integral_constant<int, 0>{});
     return;
   }
   if constexpr (KIND != kChunkDelta) {
-    grid.y = p.segs;
-    chunk_scan_kernel<T, KIND, DT, NW, HPW, 1><<<grid, block, 0, s>>>(p);
+    scan(std::integral_constant<int, 1>{});
     chunk_combine_kernel<<<dim3((p.D * p.Dv / 4 + 255) / 256, p.H, B), dim3(256), 0, s>>>(p);
-    chunk_scan_kernel<T, KIND, DT, NW, HPW, 2><<<grid, block, 0, s>>>(p);
+    scan(std::integral_constant<int, 2>{});
   }
 }
 
