@@ -67,6 +67,7 @@
  *   lv_gated_linear_recurrence   Griffin's RG-LRU: block-diagonal gates, S <- a S + sqrt(1 - a^2) i u per channel, gelu branch
  *   lv_scaled_embedding      token rows times a constant as the f32 residual
  *   lv_rows_gemm             projections of up to 64 rows
+ *   lv_delta_prep_one, lv_delta_rule_one   the delta rule on steps of one token a sequence, two launches instead of four
  *   lv_residual_split        residual update, and the residual as the sum of two bf16 numbers for a matrix product
  *
  * A "ragged step" is a batch of B sequences; sequence b brings cu_q[b+1]-cu_q[b] new tokens that
@@ -498,6 +499,19 @@ int lv_scaled_embedding(const void* ids, const void* table, int vocab, float sca
 
 /* x f32 [T, W] += y (bf16 [T, W], may be NULL);  out bf16 [T, 2W] = x rounded | (x - x rounded) rounded. */
 int lv_residual_split(void* x, const void* y, void* out, int64_t T, int W, void* stream);
+
+/* lv_delta_prep and lv_conv_state_update in one launch, for steps in which every sequence has at most one new token. Heads of 64, 128 or
+ * 256 keys and values alike, up to four taps, rows of whole four-entry pieces; -2 for others. */
+int lv_delta_prep_one(const void* proj, int64_t ld, const void* conv_w, void* conv_state, const void* A_log, const void* dt_bias,
+                      const int32_t* cu_q, const int32_t* ctx_lens, const int32_t* slots, const int32_t* tok_seq, void* qn, void* kn, void* v,
+                      void* beta, void* decay, int64_t T, int G, int H, int D, int Dv, int taps, int off_b, const void* a, int64_t ld_a,
+                      int decay_per_channel, float unit_eps, int dtype, void* stream);
+
+/* lv_gated_delta_rule and lv_head_norm_gate in one launch, for steps in which every sequence has at most one new token and heads of
+ * D = 64 or 128 keys and values: out act [T, H*D]. f32 rows and the state 16-byte aligned, gate and out four entries. */
+int lv_delta_rule_one(const void* qn, const void* kn, const void* v, const void* beta, const void* decay, void* state, const int32_t* cu_q,
+                      const int32_t* ctx_lens, const int32_t* slots, const void* gate, int64_t ld_gate, const void* norm_w, void* out,
+                      int B, int G, int H, int D, int decay_per_channel, float eps, int gate_act, int dtype, void* stream);
 
 /* y bf16 [M, N] = x bf16 [M, K] w^T, w bf16 [N, K], sums in f32. M <= 64, K a multiple of 32; row strides ldx, ldw (multiples of 8)
  * and ldy in entries; x and w 16-byte, y 8-byte aligned. */

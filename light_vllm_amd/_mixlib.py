@@ -30,6 +30,10 @@ SIGNATURES = {
     "lv_clamped_glu": (c_int, [_P, c_int64, _P, c_int64, c_int, c_float, c_float, c_int, _P]),
     "lv_delta_prep": (c_int, [_P, c_int64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, c_int64,
                               c_int, c_int, c_int, c_int, c_int, c_int, _P, c_int64, c_int, c_float, c_int, _P]),
+    "lv_delta_prep_one": (c_int, [_P, c_int64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, c_int64,
+                                  c_int, c_int, c_int, c_int, c_int, c_int, _P, c_int64, c_int, c_float, c_int, _P]),
+    "lv_delta_rule_one": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, c_int64, _P, _P, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
+                                  c_int, _P]),
     "lv_conv_state_update": (c_int, [_P, c_int64, _P, _P, _P, _P, c_int, c_int, c_int, c_int, _P]),
     "lv_gated_delta_rule": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P]),
     "lv_head_norm_gate": (c_int, [_P, _P, c_int64, _P, _P, c_int64, c_int, c_int, c_float, c_int, c_int, _P]),

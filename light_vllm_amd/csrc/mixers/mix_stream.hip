@@ -319,8 +319,12 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(DeltaPrepParams p) {
 // Bound by memory (the projection's rows in, f32 rows out). The wave-per-(token, head) form above reads every row once per tap,
 // two bytes a lane: 16 x 1024 tokens, 3072 channels, four taps 374 us, this form 109 us;
 // 64 decoded tokens 5.5 -> 4.2 us.
+//
+// new_state: every sequence has one new token (the caller knows), so the thread that holds a channel's last inputs is the only one to read
+// what the sequence carries, and writes what it carries next in the same launch: a decode step of 64 tokens, 3072 channels, takes 4.8 us
+// for both, 4.8 and 4.7 in two launches.
 template <typename T, int TAPS>
-__global__ __launch_bounds__(256) void delta_prep_tile_kernel(DeltaPrepParams p, int tile) {
+__global__ __launch_bounds__(256) void delta_prep_tile_kernel(DeltaPrepParams p, int tile, T* new_state) {
   const int64_t t0 = static_cast<int64_t>(blockIdx.y) * tile, t1 = min(t0 + tile, p.T);
   const T* proj = static_cast<const T*>(p.proj);
   const int GD = p.G * p.D, C = 2 * GD + p.H * p.Dv, cols = (C / 4 + 255) / 256, col = blockIdx.x;
@@ -388,6 +392,17 @@ __global__ __launch_bounds__(256) void delta_prep_tile_kernel(DeltaPrepParams p,
     st4(dst + t * ldd, y);
   };
   int b = p.tok_seq[t0];
+  if (new_state != nullptr) {
+    for (int64_t t = t0; t < t1; ++t) {
+      b = p.tok_seq[t];
+      history(t, b);
+      emit(t, ld4(proj + t * p.ld + c));
+      T* row = new_state + static_cast<int64_t>(p.slots[b]) * (TAPS - 1) * C + c;
+#pragma unroll
+      for (int j = 0; j < TAPS - 1; ++j) st4(row + static_cast<int64_t>(j) * C, hist[j]);
+    }
+    return;
+  }
   history(t0, b);
   if (p.tok_seq[t1 - 1] == b) {                    // one sequence: the next rows' loads need not wait for a look at its end
 #pragma unroll 4
@@ -402,7 +417,7 @@ __global__ __launch_bounds__(256) void delta_prep_tile_kernel(DeltaPrepParams p,
 }
 
 template <typename T>
-static bool delta_prep_tiles(const DeltaPrepParams& p, hipStream_t s) {
+static bool delta_prep_tiles(const DeltaPrepParams& p, void* new_state, hipStream_t s) {
   auto at = [](const void* q, uintptr_t a) { return reinterpret_cast<uintptr_t>(q) % a == 0; };
   constexpr uintptr_t piece = 4 * sizeof(T);
   if (p.D != p.Dv || (p.D != 64 && p.D != 128 && p.D != 256) || p.taps > 4 || p.ld % 4 != 0 || !at(p.proj, piece) ||
@@ -414,10 +429,10 @@ static bool delta_prep_tiles(const DeltaPrepParams& p, hipStream_t s) {
   dim3 grid(cols + 1 + (p.dec_dim > 1 ? (p.H * p.dec_dim + 255) / 256 : 0), static_cast<unsigned>((p.T + tile - 1) / tile)), block(256);
   if (grid.y > 65535) return false;
   switch (p.taps) {
-    case 1: delta_prep_tile_kernel<T, 1><<<grid, block, 0, s>>>(p, tile); break;
-    case 2: delta_prep_tile_kernel<T, 2><<<grid, block, 0, s>>>(p, tile); break;
-    case 3: delta_prep_tile_kernel<T, 3><<<grid, block, 0, s>>>(p, tile); break;
-    default: delta_prep_tile_kernel<T, 4><<<grid, block, 0, s>>>(p, tile); break;
+    case 1: delta_prep_tile_kernel<T, 1><<<grid, block, 0, s>>>(p, tile, static_cast<T*>(new_state)); break;
+    case 2: delta_prep_tile_kernel<T, 2><<<grid, block, 0, s>>>(p, tile, static_cast<T*>(new_state)); break;
+    case 3: delta_prep_tile_kernel<T, 3><<<grid, block, 0, s>>>(p, tile, static_cast<T*>(new_state)); break;
+    default: delta_prep_tile_kernel<T, 4><<<grid, block, 0, s>>>(p, tile, static_cast<T*>(new_state)); break;
   }
   return true;
 }
@@ -565,6 +580,80 @@ __global__ __launch_bounds__(256) void gated_delta_rule_kernel(DeltaRuleParams p
     for (int r = 0; r < DR; ++r)
       if (row0 + r < p.D) sbase[static_cast<int64_t>(row0 + r) * p.Dv + col] = s[r];
   }
+}
+
+// One new token a sequence (decode steps), heads of D = 64 or 128 keys and values: the rule, each head's norm and its gate in one launch, a
+// workgroup a (head, sequence). A thread owns four columns of every 256 * 4 / D-th of the rows; the state comes and goes in 16-byte
+// pieces, all requested before anything else is looked at, and both sums over its rows meet in LDS. Bound by memory (the state read and
+// written): 64 sequences, 16 heads of 128 x 128: with the
+// carried inputs written in the preparation, four launches become two, and a layer of Kagalorn's decode step takes 40 us instead of 55.
+template <typename T, int D, bool CH>
+__global__ __launch_bounds__(256) void delta_one_kernel(DeltaRuleParams p, const T* __restrict__ gate, int64_t ld_gate,
+                                                        const float* __restrict__ norm_w, T* __restrict__ out, float eps, int gate_act) {
+  constexpr int LANES = D / 4, RG = 256 / LANES, R = D / RG;         // lanes of a row, row groups, rows of a thread
+  __shared__ __attribute__((aligned(16))) float part[2][RG][D];
+  const int h = blockIdx.x, b = blockIdx.y, c = threadIdx.x % LANES * 4, rg = threadIdx.x / LANES;
+  const int64_t t = p.cu_q[b];
+  if (p.cu_q[b + 1] - t <= 0) return;
+  float* sbase = p.state + (static_cast<int64_t>(p.slots[b]) * p.H + h) * D * D + rg * R * D + c;
+  const bool carry = p.ctx_lens[b] > 0;
+  float4 s[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) s[r] = carry ? ld4(sbase + r * D) : float4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int64_t krow = (t * p.G + h / (p.H / p.G)) * D + rg * R, hrow = t * p.H + h;
+  float k[R], q[R], g[CH ? R : 1];
+#pragma unroll
+  for (int r = 0; r < R; r += 4) {
+    const float4 x = ld4(p.kn + krow + r), y = ld4(p.qn + krow + r);
+    k[r] = x.x; k[r + 1] = x.y; k[r + 2] = x.z; k[r + 3] = x.w;
+    q[r] = y.x; q[r + 1] = y.y; q[r + 2] = y.z; q[r + 3] = y.w;
+    if constexpr (CH) {
+      const float4 z = ld4(p.decay + hrow * D + rg * R + r);
+      g[r] = z.x; g[r + 1] = z.y; g[r + 2] = z.z; g[r + 3] = z.w;
+    }
+  }
+  const float beta = p.beta[hrow], dec = CH ? 1.0f : p.decay[hrow];
+  const float4 v = ld4(p.v + hrow * D + c);
+  auto axpy = [](float4 a, float x, float4 y) __attribute__((always_inline)) {
+    return float4{fmaf(x, y.x, a.x), fmaf(x, y.y, a.y), fmaf(x, y.z, a.z), fmaf(x, y.w, a.w)};
+  };
+  auto add = [](float4 a, float4 y) __attribute__((always_inline)) { return float4{a.x + y.x, a.y + y.y, a.z + y.z, a.w + y.w}; };
+  const float4 zero{0.0f, 0.0f, 0.0f, 0.0f};
+  float4 sum[4] = {zero, zero, zero, zero};            // short sums, added in pairs
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if constexpr (CH) s[r] = float4{s[r].x * g[r], s[r].y * g[r], s[r].z * g[r], s[r].w * g[r]};
+    sum[r & 3] = axpy(sum[r & 3], k[r], s[r]);
+  }
+  st4(&part[0][rg][c], add(add(sum[0], sum[1]), add(sum[2], sum[3])));
+  __syncthreads();
+  auto total = [&](int i) __attribute__((always_inline)) {
+    float4 x[4] = {zero, zero, zero, zero};
+#pragma unroll
+    for (int j = 0; j < RG; ++j) x[j & 3] = add(x[j & 3], ld4(&part[i][j][c]));
+    return add(add(x[0], x[1]), add(x[2], x[3]));
+  };
+  const float4 ks = total(0);
+  const float4 u{beta * fmaf(-dec, ks.x, v.x), beta * fmaf(-dec, ks.y, v.y), beta * fmaf(-dec, ks.z, v.z), beta * fmaf(-dec, ks.w, v.w)};
+  sum[0] = sum[1] = sum[2] = sum[3] = zero;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    // (the decayed state is rounded once, with what is added)
+    s[r] = axpy(float4{k[r] * u.x, k[r] * u.y, k[r] * u.z, k[r] * u.w}, dec, s[r]);
+    sum[r & 3] = axpy(sum[r & 3], q[r], s[r]);
+    st4(sbase + r * D, s[r]);
+  }
+  st4(&part[1][rg][c], add(add(sum[0], sum[1]), add(sum[2], sum[3])));
+  __syncthreads();
+  if (rg != 0) return;
+  const float4 o = total(1);
+  float ss = row16_sum((o.x * o.x + o.y * o.y) + (o.z * o.z + o.w * o.w));
+  if constexpr (LANES > 16) ss += __shfl_xor(ss, 16, kWave);
+  const float inv = 1.0f / sqrtf(ss / static_cast<float>(D) + eps);
+  const float4 w = ld4(norm_w + c), gv = ld4(gate + t * ld_gate + static_cast<int64_t>(h) * D + c);
+  auto act = [&](float x) { return gate_act == LV_MIX_GATE_SILU ? siluf_(x) : sigmoidf_(x); };
+  st4(out + hrow * D + c, float4{o.x * inv * w.x * act(gv.x), o.y * inv * w.y * act(gv.y), o.z * inv * w.z * act(gv.z),
+                                 o.w * inv * w.w * act(gv.w)});
 }
 
 template <int DR>
@@ -729,7 +818,7 @@ int lv_clamped_glu(const void* in, int64_t ld_in, void* out, int64_t T, int F, f
   return launched("lv_clamped_glu");
 }
 
-int lv_delta_prep(const void* proj, int64_t ld, const void* conv_w, const void* conv_state, const void* A_log,
+static int delta_prep_entry(void* new_state, const void* proj, int64_t ld, const void* conv_w, const void* conv_state, const void* A_log,
                   const void* dt_bias, const int32_t* cu_q, const int32_t* ctx_lens, const int32_t* slots,
                   const int32_t* tok_seq, void* qn, void* kn, void* v, void* beta, void* decay, int64_t T, int G,
                   int H, int D, int Dv, int taps, int off_b, const void* a, int64_t ld_a, int decay_per_channel,
@@ -749,13 +838,70 @@ int lv_delta_prep(const void* proj, int64_t ld, const void* conv_w, const void* 
                     static_cast<float*>(decay), T, G, H, D, Dv, taps, off_b, unit_eps, a, ld_a, dec_dim};
   const int units = 2 * G + H + 1 + (dec_dim > 1 ? H : 0);
   dim3 grid(static_cast<unsigned>(T), (units + 3) / 4), block(256);
-  if ((dtype == LV_MIX_BF16 && delta_prep_tiles<bf16_t>(p, as_stream(stream))) ||
-      (dtype == LV_MIX_F32 && delta_prep_tiles<float>(p, as_stream(stream))))
+  if ((dtype == LV_MIX_BF16 && delta_prep_tiles<bf16_t>(p, new_state, as_stream(stream))) ||
+      (dtype == LV_MIX_F32 && delta_prep_tiles<float>(p, new_state, as_stream(stream))))
     return launched("lv_delta_prep");
+  if (new_state != nullptr) return fail(-2, "lv_delta_prep_one: sizes or alignment that the tiled form does not take");
   if (dtype == LV_MIX_BF16) delta_prep_kernel<bf16_t><<<grid, block, 0, as_stream(stream)>>>(p);
   else if (dtype == LV_MIX_F32) delta_prep_kernel<float><<<grid, block, 0, as_stream(stream)>>>(p);
   else return fail(-1, "lv_delta_prep: dtype %d", dtype);
   return launched("lv_delta_prep");
+}
+
+int lv_delta_prep(const void* proj, int64_t ld, const void* conv_w, const void* conv_state, const void* A_log,
+                  const void* dt_bias, const int32_t* cu_q, const int32_t* ctx_lens, const int32_t* slots,
+                  const int32_t* tok_seq, void* qn, void* kn, void* v, void* beta, void* decay, int64_t T, int G,
+                  int H, int D, int Dv, int taps, int off_b, const void* a, int64_t ld_a, int decay_per_channel,
+                  float unit_eps, int dtype, void* stream) {
+  return delta_prep_entry(nullptr, proj, ld, conv_w, conv_state, A_log, dt_bias, cu_q, ctx_lens, slots, tok_seq, qn, kn, v, beta, decay, T, G,
+                          H, D, Dv, taps, off_b, a, ld_a, decay_per_channel, unit_eps, dtype, stream);
+}
+
+int lv_delta_prep_one(const void* proj, int64_t ld, const void* conv_w, void* conv_state, const void* A_log,
+                      const void* dt_bias, const int32_t* cu_q, const int32_t* ctx_lens, const int32_t* slots,
+                      const int32_t* tok_seq, void* qn, void* kn, void* v, void* beta, void* decay, int64_t T, int G,
+                      int H, int D, int Dv, int taps, int off_b, const void* a, int64_t ld_a, int decay_per_channel,
+                      float unit_eps, int dtype, void* stream) {
+  if (T != 0 && !conv_state) return fail(-1, "lv_delta_prep_one: null pointer");
+  return delta_prep_entry(conv_state, proj, ld, conv_w, conv_state, A_log, dt_bias, cu_q, ctx_lens, slots, tok_seq, qn, kn, v, beta, decay, T,
+                          G, H, D, Dv, taps, off_b, a, ld_a, decay_per_channel, unit_eps, dtype, stream);
+}
+
+int lv_delta_rule_one(const void* qn, const void* kn, const void* v, const void* beta, const void* decay, void* state, const int32_t* cu_q,
+                      const int32_t* ctx_lens, const int32_t* slots, const void* gate, int64_t ld_gate, const void* norm_w, void* out,
+                      int B, int G, int H, int D, int decay_per_channel, float eps, int gate_act, int dtype, void* stream) {
+  if (B == 0) return 0;
+  if (!qn || !kn || !v || !beta || !decay || !state || !cu_q || !ctx_lens || !slots || !gate || !norm_w || !out)
+    return fail(-1, "lv_delta_rule_one: null pointer");
+  if (B < 0 || B > 65535 || G <= 0 || H <= 0 || H % G != 0 || (D != 64 && D != 128) || ld_gate < static_cast<int64_t>(H) * D || ld_gate % 4 != 0 ||
+      (gate_act != LV_MIX_GATE_SILU && gate_act != LV_MIX_GATE_SIGMOID) || (dtype != LV_MIX_BF16 && dtype != LV_MIX_F32))
+    return fail(-1, "lv_delta_rule_one: bad arguments");
+  const uintptr_t piece = dtype == LV_MIX_BF16 ? 8 : 16;
+  for (const void* x : {qn, kn, v, static_cast<const void*>(state), norm_w})
+    if (reinterpret_cast<uintptr_t>(x) % 16 != 0) return fail(-1, "lv_delta_rule_one: alignment");
+  if (reinterpret_cast<uintptr_t>(gate) % piece != 0 || reinterpret_cast<uintptr_t>(out) % piece != 0 ||
+      (decay_per_channel && reinterpret_cast<uintptr_t>(decay) % 16 != 0))
+    return fail(-1, "lv_delta_rule_one: alignment");
+  DeltaRuleParams p{static_cast<const float*>(qn), static_cast<const float*>(kn), static_cast<const float*>(v),
+                    static_cast<const float*>(beta), static_cast<const float*>(decay), static_cast<float*>(state),
+                    cu_q, ctx_lens, slots, nullptr, G, H, D, D};
+  dim3 grid(H, B), block(256);
+  hipStream_t s = as_stream(stream);
+  const float* w = static_cast<const float*>(norm_w);
+  auto go = [&](auto type, auto size, auto channel) {
+    using A = decltype(type);
+    delta_one_kernel<A, decltype(size)::value, decltype(channel)::value><<<grid, block, 0, s>>>(p, static_cast<const A*>(gate), ld_gate, w,
+                                                                                             static_cast<A*>(out), eps, gate_act);
+  };
+  auto by_size = [&](auto type) {
+    if (D == 64 && decay_per_channel) go(type, std::integral_constant<int, 64>{}, std::true_type{});
+    else if (D == 64) go(type, std::integral_constant<int, 64>{}, std::false_type{});
+    else if (decay_per_channel) go(type, std::integral_constant<int, 128>{}, std::true_type{});
+    else go(type, std::integral_constant<int, 128>{}, std::false_type{});
+  };
+  if (dtype == LV_MIX_BF16) by_size(bf16_t{});
+  else by_size(0.0f);
+  return launched("lv_delta_rule_one");
 }
 
 int lv_conv_state_update(const void* proj, int64_t ld, void* conv_state, const int32_t* cu_q, const int32_t* ctx_lens,

@@ -271,14 +271,28 @@ def _chunk_scan(kind, q, k, v, a, decay, p0, p1, p2, state, step, H, G, D, Dv):
 
 
 # ------------------------------------------------------------------------------------- delta rule
+def _one_token(step) -> bool:
+    """Whether every sequence of the step has at most one new token (captured decode steps always)."""
+    return max(step.host_lens_q, default=0) <= 1
+
+
 def delta_prep(proj, conv_w, conv_state, A_log, dt_bias, step, G, H, D, Dv, taps, off_b, a, unit_eps,
-               decay_per_channel=False):
+               decay_per_channel=False, carry_on=False):
     """Short causal convolution + silu over the q | k | v channels of `proj` [T, ld] (taps from the
     portion's own rows, then from the carried state of the sequence's slot, zeros before position
     0), unit-norm q (times D^-1/2) and k per head, beta = sigmoid(b), decay = exp(-exp(A_log) *
     softplus(a + dt_bias)) with a [T, H] (a view of proj's columns or a tensor of its own), or
     [T, H*D] with decay_per_channel (dt_bias [H*D], A_log [H]).
-    Returns f32 (qn [T,G,D], kn [T,G,D], v [T,H,Dv], beta [T,H], decay [T,H] or [T,H,D])."""
+    Returns f32 (qn [T,G,D], kn [T,G,D], v [T,H,Dv], beta [T,H], decay [T,H] or [T,H,D]).
+    carry_on: conv_state_update as well; decode steps (one new token a sequence) do it in the same launch."""
+    if carry_on:
+        one = (proj.is_cuda and 1 < taps <= 4 and _one_token(step) and D == Dv and D in (64, 128, 256) and proj.stride(0) % 4 == 0
+               and proj.size(0) <= 65535
+               and all(x.data_ptr() % (4 * x.element_size()) == 0 for x in (proj, conv_state)))
+        if not one:
+            out = delta_prep(proj, conv_w, conv_state, A_log, dt_bias, step, G, H, D, Dv, taps, off_b, a, unit_eps, decay_per_channel)
+            conv_state_update(proj, conv_state, step, 2 * G * D + H * Dv, taps)
+            return out
     T = proj.size(0)
     dev = proj.device
     _f32(conv_w, A_log, dt_bias)
@@ -294,10 +308,11 @@ def delta_prep(proj, conv_w, conv_state, A_log, dt_bias, step, G, H, D, Dv, taps
     if proj.is_cuda:
         assert proj.stride(1) == 1 and a.stride(1) == 1
         lib = _mixlib.load()
-        _mixlib.check(lib.lv_delta_prep(_p(proj), proj.stride(0), _p(conv_w), _p(conv_state), _p(A_log), _p(dt_bias),
-                                        _p(step.cu_q), _p(step.ctx_lens), _p(step.slots), _p(step.tok_seq), _p(qn),
-                                        _p(kn), _p(v), _p(beta), _p(decay), T, G, H, D, Dv, taps, off_b, _p(a),
-                                        a.stride(0), int(decay_per_channel), unit_eps, _DT[proj.dtype], _stream(proj)),
+        prep = lib.lv_delta_prep_one if carry_on else lib.lv_delta_prep
+        _mixlib.check(prep(_p(proj), proj.stride(0), _p(conv_w), _p(conv_state), _p(A_log), _p(dt_bias),
+                           _p(step.cu_q), _p(step.ctx_lens), _p(step.slots), _p(step.tok_seq), _p(qn),
+                           _p(kn), _p(v), _p(beta), _p(decay), T, G, H, D, Dv, taps, off_b, _p(a),
+                           a.stride(0), int(decay_per_channel), unit_eps, _DT[proj.dtype], _stream(proj)),
                       "lv_delta_prep")
         return qn, kn, v, beta, decay
     q0 = 0
@@ -401,6 +416,28 @@ def head_norm_gate(o, gate, norm_w, eps, act_dtype, gate_act="silu"):
     y = o / torch.sqrt(o.pow(2).mean(-1, keepdim=True) + eps) * norm_w
     g = F.silu(gate.float()) if gate_act == "silu" else torch.sigmoid(gate.float())
     out.copy_((y * g.view(T, H, Dv)).reshape(T, H * Dv))
+    return out
+
+
+def delta_rule_norm_gate(qn, kn, v, beta, decay, state, step, gate, norm_w, eps, act_dtype, gate_act="silu"):
+    """head_norm_gate of gated_delta_rule: act [T, H*Dv]. Decode steps (one new token a sequence) with heads of 64 or 128 keys and values
+    do both in one launch."""
+    T, H, Dv = v.shape
+    if not (v.is_cuda and T > 0 and _one_token(step) and qn.size(2) == Dv and Dv in (64, 128) and len(step.host_lens_q) <= 65535
+            and gate.stride(0) % 4 == 0 and gate.data_ptr() % (4 * gate.element_size()) == 0
+            and all(x.data_ptr() % 16 == 0 for x in (qn, kn, v, decay, state, norm_w))):
+        return head_norm_gate(gated_delta_rule(qn, kn, v, beta, decay, state, step), gate, norm_w, eps, act_dtype, gate_act)
+    assert gate_act in ("silu", "sigmoid") and gate.stride(1) == 1 and gate.dtype == act_dtype
+    _f32(qn, kn, v, beta, decay, state, norm_w)
+    G, D = qn.size(1), Dv
+    per_channel = decay.dim() == 3
+    assert state.shape[1:] == (H, D, D) and decay.shape == ((T, H, D) if per_channel else (T, H))
+    out = torch.empty(T, H * Dv, dtype=act_dtype, device=v.device)
+    lib = _mixlib.load()
+    _mixlib.check(lib.lv_delta_rule_one(_p(qn), _p(kn), _p(v), _p(beta), _p(decay), _p(state), _p(step.cu_q), _p(step.ctx_lens),
+                                        _p(step.slots), _p(gate), gate.stride(0), _p(norm_w), _p(out), len(step.host_lens_q), G, H, D,
+                                        int(per_channel), eps, int(gate_act == "sigmoid"), _DT[act_dtype], _stream(v)),
+                  "lv_delta_rule_one")
     return out
 
 
