@@ -105,6 +105,7 @@ SIGNATURES = {
                                            c_int, c_int, c_int, _P, c_int, c_int, _P]),
     "lv_scaled_embedding": (c_int, [_P, _P, c_int, c_float, _P, _P, _P, c_int64, c_int, c_int, _P]),
     "lv_residual_split": (c_int, [_P, _P, _P, c_int64, c_int, _P]),
+    "lv_router_gemm": (c_int, [_P, c_int64, _P, _P, c_int64, c_int, c_int, _P]),
     "lv_rows_gemm": (c_int, [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P]),
 }
 

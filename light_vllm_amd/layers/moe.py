@@ -93,7 +93,7 @@ class SparseMoE(nn.Module):
 
     def route(self, h: torch.Tensor):
         # logits_kernel: small steps form their f32 logits straight from the activations (no widened copy)
-        logits = mix_ops.router_logits(h, self.router_weight) if self.logits_kernel else F.linear(h.float(), self.router_weight)
+        logits = mix_ops.router_logits(h, self.router_weight) if self.logits_kernel else mix_ops.router_product(h, self.router_weight)
         return mix_ops.moe_route(logits, self.correction, self.top, self.groups, self.keep, score=self.score,
                                  group_rank=self.group_rank)
 

@@ -942,7 +942,7 @@ ROUTER_KERNEL_MAX_TOKENS = 256     # steps of at most this many tokens form thei
 def router_logits(h, router_w):
     """f32 [T, E] = h router_w^T computed in f32 (h act [T, W], router_w f32 [E, W]). Steps of few tokens (decoded tokens,
     small portions, everything replayed from a graph) read the activations as they are, one workgroup per (token, four
-    experts): one small launch instead of a widening copy and a GEMM. Larger steps take the f32 vendor GEMM."""
+    experts): one small launch instead of a widening copy and a GEMM. Larger steps take router_product."""
     T, W = h.shape
     E = router_w.size(0)
     _f32(router_w)
@@ -953,7 +953,22 @@ def router_logits(h, router_w):
         _mixlib.check(lib.lv_router_logits(_p(h), h.stride(0), _p(router_w), _p(logits), T, W, E, _DT[h.dtype], _stream(h)),
                       "lv_router_logits")
         return logits
-    return F.linear(h.float(), router_w)
+    return router_product(h, router_w)
+
+
+def router_product(h, router_w):
+    """f32 [T, E] = h router_w^T in f32 products. bf16 activations are read as they are (lv_router_gemm) where their rows are whole 16-byte
+    pieces and a multiple of 32 entries; others are widened for the vendor's product."""
+    T, W = h.shape
+    if not (h.is_cuda and T > 0 and h.dtype == torch.bfloat16 and router_w.dtype == torch.float32 and router_w.is_contiguous()
+            and not _transformed(h, router_w) and W > 0 and W % 32 == 0 and h.stride(1) == 1 and h.stride(0) % 8 == 0
+            and h.data_ptr() % 16 == 0 and router_w.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled() and (h.requires_grad or router_w.requires_grad))):
+        return F.linear(h.float(), router_w)
+    logits = torch.empty(T, router_w.size(0), dtype=torch.float32, device=h.device)
+    lib = _mixlib.load()
+    _mixlib.check(lib.lv_router_gemm(_p(h), h.stride(0), _p(router_w), _p(logits), T, router_w.size(0), W, _stream(h)), "lv_router_gemm")
+    return logits
 
 
 def relu2_scale(up, dense, E, Fe):
