@@ -64,23 +64,9 @@ __device__ __forceinline__ float chunk_lane(float x, int i) {
 }
 __device__ __forceinline__ int acc_row(int i, int half) { return 8 * (i >> 2) + 4 * half + (i & 3); }
 
-// x / (1 + exp(-x)) in about half the instructions of siluf_, to the same two units in the last place: the exponent as a sum of
-// two floats in front of the hardware exp2, the hardware reciprocal with one Newton step behind it. Below -87, where the
-// function is within 1.5e-36 of zero and exp(-x) would overflow, zero (a NaN for -infinity, as siluf_).
-__device__ __forceinline__ float chunk_silu(float x) {
-  constexpr float kLog2e = 1.44269504f, kLog2eRest = 1.92596303e-8f, kLn2 = 0.69314718f;
-  const float c = __builtin_amdgcn_fmed3f(x, -87.0f, 87.0f);
-  const float t = -kLog2e * c, rest = fmaf(-kLog2e, c, -t) - kLog2eRest * c;
-  float e = __builtin_amdgcn_exp2f(t);
-  e = fmaf(e, kLn2 * rest, e);
-  const float d = 1.0f + e;
-  float q = __builtin_amdgcn_rcpf(d);
-  q = fmaf(q, fmaf(-d, q, 1.0f), q);
-  return x * (x < -87.0f ? 0.0f : q);
-}
 template <bool SILU>
 __device__ __forceinline__ float4 chunk_act(float4 x) {
-  if constexpr (SILU) return float4{chunk_silu(x.x), chunk_silu(x.y), chunk_silu(x.z), chunk_silu(x.w)};
+  if constexpr (SILU) return float4{quick_silu_(x.x), quick_silu_(x.y), quick_silu_(x.z), quick_silu_(x.w)};
   return x;
 }
 
@@ -440,7 +426,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      if constexpr (SILU) U_next[i >> 2][i & 3] = chunk_silu(__builtin_bit_cast(float, vreg[i] << 16));
+      if constexpr (SILU) U_next[i >> 2][i & 3] = quick_silu_(__builtin_bit_cast(float, vreg[i] << 16));
       else U_next[i >> 2][i & 3] = vreg[i];
     }
     if (w % WPW == 0) ge_all[buf][hw][lane] = gereg;
@@ -727,6 +713,10 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_step_kernel(ChunkParams p) {
     const unsigned char *k_lds = k_all[buf], *q_lds = q_all[buf], *p_lds = p_all[buf][MATS > 0 ? hw : 0];
     const float* ge_lds = ge_all[buf][hw];
     const f32x4 U[2] = {U_next[0], U_next[1]};
+    if constexpr (!FULL) {                             // (few products to stand among: 85 us there, 68 here, in the launch of 323)
+      stage(buf ^ 1);
+      if (c0 + 2 * kCh < s1) fetch(c0 + 2 * kCh);
+    }
     f32x4 o[2], u2[2], next[DT];
 #pragma unroll
     for (int x = 0; x < 2; ++x) u2[x] = scale4(U[x], rows4(ge_lds + kCh, x));
@@ -738,7 +728,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_step_kernel(ChunkParams p) {
       for (int x = 0; x < 2; ++x) qs[0][x] = qs[1][x] = pu[x] = zero;
       chunk_bf16x8 uc[3];
       cut8(u2[0], u2[1], uc);
-      stage(buf ^ 1);
+      if constexpr (FULL) stage(buf ^ 1);
 #pragma unroll
       for (int jj = 0; jj < DT / 2; ++jj) {
         if constexpr (FULL) {
@@ -773,10 +763,10 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_step_kernel(ChunkParams p) {
         }
         odd = !all_finite(o);                          // the state itself may hold an infinity
       }
-    } else {
+    } else if constexpr (FULL) {
       stage(buf ^ 1);
     }
-    if (c0 + 2 * kCh < s1) fetch(c0 + 2 * kCh);
+    if (FULL && c0 + 2 * kCh < s1) fetch(c0 + 2 * kCh);
     if (__builtin_expect(odd, 0)) {
       // the chunk in f32, the lower triangle token by token: a value that is not finite would reach the tokens before it through zeros
       auto row4 = [&](const unsigned char* img, int tok, int d) {

@@ -68,6 +68,20 @@ __device__ __forceinline__ float row16_sum(float x) {
 
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + expf(-x)); }
 __device__ __forceinline__ float siluf_(float x) { return x / (1.0f + expf(-x)); }
+// x / (1 + exp(-x)) in about half the instructions of siluf_, to the same two units in the last place: the exponent as a sum of
+// two floats in front of the hardware exp2, the hardware reciprocal with one Newton step behind it. Below -87, where the
+// function is within 1.5e-36 of zero and exp(-x) would overflow, zero (a NaN for -infinity, as siluf_).
+__device__ __forceinline__ float quick_silu_(float x) {
+  constexpr float kLog2e = 1.44269504f, kLog2eRest = 1.92596303e-8f, kLn2 = 0.69314718f;
+  const float c = __builtin_amdgcn_fmed3f(x, -87.0f, 87.0f);
+  const float t = -kLog2e * c, rest = fmaf(-kLog2e, c, -t) - kLog2eRest * c;
+  float e = __builtin_amdgcn_exp2f(t);
+  e = fmaf(e, kLn2 * rest, e);
+  const float d = 1.0f + e;
+  float q = __builtin_amdgcn_rcpf(d);
+  q = fmaf(q, fmaf(-d, q, 1.0f), q);
+  return x * (x < -87.0f ? 0.0f : q);
+}
 __device__ __forceinline__ float softplusf_(float x) { return x > 20.0f ? x : log1pf(expf(x)); }
 
 __device__ __forceinline__ float gelu_tanh_(float z) {

@@ -79,7 +79,7 @@ __device__ __forceinline__ void conv_emit(const ConvParams& p, int64_t t, int b,
   if constexpr (!ATT) {
     if (p.silu) {
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) y[e] = siluf_(y[e]);
+      for (int e = 0; e < VEC; ++e) y[e] = quick_silu_(y[e]);
     }
     stv<VEC>(static_cast<T*>(p.out) + t * p.C + c, y);
   } else {
@@ -130,9 +130,8 @@ __global__ __launch_bounds__(128) void causal_conv_kernel(ConvParams p) {
     }
   }
   const int r1 = min(n, r0 + kConvTile);
-  for (int r = r0; r < r1; ++r) {
-    float u[VEC], y[VEC];
-    ldv<VEC>(in + static_cast<int64_t>(r) * p.ld, u);
+  auto row = [&](int r, const float (&u)[VEC]) __attribute__((always_inline)) {
+    float y[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
       y[e] = bias[e];
@@ -144,6 +143,22 @@ __global__ __launch_bounds__(128) void causal_conv_kernel(ConvParams p) {
       if (TAPS > 1) hist[HIST - 1][e] = u[e];
     }
     conv_emit<T, VEC, ATT>(p, q0 + r, b, ctx + r, c, y);
+  };
+  // Rows requested together: behind a store the compiler asks for no row before its turn. 14000 tokens, 4096 channels, four taps: 107 us row
+  // by row, 90 this way, 65 with the shorter silu; 47 at the rate of a large copy.
+  constexpr int AHEAD = 8;
+  int r = r0;
+  for (; r + AHEAD <= r1; r += AHEAD) {
+    float u[AHEAD][VEC];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) ldv<VEC>(in + static_cast<int64_t>(r + i) * p.ld, u[i]);
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) row(r + i, u[i]);
+  }
+  for (; r < r1; ++r) {
+    float u[VEC];
+    ldv<VEC>(in + static_cast<int64_t>(r) * p.ld, u);
+    row(r, u);
   }
   if (r0 == 0 && TAPS > 1) {
 #pragma unroll
@@ -661,7 +676,7 @@ __global__ __launch_bounds__(256) void part_gate_norm_kernel(const float* __rest
       ldv<4>(z + t * ldz + c0 + i, g);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        y[x][e] *= siluf_(g[e]);
+        y[x][e] *= quick_silu_(g[e]);
         ss += y[x][e] * y[x][e];
       }
     }
