@@ -74,9 +74,11 @@ __device__ __forceinline__ float4 chunk_act(float4 x) {
 // cu_q[b] / 32 + b, which leaves at most one place a sequence empty. (A grid over sequences and the longest one's chunks
 // spent 1.57 ms on empty workgroups where two portions of 1000 tokens ran beside 250 decoded ones.) The products q k^T and k k^T do
 // not depend on the head: the waves take a share of the key dimension each, and every wave then takes heads of the group.
-template <typename T, int KIND>
-__global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
+template <typename T, int KIND, int D>
+__global__ __launch_bounds__(256, KIND == kChunkDelta ? 4 : 1) void chunk_prep_kernel(ChunkParams p) {
   constexpr bool DELTA = KIND == kChunkDelta, SILU = KIND == kChunkConst;
+  using Row4 = std::conditional_t<sizeof(T) == 2, uint2, float4>;      // four entries as they lie in memory
+  auto wide = [](Row4 x) __attribute__((always_inline)) { return ld4(reinterpret_cast<const T*>(&x)); };
   constexpr int RS = kCh + 1;
   __shared__ float prod[4][kCh * RS];                  // partial products of the waves
   __shared__ __attribute__((aligned(16))) float amat[DELTA ? 4 : 1][kCh * (kCh + kPad)];
@@ -95,11 +97,25 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
   const int cn = min(kCh, n - c0);
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, half = lane >> 5;
   const int64_t t0 = static_cast<int64_t>(q0) + c0;
+  const int rep = p.H / p.G;
+  // what the first head's decays are made of, requested with the rows
+  float first_a = 0.0f, first_g = 0.0f;
+  T first_step{};
+  if (KIND != kChunkConst && w < rep && r < cn) {
+    const int64_t at = (t0 + r) * p.H + g * rep + w;
+    if constexpr (KIND == kChunkStep) first_step = static_cast<const T*>(p.a)[(t0 + r) * p.lda + g * rep + w];
+    if constexpr (DELTA) {
+      first_a = static_cast<const float*>(p.a)[at];
+      first_g = p.decay[at];
+    }
+  }
   {
     const bool kk = DELTA && w < 2;                    // delta rule: waves 0, 1 k k^T, waves 2, 3 q k^T; otherwise all q k^T
-    const int shares = DELTA ? 2 : 4, share = DELTA ? (w & 1) : w;
-    const T* left = static_cast<const T*>(kk ? p.k : p.q) + (t0 + r) * (kk ? p.ldk : p.ldq) + static_cast<int64_t>(g) * p.D;
-    const T* right = static_cast<const T*>(p.k) + (t0 + r) * p.ldk + static_cast<int64_t>(g) * p.D;
+    constexpr int shares = DELTA ? 2 : 4;
+    const int r_in = min(r, cn - 1);                   // tokens past the end: the last one's rows, not used
+    const int share = DELTA ? (w & 1) : w;
+    const T* left = static_cast<const T*>(kk ? p.k : p.q) + (t0 + r_in) * (kk ? p.ldk : p.ldq) + static_cast<int64_t>(g) * D;
+    const T* right = static_cast<const T*>(p.k) + (t0 + r_in) * p.ldk + static_cast<int64_t>(g) * D;
     if (DELTA && !kk) {
       // q k^T in 64 bits: read-outs are sums of few of these products, each a small difference of large terms. Summed in f32 they
       // were most of an output's error (1.33e-7 at heads of 128 x 128; 0.86e-7 with these, 0.95e-7 in the token loop).
@@ -107,20 +123,24 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
       f64x4 acc[2][2];
 #pragma unroll
       for (int x = 0; x < 4; ++x) acc[x >> 1][x & 1] = f64x4{0.0, 0.0, 0.0, 0.0};
-      const T* q16 = static_cast<const T*>(p.q) + (t0 + r16) * p.ldq + static_cast<int64_t>(g) * p.D + 4 * quad;
-      const T* k16 = static_cast<const T*>(p.k) + (t0 + r16) * p.ldk + static_cast<int64_t>(g) * p.D + 4 * quad;
-      for (int d = share * 16; d < p.D; d += 32) {
-        float4 x[2], y[2];
+      const T* q16 = static_cast<const T*>(p.q) + t0 * p.ldq + static_cast<int64_t>(g) * D + 4 * quad;
+      const T* k16 = static_cast<const T*>(p.k) + t0 * p.ldk + static_cast<int64_t>(g) * D + 4 * quad;
+      Row4 x[D / 32][2], y[D / 32][2];                 // all of them on their way at once
+#pragma unroll
+      for (int i = 0; i < D / 32; ++i)
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-          const bool in = 16 * e + r16 < cn;
-          x[e] = in ? ld4(q16 + 16 * e * p.ldq + d) : float4{0, 0, 0, 0};
-          y[e] = in ? ld4(k16 + 16 * e * p.ldk + d) : float4{0, 0, 0, 0};
+          const int64_t row = min(16 * e + r16, cn - 1);
+          x[i][e] = *reinterpret_cast<const Row4*>(q16 + row * p.ldq + share * 16 + 32 * i);
+          y[i][e] = *reinterpret_cast<const Row4*>(k16 + row * p.ldk + share * 16 + 32 * i);
         }
+#pragma unroll
+      for (int i = 0; i < D / 32; ++i) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           f64x4& to = acc[e >> 1][e & 1];
-          const float4 a = x[e >> 1], b = y[e & 1];
+          const float4 none{0.0f, 0.0f, 0.0f, 0.0f};
+          const float4 a = 16 * (e >> 1) + r16 < cn ? wide(x[i][e >> 1]) : none, b = 16 * (e & 1) + r16 < cn ? wide(y[i][e & 1]) : none;
           to = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, to, 0, 0, 0);
           to = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.y, to, 0, 0, 0);
           to = __builtin_amdgcn_mfma_f64_16x16x4f64(a.z, b.z, to, 0, 0, 0);
@@ -136,12 +156,18 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
       f32x16 acc, acc2;                                  // two sums of half the length: half the roundings each
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[i] = acc2[i] = 0.0f;
-      for (int d = share * 8; d < p.D; d += shares * 8) {
-        float4 x{0, 0, 0, 0}, y{0, 0, 0, 0};
-        if (in) {
-          x = chunk_act<SILU>(ld4(left + d + 4 * half));
-          y = chunk_act<SILU>(ld4(right + d + 4 * half));
-        }
+      constexpr int N = D / (8 * shares);
+      Row4 xr[N], yr[N];                               // all of them on their way at once
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        xr[i] = *reinterpret_cast<const Row4*>(left + (share + i * shares) * 8 + 4 * half);
+        yr[i] = *reinterpret_cast<const Row4*>(right + (share + i * shares) * 8 + 4 * half);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const float4 none{0.0f, 0.0f, 0.0f, 0.0f};
+        const float4 x = in ? chunk_act<SILU>(wide(xr[i])) : none, y = in ? chunk_act<SILU>(wide(yr[i])) : none;
         acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, y.x, acc, 0, 0, 0);
         acc2 = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, y.y, acc2, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, y.z, acc, 0, 0, 0);
@@ -152,7 +178,6 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
     }
   }
   __syncthreads();
-  const int rep = p.H / p.G;
   const uint32_t p_off = static_cast<uint32_t>(4 * half * p.H * kCh) + r;
   int r_here = r, half_here = half, cn_here = cn;
 #pragma unroll 1
@@ -165,11 +190,12 @@ __global__ __launch_bounds__(256) void chunk_prep_kernel(ChunkParams p) {
     if (r < cn) {
       const int64_t at = (t0 + r) * p.H + h;
       if constexpr (KIND == kChunkStep) {
-        wr = softplusf_(ldf(static_cast<const T*>(p.a) + (t0 + r) * p.lda + h) + p.p0[h]);
+        const T step = hr == w ? first_step : static_cast<const T*>(p.a)[(t0 + r) * p.lda + h];
+        wr = softplusf_(ldf(&step) + p.p0[h]);
         dec = expf(-expf(p.p1[h]) * wr);
       } else if constexpr (DELTA) {
-        wr = static_cast<const float*>(p.a)[at];       // beta
-        dec = p.decay[at];
+        wr = hr == w ? first_a : static_cast<const float*>(p.a)[at];       // beta
+        dec = hr == w ? first_g : p.decay[at];
       }
     } else {
       wr = 0.0f;
@@ -880,9 +906,14 @@ static void chunk_waves(const ChunkParams& p, int B, hipStream_t s) {
 
 template <typename T, int KIND>
 static void chunk_dispatch(const ChunkParams& p, int64_t tokens, int B, hipStream_t s) {
-  chunk_prep_kernel<T, KIND><<<dim3(static_cast<unsigned>(tokens / kCh + B), p.G), dim3(256), 0, s>>>(p);
-  if (p.D == 64) chunk_waves<T, KIND, 4>(p, B, s);
-  else chunk_waves<T, KIND, 8>(p, B, s);
+  const dim3 grid(static_cast<unsigned>(tokens / kCh + B), p.G), block(256);
+  if (p.D == 64) {
+    chunk_prep_kernel<T, KIND, 64><<<grid, block, 0, s>>>(p);
+    chunk_waves<T, KIND, 4>(p, B, s);
+  } else {
+    chunk_prep_kernel<T, KIND, 128><<<grid, block, 0, s>>>(p);
+    chunk_waves<T, KIND, 8>(p, B, s);
+  }
 }
 
 static int chunk_segments(int kind, int max_new, int seg_len) {
