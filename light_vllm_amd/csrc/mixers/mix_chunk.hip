@@ -32,6 +32,8 @@
 // products for one, and every row to cut.
 #include "mix_common.h"
 
+#include <algorithm>
+
 namespace lvmix {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -897,11 +899,24 @@ static void chunk_launch(const ChunkParams& p, int B, hipStream_t s) {
   }
 }
 
+// Eight waves a workgroup: 128 columns of a head, or two heads of 64 that share q and k. Launches of few workgroups, which leave half of the
+// chip empty, cut them in two (the f32 scans: a compute unit then holds one wave a SIMD, and a chunk takes two thirds of the time, though q
+// and k are staged twice); beyond that the halves only take each other's place. us, 8 / 4 waves, 16 heads of 128 x 128, prompts of 1000: delta
+// rule 1 prompt 268 / 186, 8 284 / 207, 10 294 / 384; constant decays 228 / 168, 253 / 194, 259 / 294; heads of 64 x 64, delta rule, 12
+// prompts 204 / 150. Step sizes are bound by a chunk's chain either way (one prompt of 4096, 32 heads of 128 x 64, 469 / 500).
 template <typename T, int KIND, int DT>
-static void chunk_waves(const ChunkParams& p, int B, hipStream_t s) {
-  if (p.Dv % 128 == 0) chunk_launch<T, KIND, DT, 8, 1>(p, B, s);
-  else if (p.H / p.G % 2 == 0) chunk_launch<T, KIND, DT, 8, 2>(p, B, s);     // Dv == 64: two heads of a group
-  else chunk_launch<T, KIND, DT, 4, 1>(p, B, s);
+static void chunk_waves(const ChunkParams& p, int64_t tokens, int B, hipStream_t s) {
+  const int64_t pieces = p.segs > 1 ? std::min<int64_t>(static_cast<int64_t>(B) * p.segs, tokens / p.seg_len + B) : B;
+  const bool few = KIND != kChunkStep && pieces * p.H * p.Dv / 128 <= 128;
+  if (p.Dv % 128 == 0 && !few) {
+    chunk_launch<T, KIND, DT, 8, 1>(p, B, s);
+    return;
+  }
+  if (p.Dv % 128 != 0 && p.H / p.G % 2 == 0 && !few) {
+    chunk_launch<T, KIND, DT, 8, 2>(p, B, s);
+    return;
+  }
+  chunk_launch<T, KIND, DT, 4, 1>(p, B, s);
 }
 
 template <typename T, int KIND>
@@ -909,10 +924,10 @@ static void chunk_dispatch(const ChunkParams& p, int64_t tokens, int B, hipStrea
   const dim3 grid(static_cast<unsigned>(tokens / kCh + B), p.G), block(256);
   if (p.D == 64) {
     chunk_prep_kernel<T, KIND, 64><<<grid, block, 0, s>>>(p);
-    chunk_waves<T, KIND, 4>(p, B, s);
+    chunk_waves<T, KIND, 4>(p, tokens, B, s);
   } else {
     chunk_prep_kernel<T, KIND, 128><<<grid, block, 0, s>>>(p);
-    chunk_waves<T, KIND, 8>(p, B, s);
+    chunk_waves<T, KIND, 8>(p, tokens, B, s);
   }
 }
 

@@ -3,7 +3,7 @@ import pytest
 import torch
 
 from light_vllm_amd import mix_ops
-from tests.test_chunk_scan_gpu import make_step
+from tests.test_chunk_scan_gpu import REL, case, make_step, recurrence
 
 pytestmark = pytest.mark.gpu
 
@@ -40,3 +40,18 @@ def test_like_the_token_loop(monkeypatch, D, Dv, H, G, where):
         # f32 sums of D + T terms on both sides
         assert bool(((x - y)[ok].abs() <= 2.0 ** -24 * (D + 64) * 8 * (1 + x[ok].abs())).all()) or where == "huge"
     assert where in ("none", "huge") or not bool(torch.isfinite(got[1][0]).all())
+
+
+@pytest.mark.parametrize("kind", ["delta", "const"])
+@pytest.mark.parametrize("H,G,D,Dv,B", [(4, 4, 128, 128, 32), (4, 4, 128, 128, 33), (4, 2, 64, 64, 64), (4, 2, 64, 64, 65), (2, 2, 128, 256, 3), (2, 1, 128, 64, 2)])
+def test_both_workgroup_sizes(monkeypatch, kind, H, G, D, Dv, B):
+    """Launches on both sides of the rule that cuts workgroups in two, against float64 as the other shapes are."""
+    monkeypatch.setattr(mix_ops, "SCAN_KERNEL", "chunk")
+    G = H if kind == "const" else G
+    new, ctx = [33 + i % 40 for i in range(B)], [3 * (i % 2) for i in range(B)]
+    step = make_step(new, ctx)
+    call, args, skip = case(kind, new, H, G, D, Dv, 11)
+    state = torch.randn(B, H, D, Dv, device="cuda", generator=torch.Generator(device="cuda").manual_seed(12))
+    want_o, want_s = recurrence(*args, state, step)
+    o = call(state, step).view(sum(new), H, Dv)
+    assert float((o.double() - want_o - skip).norm() / want_o.norm()) <= REL and float((state.double() - want_s).norm() / want_s.norm()) <= REL
