@@ -332,6 +332,7 @@ int lv_prefill_attn(const void* q, const void* k, const void* v, void* o, int64_
        workspace_bytes < lv_prefill_workspace_bytes(total_q, num_heads, head_dim, nsplit)))
     nsplit = 1;
   p.nsplit = nsplit;
+  p.by_tile = max_seqlen_k <= 2 * static_cast<int64_t>(max_seqlen_q);
   p.ws_o = nullptr;
   p.ws_ml = nullptr;
   p.total_q = total_q;

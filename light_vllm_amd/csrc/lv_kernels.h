@@ -55,6 +55,7 @@ struct PrefillParams {
   int order_lanes;             // 0: tile_order holds codes b * qtiles + t. > 0: it holds 8-int entries
                                // {q row, valid rows, causal limit of the first row, packed K row or sequence,
                                // keys, 0, 0, 0}, [depth][lanes][order_cols]: the lists persistent workgroups walk
+  int by_tile;                 // natural mapping of the free-running kernels: every sequence's last tile first
 };
 // Lanes of an item table: workgroups per (query head, table column) that one launch keeps resident.
 int prefill_order_lanes(int num_heads, int num_kv_heads);
