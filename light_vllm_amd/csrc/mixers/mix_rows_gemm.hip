@@ -144,9 +144,9 @@ static void rows_gemm_launch(const RowsGemmParams& p, hipStream_t s) {
 // ---- logits [T, E] f32 = x [T, K] bf16 times w [E, K]^T f32 (a router's): as f32 products, without widening x.
 //
 // w is cut into three bf16 numbers an entry whose sum it is (8 bits each, nothing rounded), so that three products on the bf16 instructions,
-// exact and summed in f32, stand for an f32 one. Bound by reading x. A workgroup takes 64 rows and 32 outputs, its waves share k; x
+// exact and summed in f32, stand for an f32 one. Bound by reading x. A workgroup takes up to 64 rows and 32 outputs, its waves share k; x
 // passes through LDS as above, w is cut on its way to the registers. An infinity has no such pieces: sums that are not finite are
-// formed again in f32, one after the other. 16384 x 2048 x 32, us: widening and the vendor's f32 product 68, this 26.
+// formed again in f32, one after the other. 16384 x 2048 x 32, us: widening and the vendor's f32 product 53, this 17.
 struct RouterGemmParams {
   const uint16_t* x;
   const float* w;
@@ -155,8 +155,9 @@ struct RouterGemmParams {
   int T, E, K;
 };
 
+template <int MT, int NT>
 __global__ __launch_bounds__(kRowsWaves * kWave) void router_gemm_kernel(RouterGemmParams p) {
-  constexpr int NW = kRowsWaves, MT = 4, NT = 2, RS = NT * 16 + 4;
+  constexpr int NW = kRowsWaves, RS = NT * 16 + 4;
   constexpr int STAGE = MT * 2048, PART = MT * 16 * RS * 4, PER = STAGE > PART ? STAGE : PART;
   __shared__ __attribute__((aligned(16))) unsigned char lds[NW * PER];
   const int m0 = blockIdx.x * MT * 16, n0 = blockIdx.y * NT * 16;
@@ -306,6 +307,18 @@ extern "C" int lv_router_gemm(const void* x, int64_t ldx, const void* w, void* y
   if (ldx < 0 || ldx % 8 != 0 || reinterpret_cast<uintptr_t>(x) % 16 != 0 || reinterpret_cast<uintptr_t>(w) % 16 != 0)
     return fail(-1, "lv_router_gemm: strides or alignment");
   RouterGemmParams p{static_cast<const uint16_t*>(x), static_cast<const float*>(w), static_cast<float*>(y), ldx, static_cast<int>(T), E, K};
-  router_gemm_kernel<<<dim3(static_cast<unsigned>((T + 63) / 64), (E + 31) / 32), dim3(kRowsWaves * kWave), 0, as_stream(stream)>>>(p);
+  // Cutting w takes most of a workgroup's time, and one of few workgroups is the launch's: smaller tiles as long as they fit the chip at
+  // once. us, widening and the vendor's product / 16 x 16 / 32 x 16 / 64 x 32 rows by outputs, K 4096, 32 outputs: 300 rows 17.0 / 10.6 / 11.6 /
+  // 21.7, 3000 30.2 / 20.3 / 13.1 / 22.3, 6000 46.6 / 28.5 / 22.9 / 23.2, 16384 111 / 67 / 45 / 27.
+  hipStream_t s = as_stream(stream);
+  auto go = [&](auto mt, auto nt) {
+    constexpr int M = decltype(mt)::value, N = decltype(nt)::value;
+    router_gemm_kernel<M, N><<<dim3(static_cast<unsigned>((T + 16 * M - 1) / (16 * M)), (E + 16 * N - 1) / (16 * N)), dim3(kRowsWaves * kWave), 0, s>>>(p);
+  };
+  using std::integral_constant;
+  const int64_t halves = (E + 15) / 16;
+  if ((T + 15) / 16 * halves <= 256) go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+  else if ((T + 31) / 32 * halves <= 256) go(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+  else go(integral_constant<int, 4>{}, integral_constant<int, 2>{});
   return launched("lv_router_gemm");
 }
