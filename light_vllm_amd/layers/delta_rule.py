@@ -85,12 +85,19 @@ class GatedDeltaRule(nn.Module):
         a = proj[:, self.off_a:self.off_a + self.decay_in]
         if self.decay_up is not None:
             a = self.decay_up(a)
+        few = proj.size(0) <= len(step.host_lens_q)        # perhaps one new token a sequence; prompts' steps look no further
         qn, kn, v, beta, decay = mix_ops.delta_prep(proj, self.conv_weight, self.conv_state, self.A_log, self.dt_bias,
                                                     step, self.G, self.H, self.D, self.Dv, self.taps, self.off_b, a,
-                                                    self.unit_eps, self.decay_per_channel, carry_on=True)
+                                                    self.unit_eps, self.decay_per_channel, few)
+        if not few:
+            mix_ops.conv_state_update(proj, self.conv_state, step, self.channels, self.taps)
         gate = proj[:, self.off_gate:self.off_gate + self.gate_in]
         if self.gate_up is not None:
             gate = self.gate_up(gate)
-        y = mix_ops.delta_rule_norm_gate(qn, kn, v, beta, decay, self.state, step, gate, self.out_norm_weight, self.norm_eps, h.dtype,
-                                         self.gate_act)
+        if few:
+            y = mix_ops.delta_rule_norm_gate(qn, kn, v, beta, decay, self.state, step, gate, self.out_norm_weight, self.norm_eps, h.dtype,
+                                             self.gate_act)
+        else:
+            o = mix_ops.gated_delta_rule(qn, kn, v, beta, decay, self.state, step)
+            y = mix_ops.head_norm_gate(o, gate, self.out_norm_weight, self.norm_eps, h.dtype, self.gate_act)
         return self.o_proj(y)

@@ -19,7 +19,9 @@ from .tp import divide, tp_rank, tp_size
 
 
 def _linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
-    return mix_ops.linear(x, weight) if bias is None else F.linear(x, weight, bias)
+    if bias is not None or x.size(0) > mix_ops.ROWS_GEMM_MAX:       # prompts' steps look no further
+        return F.linear(x, weight, bias)
+    return mix_ops.linear(x, weight)
 
 
 class LinearBase(nn.Module):
@@ -135,7 +137,7 @@ class RowParallelLinear(LinearBase):
         after the sum."""
         if self.tp_size == 1 and self.bias is not None:
             return F.linear(x, self.weight, self.bias)      # one rank: the bias rides in the GEMM, one rounding
-        y = mix_ops.linear(x, self.weight)
+        y = _linear(x, self.weight, None)
         if not reduce:
             assert self.bias is None
             return y

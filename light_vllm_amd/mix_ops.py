@@ -285,14 +285,8 @@ def delta_prep(proj, conv_w, conv_state, A_log, dt_bias, step, G, H, D, Dv, taps
     [T, H*D] with decay_per_channel (dt_bias [H*D], A_log [H]).
     Returns f32 (qn [T,G,D], kn [T,G,D], v [T,H,Dv], beta [T,H], decay [T,H] or [T,H,D]).
     carry_on: conv_state_update as well; decode steps (one new token a sequence) do it in the same launch."""
-    if carry_on:
-        one = (proj.is_cuda and 1 < taps <= 4 and _one_token(step) and D == Dv and D in (64, 128, 256) and proj.stride(0) % 4 == 0
-               and proj.size(0) <= 65535
-               and all(x.data_ptr() % (4 * x.element_size()) == 0 for x in (proj, conv_state)))
-        if not one:
-            out = delta_prep(proj, conv_w, conv_state, A_log, dt_bias, step, G, H, D, Dv, taps, off_b, a, unit_eps, decay_per_channel)
-            conv_state_update(proj, conv_state, step, 2 * G * D + H * Dv, taps)
-            return out
+    one = (carry_on and proj.is_cuda and _one_token(step) and 1 < taps <= 4 and D == Dv and D in (64, 128, 256) and proj.stride(0) % 4 == 0
+           and proj.size(0) <= 65535 and all(x.data_ptr() % (4 * x.element_size()) == 0 for x in (proj, conv_state)))
     T = proj.size(0)
     dev = proj.device
     _f32(conv_w, A_log, dt_bias)
@@ -308,12 +302,14 @@ def delta_prep(proj, conv_w, conv_state, A_log, dt_bias, step, G, H, D, Dv, taps
     if proj.is_cuda:
         assert proj.stride(1) == 1 and a.stride(1) == 1
         lib = _mixlib.load()
-        prep = lib.lv_delta_prep_one if carry_on else lib.lv_delta_prep
+        prep = lib.lv_delta_prep_one if one else lib.lv_delta_prep
         _mixlib.check(prep(_p(proj), proj.stride(0), _p(conv_w), _p(conv_state), _p(A_log), _p(dt_bias),
                            _p(step.cu_q), _p(step.ctx_lens), _p(step.slots), _p(step.tok_seq), _p(qn),
                            _p(kn), _p(v), _p(beta), _p(decay), T, G, H, D, Dv, taps, off_b, _p(a),
                            a.stride(0), int(decay_per_channel), unit_eps, _DT[proj.dtype], _stream(proj)),
                       "lv_delta_prep")
+        if carry_on and not one:
+            conv_state_update(proj, conv_state, step, C, taps)
         return qn, kn, v, beta, decay
     q0 = 0
     for b, (n, ctx) in enumerate(zip(step.host_lens_q, step.host_ctx_lens)):
@@ -338,6 +334,8 @@ def delta_prep(proj, conv_w, conv_state, A_log, dt_bias, step, G, H, D, Dv, taps
         else:
             decay[q0:q0 + n] = torch.exp(-rate * sp)
         q0 += n
+    if carry_on:
+        conv_state_update(proj, conv_state, step, C, taps)
     return qn, kn, v, beta, decay
 
 
