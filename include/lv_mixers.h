@@ -67,7 +67,6 @@
  *   lv_gated_linear_recurrence   Griffin's RG-LRU: block-diagonal gates, S <- a S + sqrt(1 - a^2) i u per channel, gelu branch
  *   lv_scaled_embedding      token rows times a constant as the f32 residual
  *   lv_rows_gemm             projections of up to 64 rows
- *   lv_router_gemm           router logits of prompt steps, f32 products of bf16 activations
  *   lv_delta_prep_one, lv_delta_rule_one   the delta rule on steps of one token a sequence, two launches instead of four
  *   lv_residual_split        residual update, and the residual as the sum of two bf16 numbers for a matrix product
  *
@@ -91,7 +90,7 @@
 extern "C" {
 #endif
 
-#define LV_MIX_ABI_VERSION 12
+#define LV_MIX_ABI_VERSION 13
 #define LV_MIX_BF16 0
 #define LV_MIX_F32 1
 #define LV_MIX_MAX_STREAMS 8
@@ -513,10 +512,6 @@ int lv_delta_prep_one(const void* proj, int64_t ld, const void* conv_w, void* co
 int lv_delta_rule_one(const void* qn, const void* kn, const void* v, const void* beta, const void* decay, void* state, const int32_t* cu_q,
                       const int32_t* ctx_lens, const int32_t* slots, const void* gate, int64_t ld_gate, const void* norm_w, void* out,
                       int B, int G, int H, int D, int decay_per_channel, float eps, int gate_act, int dtype, void* stream);
-
-/* logits f32 [T, E] = x bf16 [T, K] w^T, w f32 [E, K], as f32 products. K a multiple of 32, rows of x ldx entries apart (a multiple of 8),
- * x and w 16-byte aligned. */
-int lv_router_gemm(const void* x, int64_t ldx, const void* w, void* logits, int64_t T, int E, int K, void* stream);
 
 /* y bf16 [M, N] = x bf16 [M, K] w^T, w bf16 [N, K], sums in f32. M <= 64, K a multiple of 32; row strides ldx, ldw (multiples of 8)
  * and ldy in entries; x and w 16-byte, y 8-byte aligned. */

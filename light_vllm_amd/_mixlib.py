@@ -19,7 +19,7 @@ LIB_PATH = os.path.join(_HERE, "lib", "liblvmix.so")
 SOURCES = ["mix_stream.hip", "mix_window_attn.hip", "mix_window_mfma.hip", "mix_latent.hip", "mix_moe_gemm.hip",
            "mix_moe_tiles.hip", "mix_sandwich.hip", "mix_parallel.hip", "mix_recurrent.hip", "mix_prep.hip", "mix_lru.hip", "mix_chunk.hip",
            "mix_rows_gemm.hip"]
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 _P = c_void_p
 SIGNATURES = {
@@ -105,7 +105,6 @@ SIGNATURES = {
                                            c_int, c_int, c_int, _P, c_int, c_int, _P]),
     "lv_scaled_embedding": (c_int, [_P, _P, c_int, c_float, _P, _P, _P, c_int64, c_int, c_int, _P]),
     "lv_residual_split": (c_int, [_P, _P, _P, c_int64, c_int, _P]),
-    "lv_router_gemm": (c_int, [_P, c_int64, _P, _P, c_int64, c_int, c_int, _P]),
     "lv_rows_gemm": (c_int, [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P]),
 }
 

@@ -141,126 +141,6 @@ static void rows_gemm_launch(const RowsGemmParams& p, hipStream_t s) {
   rows_gemm_kernel<MT, NT, NT == 1 ? 2 : 1><<<dim3(rows_gemm_groups(p, MT, NT)), dim3(kRowsWaves * kWave), 0, s>>>(p);
 }
 
-// ---- logits [T, E] f32 = x [T, K] bf16 times w [E, K]^T f32 (a router's): as f32 products, without widening x.
-//
-// w is cut into three bf16 numbers an entry whose sum it is (8 bits each, nothing rounded), so that three products on the bf16 instructions,
-// exact and summed in f32, stand for an f32 one. Bound by reading x. A workgroup takes up to 64 rows and 32 outputs, its waves share k; x
-// passes through LDS as above, w is cut on its way to the registers. An infinity has no such pieces: sums that are not finite are
-// formed again in f32, one after the other. 16384 x 2048 x 32, us: widening and the vendor's f32 product 53, this 17.
-struct RouterGemmParams {
-  const uint16_t* x;
-  const float* w;
-  float* y;
-  int64_t ldx;
-  int T, E, K;
-};
-
-template <int MT, int NT>
-__global__ __launch_bounds__(kRowsWaves * kWave) void router_gemm_kernel(RouterGemmParams p) {
-  constexpr int NW = kRowsWaves, RS = NT * 16 + 4;
-  constexpr int STAGE = MT * 2048, PART = MT * 16 * RS * 4, PER = STAGE > PART ? STAGE : PART;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[NW * PER];
-  const int m0 = blockIdx.x * MT * 16, n0 = blockIdx.y * NT * 16;
-  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, quad = lane >> 4;
-  const int lrow = lane >> 3, lch = lane & 7;
-  const int pieces = (p.K + 63) / 64, c0 = w * pieces / NW, c1 = (w + 1) * pieces / NW;
-  unsigned char* mine = lds + w * PER;
-  const uint16_t* xr[MT * 2];
-  const float* wr[NT];
-#pragma unroll
-  for (int i = 0; i < MT * 2; ++i) xr[i] = p.x + min(m0 + 8 * i + lrow, p.T - 1) * p.ldx + 8 * lch;
-#pragma unroll
-  for (int i = 0; i < NT; ++i) wr[i] = p.w + static_cast<int64_t>(min(n0 + 16 * i + r, p.E - 1)) * p.K + 8 * quad;
-  u32x4_t xf[MT * 2];
-  float4 wf[2][NT][2];
-  f32x4_t acc[NT][MT];
-#pragma unroll
-  for (int i = 0; i < NT; ++i)
-#pragma unroll
-    for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  auto load = [&](int c) __attribute__((always_inline)) {
-    const bool whole = 64 * c + 32 < p.K;              // k may end in the middle of a piece: its first half again
-    const int k = whole || lch < 4 ? 64 * c : 64 * c - 32;
-#pragma unroll
-    for (int i = 0; i < MT * 2; ++i) xf[i] = *reinterpret_cast<const u32x4_t*>(xr[i] + k);
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int i = 0; i < NT; ++i)
-#pragma unroll
-        for (int e = 0; e < 2; ++e) wf[h][i][e] = ld4(wr[i] + 64 * c + (whole ? 32 * h : 0) + 4 * e);
-  };
-  auto cut = [](float4 a, float4 b, bf16x8_t (&to)[3]) __attribute__((always_inline)) {
-    float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      u32x4_t u;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        u[e] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, v[2 * e + 1]), __builtin_bit_cast(uint32_t, v[2 * e]), 0x07060302u);
-      to[i] = __builtin_bit_cast(bf16x8_t, u);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] -= __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[e]) & 0xffff0000u);
-    }
-  };
-  if (c0 < c1) load(c0);
-  for (int c = c0; c < c1; ++c) {
-#pragma unroll
-    for (int i = 0; i < MT * 2; ++i) {
-      const int row = 8 * i + lrow;
-      *reinterpret_cast<u32x4_t*>(mine + row * 128 + 16 * (lch ^ ((row >> 1) & 7))) = xf[i];
-    }
-    float4 wv[2][NT][2];
-#pragma unroll
-    for (int i = 0; i < 2 * NT * 2; ++i) wv[i / (2 * NT)][i / 2 % NT][i % 2] = wf[i / (2 * NT)][i / 2 % NT][i % 2];
-    __builtin_amdgcn_wave_barrier();                   // the wave's own LDS: its operations are carried out in order
-    bf16x8_t xv[MT][2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int j = 0; j < MT; ++j) {
-        const int row = 16 * j + r;
-        xv[j][h] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(mine + row * 128 + 16 * ((4 * h + quad) ^ ((row >> 1) & 7))));
-      }
-    __builtin_amdgcn_wave_barrier();
-    if (c + 1 < c1) load(c + 1);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      if (h == 1 && 64 * c + 32 >= p.K) break;
-#pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        bf16x8_t wc[3];
-        cut(wv[h][i][0], wv[h][i][1], wc);
-#pragma unroll
-        for (int x = 2; x >= 0; --x)
-#pragma unroll
-          for (int j = 0; j < MT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[x], xv[j][h], acc[i][j], 0, 0, 0);
-      }
-    }
-  }
-  __builtin_amdgcn_wave_barrier();
-  float* part = reinterpret_cast<float*>(mine);
-#pragma unroll
-  for (int i = 0; i < NT; ++i)
-#pragma unroll
-    for (int j = 0; j < MT; ++j) *reinterpret_cast<f32x4_t*>(part + (16 * j + r) * RS + 16 * i + 4 * quad) = acc[i][j];
-  __syncthreads();
-  for (int e = threadIdx.x; e < MT * 16 * NT * 16; e += NW * kWave) {
-    const int m = e / (NT * 16), n = e % (NT * 16);
-    if (m0 + m >= p.T || n0 + n >= p.E) continue;
-    float s = 0.0f;
-#pragma unroll
-    for (int i = 0; i < NW; ++i) s += *(reinterpret_cast<const float*>(lds + i * PER) + m * RS + n);
-    if (!__builtin_isfinite(s)) {
-      const bf16_t* x = reinterpret_cast<const bf16_t*>(p.x) + (m0 + m) * p.ldx;
-      const float* wn = p.w + static_cast<int64_t>(n0 + n) * p.K;
-      s = 0.0f;
-      for (int k = 0; k < p.K; ++k) s = fmaf(ldf(x + k), wn[k], s);
-    }
-    p.y[static_cast<int64_t>(m0 + m) * p.E + n0 + n] = s;
-  }
-}
-
 }  // namespace lvmix
 
 using namespace lvmix;
@@ -298,27 +178,4 @@ extern "C" int lv_rows_gemm(const void* x, int64_t ldx, const void* w, int64_t l
     default: rows_gemm_launch<4, 2>(p, s);
   }
   return launched("lv_rows_gemm");
-}
-
-extern "C" int lv_router_gemm(const void* x, int64_t ldx, const void* w, void* y, int64_t T, int E, int K, void* stream) {
-  if (T == 0 || E == 0) return 0;
-  if (!x || !w || !y) return fail(-1, "lv_router_gemm: null pointer");
-  if (T < 0 || T > INT32_MAX / 2 || E < 0 || E > 65535 * 32 || K <= 0 || K % 32 != 0) return fail(-1, "lv_router_gemm: bad sizes");
-  if (ldx < 0 || ldx % 8 != 0 || reinterpret_cast<uintptr_t>(x) % 16 != 0 || reinterpret_cast<uintptr_t>(w) % 16 != 0)
-    return fail(-1, "lv_router_gemm: strides or alignment");
-  RouterGemmParams p{static_cast<const uint16_t*>(x), static_cast<const float*>(w), static_cast<float*>(y), ldx, static_cast<int>(T), E, K};
-  // Cutting w takes most of a workgroup's time, and one of few workgroups is the launch's: smaller tiles as long as they fit the chip at
-  // once. us, widening and the vendor's product / 16 x 16 / 32 x 16 / 64 x 32 rows by outputs, K 4096, 32 outputs: 300 rows 17.0 / 10.6 / 11.6 /
-  // 21.7, 3000 30.2 / 20.3 / 13.1 / 22.3, 6000 46.6 / 28.5 / 22.9 / 23.2, 16384 111 / 67 / 45 / 27.
-  hipStream_t s = as_stream(stream);
-  auto go = [&](auto mt, auto nt) {
-    constexpr int M = decltype(mt)::value, N = decltype(nt)::value;
-    router_gemm_kernel<M, N><<<dim3(static_cast<unsigned>((T + 16 * M - 1) / (16 * M)), (E + 16 * N - 1) / (16 * N)), dim3(kRowsWaves * kWave), 0, s>>>(p);
-  };
-  using std::integral_constant;
-  const int64_t halves = (E + 15) / 16;
-  if ((T + 15) / 16 * halves <= 256) go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
-  else if ((T + 31) / 32 * halves <= 256) go(integral_constant<int, 2>{}, integral_constant<int, 1>{});
-  else go(integral_constant<int, 4>{}, integral_constant<int, 2>{});
-  return launched("lv_router_gemm");
 }

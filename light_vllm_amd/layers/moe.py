@@ -92,9 +92,8 @@ class SparseMoE(nn.Module):
             self.up_weight, self.down_weight = share.up_weight, share.down_weight
 
     def route(self, h: torch.Tensor):
-        # bf16, or logits_kernel: f32 logits straight from the activations (no widened copy)
-        kernel = self.logits_kernel or h.dtype == torch.bfloat16
-        logits = mix_ops.router_logits(h, self.router_weight) if kernel else F.linear(h.float(), self.router_weight)
+        # logits_kernel: small steps form their f32 logits straight from the activations (no widened copy)
+        logits = mix_ops.router_logits(h, self.router_weight) if self.logits_kernel else mix_ops.router_product(h, self.router_weight)
         return mix_ops.moe_route(logits, self.correction, self.top, self.groups, self.keep, score=self.score,
                                  group_rank=self.group_rank)
 

@@ -955,18 +955,10 @@ def router_logits(h, router_w):
 
 
 def router_product(h, router_w):
-    """f32 [T, E] = h router_w^T in f32 products. bf16 activations are read as they are (lv_router_gemm) where their rows are whole 16-byte
-    pieces and a multiple of 32 entries; others are widened for the vendor's product."""
-    T, W = h.shape
-    if not (h.is_cuda and T > 0 and h.dtype == torch.bfloat16 and router_w.dtype == torch.float32 and router_w.is_contiguous()
-            and not _transformed(h, router_w) and W > 0 and W % 32 == 0 and h.stride(1) == 1 and h.stride(0) % 8 == 0
-            and h.data_ptr() % 16 == 0 and router_w.data_ptr() % 16 == 0
-            and not (torch.is_grad_enabled() and (h.requires_grad or router_w.requires_grad))):
-        return F.linear(h.float(), router_w)
-    logits = torch.empty(T, router_w.size(0), dtype=torch.float32, device=h.device)
-    lib = _mixlib.load()
-    _mixlib.check(lib.lv_router_gemm(_p(h), h.stride(0), _p(router_w), _p(logits), T, router_w.size(0), W, _stream(h)), "lv_router_gemm")
-    return logits
+    """f32 [T, E] = h router_w^T: the activations widened, the vendor's f32 product. Tokens whose experts nearly tie take one or the other by
+    the order of these sums, so the order stays: f32 sums in three bf16 pieces were 50 us faster at 16384 x 2048 x 32, no further from float64,
+    and moved such tokens to other experts."""
+    return F.linear(h.float(), router_w)
 
 
 def relu2_scale(up, dense, E, Fe):

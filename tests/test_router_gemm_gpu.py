@@ -1,5 +1,5 @@
-"""lv_router_gemm (router logits as f32 products of bf16 activations) against float64: edges of its tiles and of its loop over k, rows of a
-wider tensor, values that are not finite."""
+"""Router logits (mix_ops.router_product, f32 products of widened bf16 activations) against float64: sizes around 64 rows, rows of a wider
+tensor, values that are not finite."""
 import pytest
 import torch
 import torch.nn.functional as F
