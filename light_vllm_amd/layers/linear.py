@@ -19,9 +19,10 @@ from .tp import divide, tp_rank, tp_size
 
 
 def _linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
-    if bias is not None or x.size(0) > mix_ops.ROWS_GEMM_MAX:       # prompts' steps look no further
-        return F.linear(x, weight, bias)
-    return mix_ops.linear(x, weight)
+    if not torch.jit.is_scripting():                    # (a script holds torch's operators only)
+        if bias is None:
+            return mix_ops.linear(x, weight)
+    return F.linear(x, weight, bias)
 
 
 class LinearBase(nn.Module):

@@ -1739,14 +1739,22 @@ def mm_f32(a, b_t, add=None):
 ROWS_GEMM_MAX = 64           # rows of x that lv_rows_gemm takes
 
 
-def _transformed(*ts) -> bool:
-    """Whether something is to see or rewrite torch's own operators on these tensors: forward-mode gradients, function transforms,
-    tracing, autocast, modes (a default device is none: the engine sets one) and subclasses. A launch of our own is invisible to all of
-    them."""
-    return (any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in ts) or forward_ad._current_level >= 0
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _traced(x) -> bool:
+    """Whether x stands for other tensors: a tracer's or a subclass's operand, or one inside a compilation or a trace. It is not looked at any
+    further then: what it is asked becomes part of what is traced."""
+    return type(x) not in _PLAIN or torch.compiler.is_compiling() or torch.jit.is_tracing()
+
+
+def _transformed(w) -> bool:
+    """Whether something is to see or rewrite torch's own operators: forward-mode gradients, function transforms, autocast, modes (a default
+    device is none: the engine sets one) and subclasses. A launch of our own is invisible to all of them."""
+    return (type(w) not in _PLAIN or forward_ad._current_level >= 0
             or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0
             or any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
-            or torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing())
+            or torch.is_autocast_enabled("cuda"))
 
 
 def rows_gemm_ok(x, w) -> bool:
@@ -1754,7 +1762,7 @@ def rows_gemm_ok(x, w) -> bool:
     most 64 rows of x. Above 32 rows the rows of x that every compute unit reads weigh as much as the weights, and large products
     are the vendor's: us, vendor / own, 33, 48 and 64 rows: 10304 x 4096 29 / 26, 29 / 27, 29 / 30; 20480 x 4096 42 / 43, 44 / 45, 45 / 48;
     8192 x 2048 14.7 / 12.0, 14.8 / 12.3, 14.7 / 12.0."""
-    if x.dim() != 2 or not 0 < x.size(0) <= ROWS_GEMM_MAX or not x.is_cuda or x.dtype != torch.bfloat16 or _transformed(x, w):
+    if _traced(x) or x.dim() != 2 or not 0 < x.size(0) <= ROWS_GEMM_MAX or not x.is_cuda or x.dtype != torch.bfloat16 or _transformed(w):
         return False
     M, K = x.shape
     N = w.size(0)
