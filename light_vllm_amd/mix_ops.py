@@ -1781,11 +1781,12 @@ def _rows_gemm(x, w):
 
 
 class _RowsLinear(torch.autograd.Function):
-    """lv_rows_gemm where gradients are recorded: the same output, torch's products behind it."""
+    """lv_rows_gemm where gradients are recorded: the same output, torch's products behind it. As in torch's own product an operand is kept
+    only for the other one's gradient: the rows in front of a frozen weight may be overwritten."""
 
     @staticmethod
     def forward(ctx, x, w):
-        ctx.save_for_backward(x, w)
+        ctx.save_for_backward(x if ctx.needs_input_grad[1] else None, w if ctx.needs_input_grad[0] else None)
         return _rows_gemm(x, w)
 
     @staticmethod
