@@ -1742,19 +1742,32 @@ ROWS_GEMM_MAX = 64           # rows of x that lv_rows_gemm takes
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
-def _traced(x) -> bool:
-    """Whether x stands for other tensors: a tracer's or a subclass's operand, or one inside a compilation or a trace. It is not looked at any
-    further then: what it is asked becomes part of what is traced."""
-    return type(x) not in _PLAIN or torch.compiler.is_compiling() or torch.jit.is_tracing()
-
-
-def _transformed(w) -> bool:
+def _transformed() -> bool:
     """Whether something is to see or rewrite torch's own operators: forward-mode gradients, function transforms, autocast, modes (a default
-    device is none: the engine sets one) and subclasses. A launch of our own is invisible to all of them."""
-    return (type(w) not in _PLAIN or forward_ad._current_level >= 0
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0
-            or any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
-            or torch.is_autocast_enabled("cuda"))
+    device is none: the engine sets one). A launch of our own is invisible to all of them."""
+    modes = torch._C._len_torch_function_stack()
+    return (forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._len_torch_dispatch_stack() > 0 or torch.is_autocast_enabled("cuda")
+            or modes > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(modes)))
+
+
+def _rows_gemm_sizes(x, w):
+    """(M, N, K, row strides of x and of w, device) if linear(x, w) takes lv_rows_gemm, None if it stays with torch; rows_gemm_ok says when.
+    An operand that stands for others (a tracer's, a subclass's, one inside a compilation or a trace) is not looked at: what it is asked
+    becomes part of what is traced. Eager steps of few tokens are bound by the host and every projection asks, so nothing is asked
+    twice: us a call, 8 x 2048 x 2048: looks, allocation and launch 12.0 with each look of its own, 7.5 this way; 0.7 where more rows go on
+    to torch's linear."""
+    if (type(x) not in _PLAIN or torch.compiler.is_compiling() or torch._C._is_tracing() or x.dim() != 2
+            or not 0 < x.size(0) <= ROWS_GEMM_MAX or not x.is_cuda or x.dtype is not torch.bfloat16 or type(w) not in _PLAIN
+            or w.dim() != 2 or w.dtype is not torch.bfloat16 or _transformed()):
+        return None
+    (M, K), (N, k) = x.shape, w.shape
+    (ldx, one_x), (ldw, one_w) = x.stride(), w.stride()
+    dev = x.get_device()
+    if (k != K or K == 0 or K % 32 or N == 0 or not (M <= 32 or M * N * K <= 1 << 31) or one_x != 1 or one_w != 1 or ldx % 8 or ldw % 8
+            or ldw < K or (x.data_ptr() | w.data_ptr()) & 15 or w.get_device() != dev or dev != torch.cuda.current_device()):
+        return None
+    return M, N, K, ldx, ldw, dev
 
 
 def rows_gemm_ok(x, w) -> bool:
@@ -1762,21 +1775,15 @@ def rows_gemm_ok(x, w) -> bool:
     most 64 rows of x. Above 32 rows the rows of x that every compute unit reads weigh as much as the weights, and large products
     are the vendor's: us, vendor / own, 33, 48 and 64 rows: 10304 x 4096 29 / 26, 29 / 27, 29 / 30; 20480 x 4096 42 / 43, 44 / 45, 45 / 48;
     8192 x 2048 14.7 / 12.0, 14.8 / 12.3, 14.7 / 12.0."""
-    if _traced(x) or x.dim() != 2 or not 0 < x.size(0) <= ROWS_GEMM_MAX or not x.is_cuda or x.dtype != torch.bfloat16 or _transformed(w):
-        return False
-    M, K = x.shape
-    N = w.size(0)
-    return (w.dim() == 2 and w.dtype == torch.bfloat16 and w.device == x.device and w.size(1) == K and K > 0 and K % 32 == 0 and N > 0
-            and (M <= 32 or M * N * K <= 1 << 31) and x.stride(1) == 1 and w.stride(1) == 1 and x.stride(0) % 8 == 0
-            and w.stride(0) % 8 == 0 and w.stride(0) >= K and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and x.device.index == torch.cuda.current_device())
+    return _rows_gemm_sizes(x, w) is not None
 
 
-def _rows_gemm(x, w):
-    M, K = x.shape
-    y = torch.empty(M, w.size(0), dtype=x.dtype, device=x.device)
+def _rows_gemm(x, w, sizes):
+    M, N, K, ldx, ldw, dev = sizes
+    y = x.new_empty((M, N))
     lib = _mixlib.load()
-    _mixlib.check(lib.lv_rows_gemm(_p(x), x.stride(0), _p(w), w.stride(0), _p(y), y.stride(0), M, w.size(0), K, _stream(x)), "lv_rows_gemm")
+    _mixlib.check(lib.lv_rows_gemm(x.data_ptr(), ldx, w.data_ptr(), ldw, y.data_ptr(), N, M, N, K, torch._C._cuda_getCurrentRawStream(dev)),
+                  "lv_rows_gemm")
     return y
 
 
@@ -1785,20 +1792,21 @@ class _RowsLinear(torch.autograd.Function):
     only for the other one's gradient: the rows in front of a frozen weight may be overwritten."""
 
     @staticmethod
-    def forward(ctx, x, w):
+    def forward(ctx, x, w, sizes):
         ctx.save_for_backward(x if ctx.needs_input_grad[1] else None, w if ctx.needs_input_grad[0] else None)
-        return _rows_gemm(x, w)
+        return _rows_gemm(x, w, sizes)
 
     @staticmethod
     def backward(ctx, dy):
         x, w = ctx.saved_tensors
-        return (dy.mm(w) if ctx.needs_input_grad[0] else None), (dy.t().mm(x) if ctx.needs_input_grad[1] else None)
+        return (dy.mm(w) if ctx.needs_input_grad[0] else None), (dy.t().mm(x) if ctx.needs_input_grad[1] else None), None
 
 
 def linear(x, w):
     """x [..., K] w [N, K]^T. Few rows of bf16 (decode steps) take lv_rows_gemm, everything else torch's linear."""
-    if not rows_gemm_ok(x, w):
+    sizes = _rows_gemm_sizes(x, w)
+    if sizes is None:
         return F.linear(x, w)
     if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
-        return _RowsLinear.apply(x, w)
-    return _rows_gemm(x, w)
+        return _RowsLinear.apply(x, w, sizes)
+    return _rows_gemm(x, w, sizes)

@@ -9,7 +9,7 @@ from light_vllm_amd import mix_ops
 @pytest.fixture
 def product(monkeypatch):
     monkeypatch.setattr(mix_ops, "_rows_gemm", lambda x, w, *a: torch.mm(x, w.t()))
-    return lambda x, w: mix_ops._RowsLinear.apply(x, w)
+    return lambda x, w: mix_ops._RowsLinear.apply(x, w, None)
 
 
 def operands(gx, gw):
