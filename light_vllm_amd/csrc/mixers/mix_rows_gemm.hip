@@ -9,9 +9,9 @@
 // A row's sums are formed in the same order whatever else is in the step and whatever tile it lands in.
 //
 // us in a replayed graph over weights that no cache holds, vendor product -> this, rows x columns x k: 1 x 5152 x 2048 12.3 -> 7.2,
-// 16 x 2048 x 2048 11.1 -> 5.4, 32 x 8192 x 2048 14.2 -> 9.8, 64 x 5152 x 2048 12.8 -> 10.9, 64 x 2048 x 2048 11.7 -> 6.3,
-// 64 x 4096 x 4096 15.4 -> 12.9, 8 x 20480 x 4096 68 -> 34. Large weights on 33 to 64 rows stay with the vendor's product
-// (64 x 20480 x 4096: 45 there, 50 here): the caller's rule.
+// 16 x 2048 x 2048 11.0 -> 5.3, 32 x 8192 x 2048 13.2 -> 9.7, 64 x 5152 x 2048 12.9 -> 10.7, 64 x 2048 x 2048 11.7 -> 6.2,
+// 64 x 4096 x 4096 15.2 -> 12.9, 8 x 10304 x 4096 26.3 -> 19.2, 16 x 5120 x 17408 115 -> 43. Not everywhere: 32 x 10304 x 4096 22.4 there,
+// 25.3 here, 64 x 20480 x 4096 45 and 48. The caller's rule says where.
 #include "mix_common.h"
 
 namespace lvmix {
@@ -155,26 +155,22 @@ extern "C" int lv_rows_gemm(const void* x, int64_t ldx, const void* w, int64_t l
     return fail(-1, "lv_rows_gemm: strides or alignment");
   RowsGemmParams p{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), static_cast<uint16_t*>(y), ldx, ldw, ldy, M, N, K};
   // The tile that brings the least into a compute unit: rounds of 256 workgroups times a workgroup's rows of x and w. us at
-  // 64 x 2592 x 2048 (rows x columns of a tile): 32 x 32 7.6, 64 x 16 8.5, 16 x 16 8.9, 32 x 16 9.2; at 64 x 5152 x 2048 64 x 32 10.9,
-  // 16 x 32 12.2, 32 x 32 12.3; at 48 x 2048 x 2048 32 x 16 5.8, 16 x 32 6.3, 16 x 16 6.8.
-  int best = 0, cost = 1 << 30;
+  // 64 x 2592 x 2048 (rows x columns of a tile): 32 x 32 7.6, 16 x 16 8.9; at 64 x 5152 x 2048 64 x 32 10.9, 16 x 32 12.2, 32 x 32 12.3; at
+  // 48 x 2048 x 2048 16 x 32 6.3, 16 x 16 6.7. Tiles of more rows by 16 columns never count less than one of these (32 x 16 as much as 16 x 32,
+  // though it took 5.8 at the last), so there are none.
+  auto count = [&](int mt, int nt) { return (rows_gemm_groups(p, mt, nt) + 255) / 256 * (mt + nt); };
+  int best = 0, least = count(1, 1);
   for (int mt = 1; mt <= (M + 15) / 16; ++mt)
-    for (int nt = 1; nt <= 2; ++nt) {
-      const int c = ((rows_gemm_groups(p, mt, nt) + 255) / 256) * (mt + nt);
-      if (c < cost) {
-        best = 2 * mt + nt - 3;
-        cost = c;
-      }
+    if (count(mt, 2) < least) {
+      best = mt;
+      least = count(mt, 2);
     }
   hipStream_t s = as_stream(stream);
   switch (best) {
     case 0: rows_gemm_launch<1, 1>(p, s); break;
     case 1: rows_gemm_launch<1, 2>(p, s); break;
-    case 2: rows_gemm_launch<2, 1>(p, s); break;
-    case 3: rows_gemm_launch<2, 2>(p, s); break;
-    case 4: rows_gemm_launch<3, 1>(p, s); break;
-    case 5: rows_gemm_launch<3, 2>(p, s); break;
-    case 6: rows_gemm_launch<4, 1>(p, s); break;
+    case 2: rows_gemm_launch<2, 2>(p, s); break;
+    case 3: rows_gemm_launch<3, 2>(p, s); break;
     default: rows_gemm_launch<4, 2>(p, s);
   }
   return launched("lv_rows_gemm");

@@ -1764,17 +1764,40 @@ def _rows_gemm_sizes(x, w):
     (M, K), (N, k) = x.shape, w.shape
     (ldx, one_x), (ldw, one_w) = x.stride(), w.stride()
     dev = x.get_device()
-    if (k != K or K == 0 or K % 32 or N == 0 or not (M <= 32 or M * N * K <= 1 << 31) or one_x != 1 or one_w != 1 or ldx % 8 or ldw % 8
+    if (k != K or K == 0 or K % 32 or N == 0 or not rows_gemm_pays(M, N, K) or one_x != 1 or one_w != 1 or ldx % 8 or ldw % 8
             or ldw < K or (x.data_ptr() | w.data_ptr()) & 15 or w.get_device() != dev or dev != torch.cuda.current_device()):
         return None
     return M, N, K, ldx, ldw, dev
 
 
+def rows_gemm_pays(M, N, K) -> bool:
+    """Whether lv_rows_gemm is ahead of the vendor's product for M rows, N columns and this k. Measured in replayed graphs over weights that no
+    cache holds, 520 pairs of N and k from 64 x 64 to 65536 x 2048 at up to 16 row counts; where the answer is yes, nowhere behind by 2 %.
+    Times in us, vendor / own.
+      up to 4096 columns: to k 6400 (4096 x 6400 at 16 rows 23.3 / 13.4; at 64 21.7 / 19.4). Longer k is level (256 x 8192 8.4 / 8.6) or
+        lost (4096 x 12288, 17 rows, 24.0 / 26.5) until the vendor's product falls off behind 16384 (up to 32 rows: 5120 x
+        17408 111 / 36 at one, 121 / 52 at 32).
+      up to 8192, one round of workgroups of 32 columns: to k 4096 (8192 x 4096, 48 rows, 18.5 / 17.8); beyond 48 rows the rows of x that every
+        compute unit reads weigh as much as the weights (the same, 56 rows, 19.0 / 19.5), to k 3584 (7000 columns, 64 rows, 20.1 / 17.8).
+      more columns, up to 16 rows: to k 4096 (10304 x 4096 26.3 / 20.7); to 5120 where many rounds even out (34816 75.6 / 72.5; not 9000,
+        23.7 / 25.7).
+      more columns, up to 32 rows: what the last round leaves idle costs more than short k or the vendor's trouble with rows of whole 4 KiB
+        give back: 14336 x 1024 21.3 / 8.7, 12288 x 2048 15.4 / 14.9, 24576 x 4096 46.7 / 42.1; not
+        30000 x 640 11.6 / 12.2, 9000 x 3072 16.9 / 20.2, 10304 x 4096 22.4 / 25.3, 26000 x 4096 48.6 / 49.8.
+      more columns and more rows stay with the vendor (12288 x 2048, 64 rows, 16.6 / 17.7; 20480 x 4096 45 / 48)."""
+    if N <= 4096:
+        return K <= 6400 or (K > 16384 and N >= 2048 and M <= 32)
+    if N <= 8192:
+        return K <= (4096 if M <= 48 else 3584) or (K > 16384 and M <= 32)
+    if M <= 16:
+        return N <= 40000 and (K <= 4096 or (K <= 5120 and N >= 18432))
+    idle = -((N + 31) // 32) % 256                         # places that the last round of 256 workgroups leaves empty
+    return M <= 32 and N <= 32768 and (K <= 1024 and N <= 16384 or K == 2048 or K == 4096 and N >= 16384 and idle <= 154)
+
+
 def rows_gemm_ok(x, w) -> bool:
     """Whether linear(x, w) takes lv_rows_gemm: bf16 matrices on one device with rows of whole 16-byte pieces, k a multiple of 32, at
-    most 64 rows of x. Above 32 rows the rows of x that every compute unit reads weigh as much as the weights, and large products
-    are the vendor's: us, vendor / own, 33, 48 and 64 rows: 10304 x 4096 29 / 26, 29 / 27, 29 / 30; 20480 x 4096 42 / 43, 44 / 45, 45 / 48;
-    8192 x 2048 14.7 / 12.0, 14.8 / 12.3, 14.7 / 12.0."""
+    most 64 rows of x, where it pays."""
     return _rows_gemm_sizes(x, w) is not None
 
 

@@ -9,10 +9,10 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-def case(M, N, K, seed, lead=0):
+def case(M, N, K, seed, lead=0, lead_w=0):
     gen = torch.Generator(device=DEV).manual_seed(seed)
     x = torch.empty(M, K + lead, dtype=torch.bfloat16, device=DEV).normal_(generator=gen)[:, lead:]
-    w = torch.empty(N, K, dtype=torch.bfloat16, device=DEV).normal_(0.0, K ** -0.5, generator=gen)
+    w = torch.empty(N, K + lead_w, dtype=torch.bfloat16, device=DEV).normal_(0.0, K ** -0.5, generator=gen)[:, lead_w:]
     return x, w
 
 
@@ -21,9 +21,25 @@ def case(M, N, K, seed, lead=0):
 @pytest.mark.parametrize("N,K,lead", [(1, 32, 0), (15, 64, 8), (16, 96, 0), (33, 544, 0), (132, 2080, 64), (1040, 2048, 0), (2600, 1024, 0),
                                       (5152, 512, 0), (8208, 768, 8), (10304, 256, 0)])
 def test_against_float64(M, N, K, lead):
-    x, w = case(M, N, K, 1000 * M + N, lead)
-    assert mix_ops.rows_gemm_ok(x, w)
-    y = mix_ops.linear(x, w)
+    check(M, N, K, lead)
+
+
+# both halves of a last piece of k, first and last rows of a tile and columns that leave remainders, in tiles (16-row blocks, 16-column
+# blocks) of 1 x 1, 1 x 2, 2 x 2, 3 x 2 and 4 x 2; rows of x and of w inside wider ones
+@torch.inference_mode()
+@pytest.mark.parametrize("Ms,N", [((1, 15, 33, 48), 1041), ((2, 16), 5170), ((49, 63), 1045), ((17, 31, 32), 5170), ((50, 64), 2607), ((33, 47, 48), 5170),
+                                  ((49, 63, 64), 5170)])
+@pytest.mark.parametrize("K", [32, 544, 576])
+@pytest.mark.parametrize("lead,lead_w", [(0, 0), (8, 24)])
+def test_tiles(Ms, N, K, lead, lead_w):
+    for M in Ms:
+        check(M, N, K, lead, lead_w)
+
+
+def check(M, N, K, lead=0, lead_w=0):
+    x, w = case(M, N, K, 1000 * M + N, lead, lead_w)
+    y = mix_ops._rows_gemm(x, w, (M, N, K, K + lead, K + lead_w, x.get_device()))       # whether or not it pays
+    assert not mix_ops.rows_gemm_ok(x, w) or torch.equal(y, mix_ops.linear(x, w))
     ref = x.double() @ w.double().t()
     # one rounding to bf16 (half a unit in the last place, 2^-9 of the value at most) and K f32 additions in chains of their own
     bound = ref.abs() * 2.0 ** -8 + (x.double().abs() @ w.double().abs().t()) * K * 2.0 ** -24
@@ -62,6 +78,7 @@ def test_calls_that_stay_with_torch():
         assert not mix_ops.rows_gemm_ok(x.float(), w.float()) and not mix_ops.rows_gemm_ok(x.view(2, 4, 64), w)
         assert not mix_ops.rows_gemm_ok(x, w.t()) and not mix_ops.rows_gemm_ok(x[:, ::2], w[:, ::2])
         assert not mix_ops.rows_gemm_ok(*case(64, 20480, 4096, 8)) and mix_ops.rows_gemm_ok(*case(32, 20480, 4096, 8))
+        assert not mix_ops.rows_gemm_ok(*case(17, 10304, 4096, 8)) and mix_ops.rows_gemm_ok(*case(16, 10304, 4096, 8))
         with torch.autocast("cuda", dtype=torch.float16):
             assert not mix_ops.rows_gemm_ok(x, w)
         with torch.device("cuda"):               # a default device, as the engine sets one

@@ -48,3 +48,13 @@ def test_second_derivatives_and_batched_gradients(product):
     got = torch.autograd.grad(product(x, w), (x, w), dy, is_grads_batched=True)
     want = torch.autograd.grad(F.linear(x, w), (x, w), dy, is_grads_batched=True)
     assert all(torch.allclose(a, b, rtol=1e-5, atol=1e-6) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("N,K,pays,not_pays", [
+    (48, 2048, (1, 64), ()), (4096, 6400, (1, 16, 17, 64), ()), (256, 8192, (), (1, 16, 64)), (4096, 12288, (), (1, 17, 64)), (5120, 17408, (1, 32), (33, 64)),
+    (8192, 4096, (1, 17, 32, 48), (49, 64)), (8192, 3584, (1, 64), ()), (5120, 5120, (), (1, 17, 33, 64)), (10304, 4096, (1, 16), (17, 32, 33, 64)),
+    (12800, 5120, (), (1, 16, 32, 64)), (34816, 5120, (1, 16), (17, 64)), (9000, 3072, (1, 16), (17, 33)), (12288, 2048, (16, 32), (33, 64)),
+    (14336, 1024, (32,), (64,)), (16384, 4096, (32,), (64,)), (20480, 4096, (16, 32), (33, 64)), (26000, 4096, (16,), (32,)), (65536, 2048, (), (1, 32))])
+def test_where_the_kernel_pays(N, K, pays, not_pays):
+    """Both sides of the measured rule."""
+    assert all(mix_ops.rows_gemm_pays(M, N, K) for M in pays) and not any(mix_ops.rows_gemm_pays(M, N, K) for M in not_pays)
