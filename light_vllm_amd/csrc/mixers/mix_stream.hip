@@ -837,6 +837,7 @@ static int delta_prep_entry(void* new_state, const void* proj, int64_t ld, const
       !kn || !v || !beta || !decay || !a)
     return fail(-1, "lv_delta_prep: null pointer");
   if (G <= 0 || H <= 0 || H % G != 0 || D <= 0 || Dv <= 0 || taps < 1) return fail(-1, "lv_delta_prep: bad sizes");
+  if (dtype != LV_MIX_BF16 && dtype != LV_MIX_F32) return fail(-1, "lv_delta_prep: dtype %d", dtype);
   const int C = 2 * G * D + H * Dv;
   const int dec_dim = decay_per_channel ? D : 1;
   if (ld < C || off_b + H > ld || ld_a < static_cast<int64_t>(H) * dec_dim)
@@ -852,8 +853,7 @@ static int delta_prep_entry(void* new_state, const void* proj, int64_t ld, const
     return launched("lv_delta_prep");
   if (new_state != nullptr) return fail(-2, "lv_delta_prep_one: sizes or alignment that the tiled form does not take");
   if (dtype == LV_MIX_BF16) delta_prep_kernel<bf16_t><<<grid, block, 0, as_stream(stream)>>>(p);
-  else if (dtype == LV_MIX_F32) delta_prep_kernel<float><<<grid, block, 0, as_stream(stream)>>>(p);
-  else return fail(-1, "lv_delta_prep: dtype %d", dtype);
+  else delta_prep_kernel<float><<<grid, block, 0, as_stream(stream)>>>(p);
   return launched("lv_delta_prep");
 }
 

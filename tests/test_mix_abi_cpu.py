@@ -84,6 +84,27 @@ def test_argument_validation_happens_before_any_launch():
     assert lib.lv_embed_norm(p, p, 8, 1.0, None, 0, 0, 0, None, p, 0, p, p, 1.0, 1e-6, p, p, p, p, p, p, 1, 8, 0, None) == -1   # empty position table
     assert lib.lv_unary_act(p, p, 8, 17, 0, None) == -1
     assert lib.lv_masked_attn(p, p, p, None, None, None, 0, p, p, p, p, p, 1, 1, 4, 2, 8, 8, 16, 64, 0, 0, 0, 0.5, -1.0, 0, None, 0, 0, 1, None, 0, None) == -1   # cap
+    # decode steps: projections of few rows, the delta rule in two launches
+    rows = lambda **kw: [kw.get("x", p), kw.get("ldx", 64), kw.get("w", p), kw.get("ldw", 64), kw.get("y", p), kw.get("ldy", 8), kw.get("M", 1),  # noqa: E731
+                         kw.get("N", 8), kw.get("K", 64), None]
+    assert lib.lv_rows_gemm(*rows(M=0, x=None)) == 0 and lib.lv_rows_gemm(*rows(N=0, w=None)) == 0
+    for bad in (dict(x=None), dict(w=None), dict(y=None), dict(M=65), dict(M=-1), dict(N=-1), dict(K=0), dict(K=48), dict(ldx=-8), dict(ldx=68), dict(ldw=56),
+                dict(ldw=68), dict(ldy=7), dict(x=p + 8), dict(w=p + 8), dict(y=p + 4)):
+        assert lib.lv_rows_gemm(*rows(**bad)) == -1 and b"lv_rows_gemm" in lib.lv_mix_last_error(), bad
+    prep = lambda **kw: [p, kw.get("ld", 324), p, kw.get("state", p), p, p, p, p, p, p, kw.get("qn", p), p, p, p, p, kw.get("T", 1), 1, kw.get("H", 3),  # noqa: E731
+                         kw.get("D", 64), kw.get("Dv", 64), kw.get("taps", 4), kw.get("off_b", 320), p, 4, 0, 1e-6, kw.get("dt", 0), None]
+    assert lib.lv_delta_prep_one(*prep(T=0, state=None)) == 0
+    for bad in (dict(state=None), dict(qn=None), dict(H=0), dict(taps=0), dict(ld=316), dict(off_b=322), dict(dt=7)):
+        assert lib.lv_delta_prep_one(*prep(**bad)) == -1, bad
+    assert lib.lv_delta_prep(*prep(dt=7)) == -1 and b"dtype" in lib.lv_mix_last_error()
+    for other in (dict(D=32), dict(Dv=128, ld=520, off_b=512), dict(taps=5), dict(ld=325), dict(state=p + 4), dict(qn=p + 4)):      # what lv_delta_prep serves otherwise
+        assert lib.lv_delta_prep_one(*prep(**other)) == -2, other
+    one = lambda **kw: [kw.get("qn", p), p, p, p, kw.get("decay", p), kw.get("state", p), p, p, p, kw.get("gate", p), kw.get("ldg", 128), p, kw.get("out", p),  # noqa: E731
+                        kw.get("B", 1), kw.get("G", 1), kw.get("H", 2), kw.get("D", 64), kw.get("channel", 0), 1e-6, kw.get("act", 0), kw.get("dt", 0), None]
+    assert lib.lv_delta_rule_one(*one(B=0, qn=None)) == 0
+    for bad in (dict(qn=None), dict(B=-1), dict(B=65536), dict(G=0), dict(G=3), dict(H=0), dict(D=32), dict(D=256), dict(ldg=124), dict(ldg=130), dict(act=2), dict(dt=2),
+                dict(qn=p + 4), dict(state=p + 8), dict(gate=p + 4), dict(out=p + 4), dict(gate=p + 8, dt=1), dict(decay=p + 4, channel=1)):
+        assert lib.lv_delta_rule_one(*one(**bad)) == -1 and b"lv_delta_rule_one" in lib.lv_mix_last_error(), bad
     # the gated linear recurrence, stored norms, split residuals, extended attention
     assert lib.lv_gated_linear_recurrence(None, 0, None, 0, None, None, None, None, None, None, None, None, 0, 0, 0, 0, 8, 2, 1, None, 0, 0, None) == 0
     lru = lambda **kw: [p, kw.get("ldu", 64), p, kw.get("ldy", 64), p, p, p, p, p, p, p, p, 64, 1, 1, 1, 64, kw.get("blocks", 2), kw.get("nsplit", 1),  # noqa: E731
