@@ -36,9 +36,16 @@ def test_like_the_token_loop(monkeypatch, D, Dv, H, G, where):
         got.append((mix_ops.gated_scan(mix_ops.SCAN_STEP, q, k, v, a, p0, p1, step, st, H, G, D, Dv, p2=p2).view(T, H, Dv), st))
     for x, y in zip(*got):
         assert torch.equal(torch.isfinite(x), torch.isfinite(y))
+        if where not in ("q", "v"):
+            # one infinity a sum on both sides: the same sign. (An infinite v fills a column of the state, which a later token sums with the
+            # signs of its q; the chunk multiplies it by one sum of q and k. An infinite q the other way round.)
+            assert torch.equal(torch.isnan(x), torch.isnan(y)) and torch.equal(torch.isposinf(x), torch.isposinf(y))
         ok = torch.isfinite(x)
-        # f32 sums of D + T terms on both sides
-        assert bool(((x - y)[ok].abs() <= 2.0 ** -24 * (D + 64) * 8 * (1 + x[ok].abs())).all()) or where == "huge"
+        # f32 sums of D + T terms on both sides, relative to their terms: the state's huge entry dominates the outputs that it reaches
+        assert bool(((x - y)[ok].abs() <= 2.0 ** -24 * (D + 64) * 8 * (1 + x[ok].abs())).all())
+    if where == "huge":
+        far = got[1][0][sum(new[:3]):, H - 1, 7].abs()
+        assert float(far[0]) > 1e30 and float(got[1][0].abs().amax()) < 1.1e38
     assert where in ("none", "huge") or not bool(torch.isfinite(got[1][0]).all())
 
 

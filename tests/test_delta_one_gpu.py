@@ -14,6 +14,23 @@ NEW, CTX = [1, 1, 0, 1, 1, 1] * 16, [0, 1, 4, 2, 3, 700] * 16
 @pytest.mark.parametrize("channel", [False, True])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_preparation(G, H, D, taps, channel, dtype):
+    preparation(G, H, D, taps, channel, dtype, NEW, CTX)
+
+
+# tiles of two and five tokens, each a sequence of its own, the last tile cut short
+@pytest.mark.parametrize("G,H,D,taps,times", [(1, 1, 64, 4, 215), (1, 2, 128, 3, 530), (1, 2, 64, 2, 531)])
+@pytest.mark.parametrize("channel", [False, True])
+def test_preparation_of_many_sequences(G, H, D, taps, times, channel):
+    preparation(G, H, D, taps, channel, torch.bfloat16, NEW[:6] * times + [1], CTX[:6] * times + [2])
+
+
+# no more tokens than sequences, but not one each: the launches that longer steps take
+@pytest.mark.parametrize("new,ctx", [([3, 0, 0], [5, 4, 0]), ([0, 2, 1, 0], [0, 1, 2, 9])])
+def test_preparation_of_uneven_steps(new, ctx):
+    preparation(2, 4, 128, 4, False, torch.bfloat16, new, ctx)
+
+
+def preparation(G, H, D, taps, channel, dtype, NEW, CTX):
     gen = torch.Generator(device="cuda").manual_seed(G + D)
     rn = lambda *s: torch.randn(*s, device="cuda", generator=gen)    # noqa: E731
     T, C, wide = sum(NEW), 2 * G * D + H * D, H * D if channel else H
@@ -61,3 +78,17 @@ def test_rule_norm_gate(G, H, D, channel, dtype, act):
     assert err(ours, S) <= 1.05 * err(theirs, S) + 1e-9 and err(got, y) <= 1.05 * err(want, y) + 1e-9
     still = step.host_slots[NEW.index(0)]
     assert torch.equal(ours[still], state[still])
+
+
+@pytest.mark.parametrize("new,ctx", [([3, 0, 0], [5, 4, 0]), ([0, 2, 1, 0], [0, 1, 2, 9])])
+def test_rule_of_uneven_steps(new, ctx):
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    rn = lambda *s: torch.randn(*s, device="cuda", generator=gen)    # noqa: E731
+    T, G, H, D, step = sum(new), 2, 4, 128, make_step(new, ctx)
+    q, k = (torch.nn.functional.normalize(rn(T, G, D), dim=-1) for _ in range(2))
+    v, beta, decay, gate, w = rn(T, H, D), torch.sigmoid(rn(T, H)), torch.sigmoid(rn(T, H)), rn(T, H * D).bfloat16(), rn(D)
+    state = rn(len(new), H, D, D)
+    ours, theirs = state.clone(), state.clone()
+    got = mix_ops.delta_rule_norm_gate(q, k, v, beta, decay, ours, step, gate, w, 1e-6, torch.bfloat16)
+    want = mix_ops.head_norm_gate(mix_ops.gated_delta_rule(q, k, v, beta, decay, theirs, step), gate, w, 1e-6, torch.bfloat16)
+    assert torch.equal(got, want) and torch.equal(ours, theirs)
