@@ -1740,6 +1740,7 @@ ROWS_GEMM_MAX = 64           # rows of x that lv_rows_gemm takes
 
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+_compiling, _tracing = torch.compiler.is_compiling, torch._C._is_tracing
 
 
 def _transformed() -> bool:
@@ -1755,13 +1756,15 @@ def _rows_gemm_sizes(x, w):
     """(M, N, K, row strides of x and of w, device) if linear(x, w) takes lv_rows_gemm, None if it stays with torch; rows_gemm_ok says when.
     An operand that stands for others (a tracer's, a subclass's, one inside a compilation or a trace) is not looked at: what it is asked
     becomes part of what is traced. Eager steps of few tokens are bound by the host and every projection asks, so nothing is asked
-    twice: us a call, 8 x 2048 x 2048: looks, allocation and launch 12.0 with each look of its own, 7.5 this way; 0.7 where more rows go on
-    to torch's linear."""
-    if (type(x) not in _PLAIN or torch.compiler.is_compiling() or torch._C._is_tracing() or x.dim() != 2
-            or not 0 < x.size(0) <= ROWS_GEMM_MAX or not x.is_cuda or x.dtype is not torch.bfloat16 or type(w) not in _PLAIN
+    twice: us a call, 8 x 2048 x 2048: looks, allocation and launch 12.0 with each look of its own, 7.5 this way; half a microsecond where
+    more rows go on to torch's linear."""
+    if type(x) not in _PLAIN or _compiling() or _tracing():
+        return None
+    shape = x.shape
+    if (len(shape) != 2 or not 0 < shape[0] <= ROWS_GEMM_MAX or not x.is_cuda or x.dtype is not torch.bfloat16 or type(w) not in _PLAIN
             or w.dim() != 2 or w.dtype is not torch.bfloat16 or _transformed()):
         return None
-    (M, K), (N, k) = x.shape, w.shape
+    (M, K), (N, k) = shape, w.shape
     (ldx, one_x), (ldw, one_w) = x.stride(), w.stride()
     dev = x.get_device()
     if (k != K or K == 0 or K % 32 or N == 0 or not rows_gemm_pays(M, N, K) or one_x != 1 or one_w != 1 or ldx % 8 or ldw % 8
