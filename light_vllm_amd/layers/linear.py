@@ -17,11 +17,17 @@ from .. import mix_ops
 from . import tp
 from .tp import divide, tp_rank, tp_size
 
+_scripting, _compiling, _tracing, _Tensor = torch.jit.is_scripting, torch.compiler.is_compiling, torch._C._is_tracing, torch.Tensor
+_FEW = mix_ops.ROWS_GEMM_MAX
+
 
 def _linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
-    if not torch.jit.is_scripting():                    # (a script holds torch's operators only)
-        if bias is None:
-            return mix_ops.linear(x, weight)
+    if not _scripting():                                # (a script holds torch's operators only)
+        # mix_ops.linear's first looks, without a call: a prompt's step on few tokens is bound by the host, and goes on to torch's linear here
+        if bias is None and type(x) is _Tensor and not _compiling() and not _tracing():
+            shape = x.shape
+            if len(shape) == 2 and shape[0] <= _FEW:
+                return mix_ops.linear(x, weight)
     return F.linear(x, weight, bias)
 
 
