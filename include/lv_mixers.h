@@ -21,6 +21,7 @@
  *                            rotation of the shared positional key part, both written into the paged latent cache
  *   lv_latent_q_finish       joins the absorbed queries with their rotated positional part
  *   lv_latent_out_gate       per-head outputs [H, T, Dv] -> [T, H*Dv] times sigmoid(gate), gate per head or per channel
+ *   lv_latent_prompt_attn    what lies between lv_latent_prep and the output projection, in one launch, for prompt steps
  *   lv_moe_route             sigmoid router with a selection-only correction, group limit and top-k
  *   lv_router_logits         f32 router logits of steps of few tokens, straight from the activations
  *   lv_relu2_scale           squared relu of the experts' up projections times the routing weight
@@ -90,7 +91,7 @@
 extern "C" {
 #endif
 
-#define LV_MIX_ABI_VERSION 13
+#define LV_MIX_ABI_VERSION 14
 #define LV_MIX_BF16 0
 #define LV_MIX_F32 1
 #define LV_MIX_MAX_STREAMS 8
@@ -231,6 +232,16 @@ int lv_latent_q_finish(const void* q, const void* q_lat, const void* inv_freq, v
  * (LV_MIX_GATE_PER_HEAD) or H*Dv (LV_MIX_GATE_PER_CHANNEL). */
 int lv_latent_out_gate(const void* o, const void* gate, int64_t ld_gate, int gate_kind, void* out, int64_t T, int H,
                        int Dv, int dtype, void* stream);
+
+/* Latent attention of prompt steps, bf16: out act [T, H, Dn] = per head W_uv times the weighted sum over the cached rows that the query
+ * [W_uk q_n | rotated q_r] sees in a window, times sigmoid(gate).  q act [T, H, Dn + Dr], uk act [H, Dn, R], uv act [H, R, Dn], cache act
+ * [pages, page, R + Dr] (the new tokens' rows stored), gate rows as lv_latent_out_gate or NULL, sinks f32 [H] or NULL.  H in
+ * multiples of 4, Dn 64 or 128, R + Dr 192 + 64 (all 64 entries rotated, inv_freq f32 [32]) or 256 + 0, pages in multiples of 64; -2 for
+ * other head sizes.  q, cache, uk, uv aligned to 16 bytes, out and per-channel gates (rows in multiples of 4) to 8. */
+int lv_latent_prompt_attn(const void* q, const void* cache, const void* uk, const void* uv, const void* inv_freq, const void* gate,
+                          int64_t ld_gate, int gate_kind, void* out, const int32_t* cu_q, const int32_t* ctx_lens, const int32_t* block_tables,
+                          int bt_stride, int B, int max_new_tokens, int H, int Dn, int Dr, int R, int page, int window, float scale,
+                          const void* sinks, void* stream);
 
 /* Router of a mixture of experts. logits f32 [T, E]; scores s = sigmoid(logits); selection scores c = s + correction
  * (f32 [E], may be NULL). The experts are split into `groups` consecutive blocks of equal size; a block is ranked by its

@@ -57,6 +57,13 @@ struct WindowMfmaParams {
 
 enum ScoreForm { kPlain = 0, kCapped = 1, kExtended = 2 };
 
+// Latent attention with its two matrices in the attention kernel: q holds the heads' own queries, [T, H, Dn + Dr], and out their own
+// outputs, [T, H, Dn]; D = R + Dr and Dv = R stay those of the cached rows.
+struct LatentParams : WindowMfmaParams {
+  const uint16_t *uk, *uv;   // [H, Dn, R], [H, R, Dn]
+  const float* inv_freq;     // [Dr / 2]
+};
+
 constexpr int kTileQ = 16;
 constexpr int kTileK = 64;
 constexpr int kMaxK32 = 8;     // D <= 256: 32-wide steps over D (template K32: 2, 4 or 8)
@@ -447,8 +454,9 @@ __device__ __forceinline__ float half_max(float x) {
 // The 32 queries from row rw of sequence b, head h, key by key, each on the keys that it sees: for waves whose products met an
 // infinity or a NaN behind a mask. Lanes c and c + 32 hold query c and half of its entries each. It starts from the kernel's arguments
 // again so that nothing of it stays in registers through the kernel that ends with it.
-template <int DK, int DV, int FORM>
-__device__ __forceinline__ void prompt_redo(int b, int h, int rw) {
+// LATENT: the queries 16 pass .. 16 pass + 15 alone, whose rows lie in q_lds; their sums go to o_lds, rows of DV.
+template <int DK, int DV, int FORM, bool LATENT = false>
+__device__ __forceinline__ void prompt_redo(int b, int h, int rw, const bf16_t* q_lds = nullptr, bf16_t* o_lds = nullptr, int pass = 0) {
   typedef const __attribute__((address_space(4))) WindowMfmaParams* kernarg_t;
   kernarg_t pp = (kernarg_t)__builtin_amdgcn_kernarg_segment_ptr();
   int lane = threadIdx.x & 63;
@@ -464,7 +472,7 @@ __device__ __forceinline__ void prompt_redo(int b, int h, int rw) {
   const int early = p.P > 0 ? (p.chunk == 0 && w1 - p.window + 1 > 0 ? (w1 - p.window + 1) / p.P : 0) : min(p.keep_first, from);
   const float sink = p.sinks != nullptr ? p.sinks[h] : p.m0;
   constexpr int PARTS = DV > 128 ? DV / 64 : 1, ND = DV / 8 / PARTS;                      // wide rows in parts: registers
-  const bf16_t* q = reinterpret_cast<const bf16_t*>(p.q) + (t * p.H + h) * DK + 4 * half;
+  const bf16_t* q = (LATENT ? q_lds + (c & 15) * DK : reinterpret_cast<const bf16_t*>(p.q) + (t * p.H + h) * DK) + 4 * half;
 #pragma unroll 1
   for (int col = 0; col < DV; col += DV / PARTS) {
     float m = (sink < -1e30f ? -1e30f : sink) * kLog2e, l = p.sink, o[ND][4];
@@ -507,10 +515,10 @@ __device__ __forceinline__ void prompt_redo(int b, int h, int rw) {
         }
       }
     }
-    if (rw + c >= n) continue;
+    if (rw + c >= n || (LATENT && (c >> 4) != pass)) continue;
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    bf16_t* orow = reinterpret_cast<bf16_t*>(p.out) + t * p.out_ld + static_cast<int64_t>(h) * DV + col + 4 * half;
-    const bf16_t* grow = p.gate != nullptr ? reinterpret_cast<const bf16_t*>(p.gate) + t * p.ld_gate + static_cast<int64_t>(h) * p.gate_dv : nullptr;
+    bf16_t* orow = (LATENT ? o_lds + (c & 15) * DV : reinterpret_cast<bf16_t*>(p.out) + t * p.out_ld + static_cast<int64_t>(h) * DV) + col + 4 * half;
+    const bf16_t* grow = p.gate != nullptr && (!LATENT || p.gate_dv == 1) ? reinterpret_cast<const bf16_t*>(p.gate) + t * p.ld_gate + static_cast<int64_t>(h) * p.gate_dv : nullptr;
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
       float y[4];
@@ -522,8 +530,16 @@ __device__ __forceinline__ void prompt_redo(int b, int h, int rw) {
   }
 }
 
-template <int DK, int DV, bool SAME, int FORM>
-__global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(WindowMfmaParams p, int hpw, int tiles, int by_count) {
+// DN > 0, latent attention: a wave turns its 32 queries of DN entries into rows that meet the cached ones, rotates the DK - DV entries
+// behind them, and multiplies its sums by the head's value matrix before they leave, so that neither the DK entries a head that go in
+// nor the DV that come out pass through memory. 16 x 1024 tokens, 16 heads of 128 + 64 on rows of 192 + 64: 216 us, where this kernel took 177,
+// the two batched products around it 111 and the rotation's launch 27. A head's matrix comes in pieces of 8 KB through the wave's own part
+// of the two tiles, one piece on its way while the other is multiplied; all workgroups of a head run on one XCD (with 8 sequences times
+// head groups or a multiple), whose L2 holds it. A product's result rows are its matrix's columns in the order in which the next product
+// takes them, so that nothing is exchanged between lanes.
+template <int DK, int DV, bool SAME, int FORM, int DN = 0>
+__global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std::conditional_t<(DN > 0), LatentParams, WindowMfmaParams> p, int hpw,
+                                                                            int tiles, int by_count) {
   constexpr int KB = DK * 2, VB = SAME ? KB : DV * 2;                       // bytes of a staged row
   constexpr int KT = kTileK * KB, VT = SAME ? 0 : kTileK * VB;
   constexpr int KCH = DK / 8, VCH = DV / 8, KN = kTileK * KCH / 256, VN = SAME ? 0 : kTileK * VCH / 256;
@@ -532,6 +548,9 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(Wind
   constexpr float kLog2e = 1.44269504088896f;
   constexpr bool DMA = !FIRST;
   static_assert(!DMA || (SAME && KB == 512 && FORM == kPlain), "rows of 512 bytes, two of them a load instruction");
+  static_assert(DN == 0 || (DMA && (DK == DV || DK - DV == 64)), "own queries and outputs: latent rows, nothing or 64 entries rotated");
+  constexpr int DR = DN > 0 ? DK - DV : 0, QW = DN > 0 ? DN + DR : DK;      // entries of a query's head
+  __shared__ float turn_lds[DR > 0 ? 2 : 1][DR > 0 ? DR / 2 * kPromptQ : 1];                       // cosines, then sines: [frequency][query]
   __shared__ __attribute__((aligned(16))) unsigned char lds[DMA ? 16 : 2 * (KT + VT)];
   __shared__ __attribute__((aligned(1024))) unsigned char tile0[DMA ? KT : 16];
   __shared__ __attribute__((aligned(1024))) unsigned char tile1[DMA ? KT : 16];
@@ -560,7 +579,203 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(Wind
   const int64_t GD = static_cast<int64_t>(p.G) * DK, GDv = static_cast<int64_t>(p.G) * DV;
 
   bf16x8_t qf[NS];
-  {
+  lds_u8* const slot0 = (lds_u8*)tile0 + 8192 * wave;                       // the wave's own parts of the tiles
+  lds_u8* const slot1 = (lds_u8*)tile1 + 8192 * wave;
+  const int tq = (lane & 15) >> 2, tp = lane & 3, gi = lane >> 4;           // transposed reads: 16 lanes read 4 rows x 16 columns
+  auto landed = [&](auto later) __attribute__((always_inline)) {            // own pieces, but for the `later` youngest loads
+    constexpr int n = decltype(later)::value;
+    __builtin_amdgcn_s_waitcnt(n | 0x0f70);
+    asm volatile("" ::: "memory");
+  };
+  auto reads_done = [&]() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);                                     // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+  };
+  auto cast8 = [](const f32x16_t& x, int from) __attribute__((always_inline)) {
+    bf16x8_t y;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[i] = static_cast<__bf16>(x[from + i]);
+    return y;
+  };
+  // the lane's number, unknown to the compiler: what is made of it is not kept in registers from here to there
+  auto lane_here = [&]() __attribute__((always_inline)) {
+    int x = lane;
+    asm volatile("" : "+v"(x));
+    return x;
+  };
+  // rows of the key matrix, 16 a piece of 512-byte rows (of which a latent of 192 fills 384)
+  auto uk_piece = [&](int k, lds_u8* at, int ln) __attribute__((always_inline)) {
+    if constexpr (DN > 0) {
+      const char* from = reinterpret_cast<const char*>(p.uk + (static_cast<int64_t>(h) * DN + 16 * k) * DV);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r = 2 * i + (ln >> 5), ch = (ln & 31) ^ (((r & 3) << 2) | ((r >> 2) & 3));
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(from + static_cast<uint32_t>(r * 2 * DV + 16 * min(ch, DV / 8 - 1))),
+                                         (__attribute__((address_space(3))) void*)(at + 1024 * i), 16, 0, 0);
+      }
+    }
+  };
+  // qf = [q_n W_uk | rotated q_r]
+  auto absorb = [&](auto beside) __attribute__((always_inline)) {
+    if constexpr (DN > 0) {
+      constexpr int NP = DN / 16;
+      const int ln = lane_here(), half = ln >> 5, c = ln & 31, tq = (ln & 15) >> 2, tp = ln & 3, gi = ln >> 4;
+      uk_piece(0, slot0, ln);
+      uk_piece(1, slot1, ln);
+      const uint16_t* qrow = p.q + (static_cast<int64_t>(q0 + min(rw + c, n - 1)) * p.H + h) * QW + 8 * half;
+      bf16x8_t raw[NP];
+#pragma unroll
+      for (int k = 0; k < NP; ++k) raw[k] = *reinterpret_cast<const bf16x8_t*>(qrow + 16 * k);
+#pragma unroll
+      for (int x = 0; x < DR / 16; ++x) qf[DV / 16 + x] = *reinterpret_cast<const bf16x8_t*>(qrow + DN + 16 * x);
+      beside();
+#pragma unroll
+      for (int k = 0; k < NP; ++k) asm volatile("" ::"v"(raw[k]));
+      f32x16_t acc[ND];
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[d][i] = 0.0f;
+      // of 16 columns, fours 1 and 2 change places: a lane's results are then entries 8 half .. 8 half + 7 of two steps of K Q^T
+      int addr[2][ND < 4 ? ND : 4];
+#pragma unroll
+      for (int second = 0; second < 2; ++second)
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+          addr[second][d] = prompt_off<512>(8 * (gi >> 1) + 4 * second + tq, 4 * d + 2 * (gi & 1) + (tp & 1)) + 8 * (tp >> 1);
+      auto multiply = [&](int k, const lds_u8* at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+          const bf16x4v_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(at + addr[0][d % 4] + 256 * (d / 4)));
+          const bf16x4v_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(at + addr[1][d % 4] + 256 * (d / 4)));
+          acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), raw[k], acc[d], 0, 0, 0);
+          if (d % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+#pragma unroll
+      for (int k = 0; k < NP; k += 2) {
+        landed(std::integral_constant<int, 8>{});
+        multiply(k, slot0);
+        reads_done();
+        if (k + 2 < NP) {
+          uk_piece(k + 2, slot0, ln);
+          landed(std::integral_constant<int, 8>{});
+        } else {
+          landed(std::integral_constant<int, 0>{});
+        }
+        multiply(k + 1, slot1);
+        reads_done();
+        if (k + 3 < NP) uk_piece(k + 3, slot1, ln);
+      }
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        qf[2 * d] = cast8(acc[d], 0);
+        qf[2 * d + 1] = cast8(acc[d], 8);
+      }
+      if constexpr (DR > 0) {                                               // pairs (i, i + 32): a lane holds both
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          bf16x8_t &a = qf[DV / 16 + x], &z = qf[DV / 16 + 2 + x];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const int at = (16 * x + 8 * half + i) * kPromptQ + c;
+            const float co = turn_lds[0][at], si = turn_lds[1][at], u = static_cast<float>(a[i]), v = static_cast<float>(z[i]);
+            a[i] = static_cast<__bf16>(u * co - v * si);
+            z[i] = static_cast<__bf16>(v * co + u * si);
+          }
+        }
+      }
+    }
+  };
+  // the wave's outputs from its sums, which lie as the value matrix takes them; pass >= 0: those of 16 queries
+  auto leave = [&](const bf16x8_t* of, int pass) __attribute__((always_inline)) {
+    if constexpr (DN > 0) {
+      constexpr int UB = 2 * DN, UN = UB * 32 / 1024, NE = DN / 32;
+      const int ln = lane_here(), half = ln >> 5, c = ln & 31, tq = (ln & 15) >> 2, tp = ln & 3, gi = ln >> 4;
+      auto uv_piece = [&](int k, lds_u8* at) __attribute__((always_inline)) {      // 32 rows
+        const char* from = reinterpret_cast<const char*>(p.uv + (static_cast<int64_t>(h) * DV + 32 * k) * DN);
+#pragma unroll
+        for (int i = 0; i < UN; ++i) {
+          const int r = (1024 / UB) * i + ln / (UB / 16), pc = ln % (UB / 16);
+          const int ch = UB == 128 ? pc ^ ((((r >> 1) & 1) << 2) | ((r >> 2) & 3)) : pc ^ (((r & 3) << 2) | ((r >> 2) & 3));
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(from + static_cast<uint32_t>(r * UB + 16 * ch)),
+                                           (__attribute__((address_space(3))) void*)(at + 1024 * i), 16, 0, 0);
+        }
+      };
+      uv_piece(0, slot0);
+      uv_piece(1, slot1);
+      int addr[2][NE];
+#pragma unroll
+      for (int second = 0; second < 2; ++second)
+#pragma unroll
+        for (int e = 0; e < NE; ++e)
+          addr[second][e] = prompt_off<UB>(8 * second + 4 * (gi >> 1) + tq, 4 * e + 2 * (gi & 1) + (tp >> 1)) + 8 * (tp & 1);
+      f32x16_t y[NE];
+#pragma unroll
+      for (int e = 0; e < NE; ++e)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) y[e][i] = 0.0f;
+      auto multiply = [&](int k, const lds_u8* at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+#pragma unroll
+          for (int e = 0; e < NE; ++e) {
+            const bf16x4v_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(at + UB * 16 * x + addr[0][e]));
+            const bf16x4v_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(at + UB * 16 * x + addr[1][e]));
+            y[e] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), of[2 * k + x], y[e], 0, 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+#pragma unroll
+      for (int k = 0; k < ND; k += 2) {
+        landed(std::integral_constant<int, UN>{});
+        multiply(k, slot0);
+        reads_done();
+        if (k + 2 < ND) {
+          uv_piece(k + 2, slot0);
+          landed(std::integral_constant<int, UN>{});
+        } else {
+          landed(std::integral_constant<int, 0>{});
+        }
+        multiply(k + 1, slot1);
+        reads_done();
+        if (k + 3 < ND) uv_piece(k + 3, slot1);
+      }
+      if (rw + c >= n || (pass >= 0 && (c >> 4) != pass)) return;
+      const int64_t t = q0 + rw + c;
+      bf16_t* orow = reinterpret_cast<bf16_t*>(p.out) + t * p.out_ld + static_cast<int64_t>(h) * DN + 4 * half;
+      const bool gated = p.gate != nullptr && p.gate_dv != 1;
+      const bf16_t* grow = reinterpret_cast<const bf16_t*>(p.gate) + t * p.ld_gate + static_cast<int64_t>(h) * DN + 4 * half;
+#pragma unroll
+      for (int e = 0; e < NE; ++e)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          float4 v{y[e][4 * x], y[e][4 * x + 1], y[e][4 * x + 2], y[e][4 * x + 3]};
+          if (gated) {
+            const float4 gv = ld4(grow + 32 * e + 8 * x);
+            v = float4{v.x * sigmoidf_(gv.x), v.y * sigmoidf_(gv.y), v.z * sigmoidf_(gv.z), v.w * sigmoidf_(gv.w)};
+          }
+          st4(orow + 32 * e + 8 * x, v);
+        }
+    }
+  };
+  if constexpr (DN > 0) {
+    absorb([&]() __attribute__((always_inline)) {
+      if constexpr (DR > 0) {                                               // (the four waves have the same queries)
+#pragma unroll 1
+        for (int f = threadIdx.x >> 5; f < DR / 2; f += 8) {
+          float si, co;
+          sincosf(static_cast<float>(pos) * p.inv_freq[f], &si, &co);
+          turn_lds[0][f * kPromptQ + c] = co;
+          turn_lds[1][f * kPromptQ + c] = si;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      }
+    });
+    asm volatile("s_barrier" ::: "memory");                                 // the tiles are everyone's again
+  } else {
     const uint16_t* qrow = p.q + (t * p.H + h) * DK + 8 * half;
 #pragma unroll
     for (int s = 0; s < NS; ++s) qf[s] = *reinterpret_cast<const bf16x8_t*>(qrow + 16 * s);
@@ -630,8 +845,7 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(Wind
     }
   }
 
-  // LDS addresses inside a buffer: rows of K (lane = key), V transposed (16 lanes read 4 keys x 16 columns)
-  const int tq = (lane & 15) >> 2, tp = lane & 3, gi = lane >> 4;
+  // LDS addresses inside a buffer: rows of K (lane = key), V transposed
   // (chunks 16 further lie 256 bytes further: a turn touches the four lowest bits)
   constexpr int NKA = NS < 8 ? NS : 8, NVA = ND < 4 ? ND : 4;
   int kaddr[NKA], vaddr[2][NVA];
@@ -828,16 +1042,57 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(Wind
       }
     }
     if (__builtin_amdgcn_ballot_w64(bad) != 0) {
-      prompt_redo<DK, DV, FORM>(b, __builtin_amdgcn_readfirstlane(h), __builtin_amdgcn_readfirstlane(rw));
-      return;
+      if constexpr (DN == 0) {
+        prompt_redo<DK, DV, FORM>(b, __builtin_amdgcn_readfirstlane(h), __builtin_amdgcn_readfirstlane(rw));
+        return;
+      } else {
+        bf16_t *q_at = reinterpret_cast<bf16_t*>(tile0 + 8192 * wave), *o_at = reinterpret_cast<bf16_t*>(tile1 + 8192 * wave);
+#pragma unroll 1
+        for (int pass = 0; pass < 2; ++pass) {
+          absorb([] {});
+          if ((c >> 4) == pass) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) *reinterpret_cast<bf16x8_t*>(q_at + (c & 15) * DK + 16 * s + 8 * half) = qf[s];
+          }
+          reads_done();
+          prompt_redo<DK, DV, FORM, true>(b, __builtin_amdgcn_readfirstlane(h), __builtin_amdgcn_readfirstlane(rw), q_at, o_at, pass);
+          reads_done();
+          bf16x8_t of[2 * ND];
+#pragma unroll
+          for (int d = 0; d < 2 * ND; ++d) {
+            const uint2 lo = *reinterpret_cast<const uint2*>(o_at + (c & 15) * DV + 16 * d + 4 * half);
+            const uint2 hi = *reinterpret_cast<const uint2*>(o_at + (c & 15) * DV + 16 * d + 8 + 4 * half);
+            of[d] = __builtin_bit_cast(bf16x8_t, uint4{lo.x, lo.y, hi.x, hi.y});
+          }
+          reads_done();
+          leave(of, pass);
+        }
+        return;
+      }
     }
   }
   const float total = l + __shfl_xor(l, 32, kWave);
   const float inv = total > 0.0f ? 1.0f / total : 0.0f;
-  if (rw + c >= n) return;
+  if constexpr (DN == 0) {
+    if (rw + c >= n) return;
+  }
   uint16_t* orow = p.out + t * p.out_ld + static_cast<int64_t>(h) * DV + 4 * half;
   const uint16_t* grow = p.gate != nullptr ? p.gate + t * p.ld_gate + static_cast<int64_t>(h) * p.gate_dv : nullptr;
   const float gate1 = grow != nullptr && p.gate_dv == 1 ? sigmoidf_(ldf(reinterpret_cast<const bf16_t*>(grow))) : 1.0f;
+  if constexpr (DN > 0) {
+    bf16x8_t of[2 * ND];
+    const float f = inv * gate1;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[d][i] *= f;
+      of[2 * d] = cast8(o[d], 0);
+      of[2 * d + 1] = cast8(o[d], 8);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    leave(of, -1);
+    return;
+  }
 #pragma unroll
   for (int d = 0; d < ND; ++d)
 #pragma unroll
@@ -1005,4 +1260,39 @@ extern "C" int lv_masked_attn_mfma(const void* q, const void* k_cache, const voi
         static_cast<uint16_t*>(out), items, H, Dv, nsplit, out_ld, m0, static_cast<const float*>(sinks));
   }
   return launched("lv_window_pool_attn_mfma");
+}
+
+extern "C" int lv_latent_prompt_attn(const void* q, const void* cache, const void* uk, const void* uv, const void* inv_freq, const void* gate,
+                                     int64_t ld_gate, int gate_kind, void* out, const int32_t* cu_q, const int32_t* ctx_lens,
+                                     const int32_t* block_tables, int bt_stride, int B, int max_new_tokens, int H, int Dn, int Dr, int R,
+                                     int page, int window, float scale, const void* sinks, void* stream) {
+  if (B == 0 || max_new_tokens <= 0) return 0;
+  if (!q || !cache || !uk || !uv || !out || !cu_q || !ctx_lens || !block_tables || (Dr > 0 && !inv_freq))
+    return fail(-1, "lv_latent_prompt_attn: null pointer");
+  if (gate_kind != LV_MIX_GATE_PER_HEAD && gate_kind != LV_MIX_GATE_PER_CHANNEL) return fail(-1, "lv_latent_prompt_attn: gate kind %d", gate_kind);
+  const int gate_dv = gate_kind == LV_MIX_GATE_PER_HEAD ? 1 : Dn;
+  if (B < 0 || H <= 0 || H % 4 != 0 || page <= 0 || page % kTileK != 0 || window <= 0 || bt_stride <= 0 || !(scale > 0.0f) ||
+      (gate != nullptr && ld_gate < static_cast<int64_t>(H) * gate_dv))
+    return fail(-1, "lv_latent_prompt_attn: bad sizes");
+  if ((Dn != 64 && Dn != 128) || !((R == 192 && Dr == 64) || (R == 256 && Dr == 0)))
+    return fail(-2, "lv_latent_prompt_attn: heads of %d + %d on rows of %d", Dn, Dr, R);
+  auto off = [](const void* at, uintptr_t a) { return reinterpret_cast<uintptr_t>(at) % a != 0; };
+  if (off(q, 16) || off(cache, 16) || off(uk, 16) || off(uv, 16) || off(out, 8) || (gate != nullptr && gate_dv > 1 && (off(gate, 8) || ld_gate % 4 != 0)))
+    return fail(-1, "lv_latent_prompt_attn: alignment");
+  const int64_t row = R + Dr;
+  LatentParams p{{static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(cache), static_cast<const uint16_t*>(cache), nullptr, nullptr,
+                  static_cast<const uint16_t*>(gate), ld_gate, gate_dv, static_cast<uint16_t*>(out), cu_q, ctx_lens, block_tables, bt_stride, H, 1,
+                  static_cast<int>(row), R, page, window, 0, 0, H / 4, scale, sinks != nullptr ? 1.0f : 0.0f, magic(page), magic(1), magic(R / 8), 1,
+                  nullptr, row, row, -1e30f, 0, 0, static_cast<const float*>(sinks), 0.0f, 0.0f, nullptr, nullptr, 0,
+                  static_cast<int64_t>(H) * Dn},
+                 static_cast<const uint16_t*>(uk), static_cast<const uint16_t*>(uv), static_cast<const float*>(inv_freq)};
+  const int tiles = (max_new_tokens + kPromptQ - 1) / kPromptQ, by = B * (H / 4);
+  if (static_cast<int64_t>(tiles) * by >= (1ll << 31)) return fail(-2, "lv_latent_prompt_attn: %d sequences of %d tokens", B, max_new_tokens);
+  const dim3 grid(static_cast<unsigned>(tiles) * by), block(256);
+  hipStream_t s = as_stream(stream);
+  if (R == 192 && Dn == 128) prompt_attn_kernel<256, 192, true, kPlain, 128><<<grid, block, 0, s>>>(p, 4, tiles, by);
+  else if (R == 192) prompt_attn_kernel<256, 192, true, kPlain, 64><<<grid, block, 0, s>>>(p, 4, tiles, by);
+  else if (Dn == 128) prompt_attn_kernel<256, 256, true, kPlain, 128><<<grid, block, 0, s>>>(p, 4, tiles, by);
+  else prompt_attn_kernel<256, 256, true, kPlain, 64><<<grid, block, 0, s>>>(p, 4, tiles, by);
+  return launched("lv_latent_prompt_attn");
 }

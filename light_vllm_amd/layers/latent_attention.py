@@ -12,7 +12,8 @@ W_uv,h sum_j p_j c_j, so every head attends to the cached rows [c | k^r] themsel
 row, values: its first kv_rank entries) and the per-head matrices act on queries and outputs only,
 as two batched GEMMs. A decoded token therefore reads kv_rank + rot_dim numbers per cached token
 instead of heads * (dim + vdim), and one attention kernel serves prompts, portions and single tokens:
-the paged windowed kernel with one kv head, a window no sequence reaches, no pooled blocks and no sink.
+the paged windowed kernel with one kv head, a window no sequence reaches, no pooled blocks and no sink. Prompt steps of the usual head
+sizes do all of it, rotation, both matrices and gate, inside the attention launch (mix_ops.latent_prompt_attention).
 
 The output gate is one number per head (`gate="head"`), one per output channel (`gate="channel"`), or absent (None).
 Rotation: the first rot_dims entries of the rot_dim-wide positional part, entries i and i + rot_dims/2 (or, with `interleaved`, 2i
@@ -113,6 +114,11 @@ class LatentAttention(nn.Module):
             o = torch.bmm(self._attend(q_abs, step).view(T, H, R).transpose(0, 1), self.uv)         # [H, T, Dv]
             return self.o_proj(mix_ops.latent_out_gate(o, gate, self.gate_per_channel))
         with torch.no_grad():           # the kernels between them carry no gradient, and `out` may not ask for one
+            if self.Dv == Dn and mix_ops.latent_prompt_ok(q, self.cache, self.uk, self.uv, gate, step, H, Dn, Dr, R, self.rot_dims,
+                                                          self.gate_per_channel):
+                o = mix_ops.latent_prompt_attention(q, self.cache, self.uk, self.uv, self.inv_freq, gate, step, H, Dn, Dr, R, self.window,
+                                                    self.scale, self.gate_per_channel, self.sink)
+                return self.o_proj(o)
             # both batched products write where the next step reads; a gate per head goes on the sum that the value matrix
             # multiplies (the same product), in the attention kernel
             q_abs = torch.empty(T, H, R + Dr, dtype=h.dtype, device=h.device)

@@ -879,6 +879,34 @@ def latent_q_finish(q, q_lat, inv_freq, step, H, Dn, Dr, R, rot_dims, out=None):
     return out
 
 
+def latent_prompt_ok(q, cache, uk, uv, gate, step, H, Dn, Dr, R, rot_dims, gate_per_channel) -> bool:
+    """Whether latent_prompt_attention takes this step: prompts (more than 16 new tokens of some sequence: shorter steps have fewer
+    queries than a wave, and theirs are cut over the keys), bf16, and the head sizes and alignment that lv_latent_prompt_attn names."""
+    return (WINDOW_ATTN_KERNEL in ("auto", "prompt") and max(step.host_lens_q, default=0) > 16 and q.dtype == torch.bfloat16
+            and cache.dtype == uk.dtype == uv.dtype == q.dtype and H % 4 == 0 and Dn in (64, 128)
+            and uk.shape == (H, Dn, R) and uv.shape == (H, R, Dn) and (R, Dr, rot_dims) in ((192, 64, 64), (256, 0, 0))
+            and cache.size(1) % 64 == 0 and all(x.is_contiguous() and x.data_ptr() % 16 == 0 for x in (q, cache, uk, uv))
+            and gate.stride(1) == 1 and gate.dtype == q.dtype
+            and (not gate_per_channel or (gate.stride(0) % 4 == 0 and gate.data_ptr() % 8 == 0)))
+
+
+def latent_prompt_attention(q, cache, uk, uv, inv_freq, gate, step, H, Dn, Dr, R, window, scale, gate_per_channel, sinks=None):
+    """q act [T, H*(Dn+Dr)] -> act [T, H*Dn]: the absorbed queries, attention over the cached rows [pages, page, R+Dr], the value
+    matrices and the output gate in one launch (see latent_prompt_ok)."""
+    out = torch.empty(q.size(0), H * Dn, dtype=q.dtype, device=q.device)
+    _f32(inv_freq)
+    if sinks is not None:
+        _f32(sinks)
+        assert sinks.numel() == H
+    assert gate.shape == (q.size(0), H * Dn if gate_per_channel else H)
+    lib = _mixlib.load()
+    _mixlib.check(lib.lv_latent_prompt_attn(_p(q), _p(cache), _p(uk), _p(uv), _p(inv_freq), _p(gate), gate.stride(0), int(gate_per_channel),
+                                            _p(out), _p(step.cu_q), _p(step.ctx_lens), _p(step.block_tables), step.block_tables.stride(0),
+                                            len(step.host_lens_q), max(step.host_lens_q), H, Dn, Dr, R, cache.size(1), window, scale, _p(sinks),
+                                            _stream(q)), "lv_latent_prompt_attn")
+    return out
+
+
 def latent_out_gate(o, gate, per_channel: bool):
     """o [H, T, Dv] -> [T, H*Dv] times sigmoid(gate); gate [T, H] (one per head) or [T, H*Dv]."""
     H, T, Dv = o.shape
