@@ -15,8 +15,8 @@ matrices one [width, experts * ff] weight. Two forms compute the same sum:
   * gathered (bf16, width and ff in multiples of 32, at least GATHER_FROM experts per choice): the (token,
     choice) pairs are sorted by expert on the device and every expert multiplies only its own rows
     (mix_ops.moe_grouped_ff: sort, two grouped GEMMs on the matrix cores, weighted sum; four launches);
-  * sorted (bf16, eager steps from TILED_FROM to TILED_SURELY rows per expert on): the same sum with both products on LDS tiles of
-    128 or 256 rows (mix_ops.moe_sorted_ff). Weights whose layout those do not take go, from SORTED_FROM rows per expert,
+  * sorted (bf16, eager steps from TILED_FROM to TILED_SURELY rows per expert on): the same sum with both products on LDS tiles
+    (mix_ops.moe_sorted_ff). Weights whose layout those do not take go, from SORTED_FROM rows per expert,
     through vendor GEMMs on the sorted rows, after reading the experts' row counts back once. Steps captured into a
     hipGraph never take this form;
   * masked (f32, other sizes, few experts per choice): the up projection of every expert in one vendor

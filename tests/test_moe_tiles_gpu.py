@@ -73,8 +73,24 @@ def test_tiles_match_the_exact_sum(gpu, T, W, F, E, top, act, through):
     assert ((y.double() - ref).abs() <= 3.5 * 2.0 ** -9 * S + 1e-6).all()
 
 
+@pytest.mark.parametrize("T,W,F,E,top,act,uneven", [(70, 256, 256, 1, 1, "relu2", 0), (600, 384, 256, 3, 1, "relu2", 0.3), (1500, 256, 640, 6, 2, "gelu", 1.0),
+                                                    (2000, 2048, 512, 5, 4, "relu2", 1.0), (9000, 512, 1280, 3, 2, "gelu_tanh", 2.0),
+                                                    (24000, 256, 256, 7, 3, "relu2", 2.0)])
+def test_tiles_in_a_chain_match_the_exact_sum(gpu, T, W, F, E, top, act, uneven):
+    """k in whole pairs of steps: workgroups go from tile to tile. Experts of 0 to 256 rows past a whole tile, fewer tiles than
+    workgroups, a last round cut in two or four, and rounds that are whole."""
+    h, _, w, up, down = operands(T, W, F, E, top, 0, 1, T + E)
+    score = torch.rand(T, E, generator=torch.Generator().manual_seed(E)) + uneven * torch.linspace(0, 1, E)
+    ids = score.topk(top, 1).indices.int().contiguous().cuda()
+    for _ in range(2):                             # and the workgroups of a second launch behind those of the first
+        y = mix_ops.moe_sorted_ff(h, ids, w, up, down, E, F, act)
+    ref, S = exact(h, ids, w, up, down, E, F, act)
+    assert ((y.double() - ref).abs() <= 3.5 * 2.0 ** -9 * S + 1e-6).all()
+
+
 @pytest.mark.parametrize("T,W,F,E,top", [(1, 32, 32, 4, 2), (257, 96, 160, 1, 1), (700, 256, 288, 4, 2), (3000, 160, 96, 5, 3),
-                                           (4097, 2080, 96, 1, 1), (2500, 1568, 224, 4, 2), (1100, 96, 2080, 5, 3)])
+                                           (4097, 2080, 96, 1, 1), (2500, 1568, 224, 4, 2), (1100, 96, 2080, 5, 3),
+                                           (3000, 512, 384, 5, 3)])
 def test_gated_tiles_match_the_exact_sum(gpu, T, W, F, E, top):
     h, ids, w, up, down = operands(T, W, F, E, top, 0, 2, T)
     wide = torch.zeros(W, E * F + 64, dtype=torch.bfloat16, device=h.device)        # the experts' columns of a wider weight
