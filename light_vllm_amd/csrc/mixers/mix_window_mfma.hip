@@ -1,5 +1,6 @@
 // Matrix-core form of the windowed pooled attention for bf16 activations and caches.
 //
+// Steps of one token a sequence: decode_pool_kernel; prompts: prompt_attn_kernel; both below, for the usual head sizes. Here, for all others:
 // One workgroup = one tile of 16 consecutive new tokens of one sequence, one kv head, up to four of its
 // query heads (one per wave). Keys are walked in tiles of 64 entries, first the pooled blocks that any
 // query of the tile may see, then the tokens from the first window start to the last query; what a
@@ -381,17 +382,209 @@ __global__ __launch_bounds__(256, AHEAD ? 1 : (DVB > 8 ? 2 : (DVB > 4 ? 3 : 4)))
   }
 }
 
-// One wave per (token, query head): combines the splits' partials (each with its own running maximum), applies the gate.
+// One new token a sequence (decode steps), plain scores: up to 16 query heads of a kv head are the 16 columns of a product, so that a key
+// row is read once for all of them; the kernel above gives every head a wave of its own, with one query in sixteen columns, and every wave the
+// key rows. A wave walks tiles of 32 keys, the four waves of a workgroup and the splits share a sequence's tiles; waves meet in
+// LDS, splits in window_pool_merge_kernel. Nothing but a tile's tail is masked: the one query sees every entry of the list. The rows of the next
+// tile are requested as soon as the scores have used this one's registers. SAME: values are the first DV entries of the key rows and
+// go from the registers to LDS, where they are read transposed.
+// HBM-bound where there is enough to read, else a chain of loads: 48 sequences of 1100 tokens on average, 16 heads on latent rows of 192 + 64
+// 123 -> 11 us (27 MB), 16 heads over 4 of 128 in a window of 1024 with pooled blocks 63 -> 24; 64 of 4000, 32 over 8, window 2048: 545 MB in
+// 103 us; four of 1000 12.6 -> 5.9.
+template <int DK, int DV, bool SAME>
+__global__ __launch_bounds__(256, 2) void decode_pool_kernel(WindowMfmaParams p) {
+  constexpr int KT = 32, NK = DK / 32, ND = DV / 16, LDV = v_row(DV), VN = SAME ? 1 : DV / 16;
+  constexpr int IMAGE = KT * LDV * 2, PART = 16 * (DV + 4) * 4;
+  constexpr int OWN = IMAGE > PART ? IMAGE : PART;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * OWN];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, ln = lane & 15, lg = lane >> 4;
+  const int b = blockIdx.z, g = blockIdx.y / p.ngroups, hg = blockIdx.y % p.ngroups, split = blockIdx.x;
+  const int64_t t = p.cu_q[b];
+  if (p.cu_q[b + 1] - static_cast<int>(t) <= 0) return;
+  const int pos = p.ctx_lens[b], rep = p.H / p.G, P = p.P, page = p.page, chunk = p.chunk;
+  const int h = g * rep + min(hg * 16 + ln, rep - 1);
+  const int32_t* bt = p.block_tables + static_cast<int64_t>(b) * p.bt_stride;
+  // the entries: pooled blocks or kept first tokens, then the window's or the chunk's tokens
+  const int jlo = chunk > 0 ? pos / chunk * chunk : max(0, pos - p.window + 1);
+  const int first = P > 0 ? (chunk == 0 && pos - p.window + 1 > 0 ? (pos - p.window + 1) / P : 0) : min(p.keep_first, jlo);
+  const int npt = (first + KT - 1) / KT, ntiles = npt + (pos + 1 - jlo + KT - 1) / KT;
+  const int per = (ntiles + p.nsplit - 1) / p.nsplit, end = min(ntiles, (split + 1) * per);
+
+  bf16x8_t qf[NK];
+#pragma unroll
+  for (int kk = 0; kk < NK; ++kk) qf[kk] = *reinterpret_cast<const bf16x8_t*>(p.q + (t * p.H + h) * DK + 32 * kk + 8 * lg);
+  f32x4_t o[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d) o[d] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  float m = fmaxf(p.sinks != nullptr ? p.sinks[h] : p.m0, -1e30f), l = split == 0 && wave == 0 ? p.sink : 0.0f;
+
+  auto slot_of = [&](int tile) __attribute__((always_inline)) {             // cache row of entry `lane & 31`; past the end the last one's
+    if (tile < npt) {
+      const int e = min(tile * KT + (lane & 31), first - 1);
+      if (P > 0) {
+        const int pj = fdiv(e * P + P - 1, page, p.m_page);
+        return bt[pj] * p.PP + (e - fdiv(page * pj, P, p.m_P));
+      }
+      const int pj = fdiv(e, page, p.m_page);
+      return bt[pj] * page + (e - pj * page);
+    }
+    const int e = min(jlo + (tile - npt) * KT + (lane & 31), pos), pj = fdiv(e, page, p.m_page);
+    return bt[pj] * page + (e - pj * page);
+  };
+  const int64_t GD = static_cast<int64_t>(p.G) * DK, GDv = static_cast<int64_t>(p.G) * DV;
+  bf16x8_t kf[2][NK];
+  u32x4_t vf[VN];
+  auto request_k = [&](int tile, int slot) __attribute__((always_inline)) {
+    const bool pooled = tile < npt && P > 0;
+    const uint16_t* base = (pooled ? p.kp : p.k_cache) + g * DK + 8 * lg;
+    const int64_t ld = pooled ? GD : p.k_ld;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      const uint16_t* row = base + __shfl(slot, 16 * kb + ln, kWave) * ld;
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk) kf[kb][kk] = *reinterpret_cast<const bf16x8_t*>(row + 32 * kk);
+    }
+  };
+  auto request_v = [&](int tile, int slot) __attribute__((always_inline)) {
+    if constexpr (!SAME) {
+      const bool pooled = tile < npt && P > 0;
+      const uint16_t* base = (pooled ? p.vp : p.v_cache) + g * DV + 8 * (lane % (DV / 8));
+      const int64_t ld = pooled ? GDv : p.v_ld;
+#pragma unroll
+      for (int x = 0; x < VN; ++x)
+        vf[x] = *reinterpret_cast<const u32x4_t*>(base + __shfl(slot, (512 / DV) * x + lane / (DV / 8), kWave) * ld);
+    }
+  };
+  uint16_t* image = reinterpret_cast<uint16_t*>(lds + wave * OWN);
+  const lds_bf16* vt = (const lds_bf16*)image + (4 * lg + (ln >> 2)) * LDV + 4 * (ln & 3);
+  int tile = split * per + wave, slot = 0;
+  if (tile < end) {
+    slot = slot_of(tile);
+    request_k(tile, slot);
+    request_v(tile, slot);
+    if (tile + 4 < end) slot = slot_of(tile + 4);
+  }
+  for (; tile < end; tile += 4) {
+    f32x4_t s[2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      s[kb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk) s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[kb][kk], qf[kk], s[kb], 0, 0, 0);
+    }
+    if constexpr (SAME) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int kk = 0; kk < DV / 32; ++kk)
+          *reinterpret_cast<bf16x8_t*>(image + (16 * kb + ln) * LDV + 32 * kk + 8 * lg) = kf[kb][kk];
+    } else {
+#pragma unroll
+      for (int x = 0; x < VN; ++x)
+        *reinterpret_cast<u32x4_t*>(image + ((512 / DV) * x + lane / (DV / 8)) * LDV + 8 * (lane % (DV / 8))) = vf[x];
+    }
+    const int e0 = tile < npt ? tile * KT : jlo + (tile - npt) * KT, e_end = tile < npt ? first : pos + 1;
+    if (tile + 4 < end) {
+      request_k(tile + 4, slot);
+      request_v(tile + 4, slot);
+      if (tile + 8 < end) slot = slot_of(tile + 8);
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[kb][i] = e0 + 16 * kb + 4 * lg + i < e_end ? s[kb][i] * p.scale : -INFINITY;
+        mx = fmaxf(mx, s[kb][i]);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+    const float nm = fmaxf(m, mx), corr = __expf(m - nm);
+    float rs = 0.0f;
+    bf16x8_t pb;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float e = __expf(s[kb][i] - nm);                              // exp(-inf) = 0 for what is not there
+        rs += e;
+        pb[4 * kb + i] = static_cast<__bf16>(e);
+      }
+    rs += __shfl_xor(rs, 16, kWave);
+    rs += __shfl_xor(rs, 32, kWave);
+    l = l * corr + rs;
+    m = nm;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      const bf16x4v_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(vt + 16 * d));
+      const bf16x4v_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(vt + 16 * d + 16 * LDV));
+      o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), pb, o[d] * corr, 0, 0, 0);
+    }
+  }
+  // the waves' sums, [16 heads][DV | maximum, sum], each over its own image
+  float* part = reinterpret_cast<float*>(lds + wave * OWN) + ln * (DV + 4);
+#pragma unroll
+  for (int d = 0; d < ND; ++d) *reinterpret_cast<f32x4_t*>(part + 16 * d + 4 * lg) = o[d];
+  if (lg == 0) {
+    part[DV] = m;
+    part[DV + 1] = l;
+  }
+  __syncthreads();
+  const int heads = min(16, rep - hg * 16);
+  for (int x = threadIdx.x; x < heads * (DV / 4); x += 256) {
+    const int hh = x / (DV / 4), dv = x % (DV / 4) * 4, head = g * rep + hg * 16 + hh;
+    const float* from = reinterpret_cast<const float*>(lds) + hh * (DV + 4);
+    float M = -INFINITY, L = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) M = fmaxf(M, from[w * (OWN / 4) + DV]);
+    f32x4_t y{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float f = __expf(from[w * (OWN / 4) + DV] - M);
+      L += f * from[w * (OWN / 4) + DV + 1];
+      y += f * *reinterpret_cast<const f32x4_t*>(from + w * (OWN / 4) + dv);
+    }
+    if (p.nsplit > 1) {                                                     // unnormalised partials
+      float* to = p.ws + ((t * p.H + head) * p.nsplit + split) * (DV + 4);
+      *reinterpret_cast<f32x4_t*>(to + dv) = y;
+      if (dv == 0) {
+        to[DV] = M;
+        to[DV + 1] = L;
+      }
+      continue;
+    }
+    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    uint16_t* orow = p.out + t * p.out_ld + static_cast<int64_t>(head) * DV + dv;
+    const uint16_t* grow = p.gate != nullptr ? p.gate + t * p.ld_gate + static_cast<int64_t>(head) * p.gate_dv : nullptr;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float v = y[i] * inv;
+      if (grow != nullptr) v *= sigmoidf_(__builtin_bit_cast(float, static_cast<uint32_t>(grow[p.gate_dv > 1 ? dv + i : 0]) << 16));
+      orow[i] = static_cast<uint16_t>(bf16_bits(v));
+    }
+  }
+}
+
+// One wave per (token, query head), or four of them: combines the splits' partials (each with its own running maximum), applies the gate. Four
+// entries a lane, eight splits of a wave on their way at once, the first beside the maxima. Partials come from other XCDs' launches, some 4 us
+// for a round of loads: 32 splits of 16 heads of 192 took 17 us a split after the other, 4.4 with four waves' rounds at once.
+template <int WAVES>
 __global__ __launch_bounds__(256) void window_pool_merge_kernel(const float* __restrict__ ws, const uint16_t* __restrict__ gate,
                                                                 int64_t ld_gate, int gate_dv, uint16_t* __restrict__ out,
                                                                 int64_t items, int H, int Dv, int nsplit, int64_t out_ld, float m0,
                                                                 const float* __restrict__ sinks) {
+  constexpr int AHEAD = 8;
+  __shared__ f32x4_t sums[WAVES > 1 ? WAVES : 1][WAVES > 1 ? kWave : 1];
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int64_t item = static_cast<int64_t>(blockIdx.x) * (blockDim.x / kWave) + wave;
+  const int64_t item = static_cast<int64_t>(blockIdx.x) * (4 / WAVES) + wave / WAVES;
   if (item >= items) return;
   const int64_t t = item / H;
-  const int h = static_cast<int>(item - t * H);
+  const int h = static_cast<int>(item - t * H), own = wave % WAVES;
   const float* w = ws + item * nsplit * (Dv + 4);
+  const int dv = 4 * lane, at = min(dv, Dv - 4);
+  f32x4_t y[AHEAD];
+#pragma unroll
+  for (int s = 0; s < AHEAD; ++s) y[s] = *reinterpret_cast<const f32x4_t*>(w + min(own + WAVES * s, nsplit - 1) * (Dv + 4) + at);
   // lane s holds split s (at most kWave of them): its maximum and sum, then the factor that brings it to the common maximum
   const float m0h = sinks != nullptr ? sinks[h] : m0;
   const bool in = lane < nsplit;
@@ -400,18 +593,33 @@ __global__ __launch_bounds__(256) void window_pool_merge_kernel(const float* __r
   const float f = in ? expf(ms - mm) : 0.0f;
   const float ll = wave_sum(ls * f);
   const float inv = ll > 0.0f ? 1.0f / ll : 0.0f;
-  for (int dv0 = 0; dv0 < Dv; dv0 += kWave) {                               // the same trip count for every lane: the factors are shuffled
-    const int dv = dv0 + lane;
-    const float* col = w + min(dv, Dv - 1);
-    float acc = 0.0f;
-#pragma unroll 4
-    for (int s = 0; s < nsplit; ++s) acc += col[s * (Dv + 4)] * __shfl(f, s, kWave);
-    float val = acc * inv;
-    if (dv >= Dv) continue;
+  f32x4_t acc{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s0 = own;; ) {
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s) {
+      const float fs = __shfl(f, min(s0 + WAVES * s, kWave - 1), kWave);
+      if (s0 + WAVES * s < nsplit) acc += fs * y[s];
+    }
+    s0 += WAVES * AHEAD;
+    if (s0 >= nsplit) break;
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s) y[s] = *reinterpret_cast<const f32x4_t*>(w + min(s0 + WAVES * s, nsplit - 1) * (Dv + 4) + at);
+  }
+  if constexpr (WAVES > 1) {
+    sums[own][lane] = acc;
+    __syncthreads();
+    if (own > 0) return;
+#pragma unroll
+    for (int i = 1; i < WAVES; ++i) acc += sums[i][lane];
+  }
+  if (dv >= Dv) return;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float val = acc[i] * inv;
     if (gate != nullptr)
       val *= sigmoidf_(__builtin_bit_cast(float, static_cast<uint32_t>(gate[t * ld_gate + static_cast<int64_t>(h) * gate_dv +
-                                                                            (gate_dv > 1 ? dv : 0)]) << 16));
-    out[t * out_ld + static_cast<int64_t>(h) * Dv + dv] = static_cast<uint16_t>(bf16_bits(val));
+                                                                            (gate_dv > 1 ? dv + i : 0)]) << 16));
+    out[t * out_ld + static_cast<int64_t>(h) * Dv + dv + i] = static_cast<uint16_t>(bf16_bits(val));
   }
 }
 
@@ -1167,6 +1375,23 @@ static bool prompt_launch(const WindowMfmaParams& p, int form, int64_t T, int B,
   return false;
 }
 
+// The head sizes that decode_pool_kernel is built for; false: the launch belongs to window_pool_mfma_kernel. Rows of q, caches and workspace
+// are read 16 bytes at a time.
+static bool decode_launch(const WindowMfmaParams& p, int form, int B, hipStream_t s) {
+  auto at = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
+  if (form != kPlain || !at(p.q) || !at(p.ws) || (p.P > 0 && (!at(p.kp) || !at(p.vp)))) return false;
+  const bool same = p.P == 0 && (p.G == 1 || p.D == p.Dv) && p.k_cache == p.v_cache && p.k_ld == p.v_ld;
+  WindowMfmaParams q = p;
+  q.ngroups = (p.H / p.G + 15) / 16;
+  const dim3 grid(p.nsplit, p.G * q.ngroups, B), block(256);
+  if (p.D == 64 && p.Dv == 64 && !same) decode_pool_kernel<64, 64, false><<<grid, block, 0, s>>>(q);
+  else if (p.D == 128 && p.Dv == 128 && !same) decode_pool_kernel<128, 128, false><<<grid, block, 0, s>>>(q);
+  else if (p.D == 256 && p.Dv == 192 && same) decode_pool_kernel<256, 192, true><<<grid, block, 0, s>>>(q);
+  else if (p.D == 256 && p.Dv == 256 && same) decode_pool_kernel<256, 256, true><<<grid, block, 0, s>>>(q);
+  else return false;
+  return true;
+}
+
 }  // namespace lvmix
 
 using namespace lvmix;
@@ -1233,6 +1458,21 @@ extern "C" int lv_masked_attn_mfma(const void* q, const void* k_cache, const voi
   hipStream_t st = as_stream(stream);
   if (nsplit <= 1 && prompt_launch(p, softcap > 0.0f ? kCapped : (extended ? kExtended : kPlain), T, B, max_new_tokens, nsplit < 0, st))
     return launched("lv_masked_attn_mfma");
+  auto merge = [&]() {
+    const int64_t items = T * H;
+    auto launch = [&](auto waves) {
+      constexpr int W = decltype(waves)::value;
+      window_pool_merge_kernel<W><<<dim3(static_cast<unsigned>((items * W + 3) / 4)), dim3(256), 0, st>>>(
+          static_cast<const float*>(workspace), static_cast<const uint16_t*>(gate), ld_gate, gate_dv, static_cast<uint16_t*>(out), items, H, Dv,
+          nsplit, out_ld, m0, static_cast<const float*>(sinks));
+    };
+    if (nsplit > 8) launch(std::integral_constant<int, 4>{});
+    else launch(std::integral_constant<int, 1>{});
+  };
+  if (max_new_tokens == 1 && nsplit >= 0 && decode_launch(p, softcap > 0.0f ? kCapped : (extended ? kExtended : kPlain), B, st)) {
+    if (nsplit > 1) merge();
+    return launched("lv_masked_attn_mfma");
+  }
   size_t shm = static_cast<size_t>(kTileK) * v_row(Dv) * sizeof(uint16_t);
   if (extended) shm += sizeof(float) * (kTileK + (p.dist_bias != nullptr && p.bias_len <= kBiasLds ? 4 * static_cast<size_t>(p.bias_len) : 0));
   dim3 grid(nsplit > 1 ? nsplit : (max_new_tokens + kTileQ - 1) / kTileQ, G * ngroups, B), block(256);
@@ -1253,12 +1493,7 @@ extern "C" int lv_masked_attn_mfma(const void* q, const void* k_cache, const voi
   else LVMIX_ATT(false);
 #undef LVMIX_ATT
 #undef LVMIX_ATT_FORM
-  if (nsplit > 1) {
-    const int64_t items = T * H;
-    window_pool_merge_kernel<<<dim3(static_cast<unsigned>((items + 3) / 4)), block, 0, st>>>(
-        static_cast<const float*>(workspace), static_cast<const uint16_t*>(gate), ld_gate, gate_dv,
-        static_cast<uint16_t*>(out), items, H, Dv, nsplit, out_ld, m0, static_cast<const float*>(sinks));
-  }
+  if (nsplit > 1) merge();
   return launched("lv_window_pool_attn_mfma");
 }
 

@@ -565,7 +565,11 @@ def window_pool_attention(q, k_cache, v_cache, kp, vp, gate, step, H, G, D, Dv, 
                 most = max(c + n for c, n in zip(step.host_ctx_lens, step.host_lens_q))
                 span = min(most, chunk + 16) if chunk > 0 else min(most, window + 16 + keep_first)
                 tiles = -(-span // 64) + (-(-(max(most - window, 0) // P) // 64) if P > 0 else 0)
-                nsplit = max(1, min(tiles, SPLIT_WORKGROUPS // max(B * G * -(-(H // G) // 4), 1), 32))      # one workgroup a CU: more splits cost more in the merge than they gain (measured)
+                if (max(step.host_lens_q) <= 1 and softcap == 0.0 and key_scale is None and dist_bias is None
+                        and (D, Dv) in ((64, 64), (128, 128), (256, 192), (256, 256))):     # sixteen heads and 128 keys a workgroup
+                    nsplit = max(1, min(tiles // 2, SPLIT_WORKGROUPS // max(B * G * -(-(H // G) // 16), 1), 32))
+                else:
+                    nsplit = max(1, min(tiles, SPLIT_WORKGROUPS // max(B * G * -(-(H // G) // 4), 1), 32))      # one workgroup a CU: more splits cost more in the merge than they gain (measured)
                 if nsplit > 1:
                     ws = torch.empty(T * H * nsplit * (Dv + 4), dtype=torch.float32, device=q.device)
             _mixlib.check(lib.lv_masked_attn_mfma(_p(q), _p(k_cache), _p(v_cache), _p(kp), _p(vp), _p(gate),

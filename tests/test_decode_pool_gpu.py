@@ -1,0 +1,68 @@
+"""Windowed and latent attention of steps of one token a sequence (decode_pool_kernel, and the merge of its splits) against the vector kernel
+(f32 products of the same bf16 rows): tails of tiles, windows and chunks, pooled blocks, kept tokens, sinks, gates, head groups, empty
+splits and sequences without a new token."""
+import pytest
+import torch
+
+from light_vllm_amd import mix_ops
+from tests._ragged import ragged_step
+
+pytestmark = pytest.mark.gpu
+# probabilities and outputs are rounded to bf16 (2^-9 each); an output is an average of values of magnitude 1 to 4
+ATOL = 4 * 2.0 ** -8
+REL = 3.0 ** 0.5 * 2.0 ** -9          # rounded probabilities and both kernels' rounded outputs, independent
+
+SHAPES = [(4, 4, 64, 64, False), (16, 4, 128, 128, False), (6, 2, 128, 128, False), (40, 2, 64, 64, False), (16, 1, 256, 192, True),
+          (20, 1, 256, 256, True), (32, 1, 256, 192, True)]
+
+
+def both(monkeypatch, ctx, H, G, D, Dv, same, page=64, pool=0, gate=None, new=None, workgroups=256, out_pad=0, seed=0, **kw):
+    step, pages = ragged_step(new or [1] * len(ctx), ctx, page, "cuda", seed)
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    T = len(step.tok_seq)
+
+    def rn(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen).bfloat16()
+
+    q, kc = rn(T, H * D), rn(pages, page, G, D)
+    vc = kc[..., :Dv] if same else rn(pages, page, G, Dv)
+    pp = max(mix_ops.pooled_slots(page, pool), 1)
+    kp, vp = (rn(pages, pp, G, D), rn(pages, pp, G, Dv)) if pool else (None, None)
+    g = None if gate is None else rn(T, H if gate == "head" else H * Dv)
+    monkeypatch.setattr(mix_ops, "SPLIT_WORKGROUPS", workgroups)
+    got = []
+    for kernel in ("valu", "auto"):
+        monkeypatch.setattr(mix_ops, "WINDOW_ATTN_KERNEL", kernel)
+        wide = torch.full((T, H * Dv + out_pad), 7.0, device="cuda", dtype=torch.bfloat16)
+        mix_ops.window_pool_attention(q, kc, vc, kp, vp, g, step, H, G, D, Dv, kw.get("window", 1 << 30), pool, D ** -0.5,
+                                      gate_per_head=gate == "head", out=wide[:, :H * Dv], **{k: v for k, v in kw.items() if k != "window"})
+        assert bool((wide[:, H * Dv:] == 7.0).all())
+        got.append(wide[:, :H * Dv].float())
+    assert bool(torch.isfinite(got[1]).all())
+    assert (got[0] - got[1]).abs().max().item() <= ATOL
+    assert (got[0] - got[1]).norm().item() <= REL * got[0].norm().item()
+
+
+@pytest.mark.parametrize("H,G,D,Dv,same", SHAPES)
+@pytest.mark.parametrize("workgroups", [1, 64, 4096])
+def test_lengths_and_splits(monkeypatch, H, G, D, Dv, same, workgroups):
+    both(monkeypatch, [0, 30, 31, 32, 126, 127, 128, 700, 1, 2100], H, G, D, Dv, same, has_sink=False, workgroups=workgroups, seed=H)
+
+
+@pytest.mark.parametrize("H,G,D,Dv,same", SHAPES)
+@pytest.mark.parametrize("kw", [dict(window=70, has_sink=True), dict(window=33, keep_first=5, has_sink=False), dict(chunk=100, has_sink=False),
+                                dict(window=1, has_sink=False), dict(sinks=True)])
+def test_windows_chunks_and_sinks(monkeypatch, H, G, D, Dv, same, kw):
+    if kw.get("sinks"):
+        kw = dict(kw, sinks=torch.linspace(-2, 3, H, device="cuda"))
+    both(monkeypatch, [0, 69, 70, 99, 100, 355, 1023], H, G, D, Dv, same, gate="head", workgroups=200, seed=G, **{"has_sink": True, **kw})
+
+
+@pytest.mark.parametrize("pool,window", [(16, 40), (64, 128), (32, 1)])
+def test_pooled_blocks_and_gates(monkeypatch, pool, window):
+    for H, G, D in ((16, 4, 128), (8, 8, 64)):
+        both(monkeypatch, [5, 40, 64, 500, 1500, 127], H, G, D, D, False, page=128, pool=pool, window=window, gate="channel", out_pad=8, seed=pool)
+
+
+def test_sequences_without_a_new_token(monkeypatch):
+    both(monkeypatch, [100, 300, 7], 16, 1, 256, 192, True, new=[1, 0, 1], has_sink=False)
