@@ -10,8 +10,8 @@
 //                           rotation of the positional key part, both written into the token's cache row.
 //   latent_q_finish_kernel  one workgroup per token: [absorbed query | rotated positional query part] per head.
 //   latent_out_gate_kernel  elementwise: head-major outputs to token-major rows times sigmoid(gate).
-//   moe_route_kernel        one wave per token: sigmoid scores, correction for the choice only, group limit, top-k,
-//                           normalised (or raw) weights; the wave keeps its scores in LDS and picks maxima by shuffles.
+//   moe_route_kernel        16, 32 or 64 lanes per token: sigmoid scores, correction for the choice only, group limit, top-k,
+//                           normalised (or raw) weights; scores in LDS, maxima by shuffles.
 //   router_logits_kernel    steps of few tokens: the f32 router logits straight from the activations, one workgroup per
 //                           (token, four experts).
 //   relu2_scale_kernel      elementwise: relu(x)^2 times the token's weight for the expert the column belongs to.
@@ -241,10 +241,11 @@ __global__ __launch_bounds__(256) void latent_out_gate_kernel(const T* __restric
 }
 
 // ------------------------------------------------------------------------------------------------
-// (value, index) maximum over the wave: larger value wins, the lower index on equal values.
+// (value, index) maximum over L lanes: larger value wins, the lower index on equal values.
 // Lanes of sixteen meet by permutations of the vector ALU; only the last two steps go through the LDS unit (16384 tokens of 32 experts, 4
 // choices: 23.9 us with all six there, 22.1 this way).
-__device__ __forceinline__ void wave_argmax(float& v, int& i) {
+template <int L>
+__device__ __forceinline__ void lanes_argmax(float& v, int& i) {
   auto meet = [&](float ov, int oi) {
     if (ov > v || (ov == v && oi < i)) {
       v = ov;
@@ -261,7 +262,7 @@ __device__ __forceinline__ void wave_argmax(float& v, int& i) {
   step(std::integral_constant<int, 0x141>{});          // mirrored within eight
   step(std::integral_constant<int, 0x140>{});          // mirrored within sixteen
 #pragma unroll
-  for (int o = 16; o <= 32; o <<= 1) {
+  for (int o = 16; o < L; o <<= 1) {
     const float ov = __shfl_xor(v, o, kWave);
     const int oi = __shfl_xor(i, o, kWave);
     meet(ov, oi);
@@ -270,18 +271,20 @@ __device__ __forceinline__ void wave_argmax(float& v, int& i) {
 
 // One wave a token, four of them a workgroup: a compute unit holds sixteen workgroups, and sixteen waves are too few to hide a chain of
 // shuffles behind. 16384 tokens of 32 experts, 4 choices, us: one wave a workgroup 22.1, four 21.3.
+// L lanes a token, as many as hold its experts, choices and groups: with 32 experts two tokens share a wave's chain of shuffles, 20.3 -> 13.1.
 constexpr int kRouteWaves = 4;
+template <int L>
 __global__ __launch_bounds__(kRouteWaves * kWave) void moe_route_kernel(const float* __restrict__ logits, const float* __restrict__ correction,
                                                         int32_t* __restrict__ ids, float* __restrict__ weights,
                                                         float* __restrict__ dense, int64_t T, int E, int top, int groups, int keep,
                                                         int normalize, int score_kind, int group_rank) {
   extern __shared__ float route_lds[];
-  float* rl = route_lds + threadIdx.x / kWave * (2 * E + (groups > 1 ? groups : 1));       // the wave's own
+  float* rl = route_lds + threadIdx.x / L * (2 * E + (groups > 1 ? groups : 1));           // the token's own
   float* s_lds = rl;              // [E] scores
   float* c_lds = rl + E;          // [E] selection scores, -inf once out of the running
   float* g_lds = rl + 2 * E;      // [groups] group scores
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * (blockDim.x / kWave) + threadIdx.x / kWave;
-  const int lane = threadIdx.x % kWave;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * (blockDim.x / L) + threadIdx.x / L;
+  const int lane = threadIdx.x % L;
   if (t >= T) return;
   // a wave's LDS operations are carried out in order: only the compiler has to keep them so
   auto in_order = []() __attribute__((always_inline)) {
@@ -290,13 +293,16 @@ __global__ __launch_bounds__(kRouteWaves * kWave) void moe_route_kernel(const fl
   };
   float smax = -INFINITY, sden = 1.0f;
   if (score_kind == LV_MIX_SCORE_SOFTMAX) {            // over all experts of the row
-    for (int e = lane; e < E; e += kWave) smax = fmaxf(smax, logits[t * E + e]);
-    smax = wave_max(smax);
+    for (int e = lane; e < E; e += L) smax = fmaxf(smax, logits[t * E + e]);
+#pragma unroll
+    for (int o = L / 2; o > 0; o >>= 1) smax = fmaxf(smax, __shfl_xor(smax, o, kWave));
     float part = 0.0f;
-    for (int e = lane; e < E; e += kWave) part += expf(logits[t * E + e] - smax);
-    sden = wave_sum(part);
+    for (int e = lane; e < E; e += L) part += expf(logits[t * E + e] - smax);
+#pragma unroll
+    for (int o = L / 2; o > 0; o >>= 1) part += __shfl_xor(part, o, kWave);
+    sden = part;
   }
-  for (int e = lane; e < E; e += kWave) {
+  for (int e = lane; e < E; e += L) {
     const float s = score_kind == LV_MIX_SCORE_SOFTMAX ? expf(logits[t * E + e] - smax) / sden : sigmoidf_(logits[t * E + e]);
     s_lds[e] = s;
     c_lds[e] = s + (correction != nullptr ? correction[e] : 0.0f);
@@ -305,7 +311,7 @@ __global__ __launch_bounds__(kRouteWaves * kWave) void moe_route_kernel(const fl
   in_order();
   if (groups > 1 && keep < groups) {
     const int gs = E / groups;
-    for (int g = lane; g < groups; g += kWave) {
+    for (int g = lane; g < groups; g += L) {
       float a = -INFINITY, b2 = -INFINITY;          // the two highest
       for (int e = g * gs; e < (g + 1) * gs; ++e) {
         const float c = c_lds[e];
@@ -319,15 +325,15 @@ __global__ __launch_bounds__(kRouteWaves * kWave) void moe_route_kernel(const fl
     for (int r = 0; r < keep; ++r) {
       float bv = -INFINITY;
       int bi = 0x7fffffff;
-      for (int g = lane; g < groups; g += kWave) {
+      for (int g = lane; g < groups; g += L) {
         const float v = g_lds[g];
         if (v != INFINITY && (v > bv || bi == 0x7fffffff)) { bv = v; bi = g; }
       }
-      wave_argmax(bv, bi);
+      lanes_argmax<L>(bv, bi);
       if (lane == 0 && bi != 0x7fffffff) g_lds[bi] = INFINITY;
       in_order();
     }
-    for (int e = lane; e < E; e += kWave)
+    for (int e = lane; e < E; e += L)
       if (g_lds[e / gs] != INFINITY) c_lds[e] = -INFINITY;
     in_order();
   }
@@ -337,11 +343,11 @@ __global__ __launch_bounds__(kRouteWaves * kWave) void moe_route_kernel(const fl
   for (int r = 0; r < top; ++r) {
     float bv = -INFINITY;
     int bi = 0x7fffffff;
-    for (int e = lane; e < E; e += kWave) {
+    for (int e = lane; e < E; e += L) {
       const float v = c_lds[e];
       if (v > bv) { bv = v; bi = e; }
     }
-    wave_argmax(bv, bi);
+    lanes_argmax<L>(bv, bi);
     if (bi == 0x7fffffff) bi = 0;                  // fewer experts in the running than asked for
     const float s = s_lds[bi];
     wsum += s;
@@ -559,9 +565,16 @@ int lv_moe_route_scored(const void* logits, const void* correction, void* ids, v
   const size_t shm = sizeof(float) * (2 * static_cast<size_t>(E) + static_cast<size_t>(groups > 1 ? groups : 1));
   if (shm > 64 * 1024) return fail(-2, "lv_moe_route: %d experts need %zu bytes of LDS", E, shm);
   const int waves = shm * kRouteWaves <= 64 * 1024 ? kRouteWaves : 1;
-  moe_route_kernel<<<dim3(static_cast<unsigned>((T + waves - 1) / waves)), dim3(waves * kWave), waves * shm, as_stream(stream)>>>(
-      static_cast<const float*>(logits), static_cast<const float*>(correction), static_cast<int32_t*>(ids),
-      static_cast<float*>(weights), static_cast<float*>(dense), T, E, top, groups, keep, normalize, score_kind, group_rank);
+  auto launch = [&](auto lanes) {
+    constexpr int L = decltype(lanes)::value;
+    const int tokens = waves * kWave / L;
+    moe_route_kernel<L><<<dim3(static_cast<unsigned>((T + tokens - 1) / tokens)), dim3(waves * kWave), tokens * shm, as_stream(stream)>>>(
+        static_cast<const float*>(logits), static_cast<const float*>(correction), static_cast<int32_t*>(ids),
+        static_cast<float*>(weights), static_cast<float*>(dense), T, E, top, groups, keep, normalize, score_kind, group_rank);
+  };
+  if (E <= 16) launch(std::integral_constant<int, 16>{});      // (top <= E, and there are no more groups than experts)
+  else if (E <= 32) launch(std::integral_constant<int, 32>{});
+  else launch(std::integral_constant<int, 64>{});
   return launched("lv_moe_route");
 }
 
