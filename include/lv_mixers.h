@@ -57,6 +57,7 @@
  *   lv_gated_scan            S <- decay S + write k v^T, o = S^T q with the state in f32, decay and write from step sizes,
  *                            from log gates under a running maximum, or one decay per row of the state with a bonus
  *   lv_chunk_scan            the recurrences with one decay per head and token, 32 tokens at a time on the matrix cores
+ *   lv_chunk_delta_norm      lv_chunk_scan of the delta rule and lv_head_norm_gate in one
  *   lv_scaled_head_norm_gate lv_head_norm_gate with a weight per head and a division of every head by its own number
  *   lv_grouped_gate_norm     o * silu(z), RMS norm in equal parts, weight
  *   lv_residual_pair_norm    single f32 residual: adds the scaled sum of two RMS-normed and weighted sublayer outputs, RMS norm
@@ -444,6 +445,14 @@ int lv_chunk_scan(int kind, const void* q, int64_t ldq, const void* k, int64_t l
                   int64_t lda, const void* decay, const void* p0, const void* p1, const void* p2, void* state,
                   const int32_t* cu_q, const int32_t* ctx_lens, const int32_t* slots, void* o, void* workspace,
                   int64_t workspace_bytes, int64_t T, int B, int max_new, int H, int G, int D, int Dv, int seg_len, void* stream);
+
+/* lv_chunk_scan of the delta rule with norm and gate behind it (lv_head_norm_gate, bf16): out bf16 [T, H*Dv] = per head o / sqrt(mean(o^2) + eps)
+ * * norm_w (f32 [Dv]) * silu or sigmoid of gate (bf16 rows of stride ld_gate).  q, k f32 [T, G, D], v f32 [T, H, Dv], beta, decay f32 [T, H].
+ * Dv 128, or 64 with an even number of heads a group. */
+int lv_chunk_delta_norm(const void* q, const void* k, const void* v, const void* beta, const void* decay, void* state, const int32_t* cu_q,
+                        const int32_t* ctx_lens, const int32_t* slots, const void* gate, int64_t ld_gate, const void* norm_w, void* out,
+                        void* workspace, int64_t workspace_bytes, int64_t T, int B, int max_new, int H, int G, int D, int Dv, float eps,
+                        int gate_kind, void* stream);
 int64_t lv_chunk_scan_workspace_bytes(int kind, int64_t T, int B, int max_new, int H, int D, int Dv, int seg_len);
 
 /* lv_head_norm_gate with o[t, h] divided by den[t, h] first (den f32 [T, H] or NULL) and the norm weight of head h at

@@ -92,6 +92,8 @@ SIGNATURES = {
                               _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P]),
     "lv_chunk_scan": (c_int, [c_int, _P, c_int64, _P, c_int64, _P, c_int64, _P, c_int64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, c_int64,
                               c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P]),
+    "lv_chunk_delta_norm": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, c_int64, _P, _P, _P, c_int64, c_int64, c_int, c_int, c_int, c_int, c_int,
+                                    c_int, c_float, c_int, _P]),
     "lv_chunk_scan_workspace_bytes": (c_int64, [c_int, c_int64, c_int, c_int, c_int, c_int, c_int, c_int]),
     "lv_scaled_head_norm_gate": (c_int, [_P, _P, _P, c_int64, _P, c_int, _P, c_int64, c_int, c_int, c_float, c_int, c_int, _P]),
     "lv_grouped_gate_norm": (c_int, [_P, _P, c_int64, _P, _P, c_int64, c_int, c_int, c_float, c_int, _P]),

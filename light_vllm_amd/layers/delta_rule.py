@@ -18,7 +18,8 @@ Serving state per sequence (one slot of the engine's state manager): S in f32 an
 taps - 1 convolution inputs. A ragged step carries any number of new tokens per sequence from that
 state; a sequence without context starts from zeros without the slot being cleared.
 All input projections are one GEMM; everything between it and the output GEMM is four launches
-(mix_ops: delta_prep, conv_state_update, gated_delta_rule, head_norm_gate), two on decode steps, and the thin second factors.
+(mix_ops: delta_prep, conv_state_update, gated_delta_rule, head_norm_gate), two on decode steps, the last two in one (the scan's second) on
+steps that go in chunks, and the thin second factors.
 """
 from __future__ import annotations
 
@@ -94,10 +95,5 @@ class GatedDeltaRule(nn.Module):
         gate = proj[:, self.off_gate:self.off_gate + self.gate_in]
         if self.gate_up is not None:
             gate = self.gate_up(gate)
-        if few:
-            y = mix_ops.delta_rule_norm_gate(qn, kn, v, beta, decay, self.state, step, gate, self.out_norm_weight, self.norm_eps, h.dtype,
-                                             self.gate_act)
-        else:
-            o = mix_ops.gated_delta_rule(qn, kn, v, beta, decay, self.state, step)
-            y = mix_ops.head_norm_gate(o, gate, self.out_norm_weight, self.norm_eps, h.dtype, self.gate_act)
-        return self.o_proj(y)
+        return self.o_proj(mix_ops.delta_rule_norm_gate(qn, kn, v, beta, decay, self.state, step, gate, self.out_norm_weight, self.norm_eps,
+                                                        h.dtype, self.gate_act))

@@ -417,11 +417,51 @@ def head_norm_gate(o, gate, norm_w, eps, act_dtype, gate_act="silu"):
     return out
 
 
+def _chunk_norm_pays(lens, H, Dv) -> bool:
+    """Whether norm and gate pay in the scan's launch. They lengthen a chunk by 1.16 us (301 against 264 us over 32 chunks), in the chain of the
+    longest sequence or, on more workgroups than compute units, of a unit's share; a launch of their own moves 10 bytes an entry at 4.5 TB/s.
+    Layers, two launches / one, us: 16 x 1024 tokens of 16 heads of 128 819 / 795; 32 x 500 of 64 432 / 413; 30 x 60 187 / 184; but 12 uneven ones of
+    500 on average, 32 heads, 1042 / 1049. A fifth more than break-even is asked for."""
+    longest, chunks, wgs = -(-max(lens) // 32), sum(-(-n // 32) for n in lens), max(1, H * Dv // 128)
+    serial = longest if len(lens) * wgs <= 256 else max(longest, chunks * wgs / 256 + longest / 2)
+    return sum(lens) * H * Dv * 10 / 4.5e6 > 1.2 * 1.16 * serial
+
+
+def _chunk_norm_ok(qn, kn, v, decay, state, step, gate, act_dtype) -> bool:
+    """Whether lv_chunk_delta_norm takes this step: chunks, in workgroups of eight waves, which hold whole heads of 64 or 128 (launches of up to
+    128 of them take four waves a workgroup, half a head of 128 each)."""
+    T, H, Dv = v.shape
+    return (len(step.host_lens_q) * H * Dv // 128 > 128 and v.is_cuda and T > 0 and decay.dim() == 2 and act_dtype == gate.dtype == torch.bfloat16
+            and gate.stride(1) == 1 and (Dv == 128 or (Dv == 64 and H // qn.size(1) % 2 == 0)) and gate.stride(0) < 1 << 27
+            and _chunk_ok(CHUNK_DELTA, step, qn.size(2), Dv, state, qn, kn) and (SCAN_KERNEL == "chunk" or _chunk_norm_pays(step.host_lens_q, H, Dv)))
+
+
+def _chunk_delta_norm(qn, kn, v, beta, decay, state, step, gate, norm_w, eps, gate_act):
+    (T, G, D), (H, Dv) = qn.shape, v.shape[1:]
+    assert gate_act in ("silu", "sigmoid") and gate.size(0) == T and gate.size(1) >= H * Dv
+    _f32(qn, kn, v, beta, decay, state, norm_w)
+    assert state.shape[1:] == (H, D, Dv) and decay.shape == beta.shape == (T, H) and norm_w.numel() == Dv
+    B, longest = len(step.host_lens_q), max(step.host_lens_q)
+    lib = _mixlib.load()
+    nbytes = lib.lv_chunk_scan_workspace_bytes(CHUNK_DELTA, T, B, longest, H, D, Dv, 0)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=v.device)
+    out = torch.empty(T, H * Dv, dtype=gate.dtype, device=v.device)
+    _mixlib.check(lib.lv_chunk_delta_norm(_p(qn), _p(kn), _p(v), _p(beta), _p(decay), _p(state), _p(step.cu_q), _p(step.ctx_lens), _p(step.slots),
+                                          _p(gate), gate.stride(0), _p(norm_w), _p(out), _p(ws), nbytes, T, B, longest, H, G, D, Dv, eps,
+                                          int(gate_act == "sigmoid"), _stream(v)), "lv_chunk_delta_norm")
+    return out
+
+
 def delta_rule_norm_gate(qn, kn, v, beta, decay, state, step, gate, norm_w, eps, act_dtype, gate_act="silu"):
     """head_norm_gate of gated_delta_rule: act [T, H*Dv]. Decode steps (one new token a sequence) with heads of 64 or 128 keys and values
-    do both in one launch."""
+    do both in one launch, bf16 steps in chunks in the scan's launch."""
     T, H, Dv = v.shape
-    if not (v.is_cuda and T > 0 and _one_token(step) and qn.size(2) == Dv and Dv in (64, 128) and len(step.host_lens_q) <= 65535
+    one = _one_token(step)
+    if not one:            # (its first look, which short steps end at, is at the number of sequences)
+        if _chunk_norm_ok(qn, kn, v, decay, state, step, gate, act_dtype):
+            return _chunk_delta_norm(qn, kn, v, beta, decay, state, step, gate, norm_w, eps, gate_act)
+        return head_norm_gate(gated_delta_rule(qn, kn, v, beta, decay, state, step), gate, norm_w, eps, act_dtype, gate_act)
+    if not (v.is_cuda and T > 0 and qn.size(2) == Dv and Dv in (64, 128) and len(step.host_lens_q) <= 65535
             and gate.stride(0) % 4 == 0 and gate.data_ptr() % (4 * gate.element_size()) == 0
             and all(x.data_ptr() % 16 == 0 for x in (qn, kn, v, decay, state, norm_w))):
         return head_norm_gate(gated_delta_rule(qn, kn, v, beta, decay, state, step), gate, norm_w, eps, act_dtype, gate_act)

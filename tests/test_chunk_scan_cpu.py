@@ -112,3 +112,9 @@ def test_segments_keep_their_states_within_256_mb():
     for n in (1, 3, 40):
         seg = mix_ops._segment_length([4096] * n, 1, 1 << 20)
         assert seg == 0 or n * -(-4096 // seg) * (1 << 20) <= 1 << 28
+
+
+@pytest.mark.parametrize("lens,H,Dv,pays", [([1024] * 16, 16, 128, True), ([500] * 32, 16, 64, True), ([60] * 30, 16, 128, True), ([900] * 6 + [100] * 6, 32, 128, False),
+                                            ([4000] + [40] * 20, 16, 128, False)])
+def test_where_the_norm_rides_with_the_scan(lens, H, Dv, pays):
+    assert mix_ops._chunk_norm_pays(lens, H, Dv) == pays
