@@ -28,7 +28,7 @@
 // branch between. The token loop they replace did fewer operations, but on the vector ALU, one token behind the other. Kernels of a
 // layer, us, token loop -> f32 chunks -> staged among the products / on bf16 instructions: 16 x 1024 tokens, delta rule (16 heads, 128 x
 // 128) 993 -> 377 -> 343; constant decays (16 heads, 128 x 128) 596 -> 295 -> 281; step sizes (32 heads, 128 x 64; 7 prompts, the longest
-// 3750) 1531 -> 456 -> 323. Pieces for the other two kinds, whose q, k and v are f32, were built and gained nothing: six to eight
+// 3750) 1531 -> 456 -> 323, 314 with three waves a SIMD in front of the scan. Pieces for the other two kinds, whose q, k and v are f32, were built and gained nothing: six to eight
 // products for one, and every row to cut.
 #include "mix_common.h"
 
