@@ -81,8 +81,24 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const T* __restrict__ 
   for (int j = threadIdx.x; j < Dr; j += blockDim.x) stf(crow + R + j, rotated(row + off_kv + R, j, half, cs));
 }
 
+// The sum over the 256 entries c = 4 lane + u of s, in the order in which four waves of a thread an entry add them (wave_sum, then wave by
+// wave): what c % 64 counts meets at distances 32, 16, 8, 4, 2, 1, of which the first four are lanes. A lane keeps half of its sums
+// at each of the first two, so that seven exchanges do.
+__device__ __forceinline__ float sum_of_four_waves(const float (&s)[4], int lane) {
+  const bool hi = (lane & 8) != 0, odd = (lane & 4) != 0;
+  const float a = (hi ? s[2] : s[0]) + __shfl_xor(hi ? s[0] : s[2], 8, kWave), b = (hi ? s[3] : s[1]) + __shfl_xor(hi ? s[1] : s[3], 8, kWave);
+  float x = (odd ? b : a) + __shfl_xor(odd ? a : b, 4, kWave);
+  x += __shfl_xor(x, 2, kWave);
+  x += __shfl_xor(x, 1, kWave);
+  x += __shfl_xor(x, 8, kWave);
+  x += __shfl_xor(x, 4, kWave);
+  auto of = [&](int i) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), i)); };
+  return of(0) + of(16) + of(32) + of(48);
+}
+
 // The same where rows, offsets and rotated halves are multiples of four: a wave a token, four entries a lane and access, all of a row on its
-// way at once and kept for the second use; NQ and NK accesses for the two latents. HBM-bound: 16 x 1024 tokens of 768 and 192 + 64, 67 MB,
+// way at once and kept for the second use; NQ and NK accesses for the two latents. Sums and products in the order of the kernel above, so that
+// a token's row does not depend on which of the two wrote it. HBM-bound: 16 x 1024 tokens of 768 and 192 + 64, 67 MB,
 // 42 us for the kernel above (two bytes a lane and access, everything read twice, a barrier between), 18 us for this (a decode step of 42 tokens gains 1 us a layer).
 template <typename T, int NQ, int NK>
 __global__ __launch_bounds__(256) void latent_prep_vec_kernel(const T* __restrict__ proj, int64_t ld, int off_q, int off_kv,
@@ -96,7 +112,12 @@ __global__ __launch_bounds__(256) void latent_prep_vec_kernel(const T* __restric
   extern __shared__ __attribute__((aligned(16))) float cs_all[];
   using Row4 = std::conditional_t<sizeof(T) == 2, uint2, float4>;      // four entries as they lie in memory
   auto wide = [](Row4 x) __attribute__((always_inline)) { return ld4(reinterpret_cast<const T*>(&x)); };
-  auto square = [](float4 x) __attribute__((always_inline)) { return (x.x * x.x + x.y * x.y) + (x.z * x.z + x.w * x.w); };
+  auto square = [](float (&s)[4], float4 x) __attribute__((always_inline)) {
+    s[0] = fmaf(x.x, x.x, s[0]);
+    s[1] = fmaf(x.y, x.y, s[1]);
+    s[2] = fmaf(x.z, x.z, s[2]);
+    s[3] = fmaf(x.w, x.w, s[3]);
+  };
   const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave, half = rot_dims / 2, Dk = R + Dr;
   const int64_t t = static_cast<int64_t>(blockIdx.x) * (blockDim.x / kWave) + w;
   if (t >= Tn) return;
@@ -125,15 +146,15 @@ __global__ __launch_bounds__(256) void latent_prep_vec_kernel(const T* __restric
   }
   __builtin_amdgcn_wave_barrier();                 // a wave's LDS operations are carried out in order: only the compiler has to keep them so
   asm volatile("" : : : "memory");
-  float sq = 0.0f, sk = 0.0f;
+  float sq[4] = {}, sk[4] = {};
 #pragma unroll
   for (int i = 0; i < NQ; ++i)
-    if (4 * lane + 256 * i < Rq) sq += square(wide(q[i]));
+    if (4 * lane + 256 * i < Rq) square(sq, wide(q[i]));
 #pragma unroll
   for (int i = 0; i < NK; ++i)
-    if (4 * lane + 256 * i < R) sk += square(wide(k[i]));
-  const float inv_q = 1.0f / sqrtf(wave_sum(sq) / static_cast<float>(Rq) + eps);
-  const float inv_k = 1.0f / sqrtf(wave_sum(sk) / static_cast<float>(R) + eps);
+    if (4 * lane + 256 * i < R) square(sk, wide(k[i]));
+  const float inv_q = 1.0f / sqrtf(sum_of_four_waves(sq, lane) / static_cast<float>(Rq) + eps);
+  const float inv_k = 1.0f / sqrtf(sum_of_four_waves(sk, lane) / static_cast<float>(R) + eps);
 #pragma unroll
   for (int i = 0; i < NQ; ++i) {
     const int c = 4 * lane + 256 * i;
@@ -153,9 +174,9 @@ __global__ __launch_bounds__(256) void latent_prep_vec_kernel(const T* __restric
     } else if (j < rot_dims) {
       const int a = j < half ? j : j - half;
       const float4 u = wide(other[i]), co = ld4(cs + a), sn = ld4(cs + half + a);
-      const float turn = j < half ? -1.0f : 1.0f;
-      x = float4{x.x * co.x + turn * (u.x * sn.x), x.y * co.y + turn * (u.y * sn.y), x.z * co.z + turn * (u.z * sn.z),
-                 x.w * co.w + turn * (u.w * sn.w)};
+      const float4 y{u.x * sn.x, u.y * sn.y, u.z * sn.z, u.w * sn.w};
+      x = j < half ? float4{fmaf(x.x, co.x, -y.x), fmaf(x.y, co.y, -y.y), fmaf(x.z, co.z, -y.z), fmaf(x.w, co.w, -y.w)}
+                   : float4{fmaf(x.x, co.x, y.x), fmaf(x.y, co.y, y.y), fmaf(x.z, co.z, y.z), fmaf(x.w, co.w, y.w)};
     }
     st4(crow + c, x);
   }

@@ -29,3 +29,23 @@ def test_norms_and_rotation(Rq, R, Dr, dims, new, ctx, dtype):
     assert (got[1][1].cpu().float() - got[0][1].float()).abs().max().item() <= tol * 4
     untouched = got[0][1] == 9.0
     assert bool((got[1][1].cpu()[untouched] == 9.0).all())
+
+
+@pytest.mark.parametrize("Rq,R,Dr,dims", [(768, 192, 64, 64), (1536, 256, 0, 0), (4, 4, 8, 8), (2048, 512, 64, 32), (772, 196, 60, 56), (260, 640, 128, 128)])
+@pytest.mark.parametrize("new,ctx", [([70, 1, 6], [5, 0, 63]), ([2045, 1, 5], [3, 100, 0])])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_do_not_depend_on_the_kernel(Rq, R, Dr, dims, new, ctx, dtype):
+    """Rows whose stride is no multiple of four go through the kernel of a thread an entry: the same bits."""
+    gen = torch.Generator(device="cuda").manual_seed(R)
+    T, page = sum(new), 64
+    rows = torch.randn(T, Rq + R + Dr, device="cuda", generator=gen).to(dtype)
+    qw, kw = (1 + 0.3 * torch.randn(n, device="cuda", generator=gen) for n in (Rq, R))
+    step, pages = ragged_step(new, ctx, page, "cuda")
+    got = []
+    for pad in (0, 1):
+        proj = torch.zeros(T, Rq + R + Dr + pad, dtype=dtype, device="cuda")
+        proj[:, :Rq + R + Dr] = rows
+        cache = torch.zeros(pages, page, R + Dr, dtype=dtype, device="cuda")
+        cq = mix_ops.latent_prep(proj, 0, Rq, qw, kw, mix_ops.rotary_inv_freq(max(dims, 2), 10000.0, "cuda"), cache, step, Rq, R, Dr, dims, 1e-6)
+        got.append((cq, cache))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
