@@ -806,6 +806,11 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std:
     for (int i = 0; i < 8; ++i) y[i] = static_cast<__bf16>(x[from + i]);
     return y;
   };
+  // a sum of rounded products, as the launch that rotates queries by itself forms it (no product goes into the addition unrounded)
+  auto rounded_sum = [](float x, float y) __attribute__((always_inline)) {
+    asm volatile("" : "+v"(x), "+v"(y));
+    return x + y;
+  };
   // the lane's number, unknown to the compiler: what is made of it is not kept in registers from here to there
   auto lane_here = [&]() __attribute__((always_inline)) {
     int x = lane;
@@ -889,8 +894,8 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std:
           for (int i = 0; i < 8; ++i) {
             const int at = (16 * x + 8 * half + i) * kPromptQ + c;
             const float co = turn_lds[0][at], si = turn_lds[1][at], u = static_cast<float>(a[i]), v = static_cast<float>(z[i]);
-            a[i] = static_cast<__bf16>(u * co - v * si);
-            z[i] = static_cast<__bf16>(v * co + u * si);
+            a[i] = static_cast<__bf16>(rounded_sum(u * co, -(v * si)));
+            z[i] = static_cast<__bf16>(rounded_sum(v * co, u * si));
           }
         }
       }
@@ -1289,11 +1294,10 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std:
   const float gate1 = grow != nullptr && p.gate_dv == 1 ? sigmoidf_(ldf(reinterpret_cast<const bf16_t*>(grow))) : 1.0f;
   if constexpr (DN > 0) {
     bf16x8_t of[2 * ND];
-    const float f = inv * gate1;
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) o[d][i] *= f;
+      for (int i = 0; i < 16; ++i) o[d][i] = o[d][i] * inv * gate1;         // (the order of the outputs without matrices)
       of[2 * d] = cast8(o[d], 0);
       of[2 * d + 1] = cast8(o[d], 8);
       __builtin_amdgcn_sched_barrier(0);

@@ -120,3 +120,16 @@ def test_what_stays_with_the_batched_products():
     assert not ok(uk=torch.empty(4, 192, 64, device="cuda", dtype=torch.bfloat16).transpose(1, 2))
     assert not ok(uv=torch.empty(4 * 192 * 64 + 4, device="cuda", dtype=torch.bfloat16)[4:].view(4, 192, 64))
     assert not ok(gate=torch.empty(40, 4 * 64 + 2, device="cuda", dtype=torch.bfloat16)[:, 2:], gate_per_channel=True)
+
+
+@pytest.mark.parametrize("H,dim,rot", [(4, 64, 64), (16, 128, 64), (8, 128, 0)])
+def test_outputs_are_those_of_the_separate_launches(H, dim, rot, monkeypatch):
+    """With matrices that hand entries through, sums have one term and any order is the same: rotation, attention and a gate per head
+    leave the bits that they leave in launches of their own."""
+    m, step, h = layer(H, dim, rot, "head", new=[130, 33, 1], ctx=[70, 0, 64], seed=H)
+    with torch.no_grad():
+        m.uk.copy_(torch.eye(dim, m.R))
+        m.uv.copy_(torch.eye(m.R, dim))
+    got = inner(m, step, h)
+    monkeypatch.setattr(mix_ops, "latent_prompt_ok", lambda *a: False)
+    assert torch.equal(got, inner(m, step, h))
