@@ -115,7 +115,7 @@ class LatentAttention(nn.Module):
             return self.o_proj(mix_ops.latent_out_gate(o, gate, self.gate_per_channel))
         with torch.no_grad():           # the kernels between them carry no gradient, and `out` may not ask for one
             if self.Dv == Dn and mix_ops.latent_prompt_ok(q, self.cache, self.uk, self.uv, gate, step, H, Dn, Dr, R, self.rot_dims,
-                                                          self.gate_per_channel):
+                                                          self.gate_per_channel, self.scale):
                 o = mix_ops.latent_prompt_attention(q, self.cache, self.uk, self.uv, self.inv_freq, gate, step, H, Dn, Dr, R, self.window,
                                                     self.scale, self.gate_per_channel, self.sink)
                 return self.o_proj(o)

@@ -923,10 +923,13 @@ def latent_q_finish(q, q_lat, inv_freq, step, H, Dn, Dr, R, rot_dims, out=None):
     return out
 
 
-def latent_prompt_ok(q, cache, uk, uv, gate, step, H, Dn, Dr, R, rot_dims, gate_per_channel) -> bool:
+def latent_prompt_ok(q, cache, uk, uv, gate, step, H, Dn, Dr, R, rot_dims, gate_per_channel, scale=1.0) -> bool:
     """Whether latent_prompt_attention takes this step: prompts (more than 16 new tokens of some sequence: shorter steps have fewer
-    queries than a wave, and theirs are cut over the keys), bf16, and the head sizes and alignment that lv_latent_prompt_attn names."""
-    return (WINDOW_ATTN_KERNEL in ("auto", "prompt") and max(step.host_lens_q, default=0) > 16 and q.dtype == torch.bfloat16
+    queries than a wave, and theirs are cut over the keys), bf16, a positive scale (the maximum is taken before it is applied), and the
+    head sizes, alignment and number of workgroups that lv_latent_prompt_attn names."""
+    longest = max(step.host_lens_q, default=0)
+    return (WINDOW_ATTN_KERNEL in ("auto", "prompt") and longest > 16 and scale > 0 and q.dtype == torch.bfloat16
+            and -(-longest // 32) * len(step.host_lens_q) * (H // 4) < 1 << 31
             and cache.dtype == uk.dtype == uv.dtype == q.dtype and H % 4 == 0 and Dn in (64, 128)
             and uk.shape == (H, Dn, R) and uv.shape == (H, R, Dn) and (R, Dr, rot_dims) in ((192, 64, 64), (256, 0, 0))
             and cache.size(1) % 64 == 0 and all(x.is_contiguous() and x.data_ptr() % 16 == 0 for x in (q, cache, uk, uv))

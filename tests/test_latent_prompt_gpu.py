@@ -133,3 +133,11 @@ def test_outputs_are_those_of_the_separate_launches(H, dim, rot, monkeypatch):
     got = inner(m, step, h)
     monkeypatch.setattr(mix_ops, "latent_prompt_ok", lambda *a: False)
     assert torch.equal(got, inner(m, step, h))
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.07])
+def test_scales_that_are_not_positive(scale):
+    m, step, h = layer(4, 128, 64, "head", new=[40, 3], ctx=[0, 70], seed=2)
+    m.scale = scale
+    got, want = inner(m, step, h), exact(m, step, h)
+    assert (got.double() - want).norm().item() <= REL * want.norm().item()
