@@ -118,21 +118,25 @@ class LatentAttention(nn.Module):
                                                           self.gate_per_channel, self.scale):
                 o = mix_ops.latent_prompt_attention(q, self.cache, self.uk, self.uv, self.inv_freq, gate, step, H, Dn, Dr, R, self.window,
                                                     self.scale, self.gate_per_channel, self.sink)
-                return self.o_proj(o)
-            # both batched products write where the next step reads; a gate per head goes on the sum that the value matrix
-            # multiplies (the same product), in the attention kernel
-            q_abs = torch.empty(T, H, R + Dr, dtype=h.dtype, device=h.device)
-            torch.bmm(q.view(T, H, Dn + Dr)[:, :, :Dn].transpose(0, 1), self.uk, out=q_abs[:, :, :R].transpose(0, 1))
-            if Dr > 0:
-                mix_ops.latent_q_finish(q, None, self.inv_freq, step, H, Dn, Dr, R, self.rot_dims, out=q_abs.view(T, H * (R + Dr)))
-            if self.gate_per_channel:
-                o = torch.bmm(self._attend(q_abs.view(T, H * (R + Dr)), step).view(T, H, R).transpose(0, 1), self.uv)   # [H, T, Dv]
-                o = mix_ops.latent_out_gate(o, gate, True)
             else:
-                o_lat = self._attend(q_abs.view(T, H * (R + Dr)), step, gate)
-                o = torch.empty(T, H * self.Dv, dtype=h.dtype, device=h.device)
-                torch.bmm(o_lat.view(T, H, R).transpose(0, 1), self.uv, out=o.view(T, H, self.Dv).transpose(0, 1))
+                o = self._batched(q, gate, step)
         return self.o_proj(o)
+
+    def _batched(self, q, gate, step):
+        """Gated head outputs [T, H * Dv] with both matrices as batched products, which write where the next step reads; a gate per head
+        goes on the sum that the value matrix multiplies (the same product), in the attention kernel."""
+        T, H, R, Dn, Dr = q.size(0), self.H, self.R, self.Dn, self.Dr
+        q_abs = torch.empty(T, H, R + Dr, dtype=q.dtype, device=q.device)
+        torch.bmm(q.view(T, H, Dn + Dr)[:, :, :Dn].transpose(0, 1), self.uk, out=q_abs[:, :, :R].transpose(0, 1))
+        if Dr > 0:
+            mix_ops.latent_q_finish(q, None, self.inv_freq, step, H, Dn, Dr, R, self.rot_dims, out=q_abs.view(T, H * (R + Dr)))
+        if self.gate_per_channel:
+            o = torch.bmm(self._attend(q_abs.view(T, H * (R + Dr)), step).view(T, H, R).transpose(0, 1), self.uv)   # [H, T, Dv]
+            return mix_ops.latent_out_gate(o, gate, True)
+        o_lat = self._attend(q_abs.view(T, H * (R + Dr)), step, gate)
+        o = torch.empty(T, H * self.Dv, dtype=q.dtype, device=q.device)
+        torch.bmm(o_lat.view(T, H, R).transpose(0, 1), self.uv, out=o.view(T, H, self.Dv).transpose(0, 1))
+        return o
 
     def _forward_direct(self, h, step, proj, col0, out):
         T, H, R, Dn, Dr = h.size(0), self.H, self.R, self.Dn, self.Dr

@@ -141,3 +141,22 @@ def test_scales_that_are_not_positive(scale):
     m.scale = scale
     got, want = inner(m, step, h), exact(m, step, h)
     assert (got.double() - want).norm().item() <= REL * want.norm().item()
+
+
+@pytest.mark.parametrize("new", [[40, 3], [9, 3]])
+def test_the_output_projection_keeps_its_gradient(new, monkeypatch):
+    """The kernels between carry none, on steps of either length and with either form of the products: the same weights have one."""
+    m, step, h = layer(4, 64, 64, "head", new=new, ctx=[0, 70], seed=1)
+    m.requires_grad_(True)
+    set_context(True, ragged=step)
+    try:
+        grads = []
+        for general in (False, True):
+            if general:
+                monkeypatch.setattr(mix_ops, "latent_prompt_ok", lambda *a: False)
+            m.zero_grad()
+            m(h).float().square().sum().backward()
+            grads.append({n for n, p in m.named_parameters() if p.grad is not None})
+        assert grads == [{"o_proj.weight"}] * 2
+    finally:
+        reset_context()
