@@ -1380,7 +1380,7 @@ static bool prompt_launch(const WindowMfmaParams& p, int form, int64_t T, int B,
 }
 
 // The head sizes that decode_pool_kernel is built for; false: the launch belongs to window_pool_mfma_kernel. Rows of q, caches and workspace
-// are read 16 bytes at a time.
+// are read 16 bytes at a time. (mix_ops.decode_heads restates this for the count of splits.)
 static bool decode_launch(const WindowMfmaParams& p, int form, int B, hipStream_t s) {
   auto at = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
   if (form != kPlain || !at(p.q) || !at(p.ws) || (p.P > 0 && (!at(p.kp) || !at(p.vp)))) return false;
@@ -1389,7 +1389,9 @@ static bool decode_launch(const WindowMfmaParams& p, int form, int B, hipStream_
   q.ngroups = (p.H / p.G + 15) / 16;
   const dim3 grid(p.nsplit, p.G * q.ngroups, B), block(256);
   if (p.D == 64 && p.Dv == 64 && !same) decode_pool_kernel<64, 64, false><<<grid, block, 0, s>>>(q);
+  else if (p.D == 64 && p.Dv == 64) decode_pool_kernel<64, 64, true><<<grid, block, 0, s>>>(q);
   else if (p.D == 128 && p.Dv == 128 && !same) decode_pool_kernel<128, 128, false><<<grid, block, 0, s>>>(q);
+  else if (p.D == 128 && p.Dv == 128) decode_pool_kernel<128, 128, true><<<grid, block, 0, s>>>(q);
   else if (p.D == 256 && p.Dv == 192 && same) decode_pool_kernel<256, 192, true><<<grid, block, 0, s>>>(q);
   else if (p.D == 256 && p.Dv == 256 && same) decode_pool_kernel<256, 256, true><<<grid, block, 0, s>>>(q);
   else return false;

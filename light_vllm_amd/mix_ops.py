@@ -555,6 +555,15 @@ def pool_update(k_cache, v_cache, kp, vp, step, G, D, Dv, P):
             vpf[dst] = vc[rows].float().mean(0)
 
 
+def decode_heads(q, k_cache, v_cache, kp, vp, G, D, Dv, P) -> int:
+    """Query heads of a kv head that a workgroup takes on a step of one token a sequence and plain scores: 16 where lv_masked_attn_mfma
+    launches decode_pool_kernel, else 4. 16 heads over one row of 128 that is key and value, in the other kernel with a count made for
+    sixteen: 16 sequences of 1100 tokens 31.7 us, 26.1 with its own; eight heads over two of 256, one of 1100 25.1 / 15.5."""
+    same = P == 0 and (G == 1 or D == Dv) and k_cache.data_ptr() == v_cache.data_ptr() and k_cache.stride(1) == v_cache.stride(1)
+    built = (D, Dv) in ((64, 64), (128, 128)) or (same and (D, Dv) in ((256, 192), (256, 256)))
+    return 16 if built and all(x.data_ptr() % 16 == 0 for x in ((q, kp, vp) if P > 0 else (q,))) else 4
+
+
 def window_pool_attention(q, k_cache, v_cache, kp, vp, gate, step, H, G, D, Dv, window, P, scale, has_sink=True,
                           gate_per_head=False, keep_first=0, chunk=0, sinks=None, softcap=0.0, key_scale=None, dist_bias=None,
                           out=None):
@@ -605,11 +614,12 @@ def window_pool_attention(q, k_cache, v_cache, kp, vp, gate, step, H, G, D, Dv, 
                 most = max(c + n for c, n in zip(step.host_ctx_lens, step.host_lens_q))
                 span = min(most, chunk + 16) if chunk > 0 else min(most, window + 16 + keep_first)
                 tiles = -(-span // 64) + (-(-(max(most - window, 0) // P) // 64) if P > 0 else 0)
-                if (max(step.host_lens_q) <= 1 and softcap == 0.0 and key_scale is None and dist_bias is None
-                        and (D, Dv) in ((64, 64), (128, 128), (256, 192), (256, 256))):     # sixteen heads and 128 keys a workgroup
-                    nsplit = max(1, min(tiles // 2, SPLIT_WORKGROUPS // max(B * G * -(-(H // G) // 16), 1), 32))
-                else:
-                    nsplit = max(1, min(tiles, SPLIT_WORKGROUPS // max(B * G * -(-(H // G) // 4), 1), 32))      # one workgroup a CU: more splits cost more in the merge than they gain (measured)
+                heads = 4
+                if max(step.host_lens_q) <= 1 and softcap == 0.0 and key_scale is None and dist_bias is None:
+                    heads = decode_heads(q, k_cache, v_cache, kp, vp, G, D, Dv, P)
+                # a workgroup of sixteen heads takes 128 keys at a time, one of four 64; one workgroup a CU: more splits cost more in the
+                # merge than they gain (measured)
+                nsplit = max(1, min(tiles // 2 if heads == 16 else tiles, SPLIT_WORKGROUPS // max(B * G * -(-(H // G) // heads), 1), 32))
                 if nsplit > 1:
                     ws = torch.empty(T * H * nsplit * (Dv + 4), dtype=torch.float32, device=q.device)
             _mixlib.check(lib.lv_masked_attn_mfma(_p(q), _p(k_cache), _p(v_cache), _p(kp), _p(vp), _p(gate),

@@ -13,7 +13,8 @@ ATOL = 4 * 2.0 ** -8
 REL = 3.0 ** 0.5 * 2.0 ** -9          # rounded probabilities and both kernels' rounded outputs, independent
 
 SHAPES = [(4, 4, 64, 64, False), (16, 4, 128, 128, False), (6, 2, 128, 128, False), (40, 2, 64, 64, False), (16, 1, 256, 192, True),
-          (20, 1, 256, 256, True), (32, 1, 256, 192, True)]
+          (20, 1, 256, 256, True), (32, 1, 256, 192, True), (16, 1, 128, 128, True), (8, 4, 128, 128, True), (20, 1, 64, 64, True),
+          (8, 2, 256, 256, False)]
 
 
 def both(monkeypatch, ctx, H, G, D, Dv, same, page=64, pool=0, gate=None, new=None, workgroups=256, out_pad=0, seed=0, **kw):
@@ -66,3 +67,29 @@ def test_pooled_blocks_and_gates(monkeypatch, pool, window):
 
 def test_sequences_without_a_new_token(monkeypatch):
     both(monkeypatch, [100, 300, 7], 16, 1, 256, 192, True, new=[1, 0, 1], has_sink=False)
+
+
+@pytest.mark.parametrize("H,G,D,Dv,same", SHAPES + [(8, 2, 128, 64, False), (8, 1, 96, 96, True)])
+@pytest.mark.parametrize("off", [False, True])
+def test_splits_are_counted_for_the_kernel_that_runs(monkeypatch, H, G, D, Dv, same, off):
+    """Workgroups of the launch, from the kernel's name and the rule: at most SPLIT_WORKGROUPS, in either kernel."""
+    from torch.profiler import ProfilerActivity, profile
+    ctx, page = [1500] * 6, 64
+    step, pages = ragged_step([1] * 6, ctx, page, "cuda")
+    q = torch.randn(6 * H * D + 8, device="cuda").bfloat16()[4 if off else 0:][:6 * H * D].view(6, H * D)
+    kc = torch.randn(pages, page, G, D, device="cuda").bfloat16()
+    vc = kc[..., :Dv] if same else torch.randn(pages, page, G, Dv, device="cuda").bfloat16()
+    heads = mix_ops.decode_heads(q, kc, vc, None, None, G, D, Dv, 0)
+    seen = []
+    lib = mix_ops._mixlib.load()
+    call = lib.lv_masked_attn_mfma
+    monkeypatch.setattr(lib, "lv_masked_attn_mfma", lambda *a: seen.append(a[27]) or call(*a))
+    run = lambda: mix_ops.window_pool_attention(q, kc, vc, None, None, None, step, H, G, D, Dv, 1 << 30, 0, D ** -0.5, has_sink=False)  # noqa: E731
+    run()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        run()
+        torch.cuda.synchronize()
+    names = " ".join(e.key for e in prof.key_averages())
+    assert ("decode_pool_kernel" in names) == (heads == 16) and ("window_pool_mfma_kernel" in names) == (heads == 4)
+    assert seen[-1] == max(1, min(24 // (2 if heads == 16 else 1), 256 // (6 * G * -(-(H // G) // heads)), 32))
