@@ -767,8 +767,9 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std:
   lds_u8* const base3 = (lds_u8*)lds;
   // sequences and kv heads fastest: with a multiple of 8 of them all tiles of one run on one XCD; last queries (most keys) first
   const int by = blockIdx.x % by_count, xt = tiles - 1 - blockIdx.x / by_count;
-  const int groups = p.G * p.ngroups, b = by / groups, gy = by % groups;
-  const int g = gy / p.ngroups, hg = gy % p.ngroups;
+  constexpr bool LATENT = DN > 0;                                           // one kv head, no chunks, rows without gaps: known here, not read
+  const int groups = LATENT ? p.ngroups : p.G * p.ngroups, b = by / groups, gy = by % groups;
+  const int g = LATENT ? 0 : gy / p.ngroups, hg = LATENT ? gy : gy % p.ngroups;
   const int q0 = p.cu_q[b], n = p.cu_q[b + 1] - q0;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane & 31, half = lane >> 5;
   const int r0 = xt * kPromptQ * (4 / hpw);
@@ -781,10 +782,10 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std:
   const int w0 = ctx + rw, w1 = ctx + min(n, rw + kPromptQ) - 1;            // positions of this wave's first and last query
   const int row = min(rw + c, n - 1), pos = ctx + row;
   const int64_t t = q0 + row;
-  const int page = p.page, P = p.P, W = p.window, chunk = p.chunk, keep = p.keep_first;
+  const int page = p.page, P = LATENT ? 0 : p.P, W = p.window, chunk = LATENT ? 0 : p.chunk, keep = LATENT ? 0 : p.keep_first;
   const int cstart = chunk > 0 ? (pos / chunk) * chunk : 0;
   const int32_t* bt = p.block_tables + static_cast<int64_t>(b) * p.bt_stride;
-  const int64_t GD = static_cast<int64_t>(p.G) * DK, GDv = static_cast<int64_t>(p.G) * DV;
+  const int64_t GD = static_cast<int64_t>(p.G) * DK, GDv = static_cast<int64_t>(p.G) * DV, k_ld = LATENT ? DK : p.k_ld;
 
   bf16x8_t qf[NS];
   lds_u8* const slot0 = (lds_u8*)tile0 + 8192 * wave;                       // the wave's own parts of the tiles
@@ -817,10 +818,23 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std:
     asm volatile("" : "+v"(x));
     return x;
   };
+  // The same of the arguments and of what this workgroup has to do: the code in front of the tile loop and behind it starts from them again. Kept
+  // through the loop they left it too few registers to read four fragments ahead (17 or 1024 tokens behind 16000, 16 heads, us: batched products
+  // 571 / 652, this launch 634 / 711 with them kept, 550 / 621 without).
+  struct LatentArgs { LatentParams p; int hpw, tiles, by_count; };
+  typedef const __attribute__((address_space(4))) LatentArgs* args_t;
+  struct Own { args_t a; int h, rw, q0, n; };
+  auto again = [&]() __attribute__((always_inline)) {
+    args_t a = (args_t)__builtin_amdgcn_kernarg_segment_ptr();
+    int block = blockIdx.x;
+    asm volatile("" : "+s"(a), "+s"(block));
+    const int by = block % a->by_count, b = by / a->p.ngroups, q0 = a->p.cu_q[b];
+    return Own{a, by % a->p.ngroups * 4 + wave, (a->tiles - 1 - block / a->by_count) * kPromptQ, q0, a->p.cu_q[b + 1] - q0};
+  };
   // rows of the key matrix, 16 a piece of 512-byte rows (of which a latent of 192 fills 384)
-  auto uk_piece = [&](int k, lds_u8* at, int ln) __attribute__((always_inline)) {
+  auto uk_piece = [&](const Own& own, int k, lds_u8* at, int ln) __attribute__((always_inline)) {
     if constexpr (DN > 0) {
-      const char* from = reinterpret_cast<const char*>(p.uk + (static_cast<int64_t>(h) * DN + 16 * k) * DV);
+      const char* from = reinterpret_cast<const char*>(own.a->p.uk + (static_cast<int64_t>(own.h) * DN + 16 * k) * DV);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int r = 2 * i + (ln >> 5), ch = (ln & 31) ^ (((r & 3) << 2) | ((r >> 2) & 3));
@@ -833,10 +847,11 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std:
   auto absorb = [&](auto beside) __attribute__((always_inline)) {
     if constexpr (DN > 0) {
       constexpr int NP = DN / 16;
+      const Own own = again();
       const int ln = lane_here(), half = ln >> 5, c = ln & 31, tq = (ln & 15) >> 2, tp = ln & 3, gi = ln >> 4;
-      uk_piece(0, slot0, ln);
-      uk_piece(1, slot1, ln);
-      const uint16_t* qrow = p.q + (static_cast<int64_t>(q0 + min(rw + c, n - 1)) * p.H + h) * QW + 8 * half;
+      uk_piece(own, 0, slot0, ln);
+      uk_piece(own, 1, slot1, ln);
+      const uint16_t* qrow = own.a->p.q + (static_cast<int64_t>(own.q0 + min(own.rw + c, own.n - 1)) * own.a->p.H + own.h) * QW + 8 * half;
       bf16x8_t raw[NP];
 #pragma unroll
       for (int k = 0; k < NP; ++k) raw[k] = *reinterpret_cast<const bf16x8_t*>(qrow + 16 * k);
@@ -872,14 +887,14 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std:
         multiply(k, slot0);
         reads_done();
         if (k + 2 < NP) {
-          uk_piece(k + 2, slot0, ln);
+          uk_piece(own, k + 2, slot0, ln);
           landed(std::integral_constant<int, 8>{});
         } else {
           landed(std::integral_constant<int, 0>{});
         }
         multiply(k + 1, slot1);
         reads_done();
-        if (k + 3 < NP) uk_piece(k + 3, slot1, ln);
+        if (k + 3 < NP) uk_piece(own, k + 3, slot1, ln);
       }
 #pragma unroll
       for (int d = 0; d < ND; ++d) {
@@ -905,9 +920,11 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std:
   auto leave = [&](const bf16x8_t* of, int pass) __attribute__((always_inline)) {
     if constexpr (DN > 0) {
       constexpr int UB = 2 * DN, UN = UB * 32 / 1024, NE = DN / 32;
+      const Own own = again();
+      const auto& p = own.a->p;
       const int ln = lane_here(), half = ln >> 5, c = ln & 31, tq = (ln & 15) >> 2, tp = ln & 3, gi = ln >> 4;
       auto uv_piece = [&](int k, lds_u8* at) __attribute__((always_inline)) {      // 32 rows
-        const char* from = reinterpret_cast<const char*>(p.uv + (static_cast<int64_t>(h) * DV + 32 * k) * DN);
+        const char* from = reinterpret_cast<const char*>(p.uv + (static_cast<int64_t>(own.h) * DV + 32 * k) * DN);
 #pragma unroll
         for (int i = 0; i < UN; ++i) {
           const int r = (1024 / UB) * i + ln / (UB / 16), pc = ln % (UB / 16);
@@ -956,11 +973,11 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std:
         reads_done();
         if (k + 3 < ND) uv_piece(k + 3, slot1);
       }
-      if (rw + c >= n || (pass >= 0 && (c >> 4) != pass)) return;
-      const int64_t t = q0 + rw + c;
-      bf16_t* orow = reinterpret_cast<bf16_t*>(p.out) + t * p.out_ld + static_cast<int64_t>(h) * DN + 4 * half;
+      if (own.rw + c >= own.n || (pass >= 0 && (c >> 4) != pass)) return;
+      const int64_t t = own.q0 + own.rw + c;
+      bf16_t* orow = reinterpret_cast<bf16_t*>(p.out) + t * p.out_ld + static_cast<int64_t>(own.h) * DN + 4 * half;
       const bool gated = p.gate != nullptr && p.gate_dv != 1;
-      const bf16_t* grow = reinterpret_cast<const bf16_t*>(p.gate) + t * p.ld_gate + static_cast<int64_t>(h) * DN + 4 * half;
+      const bf16_t* grow = reinterpret_cast<const bf16_t*>(p.gate) + t * p.ld_gate + static_cast<int64_t>(own.h) * DN + 4 * half;
 #pragma unroll
       for (int e = 0; e < NE; ++e)
 #pragma unroll
@@ -1134,6 +1151,7 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std:
         }
       }
       if (!whole) {
+        if constexpr (LATENT) asm volatile("");                             // a branch: most tiles have no mask
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const int ke = ks0 + (i & 3) + 8 * (i >> 2) + 4 * half;
@@ -1187,12 +1205,12 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std:
     auto request = [&](int tile, lds_u8* at) __attribute__((always_inline)) {
       const int e0 = jlo + tile * kTileK, pj = fdiv(e0, page, p.m_page), last = i1 - e0;
       const int64_t slot = static_cast<int64_t>(bt[pj]) * page + (e0 - pj * page);
-      const char* kb = reinterpret_cast<const char*>(p.k_cache + slot * p.k_ld + g * DK);
+      const char* kb = reinterpret_cast<const char*>(p.k_cache + slot * k_ld + g * DK);
 #pragma unroll
       for (int i = 0; i < KT / 4096; ++i) {
         const int r = 8 * i + d_r, ch = (lane & 31) ^ (((r & 3) << 2) | ((r >> 2) & 3));
         __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) void*)(kb + static_cast<uint32_t>(min(r, last)) * static_cast<uint32_t>(2 * p.k_ld) + 16 * ch),
+            (const __attribute__((address_space(1))) void*)(kb + static_cast<uint32_t>(min(r, last)) * static_cast<uint32_t>(2 * k_ld) + 16 * ch),
             (__attribute__((address_space(3))) void*)(at + 1024 * (wave + 4 * i)), 16, 0, 0);
       }
     };
@@ -1286,13 +1304,12 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std:
   }
   const float total = l + __shfl_xor(l, 32, kWave);
   const float inv = total > 0.0f ? 1.0f / total : 0.0f;
-  if constexpr (DN == 0) {
-    if (rw + c >= n) return;
-  }
-  uint16_t* orow = p.out + t * p.out_ld + static_cast<int64_t>(h) * DV + 4 * half;
-  const uint16_t* grow = p.gate != nullptr ? p.gate + t * p.ld_gate + static_cast<int64_t>(h) * p.gate_dv : nullptr;
-  const float gate1 = grow != nullptr && p.gate_dv == 1 ? sigmoidf_(ldf(reinterpret_cast<const bf16_t*>(grow))) : 1.0f;
   if constexpr (DN > 0) {
+    const Own own = again();
+    const int c = lane_here() & 31;
+    const bf16_t* gate = reinterpret_cast<const bf16_t*>(own.a->p.gate);
+    const int64_t t = own.q0 + min(own.rw + c, own.n - 1);
+    const float gate1 = gate != nullptr && own.a->p.gate_dv == 1 ? sigmoidf_(ldf(gate + t * own.a->p.ld_gate + own.h)) : 1.0f;
     bf16x8_t of[2 * ND];
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
@@ -1305,6 +1322,10 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void prompt_attn_kernel(std:
     leave(of, -1);
     return;
   }
+  if (rw + c >= n) return;
+  uint16_t* orow = p.out + t * p.out_ld + static_cast<int64_t>(h) * DV + 4 * half;
+  const uint16_t* grow = p.gate != nullptr ? p.gate + t * p.ld_gate + static_cast<int64_t>(h) * p.gate_dv : nullptr;
+  const float gate1 = grow != nullptr && p.gate_dv == 1 ? sigmoidf_(ldf(reinterpret_cast<const bf16_t*>(grow))) : 1.0f;
 #pragma unroll
   for (int d = 0; d < ND; ++d)
 #pragma unroll
