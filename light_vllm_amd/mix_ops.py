@@ -933,10 +933,21 @@ def latent_q_finish(q, q_lat, inv_freq, step, H, Dn, Dr, R, rot_dims, out=None):
     return out
 
 
+def _latent_prompt_pays(step, T, H, Dn, R) -> bool:
+    """Whether one launch beats the batched products beside many short sequences. Each of them costs it both matrices of a head for 32 queries,
+    however few there are; the products cost by the token, and three or four launches. Layers, products / one launch, us, 16 heads
+    of 128: 400 sequences with one new token and one with 100, contexts of 100, rows of 192 + 64 123 / 127, of 256 140 / 163; 1000 beside 1000 306 / 328,
+    346 / 404; contexts of 1000 742 / 705 in rows of 256, whose tile loop is the better one here; 250 beside 1000 + 1000 216 / 192. Lines
+    through 165 such steps of 16 and 32 heads, in us: the choice is within 6 % of the better one."""
+    cost = 0.0013 if Dn == 64 else 0.0025 if R == 192 else 0.0055
+    behind = H * (cost * len(step.host_lens_q) - 0.0005 * T) - 11
+    return behind <= 0 or behind <= H * (1e-6 if R == 192 else 6e-6) * sum(step.host_ctx_lens)
+
+
 def latent_prompt_ok(q, cache, uk, uv, gate, step, H, Dn, Dr, R, rot_dims, gate_per_channel, scale=1.0) -> bool:
     """Whether latent_prompt_attention takes this step: prompts (more than 16 new tokens of some sequence: shorter steps have fewer
     queries than a wave, and theirs are cut over the keys), bf16, a positive scale (the maximum is taken before it is applied), and the
-    head sizes, alignment and number of workgroups that lv_latent_prompt_attn names."""
+    head sizes, alignment and number of workgroups that lv_latent_prompt_attn names; not beside so many short sequences that it loses."""
     longest = max(step.host_lens_q, default=0)
     return (WINDOW_ATTN_KERNEL in ("auto", "prompt") and longest > 16 and scale > 0 and q.dtype == torch.bfloat16
             and -(-longest // 32) * len(step.host_lens_q) * (H // 4) < 1 << 31
@@ -944,7 +955,8 @@ def latent_prompt_ok(q, cache, uk, uv, gate, step, H, Dn, Dr, R, rot_dims, gate_
             and uk.shape == (H, Dn, R) and uv.shape == (H, R, Dn) and (R, Dr, rot_dims) in ((192, 64, 64), (256, 0, 0))
             and cache.size(1) % 64 == 0 and all(x.is_contiguous() and x.data_ptr() % 16 == 0 for x in (q, cache, uk, uv))
             and gate.stride(1) == 1 and gate.dtype == q.dtype
-            and (not gate_per_channel or (gate.stride(0) % 4 == 0 and gate.data_ptr() % 8 == 0)))
+            and (not gate_per_channel or (gate.stride(0) % 4 == 0 and gate.data_ptr() % 8 == 0))
+            and (WINDOW_ATTN_KERNEL == "prompt" or _latent_prompt_pays(step, q.size(0), H, Dn, R)))
 
 
 def latent_prompt_attention(q, cache, uk, uv, inv_freq, gate, step, H, Dn, Dr, R, window, scale, gate_per_channel, sinks=None):
