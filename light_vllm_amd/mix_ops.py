@@ -417,14 +417,15 @@ def head_norm_gate(o, gate, norm_w, eps, act_dtype, gate_act="silu"):
     return out
 
 
-def _chunk_norm_pays(lens, H, Dv) -> bool:
-    """Whether norm and gate pay in the scan's launch. They lengthen a chunk by 1.16 us (301 against 264 us over 32 chunks), in the chain of the
-    longest sequence or, on more workgroups than compute units, of a unit's share; a launch of their own moves 10 bytes an entry at 4.5 TB/s.
-    Layers, two launches / one, us: 16 x 1024 tokens of 16 heads of 128 819 / 795; 32 x 500 of 64 432 / 413; 30 x 60 187 / 184; but 12 uneven ones of
-    500 on average, 32 heads, 1042 / 1049. A fifth more than break-even is asked for."""
+def _chunk_norm_pays(lens, H, Dv, D=128) -> bool:
+    """Whether norm and gate pay in the scan's launch. They lengthen a chunk by 1.25 us (64 x 64 by 1.05: the even launches of 78, one to four
+    workgroups a unit, 1.11 to 1.40 and 0.89 to 1.37), in the chain of the longest sequence or, on more workgroups than compute units, of a unit's
+    share; a launch of their own takes 3 us and moves 10 bytes an entry at 5.8 TB/s. Scan, norm and gate in two launches / one, us: 16 x 1024
+    tokens of 16 heads of 128 393 / 372, 64 x 256 413 / 391, 9 x 64 46.8 / 44.2; 32 x 1024 of 32 heads of 64 668 / 615; but 32 uneven ones of 400 on
+    average, 16 heads, 382 / 387, one of 1500 beside 15 of 150 414 / 455. A tenth more than break-even is asked for."""
     longest, chunks, wgs = -(-max(lens) // 32), sum(-(-n // 32) for n in lens), max(1, H * Dv // 128)
     serial = longest if len(lens) * wgs <= 256 else max(longest, chunks * wgs / 256 + longest / 2)
-    return sum(lens) * H * Dv * 10 / 4.5e6 > 1.2 * 1.16 * serial
+    return 3 + sum(lens) * H * Dv * 10 / 5.8e6 > 1.1 * (1.05 if D == Dv == 64 else 1.25) * serial
 
 
 def _chunk_norm_ok(qn, kn, v, decay, state, step, gate, act_dtype) -> bool:
@@ -433,7 +434,7 @@ def _chunk_norm_ok(qn, kn, v, decay, state, step, gate, act_dtype) -> bool:
     T, H, Dv = v.shape
     return (len(step.host_lens_q) * H * Dv // 128 > 128 and v.is_cuda and T > 0 and decay.dim() == 2 and act_dtype == gate.dtype == torch.bfloat16
             and gate.stride(1) == 1 and (Dv == 128 or (Dv == 64 and H // qn.size(1) % 2 == 0)) and gate.stride(0) < 1 << 27
-            and _chunk_ok(CHUNK_DELTA, step, qn.size(2), Dv, state, qn, kn) and (SCAN_KERNEL == "chunk" or _chunk_norm_pays(step.host_lens_q, H, Dv)))
+            and _chunk_ok(CHUNK_DELTA, step, qn.size(2), Dv, state, qn, kn) and (SCAN_KERNEL == "chunk" or _chunk_norm_pays(step.host_lens_q, H, Dv, qn.size(2))))
 
 
 def _chunk_delta_norm(qn, kn, v, beta, decay, state, step, gate, norm_w, eps, gate_act):

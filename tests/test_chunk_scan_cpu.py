@@ -118,3 +118,10 @@ def test_segments_keep_their_states_within_256_mb():
                                             ([4000] + [40] * 20, 16, 128, False)])
 def test_where_the_norm_rides_with_the_scan(lens, H, Dv, pays):
     assert mix_ops._chunk_norm_pays(lens, H, Dv) == pays
+
+
+@pytest.mark.parametrize("lens,H,Dv,D,pays", [
+    ([750, 50, 400, 600] * 8, 16, 128, 128, False), ([750, 50, 400, 600] * 8, 32, 64, 64, True),
+    ([700, 100, 350, 600] * 4, 32, 64, 128, False), ([1024] * 9, 16, 128, 128, False), ([64] * 9, 16, 128, 128, True)])
+def test_where_the_norm_rides_by_head_sizes(lens, H, Dv, D, pays):
+    assert mix_ops._chunk_norm_pays(lens, H, Dv, D) == pays
