@@ -123,7 +123,8 @@ struct MoeTileParams {
 // has to wait for.
 // CHAIN (k in whole pairs of steps): a workgroup goes from tile to tile. The last two steps request the next tile's first two, which arrive while
 // the outputs leave through LDS of their own, and nothing waits for a store until a step later; a tile by itself spent some 15 us on
-// its way in and out. Other k drain the slots between tiles.
+// its way in and out. Other k drain the slots between tiles, and request the next tile's first steps in front of the outputs too (7000 tokens, 16 experts of
+// 1024 x 352, 4 each: the layer's experts 112 -> 107 us, 107 with the tiles of 128 rows that came before; 16384 tokens 222 -> 217, 240).
 // GLU: LDS rows 64 j .. 64 j + 31 of the weights hold gate columns 32 j .., the 32 after them the up columns of the same numbers.
 template <bool UP, bool GLU, bool CHAIN>
 __global__ __launch_bounds__(256, 1) void moe_tile_kernel(MoeTileParams p) {
@@ -233,12 +234,10 @@ __global__ __launch_bounds__(256, 1) void moe_tile_kernel(MoeTileParams p) {
 
   look_up(cur);
   aim(cur);
-  if constexpr (CHAIN) {
-    request(slot0, 0, I4{}, I0{}, I16{});
-    request(slot1, 1, I4{}, I0{}, I16{});
-    turn();
-  }
-  // one tile of up to 64 MB rows; with CHAIN its first step lies in slot0, the second is in slot1 or on its way there
+  request(slot0, 0, I4{}, I0{}, I16{});
+  request(slot1, 1, I4{}, I0{}, I16{});
+  turn();
+  // one tile of up to 64 MB rows, whose first two steps lie in the slots or (CHAIN) the second is on its way there
   auto tile = [&](auto mb) __attribute__((always_inline)) {
     constexpr int MB = decltype(mb)::value;
     constexpr int MUL = 8 * MB, READS = 2 * (MB + 4), EARLY = MUL * 3 / 8;
@@ -316,9 +315,9 @@ __global__ __launch_bounds__(256, 1) void moe_tile_kernel(MoeTileParams p) {
     };
 
     Tile following;
+    asm volatile("s_barrier" ::: "memory");                          // every wave's share of the first two steps has landed (awaited in front of its stores)
+    fetch(slot0, 0, f0);
     if constexpr (CHAIN) {
-      asm volatile("s_barrier" ::: "memory");                        // every wave's share of the first two steps has landed (awaited in front of its stores)
-      fetch(slot0, 0, f0);
       following = find(cur.q + stride);
       if (following.nrows > 0) look_up(following);
       // (its first turn apart and without a condition: where it may be either, the compiler waits for loads that were requested behind it)
@@ -332,10 +331,6 @@ __global__ __launch_bounds__(256, 1) void moe_tile_kernel(MoeTileParams p) {
       step(slot0, slot1, 0, std::false_type{}, std::true_type{}, I4{});
       step(slot1, slot0, 1, std::false_type{}, std::false_type{}, I4{});
     } else {
-      request(slot0, 0, mb, I0{}, std::integral_constant<int, 8 + 2 * MB>{});
-      request(slot1, 1, mb, I0{}, std::integral_constant<int, 8 + 2 * MB>{});
-      turn();
-      fetch(slot0, 0, f0);
       int c = 0;
       for (; c + 2 <= full; c += 2) {
         step(slot0, slot1, c + 2, std::false_type{}, std::true_type{}, mb);
@@ -348,6 +343,8 @@ __global__ __launch_bounds__(256, 1) void moe_tile_kernel(MoeTileParams p) {
       if (following.nrows > 0) {
         look_up(following);
         aim(following);
+        request(slot0, 0, I4{}, I0{}, I16{});
+        request(slot1, 1, I4{}, I0{}, I16{});
       }
     }
 
@@ -391,7 +388,7 @@ __global__ __launch_bounds__(256, 1) void moe_tile_kernel(MoeTileParams p) {
           *reinterpret_cast<__attribute__((address_space(3))) uint64_t*>(mine + er * WC * 2 + piece * 16 + ((eh ^ (er >> 4)) & 1) * 8) =
               static_cast<uint64_t>(pair[0]) | (static_cast<uint64_t>(pair[1]) << 32);
         }
-      if (CHAIN && j == 0) __builtin_amdgcn_s_waitcnt(0x0f70);       // the next tile's first two steps have landed: nothing there waits for a store
+      if (j == 0) __builtin_amdgcn_s_waitcnt(0x0f70);       // the next tile's first two steps have landed: nothing there waits for a store
       auto leave = [&](int i, auto unary) __attribute__((always_inline)) {
         const int r = i * RPI + ln / PIECES, c = ln % PIECES;
         const int n = cur.n0 + wn * WC + 8 * c;
