@@ -290,9 +290,9 @@ __device__ __forceinline__ void lanes_argmax(float& v, int& i) {
   }
 }
 
-// One wave a token, four of them a workgroup: a compute unit holds sixteen workgroups, and sixteen waves are too few to hide a chain of
-// shuffles behind. 16384 tokens of 32 experts, 4 choices, us: one wave a workgroup 22.1, four 21.3.
-// L lanes a token, as many as hold its experts, choices and groups: with 32 experts two tokens share a wave's chain of shuffles, 20.3 -> 13.1.
+// L lanes a token, as many as hold its experts, choices and groups: with 32 experts two tokens share a wave's chain of shuffles. Four waves a
+// workgroup: a compute unit holds sixteen workgroups, and sixteen waves are too few to hide a chain of shuffles behind. 16384 tokens of 32
+// experts, 4 choices, us: a wave a token 22.1 with one a workgroup, 20.3 with four; half a wave a token 13.1.
 constexpr int kRouteWaves = 4;
 template <int L>
 __global__ __launch_bounds__(kRouteWaves * kWave) void moe_route_kernel(const float* __restrict__ logits, const float* __restrict__ correction,

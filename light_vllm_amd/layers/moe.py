@@ -48,14 +48,14 @@ from .tp import tp_size
 
 
 GATHER_FROM = 2.0     # experts / top from which the gathered form is taken
-# Rows per expert from which an eager step multiplies on LDS tiles. 32 experts of 2048 x 1536: 118 against 160 us for the
-# gathered form at 16 rows, 129 / 254 at 64, 246 / 539 at 256, 1006 / 3412 at 2048; below 16 the gathered form's tiles of 16
-# rows read each weight once and pad little.
+# Rows per expert from which an eager step multiplies on LDS tiles. 32 experts of 2048 x 1536: 102 against 160 us for the
+# gathered form at 16 rows, 111 / 260 at 64, 193 / 543 at 256, 840 / 3479 at 2048; below 16 the gathered form's tiles of 16
+# rows read each weight once and pad little (16 experts of 1024 x 512 35 / 25 at 8).
 TILED_FROM = 16
 TILED_SURELY = 48     # rows per expert from which they always do
 # In between, entries of the sorted activations (of width, or twice ff where that is less) from which the tiles' longer sort and fewer,
-# larger workgroups pay. Tiled / gathered, us: 4 experts of 2048 x 1536 57 / 39 at 16 rows, 60 / 50 at 32, 61 / 111 at 48; 16 of
-# 1024 x 512 36 / 29 at 16, level at 32; 64 of 512 x 256 31 / 35 at 16; 32 of 2048 x 256 51 / 43 at 16, level at 32.
+# larger workgroups pay. Tiled / gathered, us: 4 experts of 2048 x 1536 53 / 40 at 16 rows, 54 / 50 at 32, 55 / 114 at 48; 16 of
+# 1024 x 512 35 / 30 at 16, 36 / 42 at 32; 64 of 512 x 256 30 / 34 at 16; 32 of 2048 x 256 45 / 42 at 16, 47 / 64 at 32.
 TILED_ENTRIES = 1 << 19
 SORTED_FROM = 256     # rows per expert for weights that the tiles do not take: vendor GEMMs on sorted rows
 MOE_KERNEL = "auto"   # "auto" | "masked" | "gathered" | "sorted" (tests force one or the other)

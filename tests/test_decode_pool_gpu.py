@@ -93,3 +93,62 @@ def test_splits_are_counted_for_the_kernel_that_runs(monkeypatch, H, G, D, Dv, s
     names = " ".join(e.key for e in prof.key_averages())
     assert ("decode_pool_kernel" in names) == (heads == 16) and ("window_pool_mfma_kernel" in names) == (heads == 4)
     assert seen[-1] == max(1, min(24 // (2 if heads == 16 else 1), 256 // (6 * G * -(-(H // G) // heads)), 32))
+
+
+def exact(q, kc, vc, step, H, G, D, Dv, window, sinks):
+    outs, rep = [], H // G
+    for b, ctx in enumerate(step.host_ctx_lens):
+        pages = torch.tensor(step.host_block_tables[b], device="cuda")
+        k, v = (x[pages].reshape(-1, G, x.size(-1))[max(0, ctx - window + 1):ctx + 1].double() for x in (kc, vc))
+        s = torch.einsum("grd,ngd->grn", q[b].view(G, rep, D).double(), k) * D ** -0.5
+        if sinks is not None:
+            s = torch.cat([s, sinks.double().view(G, rep, 1)], -1)
+        outs.append(torch.einsum("grn,ngd->grd", torch.softmax(s, -1)[..., :k.size(0)], v).reshape(-1))
+    return torch.stack(outs)
+
+
+def run(q, kc, vc, step, H, G, D, Dv, window, sinks=None):
+    return mix_ops.window_pool_attention(q, kc, vc, None, None, None, step, H, G, D, Dv, window, 0, D ** -0.5, has_sink=False, sinks=sinks)
+
+
+def operands(ctx, H, G, D, Dv, same, page, seed):
+    step, pages = ragged_step([1] * len(ctx), ctx, page, "cuda", seed)
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    kc = torch.randn(pages, page, G, D, device="cuda", generator=gen).bfloat16()
+    vc = kc[..., :Dv] if same else torch.randn(pages, page, G, Dv, device="cuda", generator=gen).bfloat16()
+    return step, torch.randn(len(ctx), H * D, device="cuda", generator=gen).bfloat16(), kc, vc
+
+
+@pytest.mark.parametrize("H,G,D,Dv,same", SHAPES)
+@pytest.mark.parametrize("sunk", [False, True])
+def test_against_float64(H, G, D, Dv, same, sunk):
+    """Sinks of minus infinity, which count nothing, among finite ones."""
+    step, q, kc, vc = operands([0, 31, 64, 700, 2100], H, G, D, Dv, same, 64, H + D)
+    sinks = torch.linspace(-3, 3, H, device="cuda") if sunk else None
+    if sunk:
+        sinks[::3] = float("-inf")
+    got, want = run(q, kc, vc, step, H, G, D, Dv, 1500, sinks), exact(q, kc, vc, step, H, G, D, Dv, 1500, sinks)
+    assert (got.double() - want).norm().item() <= 2 ** 0.5 * 2.0 ** -9 * want.norm().item()      # rounded probabilities and outputs, independent
+
+
+@pytest.mark.parametrize("H,G,D,Dv,same", SHAPES)
+def test_rows_that_are_not_finite_reach_only_the_queries_that_see_them(H, G, D, Dv, same):
+    ctx, page, window = [100, 63, 500], 64, 80
+    step, q, kc, vc = operands(ctx, H, G, D, Dv, same, page, 3)
+    clean = run(q, kc, vc, step, H, G, D, Dv, window)
+    table = step.host_block_tables
+    for rows in ({kc.data_ptr(): kc, vc.data_ptr(): vc}).values():
+        for b, c in enumerate(ctx):
+            rows[table[b][c // page], c % page + 1:] = float("nan")                 # behind the last token
+        rows[torch.tensor(table[2][:421 // page])] = float("inf")                   # whole pages in front of the window's first token, 421
+    assert torch.equal(run(q, kc, vc, step, H, G, D, Dv, window), clean)
+    for at in (90, 100):                                                            # inside the window, and the last token
+        keep = vc[table[0][at // page], at % page, 0, 3].clone()
+        vc[table[0][at // page], at % page, 0, 3] = float("inf")
+        got = run(q, kc, vc, step, H, G, D, Dv, window)
+        first = got[0, :H // G * Dv].view(-1, Dv)                                   # the kv head's query heads
+        assert torch.equal(got[1:], clean[1:]) and torch.equal(got[0, H // G * Dv:], clean[0, H // G * Dv:])
+        assert not torch.isfinite(first[:, 3]).any()
+        if not same:                                                                # (a key with an infinity takes its head along)
+            assert torch.equal(first[:, 4:], clean[0, :H // G * Dv].view(-1, Dv)[:, 4:])
+        vc[table[0][at // page], at % page, 0, 3] = keep

@@ -160,3 +160,15 @@ def test_the_output_projection_keeps_its_gradient(new, monkeypatch):
         assert grads == [{"o_proj.weight"}] * 2
     finally:
         reset_context()
+
+
+@pytest.mark.parametrize("H,dim,rot,gate", [(4, 128, 64, "head"), (8, 64, 0, "channel")])
+def test_a_prompt_beside_many_decoded_sequences(H, dim, rot, gate, monkeypatch):
+    """One query of a wave's 32 in use, or none, at contexts around tiles and pages."""
+    new, ctx = [1] * 30 + [37, 0, 1], [63 * i % 200 for i in range(30)] + [0, 5, 64]
+    m, step, h = layer(H, dim, rot, gate, new=new, ctx=ctx, seed=4)
+    calls = []
+    one = mix_ops.latent_prompt_attention
+    monkeypatch.setattr(mix_ops, "latent_prompt_attention", lambda *a, **k: calls.append(1) or one(*a, **k))
+    got, want = inner(m, step, h), exact(m, step, h)
+    assert calls and (got.double() - want).norm().item() <= REL * want.norm().item()

@@ -1,6 +1,6 @@
-"""The experts' products on LDS tiles (lv_moe_tiled_ff) against the sum in float64, at sizes where tiles end: one row, 128 and
-256 rows and one more, widths beside a multiple of the 256 columns and of four steps over k, experts without rows, experts
-that hand their input through.
+"""The experts' products on LDS tiles (lv_moe_tiled_ff) against the sum in float64, at sizes where tiles end: one row, blocks of 64 and tiles of
+256 rows and one more, widths beside a multiple of the 256 columns, k of half a step of 64 and in whole pairs of steps, experts without
+rows, experts that hand their input through.
 
 Bound: the intermediate row, the expert's output row and the result are each rounded to bf16 once (2^-9 relative; the gelus
 also read a rounded product, whose error they pass on at most 1.13 times), sums are in f32. So the error of an element is at
@@ -15,14 +15,14 @@ pytestmark = pytest.mark.gpu
 
 #        T     W    F    E  top  act         through   rows per expert about
 CASES = [(1, 32, 32, 4, 2, "relu2", 0),
-         (257, 64, 96, 1, 1, "relu2", 0),          # one expert: 257 rows, one past a tall tile
-         (129, 288, 32, 2, 1, "gelu_tanh", 0),     # short tiles, one past or two part tiles
+         (257, 64, 96, 1, 1, "relu2", 0),          # one expert: 257 rows, one past a tile
+         (129, 288, 32, 2, 1, "gelu_tanh", 0),     # one past two blocks of 64 rows; k of half a step
          (256, 160, 288, 1, 1, "gelu", 0),
          (333, 32, 32, 16, 5, "relu2", 3),
-         (2500, 544, 224, 5, 3, "relu2", 1),       # tall tiles, several runs of the sort
+         (2500, 544, 224, 5, 3, "relu2", 1),       # several runs of the sort
          (9000, 128, 128, 70, 2, "relu2", 0)]      # more experts than a wave scans at once
-# tiles of 256 rows, which launches of more than 256 short tiles take from 96 rows an expert on: one row past the last tile, a part
-# tile, several experts with one that no one chose, handed through
+# more tiles than a round of 256 workgroups holds uncut: one row past the last tile, a part tile, several experts with one that no one
+# chose, handed through
 TALL = [(4097, 2080, 96, 1, 1, "relu2", 0), (4200, 2080, 224, 1, 1, "gelu", 0), (3000, 1568, 160, 4, 2, "relu2", 0),
         (1500, 2336, 288, 5, 4, "gelu_tanh", 2)]
 
@@ -86,6 +86,25 @@ def test_tiles_in_a_chain_match_the_exact_sum(gpu, T, W, F, E, top, act, uneven)
         y = mix_ops.moe_sorted_ff(h, ids, w, up, down, E, F, act)
     ref, S = exact(h, ids, w, up, down, E, F, act)
     assert ((y.double() - ref).abs() <= 3.5 * 2.0 ** -9 * S + 1e-6).all()
+
+
+@pytest.mark.parametrize("T,W,F,E,top,through", [(3000, 256, 384, 5, 3, 2), (9000, 512, 256, 2, 2, 3), (40, 256, 256, 3, 1, 1)])
+def test_chains_pass_over_the_tiles_of_experts_that_hand_through(gpu, T, W, F, E, top, through):
+    h, ids, w, up, down = operands(T, W, F, E, top, through, 1, T + through)
+    y = mix_ops.moe_sorted_ff(h, ids, w, up, down, E, F, "relu2", through)
+    ref, S = exact(h, ids, w, up, down, E, F, "relu2")
+    assert ((y.double() - ref).abs() <= 3.5 * 2.0 ** -9 * S + 1e-6).all()
+
+
+@pytest.mark.parametrize("T,W,F", [(43000, 1024, 128), (43000, 128, 1024)])
+def test_rows_written_past_the_caches(gpu, T, W, F):
+    """Two choices of 43000 tokens: 176 MB of rows of 1024, the outputs of either product; every 41st token."""
+    E, top = 3, 2
+    h, ids, w, up, down = operands(T, W, F, E, top, 0, 1, W)
+    y = mix_ops.moe_sorted_ff(h, ids, w, up, down, E, F)
+    some = torch.arange(0, T, 41, device=h.device)
+    ref, S = exact(h[some], ids[some], w[some], up, down, E, F, "relu2")
+    assert ((y[some].double() - ref).abs() <= 3.5 * 2.0 ** -9 * S + 1e-6).all()
 
 
 @pytest.mark.parametrize("T,W,F,E,top", [(1, 32, 32, 4, 2), (257, 96, 160, 1, 1), (700, 256, 288, 4, 2), (3000, 160, 96, 5, 3),
