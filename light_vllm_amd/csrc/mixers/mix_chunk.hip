@@ -304,7 +304,7 @@ __global__ __launch_bounds__(256, KIND == kChunkDelta ? 4 : KIND == kChunkStep ?
 // holds two waves a SIMD, and one's LDS reads, staging and row factors run beside the other's products.
 // NORM (delta rule, workgroups that hold whole heads): a chunk's outputs wait in registers for the barrier behind which the other waves' sums of
 // squares are there, and leave normed and gated with the next chunk: no f32 rows through memory and no launch to read them back. 16 x 1024 tokens, 16
-// heads of 128: 264 + 59 us in two launches, 301 in one (the layer 819 -> 795).
+// heads of 128: 267 + 59 us in two launches, 307 in one (the layer 829 -> 814).
 template <typename T, int KIND, int DT, int NW, int HPW, int MODE, bool NORM = false>
 __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
   static_assert(!NORM || (KIND == kChunkDelta && MODE == 0), "the norm follows the delta rule's whole sequences");

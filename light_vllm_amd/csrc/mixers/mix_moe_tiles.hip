@@ -107,7 +107,7 @@ struct MoeTileParams {
 };
 
 // Bound by the matrix cores at the rate that the card's power allows, and by the loads that feed them. 65536 rows through 2048 x 1536 and
-// back, on experts of 328 to 5490 rows: 385 + 385 us = 1071 TFLOP/s (372 + 371 with the rows past the caches), where steps of 32 k, one workgroup a tile and tiles of 256 or 128 rows
+// back, on experts of 328 to 5490 rows: 371 + 369 us = 1114 TFLOP/s (385 + 385 with the rows through the caches), where steps of 32 k, one workgroup a tile and tiles of 256 or 128 rows
 // took 432 + 499; 2048 rows an expert 396 + 396 (420 + 490); 16 to 400 rows an expert 1.02 to 1.23 times faster, whole layers.
 // Vendor GEMMs expert by expert took 1500 us for both, fragments straight from memory (moe_gemm_kernel) 3200.
 //

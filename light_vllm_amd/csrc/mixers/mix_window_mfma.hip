@@ -740,8 +740,8 @@ __device__ __forceinline__ void prompt_redo(int b, int h, int rw, const bf16_t* 
 
 // DN > 0, latent attention: a wave turns its 32 queries of DN entries into rows that meet the cached ones, rotates the DK - DV entries
 // behind them, and multiplies its sums by the head's value matrix before they leave, so that neither the DK entries a head that go in
-// nor the DV that come out pass through memory. 16 x 1024 tokens, 16 heads of 128 + 64 on rows of 192 + 64: 216 us, where this kernel took 177,
-// the two batched products around it 111 and the rotation's launch 27. A head's matrix comes in pieces of 8 KB through the wave's own part
+// nor the DV that come out pass through memory. 16 x 1024 tokens, 16 heads of 128 + 64 on rows of 192 + 64: 201 us, where this kernel took 177,
+// the two batched products around it 111 and the rotation's launch 27 (another box). A head's matrix comes in pieces of 8 KB through the wave's own part
 // of the two tiles, one piece on its way while the other is multiplied; all workgroups of a head run on one XCD (with 8 sequences times
 // head groups or a multiple), whose L2 holds it. A product's result rows are its matrix's columns in the order in which the next product
 // takes them, so that nothing is exchanged between lanes.
