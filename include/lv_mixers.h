@@ -237,8 +237,8 @@ int lv_latent_out_gate(const void* o, const void* gate, int64_t ld_gate, int gat
 /* Latent attention of prompt steps, bf16: out act [T, H, Dn] = per head W_uv times the weighted sum over the cached rows that the query
  * [W_uk q_n | rotated q_r] sees in a window, times sigmoid(gate).  q act [T, H, Dn + Dr], uk act [H, Dn, R], uv act [H, R, Dn], cache act
  * [pages, page, R + Dr] (the new tokens' rows stored), gate rows as lv_latent_out_gate or NULL, sinks f32 [H] or NULL.  H in
- * multiples of 4, Dn 64 or 128, R + Dr 192 + 64 (all 64 entries rotated, inv_freq f32 [32]) or 256 + 0, pages in multiples of 64; -2 for
- * other head sizes.  q, cache, uk, uv aligned to 16 bytes, out and per-channel gates (rows in multiples of 4) to 8. */
+ * multiples of 4, Dn 64 or 128, R + Dr 192 + 64 (all 64 entries rotated, inv_freq f32 [32]) or 256 + 0, pages in multiples of 64, scale
+ * above zero; -2 for other head sizes and 2^31 workgroups (32 queries of four heads each).  q, cache, uk, uv aligned to 16 bytes, out and per-channel gates (rows in multiples of 4) to 8. */
 int lv_latent_prompt_attn(const void* q, const void* cache, const void* uk, const void* uv, const void* inv_freq, const void* gate,
                           int64_t ld_gate, int gate_kind, void* out, const int32_t* cu_q, const int32_t* ctx_lens, const int32_t* block_tables,
                           int bt_stride, int B, int max_new_tokens, int H, int Dn, int Dr, int R, int page, int window, float scale,
