@@ -12,7 +12,9 @@
 namespace lvmix {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
-typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+typedef __attribute__((ext_vector_type(2))) float f32x2_t;
 typedef __attribute__((address_space(3))) uint8_t lds_u8;
 
 constexpr int kTileRows = 256;
@@ -106,9 +108,12 @@ struct MoeTileParams {
   bool past;               // outputs do not stay in the caches: they are written past them
 };
 
-// Bound by the matrix cores at the rate that the card's power allows, and by the loads that feed them. 65536 rows through 2048 x 1536 and
-// back, on experts of 328 to 5490 rows: 371 + 369 us = 1114 TFLOP/s (385 + 385 with the rows through the caches), where steps of 32 k, one workgroup a tile and tiles of 256 or 128 rows
-// took 432 + 499; 2048 rows an expert 396 + 396 (420 + 490); 16 to 400 rows an expert 1.02 to 1.23 times faster, whole layers.
+// Bound by the power that the products take: 16384 x 4096 x 4096 takes 404 us on 32 x 32 x 16 products and 376 on 16 x 16 x 32 ones, 290 both on zeros,
+// and where a step's reads, barriers and requests stand moves neither. Half as many passes over the accumulators for the same products
+// are what the smaller ones save (in a loop of products alone, without operands to bring, they are 5 % slower). The vendor's product takes 355 (265).
+// 65536 rows through 2048 x 1536 and back, on 32 experts of 1940 to 2200 rows: the layer 888 -> 842 us. Other experts, launches in a graph, 32 x 32 x 16
+// -> 16 x 16 x 32: 2048 x 1536, 32 experts, 4 each, 3000 tokens 212 -> 210, 7000 390 -> 362; 4096 x 3072, 6000 tokens 1225 -> 1150; gated units
+// 2048 x 1536, 16384 tokens 1280 -> 1195; up to 64 rows an expert, where memory is the bound, level to 1 % (96 x 160, 16384 tokens 61 -> 52).
 // Vendor GEMMs expert by expert took 1500 us for both, fragments straight from memory (moe_gemm_kernel) 3200.
 //
 // Four waves, one per SIMD: 64 MB rows x 256 columns of the product, each wave 32 MB x 128 of it in 64 MB accumulators. MB follows the
@@ -119,16 +124,15 @@ struct MoeTileParams {
 // straight from memory (global_load_lds); the swizzle is applied to the address a lane loads from. A wave multiplies fragments that it read
 // half a step before; 3/8 into a step everyone has read the rest of its slot, and the step after next is requested into it, spread over
 // the remaining 5/8 and most of the second half: in a row behind one barrier, as many as the L1 takes 1024 clocks for, they held up the
-// products behind them (408 us; with no requests at all 300). The slots are arrays of their own so that the compiler knows which loads a read
-// has to wait for.
+// products behind them. The slots are arrays of their own so that the compiler knows which loads a read has to wait for.
 // CHAIN (k in whole pairs of steps): a workgroup goes from tile to tile. The last two steps request the next tile's first two, which arrive while
 // the outputs leave through LDS of their own, and nothing waits for a store until a step later; a tile by itself spent some 15 us on
 // its way in and out. Other k drain the slots between tiles, and request the next tile's first steps in front of the outputs too (7000 tokens, 16 experts of
 // 1024 x 352, 4 each: the layer's experts 112 -> 107 us, 107 with the tiles of 128 rows that came before; 16384 tokens 222 -> 217, 240).
 // GLU: LDS rows 64 j .. 64 j + 31 of the weights hold gate columns 32 j .., the 32 after them the up columns of the same numbers.
-template <bool UP, bool GLU, bool CHAIN>
+template <bool UP, bool GLU, bool CHAIN, bool UNARY = false>
 __global__ __launch_bounds__(256, 1) void moe_tile_kernel(MoeTileParams p) {
-  static_assert(!GLU || UP, "the gated unit follows the first product");
+  static_assert((!GLU || UP) && (!UNARY || (UP && !GLU)), "gated units and activations follow the first product");
   constexpr int CW = GLU ? 128 : 256, WC = CW / 2;                   // output columns of a tile and of a wave
   constexpr int SLOT = 512 * 128, STAGE = 32 * WC * 2;               // bytes of a step's operands and of a wave's 32 output rows
   __shared__ __attribute__((aligned(1024))) uint8_t slot0[SLOT];
@@ -210,22 +214,21 @@ __global__ __launch_bounds__(256, 1) void moe_tile_kernel(MoeTileParams p) {
   };
   // half a step: the pieces past the end repeat those in front of them
   const uint32_t back = ((lane & 7) ^ (((w & 1) << 2) | ((lane >> 4) & 3))) >= 4 ? 64u : 0u;
-  auto request = [&](uint8_t* slot, int c, auto rows64, auto from, auto to) __attribute__((always_inline)) {      // loads from .. to - 1 of a tile of 64 rows64
+  auto request = [&](uint8_t* slot, int c, auto rows64, int x) __attribute__((always_inline)) {      // the x-th load of a tile of 64 rows64
     int at_k = c + first;                                            // requests past the end repeat some step; never used
     at_k = c < full ? (at_k < full ? at_k : at_k - full) : 64 * full < p.K ? full : 0;
     const uint32_t less = !CHAIN && at_k == full ? back : 0u;
     lds_u8* const at = (lds_u8*)slot;
     constexpr int na = 2 * decltype(rows64)::value;
-#pragma unroll
-    for (int x = decltype(from)::value; x < decltype(to)::value; ++x) {
-      const int i = x < na ? x : x - na;
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((x < na ? abase : bbase) + 128 * static_cast<int64_t>(at_k) + ((x < na ? aoff[i] : boff[i]) - less)),
-                                       (__attribute__((address_space(3))) void*)(at + (x < na ? 0 : 256 * 128) + 1024 * (w + 4 * i)), 16, 0, 0);
-    }
+    const int i = x < na ? x : x - na;
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((x < na ? abase : bbase) + 128 * static_cast<int64_t>(at_k) + ((x < na ? aoff[i] : boff[i]) - less)),
+                                     (__attribute__((address_space(3))) void*)(at + (x < na ? 0 : 256 * 128) + 1024 * (w + 4 * i)), 16, 0, 0);
   };
-  using I0 = std::integral_constant<int, 0>;
   using I4 = std::integral_constant<int, 4>;
-  using I16 = std::integral_constant<int, 16>;
+  auto request_all = [&](uint8_t* slot, int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int x = 0; x < 16; ++x) request(slot, c, I4{}, x);
+  };
   // own LDS reads done, own requests landed (and stores on their way out); then everyone's
   auto turn = [&]() __attribute__((always_inline)) {
     __builtin_amdgcn_s_waitcnt(0x0070);
@@ -234,95 +237,100 @@ __global__ __launch_bounds__(256, 1) void moe_tile_kernel(MoeTileParams p) {
 
   look_up(cur);
   aim(cur);
-  request(slot0, 0, I4{}, I0{}, I16{});
-  request(slot1, 1, I4{}, I0{}, I16{});
+  request_all(slot0, 0);
+  request_all(slot1, 1);
   turn();
   // one tile of up to 64 MB rows, whose first two steps lie in the slots or (CHAIN) the second is on its way there
   auto tile = [&](auto mb) __attribute__((always_inline)) {
     constexpr int MB = decltype(mb)::value;
-    constexpr int MUL = 8 * MB, READS = 2 * (MB + 4), EARLY = MUL * 3 / 8;
-    // fragments: lane l holds row l % 32 of a block, eight k from 8 (l / 32); half a step is 64 bytes across, its second part 32
-    const int here = lane_here(), lr = here & 31, lh = here >> 5;
-    const int fa0 = lr * 128 + ((lh ^ ((lr >> 1) & 7)) * 16) + wm * 32 * MB * 128;
-    const int fb0 = lr * 128 + ((lh ^ ((lr >> 1) & 7)) * 16) + 256 * 128 + wn * 128 * 128;
-    struct Frags { bf16x8_t a[2][MB], b[2][4]; };
-    auto fetch = [&](const uint8_t* slot, int second, Frags& f) __attribute__((always_inline)) {
-      const lds_u8* const at = (const lds_u8*)slot;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          f.b[h][i] = *reinterpret_cast<const __attribute__((address_space(3))) bf16x8_t*>(at + (fb0 ^ (64 * second + 32 * h)) + 4096 * i);
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
-          f.a[h][i] = *reinterpret_cast<const __attribute__((address_space(3))) bf16x8_t*>(at + (fa0 ^ (64 * second + 32 * h)) + 4096 * i);
-      }
+    constexpr int NB = 2 * MB, MUL = 8 * NB, READS = NB + 8, EARLY = MUL * 3 / 8;
+    // fragments: lane l holds row l % 16 of a block, eight k from 8 (l / 16); half a step is 64 bytes across
+    const int here = lane_here(), lr = here & 15, lq = here >> 4;
+    const int fa0 = lr * 128 + ((lq ^ ((lr >> 1) & 7)) * 16) + wm * 32 * MB * 128;
+    const int fb0 = lr * 128 + ((lq ^ ((lr >> 1) & 7)) * 16) + 256 * 128 + wn * 128 * 128;
+    struct Frags { bf16x8_t a[NB], b[8]; };
+    auto fetch = [&](const uint8_t* slot, int second, Frags& f, int x) __attribute__((always_inline)) {      // the x-th, in the products' order
+      auto at = [&](int where) __attribute__((always_inline)) {
+        return *reinterpret_cast<const __attribute__((address_space(3))) bf16x8_t*>((const lds_u8*)slot + where);
+      };
+      if (x == 0) f.b[0] = at(fb0 ^ (64 * second));
+      else if (x <= NB) f.a[x - 1] = at((fa0 ^ (64 * second)) + 2048 * (x - 1));
+      else f.b[x - NB] = at((fb0 ^ (64 * second)) + 2048 * (x - NB));
     };
-    f32x16_t acc[4][MB];
+    // The accumulators are tied to the accumulation registers: left to the compiler, 64 MB blocks of four are moved to and fro at every step.
+    // It does not know of the products' latency then: what reads the sums stands behind eight other products or the wait in front of the output.
+    f32x4_t acc[8][NB];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int j = 0; j < MB; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-    auto products = [&](const Frags& f, auto from, auto to) __attribute__((always_inline)) {
-#pragma unroll
-      for (int q = decltype(from)::value; q < decltype(to)::value; ++q) {
-        const int h = q / (4 * MB), i = q / MB % 4, j = q % MB;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.b[h][i], f.a[h][j], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < NB; ++j) {
+        acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        asm volatile("" : "+a"(acc[i][j]));                          // (in front of the barrier, and so of the first product)
       }
+    auto product = [&](const Frags& f, int i, int j) __attribute__((always_inline)) {
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(f.b[i]), "v"(f.a[j]));
     };
-    using IE = std::integral_constant<int, EARLY>;
-    using IM = std::integral_constant<int, MUL>;
     Frags f0, f1;                                                    // first and second half of a step
     auto step = [&](uint8_t* mine, const uint8_t* next, int c, auto landed, auto more, auto rows64) __attribute__((always_inline)) {
       constexpr bool MORE = decltype(more)::value;
       constexpr int LOADS = 8 + 2 * decltype(rows64)::value, R1 = MORE ? LOADS * 3 / 8 : LOADS, R2 = LOADS - R1, LATE = MUL - EARLY;
-      using IR = std::integral_constant<int, R1>;
-      using IL = std::integral_constant<int, LOADS>;
-      fetch(mine, 1, f1);
-      products(f0, I0{}, IE{});
 #pragma unroll
-      for (int g = 0; g < EARLY; ++g) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, (READS + EARLY - 1) / EARLY, 0);
+      for (int q = 0; q < EARLY; ++q) {
+        product(f0, q / NB, q % NB);
+#pragma unroll
+        for (int x = q * READS / EARLY; x < (q + 1) * READS / EARLY; ++x) fetch(mine, 1, f1, x);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_waitcnt(0xc07f);                            // nobody reads this slot any more
       asm volatile("s_barrier" ::: "memory");
-      request(mine, c, rows64, I0{}, IR{});
-      products(f0, IE{}, IM{});
 #pragma unroll
-      for (int g = 0; g < LATE; ++g) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if ((g + 1) * R1 / LATE > g * R1 / LATE) __builtin_amdgcn_sched_group_barrier(0x010, (R1 + LATE - 1) / LATE, 0);
+      for (int q = 0; q < LATE; ++q) {
+        product(f0, (EARLY + q) / NB, q % NB);
+#pragma unroll
+        for (int x = q * R1 / LATE; x < (q + 1) * R1 / LATE; ++x) request(mine, c, rows64, x);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (MORE) {
+      if constexpr (MORE) {                                          // (otherwise f1's products are left to the output)
         if constexpr (!decltype(landed)::value) __builtin_amdgcn_s_waitcnt((R1 & 15) | ((R1 >> 4) << 14) | 0x0f70);
         asm volatile("s_barrier" ::: "memory");                      // the other one is complete
-        fetch(next, 0, f0);
-        request(mine, c, rows64, IR{}, IL{});
-      }
-      products(f1, I0{}, IM{});
 #pragma unroll
-      for (int g = 0; g < MUL; ++g) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (MORE && g < READS) __builtin_amdgcn_sched_group_barrier(0x100, READS > MUL ? 2 : 1, 0);
-        if (MORE && (g + 1) * R2 / MUL > g * R2 / MUL) __builtin_amdgcn_sched_group_barrier(0x010, (R2 + MUL - 1) / MUL, 0);
+        for (int q = 0; q < MUL; ++q) {
+          product(f1, q / NB, q % NB);
+          if (q < EARLY) {
+#pragma unroll
+            for (int x = q * READS / EARLY; x < (q + 1) * READS / EARLY; ++x) fetch(next, 0, f0, x);
+          }
+#pragma unroll
+          for (int x = q * R2 / MUL; x < (q + 1) * R2 / MUL; ++x) request(mine, c, rows64, R1 + x);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
-      __builtin_amdgcn_sched_barrier(0);
     };
 
     Tile following;
     asm volatile("s_barrier" ::: "memory");                          // every wave's share of the first two steps has landed (awaited in front of its stores)
-    fetch(slot0, 0, f0);
+    // the rows' scales, asked for before a store is on its way: a load behind it would wait for it
+    int who[GLU ? NB : 1];
+    float rs[GLU ? NB : 1];
+    if constexpr (GLU) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) who[j] = p.sorted_pair[cur.row0 + min(wm * 32 * MB + 16 * j + lr, cur.nrows - 1)];
+    }
+    auto scales = [&]() __attribute__((always_inline)) {
+      if constexpr (GLU) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) rs[j] = p.row_scale[who[j]];
+      }
+    };
+#pragma unroll
+    for (int x = 0; x < READS; ++x) fetch(slot0, 0, f0, x);
     if constexpr (CHAIN) {
       following = find(cur.q + stride);
       if (following.nrows > 0) look_up(following);
       // (its first turn apart and without a condition: where it may be either, the compiler waits for loads that were requested behind it)
       step(slot0, slot1, 2, std::true_type{}, std::true_type{}, mb);
       step(slot1, slot0, 3, std::false_type{}, std::true_type{}, mb);
+      scales();
       for (int c = 4; c < full; c += 2) {
         step(slot0, slot1, c, std::false_type{}, std::true_type{}, mb);
         step(slot1, slot0, c + 1, std::false_type{}, std::true_type{}, mb);
@@ -337,83 +345,95 @@ __global__ __launch_bounds__(256, 1) void moe_tile_kernel(MoeTileParams p) {
         step(slot1, slot0, c + 3, std::false_type{}, std::true_type{}, mb);
       }
       if (c < full) step(slot0, slot1, c + 2, std::false_type{}, std::true_type{}, mb);
-      if (64 * full < p.K) products(f0, I0{}, IM{});
+      if (64 * full < p.K) {
+#pragma unroll
+        for (int q = 0; q < MUL; ++q) product(f0, q / NB, q % NB);
+      }
       following = find(cur.q + stride);
+      scales();
       turn();                                                   // nobody reads or fills the slots any more
       if (following.nrows > 0) {
         look_up(following);
         aim(following);
-        request(slot0, 0, I4{}, I0{}, I16{});
-        request(slot1, 1, I4{}, I0{}, I16{});
+        request_all(slot0, 0);
+        request_all(slot1, 1);
       }
     }
 
-    // Through the wave's own rows in LDS, 32 at a time, so that they leave in whole lines. acc[i][j][4 g + u] is column 32 i + 8 g + 4 lh + u
-    // of row 32 j + lr. The eight bytes of a lane go to 16-byte piece c ^ swizzle(row), the two halves of a piece swapped in every other
-    // block of 16 rows.
-    constexpr int PIECES = WC / 8, RPI = 64 / PIECES;                // 16-byte pieces of a row; rows per store instruction
+    // Through the wave's own rows in LDS, 16 at a time in one of two places, so that they leave in whole lines. acc[i][j][u] is column
+    // 16 i + 4 (lane / 16) + u of row 16 j + lane % 16. The eight bytes of a lane go to 16-byte piece c ^ swizzle(row).
+    constexpr int PIECES = WC / 8, RPI = 64 / PIECES, PARTS = 16 / RPI, OUT = GLU ? 4 : 8;      // 16-byte pieces of a row; rows per store instruction
     auto swz = [&](int r) { return (PIECES == 16 ? r : r >> 1) & (PIECES - 1); };
     lds_u8* const mine = (lds_u8*)stage + w * STAGE;
-    const int m0 = wm * 32 * MB, ln = lane_here(), er = ln & 31, eh = ln >> 5;
+    const int m0 = wm * 32 * MB, ln = lane_here(), er = ln & 15, eq = ln >> 4;
     typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+    auto put = [&](int j, int i) __attribute__((always_inline)) {    // columns 16 i .. of rows 16 j .. to their place
+      const int src = GLU ? 4 * (i >> 1) + (i & 1) : i;
+      asm volatile("" : "+a"(acc[src][j]));
+      if constexpr (GLU) asm volatile("" : "+a"(acc[src + 2][j]));
+      float v[4];
 #pragma unroll
-    for (int j = 0; j < MB; ++j) {
-      float rs = 1.0f;
-      if constexpr (GLU) rs = p.row_scale[p.sorted_pair[cur.row0 + min(m0 + 32 * j + er, cur.nrows - 1)]];
-#pragma unroll
-      for (int i = 0; i < (GLU ? 2 : 4); ++i)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          float v[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            if constexpr (GLU) {
-              const float x = fminf(acc[2 * i][j][4 * g + u] * rs, p.limit);
-              const float y = fminf(fmaxf(acc[2 * i + 1][j][4 * g + u] * rs, -p.limit), p.limit);
-              v[u] = rs != 0.0f ? x * sigmoidf_(p.alpha * x) * (y + 1.0f) : 0.0f;
-            } else {
-              v[u] = acc[i][j][4 * g + u];
-              if (UP && p.act == LV_MIX_ACT_RELU2) v[u] = v[u] < 0.0f ? 0.0f : v[u] * v[u];
-            }
-          }
-          uint32_t pair[2];
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            bf16_t lo, hi;
-            stf(&lo, v[2 * u]);
-            stf(&hi, v[2 * u + 1]);
-            pair[u] = static_cast<uint32_t>(lo.bits) | (static_cast<uint32_t>(hi.bits) << 16);
-          }
-          const int piece = (4 * i + g) ^ swz(er);
-          *reinterpret_cast<__attribute__((address_space(3))) uint64_t*>(mine + er * WC * 2 + piece * 16 + ((eh ^ (er >> 4)) & 1) * 8) =
-              static_cast<uint64_t>(pair[0]) | (static_cast<uint64_t>(pair[1]) << 32);
+      for (int u = 0; u < 4; ++u) {
+        if constexpr (GLU) {
+          const float x = fminf(acc[src][j][u] * rs[j], p.limit);
+          const float y = fminf(fmaxf(acc[src + 2][j][u] * rs[j], -p.limit), p.limit);
+          v[u] = rs[j] != 0.0f ? x * sigmoidf_(p.alpha * x) * (y + 1.0f) : 0.0f;
+        } else {
+          v[u] = acc[src][j][u];
+          if (UP && !UNARY) v[u] = v[u] < 0.0f ? 0.0f : v[u] * v[u];
         }
-      if (j == 0) __builtin_amdgcn_s_waitcnt(0x0f70);       // the next tile's first two steps have landed: nothing there waits for a store
-      auto leave = [&](int i, auto unary) __attribute__((always_inline)) {
-        const int r = i * RPI + ln / PIECES, c = ln % PIECES;
-        const int n = cur.n0 + wn * WC + 8 * c;
-        if (m0 + 32 * j + r >= cur.nrows || n >= p.N) return;        // N is a multiple of 8: a piece is in or out as a whole
-        u32x4 v = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(mine + r * WC * 2 + (c ^ swz(r)) * 16);
-        if ((r >> 4) & 1) v = u32x4{v[2], v[3], v[0], v[1]};
-        if constexpr (decltype(unary)::value) {
+      }
+      uint2 pair;
+      pair.x = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{v[0], v[1]}), bf16x2_t));
+      pair.y = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{v[2], v[3]}), bf16x2_t));
+      const int piece = (2 * i + (eq >> 1)) ^ swz(er);
+      *reinterpret_cast<__attribute__((address_space(3))) uint64_t*>(mine + (j & 1) * (STAGE / 2) + er * WC * 2 + piece * 16 + (((eq & 1) ^ (er >> 3)) & 1) * 8) =
+          static_cast<uint64_t>(pair.x) | (static_cast<uint64_t>(pair.y) << 32);
+    };
+    auto leave = [&](int j, int i) __attribute__((always_inline)) {  // part i of rows 16 j ..
+      const int r = i * RPI + ln / PIECES, c = ln % PIECES;
+      const int n = cur.n0 + wn * WC + 8 * c;
+      u32x4 v = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(mine + (j & 1) * (STAGE / 2) + r * WC * 2 + (c ^ swz(r)) * 16);
+      if (m0 + 16 * j + r >= cur.nrows || n >= p.N) return;          // N is a multiple of 8: a piece is in or out as a whole
+      if ((r >> 3) & 1) v = u32x4{v[2], v[3], v[0], v[1]};
+      if constexpr (UNARY) {
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            bf16_t lo, hi;
-            stf(&lo, mix_act(__builtin_bit_cast(float, v[u] << 16), p.act));
-            stf(&hi, mix_act(__builtin_bit_cast(float, v[u] & 0xffff0000u), p.act));
-            v[u] = static_cast<uint32_t>(lo.bits) | (static_cast<uint32_t>(hi.bits) << 16);
-          }
+        for (int u = 0; u < 4; ++u) {
+          bf16_t lo, hi;
+          stf(&lo, mix_act(__builtin_bit_cast(float, v[u] << 16), p.act));
+          stf(&hi, mix_act(__builtin_bit_cast(float, v[u] & 0xffff0000u), p.act));
+          v[u] = static_cast<uint32_t>(lo.bits) | (static_cast<uint32_t>(hi.bits) << 16);
         }
-        u32x4* const to = reinterpret_cast<u32x4*>(p.C + static_cast<int64_t>(cur.row0 + m0 + 32 * j + r) * p.ldc + n);
-        if (p.past) __builtin_nontemporal_store(v, to);
-        else *to = v;
-      };
-      if (!UP || GLU || p.act == LV_MIX_ACT_RELU2) {
-#pragma unroll
-        for (int i = 0; i < 32 / RPI; ++i) leave(i, std::false_type{});
+      }
+      auto to = (__attribute__((address_space(1))) u32x4*)(p.C + static_cast<int64_t>(cur.row0 + m0 + 16 * j + r) * p.ldc + n);
+      if (p.past) {
+        asm volatile("" : "+v"(to));                                 // (keeps the two stores apart: as one they are both plain)
+        __builtin_nontemporal_store(v, to);
+        asm volatile("" ::: "memory");
       } else {
+        *to = v;
+      }
+    };
+    if constexpr (CHAIN) {                                           // the last half step
+#pragma unroll
+      for (int q = 0; q < MUL; ++q) product(f1, q / NB, q % NB);
+    }
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");               // the last sums are there
+    __builtin_amdgcn_sched_barrier(0);
+    // rows 16 (j + 1) go to LDS in front of the stores of rows 16 j
+#pragma unroll
+    for (int j = 0; j <= NB; ++j) {
+      if (j < NB) {
+#pragma unroll
+        for (int i = 0; i < OUT; ++i) put(j, i);
+      }
+      if (j == 0) __builtin_amdgcn_s_waitcnt(0x0f70);                // the next tile's first two steps have landed: nothing there waits for a store
+      if (j > 0 && !UNARY) {
+#pragma unroll
+        for (int i = 0; i < PARTS; ++i) leave(j - 1, i);
+      } else if (j > 0) {
 #pragma unroll 1
-        for (int i = 0; i < 32 / RPI; ++i) leave(i, std::true_type{});
+        for (int i = 0; i < PARTS; ++i) leave(j - 1, i);
       }
     }
     cur = following;
@@ -455,10 +475,17 @@ template <bool UP, bool GLU>
 void tile_launch(const MoeTileParams& p, int64_t most, hipStream_t s) {
   const int64_t groups = 4 * most * ((p.N + (GLU ? 127 : 255)) / (GLU ? 128 : 256));      // one round: tiles may be cut in four
   const dim3 grid(static_cast<unsigned>(groups < 256 ? (groups + 7) / 8 * 8 : 256)), block(256);
-  if (p.K % 128 == 0 && p.K >= 256)
-    moe_tile_kernel<UP, GLU, true><<<grid, block, 0, s>>>(p);
-  else
-    moe_tile_kernel<UP, GLU, false><<<grid, block, 0, s>>>(p);
+  auto go = [&](auto unary) {
+    constexpr bool U = decltype(unary)::value;
+    if (p.K % 128 == 0 && p.K >= 256)
+      moe_tile_kernel<UP, GLU, true, U><<<grid, block, 0, s>>>(p);
+    else
+      moe_tile_kernel<UP, GLU, false, U><<<grid, block, 0, s>>>(p);
+  };
+  if constexpr (UP && !GLU) {
+    if (p.act != LV_MIX_ACT_RELU2) return go(std::true_type{});
+  }
+  go(std::false_type{});
 }
 
 }  // namespace
@@ -507,8 +534,8 @@ int lv_moe_tiled_ff(const void* h, const void* ids, const void* weights, const v
                                                                                counts);
   moe_place_kernel<<<dim3(runs), dim3(kPlaceThreads), 3 * sizeof(int32_t) * E, s>>>(
       pid, static_cast<int>(M), static_cast<int>(E), run, counts, sorted_pair, inv, tiles, num_tiles, static_cast<int>(most));
-  // The operands of a tile's neighbours are what the L2s are for. Layers on 16384 tokens (201 and 268 MB) 918 us with outputs through them,
-  // 907 past them; up to 6900 tokens (112 MB) the step behind finds some of them and reading them again takes 1 % longer.
+  // The operands of a tile's neighbours are what the L2s are for. Layers on 16384 tokens (201 and 268 MB) 855 us with outputs through them,
+  // 845 past them; up to 6900 tokens (112 MB) the step behind finds some of them and reading them again takes 1 % longer.
   auto past = [&](int64_t width) { return M * width * 2 > int64_t{160} << 20; };
   MoeTileParams up{static_cast<const uint16_t*>(h), static_cast<const uint16_t*>(up_w), mid, sorted_pair, tiles, num_tiles,
                    F, W, top, E_real, W, W, F, static_cast<int64_t>(glu ? 2 : 1) * F * W,
