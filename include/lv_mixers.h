@@ -24,6 +24,7 @@
  *   lv_latent_prompt_attn    what lies between lv_latent_prep and the output projection, in one launch, for prompt steps
  *   lv_moe_route             sigmoid router with a selection-only correction, group limit and top-k
  *   lv_router_logits         f32 router logits of steps of few tokens, straight from the activations
+ *   lv_router_tiles          the same for prompt steps of bf16 activations
  *   lv_relu2_scale           squared relu of the experts' up projections times the routing weight
  *   lv_moe_grouped_ff        the experts' feed-forward on rows sorted by expert (grouped GEMMs on the matrix cores)
  *   lv_moe_tiled_ff          the same for prompt steps, on LDS tiles
@@ -92,7 +93,7 @@
 extern "C" {
 #endif
 
-#define LV_MIX_ABI_VERSION 14
+#define LV_MIX_ABI_VERSION 15
 #define LV_MIX_BF16 0
 #define LV_MIX_F32 1
 #define LV_MIX_MAX_STREAMS 8
@@ -257,6 +258,11 @@ int lv_moe_route(const void* logits, const void* correction, void* ids, void* we
  * f32 [E, W]), without a widened copy of h; one workgroup per (token, four experts). */
 int lv_router_logits(const void* h, int64_t ld_h, const void* router_w, void* logits, int64_t T, int W, int E, int dtype,
                      void* stream);
+
+/* Router logits of prompt steps: the same product for bf16 h on the f32 matrix instructions, 64 tokens a workgroup. One chain of sums over W in
+ * blocks of 16, four entries 4 apart a step. W a multiple of 256, E 16, 32, 48 or 64, ld_h a multiple of 8, h, router_w and logits at
+ * multiples of 16 bytes, T < 2^30. */
+int lv_router_tiles(const void* h, int64_t ld_h, const void* router_w, void* logits, int64_t T, int W, int E, void* stream);
 
 /* up act [T, E*F] (all experts' up projections side by side), dense f32 [T, E]:
  * out act [T, E*F] = relu(up)^2 * dense[t, e]. */

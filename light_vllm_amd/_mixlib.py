@@ -18,8 +18,8 @@ CSRC = os.path.join(_HERE, "csrc", "mixers")
 LIB_PATH = os.path.join(_HERE, "lib", "liblvmix.so")
 SOURCES = ["mix_stream.hip", "mix_window_attn.hip", "mix_window_mfma.hip", "mix_latent.hip", "mix_moe_gemm.hip",
            "mix_moe_tiles.hip", "mix_sandwich.hip", "mix_parallel.hip", "mix_recurrent.hip", "mix_prep.hip", "mix_lru.hip", "mix_chunk.hip",
-           "mix_rows_gemm.hip"]
-ABI_VERSION = 14
+           "mix_rows_gemm.hip", "mix_router.hip"]
+ABI_VERSION = 15
 
 _P = c_void_p
 SIGNATURES = {
@@ -54,6 +54,7 @@ SIGNATURES = {
                                       c_int, c_int, c_float, _P, _P]),
     "lv_moe_route": (c_int, [_P, _P, _P, _P, _P, c_int64, c_int, c_int, c_int, c_int, c_int, _P]),
     "lv_router_logits": (c_int, [_P, c_int64, _P, _P, c_int64, c_int, c_int, c_int, _P]),
+    "lv_router_tiles": (c_int, [_P, c_int64, _P, _P, c_int64, c_int, c_int, _P]),
     "lv_relu2_scale": (c_int, [_P, _P, _P, c_int64, c_int, c_int, c_int, _P]),
     "lv_moe_grouped_ff": (c_int, [_P, _P, _P, _P, _P, _P, _P, c_int64, c_int, c_int, c_int, c_int, _P]),
     "lv_moe_grouped_workspace_bytes": (c_int64, [c_int64, c_int, c_int, c_int, c_int]),
