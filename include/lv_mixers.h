@@ -70,6 +70,7 @@
  *   lv_gated_linear_recurrence   Griffin's RG-LRU: block-diagonal gates, S <- a S + sqrt(1 - a^2) i u per channel, gelu branch
  *   lv_scaled_embedding      token rows times a constant as the f32 residual
  *   lv_rows_gemm             projections of up to 64 rows
+ *   lv_columns_gemm          up to 64 columns of a projection of many rows
  *   lv_delta_prep_one, lv_delta_rule_one   the delta rule on steps of one token a sequence, two launches instead of four
  *   lv_residual_split        residual update, and the residual as the sum of two bf16 numbers for a matrix product
  *
@@ -542,6 +543,9 @@ int lv_delta_rule_one(const void* qn, const void* kn, const void* v, const void*
 /* y bf16 [M, N] = x bf16 [M, K] w^T, w bf16 [N, K], sums in f32. M <= 64, K a multiple of 32; row strides ldx, ldw (multiples of 8)
  * and ldy in entries; x and w 16-byte, y 8-byte aligned. */
 int lv_rows_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, int64_t ldy, int M, int N, int K, void* stream);
+
+/* The same for any number of rows and at most 64 columns (N <= 64, ldx >= K). */
+int lv_columns_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, int64_t ldy, int64_t M, int N, int K, void* stream);
 
 #ifdef __cplusplus
 }

@@ -1,6 +1,6 @@
 """Tensor-parallel linear layers (reference: lightvllm/layers/linear.py).
 
-The GEMMs are mix_ops.linear: hipBLASLt, and a kernel of our own for the few rows of a decode step. What matters to the attention path is the
+The GEMMs are mix_ops.linear: hipBLASLt, and kernels of our own for the few rows of a decode step and the few columns beside whole tiles. What matters to the attention path is the
 sharding: QKVParallelLinear gives rank r the query heads [r*Hq/tp, (r+1)*Hq/tp) and kv heads
 [r*Hkv/tp, (r+1)*Hkv/tp) in a fused [q | k | v] output (linear.py:240-310), so attention needs no
 communication, and RowParallelLinear sums the per-rank partial outputs with one in-place
@@ -18,7 +18,7 @@ from . import tp
 from .tp import divide, tp_rank, tp_size
 
 _scripting, _compiling, _tracing, _Tensor = torch.jit.is_scripting, torch.compiler.is_compiling, torch._C._is_tracing, torch.Tensor
-_FEW = mix_ops.ROWS_GEMM_MAX
+_FEW, _MANY = mix_ops.ROWS_GEMM_MAX, mix_ops.SPLIT_FROM
 
 
 def _linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
@@ -26,7 +26,7 @@ def _linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) ->
         # mix_ops.linear's first looks, without a call: a prompt's step on few tokens is bound by the host, and goes on to torch's linear here
         if bias is None and type(x) is _Tensor and not _compiling() and not _tracing():
             shape = x.shape
-            if len(shape) == 2 and shape[0] <= _FEW:
+            if len(shape) == 2 and (shape[0] <= _FEW or shape[0] >= _MANY):
                 return mix_ops.linear(x, weight)
     return F.linear(x, weight, bias)
 

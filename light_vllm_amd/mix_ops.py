@@ -1951,11 +1951,52 @@ class _RowsLinear(torch.autograd.Function):
         return (dy.mm(w) if ctx.needs_input_grad[0] else None), (dy.t().mm(x) if ctx.needs_input_grad[1] else None), None
 
 
+COLUMNS_GEMM_MAX = 64        # columns that lv_columns_gemm takes
+SPLIT_FROM = 4096            # rows from which a product may leave its last columns to lv_columns_gemm
+
+
+def _split_sizes(x, w):
+    """(M, N, columns of the vendor's part, K, row strides of x and of w) if linear(x, w) is formed in two launches, the vendor's product of whole
+    tiles and lv_columns_gemm for the columns beside them; None otherwise. Taken where the vendor's 256 x 256 tiles fill whole rounds of the
+    256 compute units without the columns and open one more with them. us, whole / in two (16384 x 2048 x 32 takes the second 13):
+    16384 rows of 2048: 1040 columns 78 / 65, 3088 202 / 155, 4128 250 / 200, 5152 274 / 245, 6176 343 / 285; 8192: 4128 137 / 104,
+    6176 213 / 148; 4096: 4128 73 / 55; 8192 rows of 4096: 10304 527 / 446. Where rounds end in the middle the vendor's choices for the two
+    products are what decides: 9500 x 5152 212 / 246, 17233 x 6176 332 / 370, 12500 x 5152 232 / 188, 8192 x 5152 136 / 154."""
+    if type(x) not in _PLAIN or type(w) not in _PLAIN or _compiling() or _tracing():
+        return None
+    shape = x.shape
+    if len(shape) != 2 or w.dim() != 2:
+        return None
+    (M, K), (N, k) = shape, w.shape
+    if M < SPLIT_FROM or M % 256 or not 0 < N % 256 <= COLUMNS_GEMM_MAX or N % 4 or (M // 256 * (N // 256)) % 256 or N < 256 or k != K or K < 1024 or K % 64:
+        return None
+    if not x.is_cuda or x.dtype is not torch.bfloat16 or w.dtype is not torch.bfloat16 or _transformed():
+        return None
+    (ldx, one_x), (ldw, one_w) = x.stride(), w.stride()
+    dev = x.get_device()
+    if (one_x != 1 or one_w != 1 or ldx < K or ldw < K or ldx % 8 or ldw % 8 or (x.data_ptr() | w.data_ptr()) & 15 or w.get_device() != dev
+            or dev != torch.cuda.current_device() or torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
+        return None
+    return M, N, N // 256 * 256, K, ldx, ldw
+
+
+def _split_linear(x, w, sizes):
+    M, N, N0, K, ldx, ldw = sizes
+    y = x.new_empty((M, N))
+    torch.mm(x, w[:N0].t(), out=y[:, :N0])
+    lib = _mixlib.load()
+    _mixlib.check(lib.lv_columns_gemm(x.data_ptr(), ldx, w.data_ptr() + 2 * N0 * ldw, ldw, y.data_ptr() + 2 * N0, N, M, N - N0, K,
+                                      torch._C._cuda_getCurrentRawStream(x.get_device())), "lv_columns_gemm")
+    return y
+
+
 def linear(x, w):
-    """x [..., K] w [N, K]^T. Few rows of bf16 (decode steps) take lv_rows_gemm, everything else torch's linear."""
+    """x [..., K] w [N, K]^T. Few rows of bf16 (decode steps) take lv_rows_gemm, many rows and a few columns more than whole tiles two launches
+    (_split_sizes), everything else torch's linear."""
     sizes = _rows_gemm_sizes(x, w)
     if sizes is None:
-        return F.linear(x, w)
+        sizes = _split_sizes(x, w)
+        return F.linear(x, w) if sizes is None else _split_linear(x, w, sizes)
     if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
         return _RowsLinear.apply(x, w, sizes)
     return _rows_gemm(x, w, sizes)
