@@ -28,7 +28,7 @@
 // branch between. The token loop they replace did fewer operations, but on the vector ALU, one token behind the other. Kernels of a
 // layer, us, token loop -> f32 chunks -> staged among the products / on bf16 instructions: 16 x 1024 tokens, delta rule (16 heads, 128 x
 // 128) 993 -> 377 -> 343; constant decays (16 heads, 128 x 128) 596 -> 295 -> 281; step sizes (32 heads, 128 x 64; 7 prompts, the longest
-// 3750) 1531 -> 456 -> 323, 314 with three waves a SIMD in front of the scan. Pieces for the other two kinds, whose q, k and v are f32, were built and gained nothing: six to eight
+// 3750) 1531 -> 456 -> 323, 314 with three waves a SIMD in front of the scan. Pieces for all products of the other two kinds, whose q, k and v are f32, were built and gained nothing: six to eight
 // products for one, and every row to cut.
 #include "mix_common.h"
 
@@ -298,6 +298,27 @@ __global__ __launch_bounds__(256, KIND == kChunkDelta ? 4 : KIND == kChunkStep ?
   }
 }
 
+// Three bf16 numbers whose sum is a finite f32 value: its 24 bits cut into eights, so that nothing is rounded. As operands of the bf16
+// matrix instructions (exact products, f32 sums) they give f32 products at four to eight times the f32 instructions' rate. An
+// infinity has no such pieces: a wave that meets one computes its chunk on the f32 instructions.
+struct Pieces4 { uint2 p[3]; };
+__device__ __forceinline__ uint32_t high_halves(float a, float b) {
+  return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
+}
+__device__ __forceinline__ float below_high(float a) { return a - __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, a) & 0xffff0000u); }
+__device__ __forceinline__ Pieces4 cut4(float x, float y, float z, float w) {
+  Pieces4 r;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    r.p[i] = uint2{high_halves(x, y), high_halves(z, w)};
+    if (i < 2) { x = below_high(x); y = below_high(y); z = below_high(z); w = below_high(w); }
+  }
+  return r;
+}
+__device__ __forceinline__ chunk_bf16x8 join8(uint2 lo, uint2 hi) {
+  return __builtin_bit_cast(chunk_bf16x8, uint4{lo.x, lo.y, hi.x, hi.y});
+}
+
 // MODE 0: the whole sequence; 1: what a segment adds to the state, and its decay; 2: a segment from its starting state.
 // grid: (heads / HPW * column parts, segments, sequences), NW waves on 16 columns of the state each: the columns of one head,
 // or of HPW heads of one group (they share q and k). Sixteen columns and not 32: a compute unit that gets one workgroup then
@@ -305,12 +326,21 @@ __global__ __launch_bounds__(256, KIND == kChunkDelta ? 4 : KIND == kChunkStep ?
 // NORM (delta rule, workgroups that hold whole heads): a chunk's outputs wait in registers for the barrier behind which the other waves' sums of
 // squares are there, and leave normed and gated with the next chunk: no f32 rows through memory and no launch to read them back. 16 x 1024 tokens, 16
 // heads of 128: 267 + 59 us in two launches, 307 in one (the layer 829 -> 814).
+// CUT (delta rule, 128 rows of the state, eight waves): K^T U on the bf16 instructions, K and U cut into three pieces each (K once, where it is
+// staged; the state's other products would have it cut in every chunk): 1024 clocks a wave and chunk for 2048 of the chain's 6900 at the f32 rate. Sixteen
+// prompts of 1024 tokens, the layer 818 -> 803 us; 32 of 500 904 -> 888. States are 5.4 to 5.6e-8 off 64 bits (5.6 to 6.0 on f32 products: fewer roundings at the
+// state's magnitude), outputs 0.866e-7 either way. Constant decays gain nothing (833 / 836: their time is the silu of q, k and v), nor
+// do launches of four waves (one prompt of 1000 250 / 255). Chunks with a value that is not finite take the f32 products.
 template <typename T, int KIND, int DT, int NW, int HPW, int MODE, bool NORM = false>
 __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
   static_assert(!NORM || (KIND == kChunkDelta && MODE == 0), "the norm follows the delta rule's whole sequences");
   constexpr bool DELTA = KIND == kChunkDelta, SILU = KIND == kChunkConst, FULL = MODE != 1;
   constexpr int D = DT * 16, RS = D + kPad, PS = kCh + kPad, NT = NW * 64, WPW = NW / HPW;
   constexpr int MATS = FULL ? HPW * (DELTA ? 2 : 1) : 0;       // P of every head, then T of every head
+  constexpr bool CUT = DELTA && DT == 8 && NW == 8;            // K^T U from pieces
+  constexpr int KB = D * 2 + 16, kImg = kCh * KB;              // bytes of a row and of an image of pieces
+  __shared__ __attribute__((aligned(16))) unsigned char kc_all[2][CUT ? 3 * kImg : 16];
+  __shared__ int odd_all[2][NW];                               // whether a wave staged a k that is not finite
   __shared__ __attribute__((aligned(16))) float k_all[2][kCh * RS];
   __shared__ __attribute__((aligned(16))) float q_all[2][FULL ? kCh * RS : 4];
   __shared__ __attribute__((aligned(16))) float pt_all[2][MATS > 0 ? MATS : 1][MATS > 0 ? kCh * PS : 4];
@@ -476,11 +506,23 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
   };
   f32x4 U_next[2];
   auto stage = [&](int buf) __attribute__((always_inline)) {
+    float odd_k = 0.0f;                                // NaN if a value is not finite
 #pragma unroll
     for (int it = 0; it < KQ; ++it) {
-      const int at = (kq_tok + it * (NT / (D / 4))) * RS + kq_off;
-      st4(k_all[buf] + at, four(kreg[it]));
+      const int tok = kq_tok + it * (NT / (D / 4)), at = tok * RS + kq_off;
+      const float4 kv = four(kreg[it]);
+      st4(k_all[buf] + at, kv);
+      if constexpr (CUT) {
+        odd_k = fmaf(kv.x, 0.0f, fmaf(kv.y, 0.0f, fmaf(kv.z, 0.0f, fmaf(kv.w, 0.0f, odd_k))));
+        const Pieces4 c = cut4(kv.x, kv.y, kv.z, kv.w);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) *reinterpret_cast<uint2*>(kc_all[buf] + i * kImg + tok * KB + 2 * kq_off) = c.p[i];
+      }
       if constexpr (FULL) st4(q_all[buf] + at, four(qreg[it]));
+    }
+    if constexpr (CUT) {
+      const bool odd = __builtin_amdgcn_ballot_w64(odd_k != 0.0f) != 0;
+      if (lane == 0) odd_all[buf][w] = odd;
     }
 #pragma unroll
     for (int it = 0; it < PN; ++it) {
@@ -545,20 +587,61 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
 #pragma unroll
     for (int x = 0; x < 2; ++x) u2[x] = scale4(U[x], rows4(ge_lds[hw] + kCh, x));
     const float g_last = ge_lds[hw][cn - 1];
-    stage(buf ^ 1);                                    // (behind the last chunk for nobody: without a branch, among the products)
+    bool odd = !CUT;
+    if constexpr (CUT) {
+      float z = 0.0f;
 #pragma unroll
-    for (int j = 0; j < DT; ++j) {
-      // constant decays, slow as a rule: what the chunk adds in two sums of its own, for fewer roundings at the state's magnitude
-      constexpr bool APART = KIND == kChunkConst;
-      f32x4 add[2] = {APART ? zero : S[j] * g_last, zero};
+      for (int i = 0; i < 8; ++i) z = fmaf(u2[i >> 2][i & 3], 0.0f, z);
+      odd = __builtin_amdgcn_ballot_w64(z != 0.0f || odd_all[buf][lane & (NW - 1)] != 0) != 0;
+    }
+    if (CUT && __builtin_expect(!odd, 1)) {
+      // lane slots of a product: tokens 4 quad .. + 3 and 16 + 4 quad .. + 3, as u2 has them; K^T comes transposed out of LDS
+      using lds_bf16x4 = __attribute__((address_space(3))) chunk_bf16x4;
+      const unsigned char* kt = kc_all[buf] + (4 * quad + (r >> 2)) * KB + 8 * (r & 3);
+      const Pieces4 ua = cut4(u2[0][0], u2[0][1], u2[0][2], u2[0][3]), ub = cut4(u2[1][0], u2[1][1], u2[1][2], u2[1][3]);
+      chunk_bf16x8 uc[3];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        f32x4& to = add[APART ? i >> 2 : 0];
-        to = __builtin_amdgcn_mfma_f32_16x16x4f32(k_lds[(16 * (i >> 2) + 4 * quad + (i & 3)) * RS + 16 * j + r], u2[i >> 2][i & 3], to, 0, 0, 0);
+      for (int i = 0; i < 3; ++i) uc[i] = join8(ua.p[i], ub.p[i]);
+      stage(buf ^ 1);                                  // (behind the last chunk for nobody: without a branch, among the products)
+#pragma unroll
+      for (int j = 0; j < DT; ++j) {
+        chunk_bf16x8 kc[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const chunk_bf16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(kt + i * kImg + 32 * j));
+          const chunk_bf16x4 c = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(kt + i * kImg + 16 * KB + 32 * j));
+          kc[i] = chunk_bf16x8{a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
+        }
+        f32x4 add = zero;
+        auto mm = [&](int a, int c) __attribute__((always_inline)) { add = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kc[a], uc[c], add, 0, 0, 0); };
+        mm(2, 1);                                      // smallest products first; the two least pieces' is below a rounding
+        mm(1, 2);
+        mm(2, 0);
+        mm(0, 2);
+        mm(1, 1);
+        mm(1, 0);
+        mm(0, 1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) add[i] = fmaf(S[j][i], g_last, add[i]);
+        mm(0, 0);
+        S[j] = add;
       }
+    } else {
+      stage(buf ^ 1);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        S[j][i] = APART ? fmaf(S[j][i], g_last, fmaf(S[j][i], cn == kCh ? g_rest : 0.0f, add[0][i] + add[1][i])) : add[0][i];
+      for (int j = 0; j < DT; ++j) {
+        // constant decays, slow as a rule: what the chunk adds in two sums of its own, for fewer roundings at the state's magnitude
+        constexpr bool APART = KIND == kChunkConst;
+        f32x4 add[2] = {APART ? zero : S[j] * g_last, zero};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          f32x4& to = add[APART ? i >> 2 : 0];
+          to = __builtin_amdgcn_mfma_f32_16x16x4f32(k_lds[(16 * (i >> 2) + 4 * quad + (i & 3)) * RS + 16 * j + r], u2[i >> 2][i & 3], to, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          S[j][i] = APART ? fmaf(S[j][i], g_last, fmaf(S[j][i], cn == kCh ? g_rest : 0.0f, add[0][i] + add[1][i])) : add[0][i];
+      }
     }
     if (c0 + 2 * kCh < s1) fetch(c0 + 2 * kCh);
     if constexpr (NORM) {
@@ -590,27 +673,6 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
       for (int i = 0; i < 4; ++i) to[(16 * j + i) * p.Dv + st_off] = S[j][i];
   }
   if (MODE == 1 && lane == 0) p.seg_decay[(static_cast<int64_t>(b) * p.segs + blockIdx.y) * p.H + h] = static_cast<float>(seg_dec);
-}
-
-// Three bf16 numbers whose sum is a finite f32 value: its 24 bits cut into eights, so that nothing is rounded. As operands of the bf16
-// matrix instructions (exact products, f32 sums) they give f32 products at four to eight times the f32 instructions' rate. An
-// infinity has no such pieces: a wave that meets one computes its chunk on the f32 instructions.
-struct Pieces4 { uint2 p[3]; };
-__device__ __forceinline__ uint32_t high_halves(float a, float b) {
-  return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
-}
-__device__ __forceinline__ float below_high(float a) { return a - __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, a) & 0xffff0000u); }
-__device__ __forceinline__ Pieces4 cut4(float x, float y, float z, float w) {
-  Pieces4 r;
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    r.p[i] = uint2{high_halves(x, y), high_halves(z, w)};
-    if (i < 2) { x = below_high(x); y = below_high(y); z = below_high(z); w = below_high(w); }
-  }
-  return r;
-}
-__device__ __forceinline__ chunk_bf16x8 join8(uint2 lo, uint2 hi) {
-  return __builtin_bit_cast(chunk_bf16x8, uint4{lo.x, lo.y, hi.x, hi.y});
 }
 
 // The same scan for step sizes, whose q, k and v rows are bf16: an f32 value on the other side of a product is cut into its pieces, and

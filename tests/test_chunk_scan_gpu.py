@@ -275,3 +275,41 @@ def test_segments_of_every_instance(kind, H, G, D, Dv, new, seg, monkeypatch):
         assert rel(o, want_o + skip) < 2 * REL and rel(s, want_s) < 2 * REL
         err.append(rel(o, want_o + skip))
     assert asked == [0, seg] and err[1] <= 1.15 * err[0]
+
+
+# launches of more than 128 workgroups: eight waves each, and the delta rule's states of 128 rows grow by products of bf16 pieces
+@pytest.mark.parametrize("H,G,Dv", [(32, 8, 128), (48, 8, 64), (24, 24, 128)])
+def test_large_delta_launches(H, G, Dv):
+    new = [33, 64, 95, 1, 40, 71, 130]
+    call, args, _ = case("delta", new, H, G, 128, Dv, seed=H + Dv)
+    step = make_step(new, [0, 4, 0, 9, 1, 0, 2])
+    state = 0.3 * torch.randn(len(new), H, 128, Dv, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    want_o, want_s = recurrence(*args, state, step)
+    o = call(state, step)
+    assert rel(o, want_o) < REL and rel(state, want_s) < REL
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan"), -3e38])
+def test_large_delta_launches_with_values_that_are_not_finite(bad):
+    """A key, a value, a state entry or sums that are not finite reach the tokens behind them and no earlier or other row."""
+    H, G, D, Dv, new = 32, 8, 128, 128, [100] * 6
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    T = sum(new)
+    q, k = (F.normalize(torch.randn(T, G, D, device="cuda", generator=gen), dim=-1) for _ in range(2))
+    v = torch.randn(T, H, Dv, device="cuda", generator=gen)
+    beta, g = torch.rand(T, H, device="cuda", generator=gen), 0.5 + 0.5 * torch.rand(T, H, device="cuda", generator=gen)
+    state = torch.randn(6, H, D, Dv, device="cuda", generator=gen)
+    s0 = state.clone()
+    want = mix_ops.gated_delta_rule(q, k, v, beta, g, s0, make_step(new, [3] * 6))
+    k[140, 2, 7], v[270, 9, 5], v[310, 3, 100] = bad, bad, bad      # sequences 1, 2 and 3
+    state[1, 20, 3, 4] = bad                                        # slot 1: sequence 4
+    s1 = state.clone()
+    got = mix_ops.gated_delta_rule(q, k, v, beta, g, s1, make_step(new, [3] * 6))
+    heads = [h for h in range(H) if not 8 <= h < 12]                # heads that do not read the key
+    cols = [c for c in range(Dv) if c not in (4, 5, 100)]
+    # a wave that sees such a value sums its chunk in another order: what it does not reach is off by the two sums' roundings
+    for x, y in [(got[:140], want[:140]), (got[140:200, heads], want[140:200, heads]), (got[200:270], want[200:270]), (got[300:310], want[300:310]),
+                 (got[200:][:, :, cols], want[200:][:, :, cols]), (s1[0], s0[0]), (s1[5], s0[5]), (s1[1][:, :, cols], s0[1][:, :, cols])]:
+        assert rel(x, y.to(F64)) < 2 * REL
+    if bad == bad and abs(bad) > 3.4e38:
+        assert not torch.isfinite(got[140, 8:12]).all() and not torch.isfinite(got[270, 9, 5])
