@@ -10,7 +10,7 @@
 //   O = diag(G) Q S + P U,      P_tj = D_tj (q_t . k_j) w_j for j <= t   (w = 1 for the delta rule)
 //   S <- G_last S + K^T diag(E w) U
 //
-// chunk_prep_kernel      T, P, G and E w of every chunk, all of them side by side
+// chunk_prep_kernel      T, P, G and E w of every chunk, all of them side by side (large launches of constant decays form them in the scan)
 // chunk_scan_kernel      the chain over a sequence's chunks; a wave owns all D rows of 16 columns of the state
 // chunk_step_kernel      the same for step sizes, on the bf16 matrix instructions
 // chunk_combine_kernel   starting states of a sequence's segments, where there are too few sequences for the chip
@@ -331,20 +331,23 @@ __device__ __forceinline__ chunk_bf16x8 join8(uint2 lo, uint2 hi) {
 // prompts of 1024 tokens, the layer 818 -> 803 us; 32 of 500 904 -> 888. States are 5.4 to 5.6e-8 off 64 bits (5.6 to 6.0 on f32 products: fewer roundings at the
 // state's magnitude), outputs 0.866e-7 either way. Constant decays gain nothing (833 / 836: their time is the silu of q, k and v), nor
 // do launches of four waves (one prompt of 1000 250 / 255). Chunks with a value that is not finite take the f32 products.
-template <typename T, int KIND, int DT, int NW, int HPW, int MODE, bool NORM = false>
+template <typename T, int KIND, int DT, int NW, int HPW, int MODE, bool NORM = false, bool OWN = false>
 __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
   static_assert(!NORM || (KIND == kChunkDelta && MODE == 0), "the norm follows the delta rule's whole sequences");
+  static_assert(!OWN || KIND == kChunkConst, "the other decays are the tokens' own");
   constexpr bool DELTA = KIND == kChunkDelta, SILU = KIND == kChunkConst, FULL = MODE != 1;
   constexpr int D = DT * 16, RS = D + kPad, PS = kCh + kPad, NT = NW * 64, WPW = NW / HPW;
-  constexpr int MATS = FULL ? HPW * (DELTA ? 2 : 1) : 0;       // P of every head, then T of every head
+  constexpr int SLOTS = OWN ? 3 : 2, RAW = 20;                 // RAW: floats of a row of q k^T
+  constexpr int MATS = FULL && !OWN ? HPW * (DELTA ? 2 : 1) : 0;       // P of every head, then T of every head
   constexpr bool CUT = DELTA && DT == 8 && NW == 8;            // K^T U from pieces
   constexpr int KB = D * 2 + 16, kImg = kCh * KB;              // bytes of a row and of an image of pieces
   __shared__ __attribute__((aligned(16))) unsigned char kc_all[2][CUT ? 3 * kImg : 16];
   __shared__ int odd_all[2][NW];                               // whether a wave staged a k that is not finite
-  __shared__ __attribute__((aligned(16))) float k_all[2][kCh * RS];
-  __shared__ __attribute__((aligned(16))) float q_all[2][FULL ? kCh * RS : 4];
+  __shared__ __attribute__((aligned(16))) float k_all[SLOTS][kCh * RS];
+  __shared__ __attribute__((aligned(16))) float q_all[SLOTS][FULL ? kCh * RS : 4];
+  __shared__ __attribute__((aligned(16))) float raw_all[2][OWN && FULL ? 8 * 16 * RAW : 4], pw_all[OWN ? NW : 1][OWN ? kCh + 4 : 4];
   __shared__ __attribute__((aligned(16))) float pt_all[2][MATS > 0 ? MATS : 1][MATS > 0 ? kCh * PS : 4];
-  __shared__ __attribute__((aligned(16))) float ge_all[2][HPW][2 * kCh];      // G, then E
+  __shared__ __attribute__((aligned(16))) float ge_all[2][HPW][OWN ? 4 : 2 * kCh];      // G, then E
   __shared__ __attribute__((aligned(16))) float sq_all[2][NORM ? NW : 1][NORM ? kCh : 4], inv_all[NORM ? NW : 1][NORM ? kCh : 4];
   const int b = blockIdx.z;
   const int q0 = p.cu_q[b], n_all = p.cu_q[b + 1] - q0;
@@ -385,6 +388,28 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
     for (int i = 1; i < kCh; i *= 2) g_chunk *= g_chunk;
     g_rest = static_cast<float>(g_chunk - static_cast<double>(static_cast<float>(g_chunk)));
   }
+  // constant decays: their powers, formed in 64 bits and rounded once; G and E of a whole chunk, and D of this lane's entries of P
+  float4 g_fac[2], e_fac[2];
+  float d_diag[4], d_low[4];
+  if constexpr (OWN) {
+    double pw = 1.0, sq = p.decay[h];
+    for (int e = lane; e > 0; e >>= 1, sq *= sq)
+      if (e & 1) pw *= sq;
+    if (lane <= kCh) pw_all[w][lane] = static_cast<float>(pw);
+    __builtin_amdgcn_wave_barrier();                   // (a wave's LDS operations keep their order)
+    const float* of = pw_all[w];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const int t = 16 * x + 4 * quad;
+      g_fac[x] = float4{of[t + 1], of[t + 2], of[t + 3], of[t + 4]};
+      e_fac[x] = float4{of[31 - t], of[30 - t], of[29 - t], of[28 - t]};
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      d_diag[i] = of[max(r - 4 * quad - i, 0)];
+      d_low[i] = of[16 + r - 4 * quad - i];
+    }
+  }
 
   // the next chunk's rows on their way, as they lie in memory (a conversion here would wait for them): q and k four entries a thread, P
   // and T too, a value for each of the wave's 32 x 16
@@ -412,7 +437,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
     if constexpr (SILU) return chunk_act<true>(ld4(reinterpret_cast<const bf16_t*>(&x)));
     else return x;
   };
-  auto fetch_rows = [&](int c0, auto whole) __attribute__((always_inline)) {
+  auto fetch_kq = [&](int c0, auto whole) __attribute__((always_inline)) {
     constexpr bool WHOLE = decltype(whole)::value;     // all 32 tokens are there: loads without conditions
     const int cn = s1 - c0;
 #pragma unroll
@@ -422,6 +447,10 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
       kreg[it] = in ? *reinterpret_cast<const Row4*>(kp + static_cast<int64_t>(c0 + it * per) * p.ldk + k_off) : Row4{};
       if constexpr (FULL) qreg[it] = in ? *reinterpret_cast<const Row4*>(qp + static_cast<int64_t>(c0 + it * per) * p.ldq + q_off) : Row4{};
     }
+  };
+  auto fetch_rest = [&](int c0, auto whole) __attribute__((always_inline)) {
+    constexpr bool WHOLE = decltype(whole)::value;
+    const int cn = s1 - c0;
 #pragma unroll
     for (int it = 0; it < PN; ++it) {
       const int m = (it * NT + (w << 6)) >> 8;         // matrix of this wave's pieces
@@ -435,13 +464,20 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
       const int lo = 16 * (i >> 2) + (i & 3);
       vreg[i] = WHOLE || lo + 4 * quad < cn ? entry(vp + static_cast<int64_t>(c0 + lo) * p.ldv + v_off) : Entry{};
     }
+    if constexpr (OWN) return;
     const bool in = WHOLE || (lane & 31) < cn;         // lane = token, G in the lower half of the lanes, E in the upper
     const int64_t at = row0 + static_cast<int64_t>(c0) * p.H + h0;
     gereg = in ? (lane >= 32 ? p.Ef : p.Gf)[at + ge_off] : 0.0f;
   };
+  auto whole_or_not = [&](int c0, auto&& f) __attribute__((always_inline)) {
+    if (s1 - c0 >= kCh) f(c0, std::true_type{});
+    else f(c0, std::false_type{});
+  };
   auto fetch = [&](int c0) __attribute__((always_inline)) {
-    if (s1 - c0 >= kCh) fetch_rows(c0, std::true_type{});
-    else fetch_rows(c0, std::false_type{});
+    whole_or_not(c0, [&](int at, auto whole) __attribute__((always_inline)) {
+      fetch_kq(at, whole);
+      fetch_rest(at, whole);
+    });
   };
   // rows 16 x + 4 quad .. + 3 of a vector, a row of a left-hand matrix from column 16 j on
   auto rows4 = [&](const float* from, int x) __attribute__((always_inline)) {
@@ -505,7 +541,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
     }
   };
   f32x4 U_next[2];
-  auto stage = [&](int buf) __attribute__((always_inline)) {
+  auto stage_kq = [&](int buf) __attribute__((always_inline)) {
     float odd_k = 0.0f;                                // NaN if a value is not finite
 #pragma unroll
     for (int it = 0; it < KQ; ++it) {
@@ -524,6 +560,8 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
       const bool odd = __builtin_amdgcn_ballot_w64(odd_k != 0.0f) != 0;
       if (lane == 0) odd_all[buf][w] = odd;
     }
+  };
+  auto stage_rest = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int it = 0; it < PN; ++it) {
       const int m = (it * NT + (w << 6)) >> 8;
@@ -534,18 +572,102 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
       if constexpr (SILU) U_next[i >> 2][i & 3] = quick_silu_(__builtin_bit_cast(float, vreg[i] << 16));
       else U_next[i >> 2][i & 3] = vreg[i];
     }
-    if (w % WPW == 0) ge_all[buf][hw][lane] = gereg;
+    if (!OWN && w % WPW == 0) ge_all[buf][hw][lane] = gereg;
+  };
+  auto stage = [&](int buf) __attribute__((always_inline)) {
+    stage_kq(buf);
+    stage_rest(buf);
+  };
+  // OWN: parts of q k^T, which does not depend on the head, of the chunk in a slot: the waves' shares of the blocks (0, 0), (1, 1) by halves of the
+  // key dimension and of (1, 0) by quarters. A lane gets four keys of its query: entries as `left` reads them.
+  auto raw_parts = [&](int slot, float* to) __attribute__((always_inline)) {
+    auto part = [&](int number, int xq, int xk, int from, auto count) __attribute__((always_inline)) {
+      constexpr int N = decltype(count)::value;
+      constexpr int M = DT == 4 ? 2 * N : N;           // sums of 16 products, of eight at 64 rows
+      f32x4 sum[M];
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const float4 qv = left(q_all[slot], RS, xq, from + j), kv = left(k_all[slot], RS, xk, from + j);
+        sum[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.x, qv.x, zero, 0, 0, 0);
+        sum[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.y, qv.y, sum[j], 0, 0, 0);
+        f32x4& rest = sum[M - N + j];
+        rest = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.z, qv.z, M > N ? zero : rest, 0, 0, 0);
+        rest = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.w, qv.w, rest, 0, 0, 0);
+      }
+#pragma unroll
+      for (int o = M / 2; o > 0; o /= 2)
+#pragma unroll
+        for (int j = 0; j < o; ++j) sum[j] += sum[j + o];
+      *reinterpret_cast<f32x4*>(to + (number * 16 + r) * RAW + 4 * quad) = sum[0];
+    };
+    const int a = w & 3;
+    if (NW == 4 || w < 4) part(a, a >> 1, a >> 1, (a & 1) * (DT / 2), std::integral_constant<int, DT / 2>{});
+    if (NW == 4 || w >= 4) part(4 + a, 1, 0, a * (DT / 4), std::integral_constant<int, DT / 4>{});
+  };
+  auto raw4 = [&](const float* raw, int number) __attribute__((always_inline)) { return ld4(raw + (number * 16 + r) * RAW + 4 * quad); };
+  auto add4 = [](float4 a, float4 b) __attribute__((always_inline)) { return float4{a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w}; };
+  // y += P x with P = D o q k^T (compare triangle)
+  auto own_triangle = [&](f32x4 (&y)[2], const float* raw, const f32x4 (&x)[2]) __attribute__((always_inline)) {
+    float z = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) z = fmaf(x[i >> 2][i & 3], 0.0f, z);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(z != 0.0f) == 0, 1)) {
+      auto diagonal = [&](int number) __attribute__((always_inline)) {
+        const float4 a = add4(raw4(raw, number), raw4(raw, number + 1));
+        const int e = r - 4 * quad;                    // selected: what a later token brings may not be finite
+        return float4{e >= 0 ? a.x * d_diag[0] : 0.0f, e >= 1 ? a.y * d_diag[1] : 0.0f, e >= 2 ? a.z * d_diag[2] : 0.0f, e >= 3 ? a.w * d_diag[3] : 0.0f};
+      };
+      const float4 a = add4(add4(raw4(raw, 4), raw4(raw, 5)), add4(raw4(raw, 6), raw4(raw, 7)));
+      const float4 low{a.x * d_low[0], a.y * d_low[1], a.z * d_low[2], a.w * d_low[3]};
+      y[0] += mul4(zero, diagonal(0), x[0]);
+      y[1] += mul4(mul4(zero, low, x[0]), diagonal(2), x[1]);
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll 1
+      for (int from = 0; from < 4; ++from) {
+        const int j = 16 * (i >> 2) + 4 * from + (i & 3);
+        const float v = __shfl(x[i >> 2][i & 3], 16 * from + r, kWave);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const int t = 16 * (k >> 2) + 4 * quad + (k & 3);
+          const float* at = raw + (t & 15) * RAW + (j & 15);
+          constexpr int next = 16 * RAW;
+          const float m = (t >> 4) == (j >> 4) ? at[2 * (t >> 4) * next] + at[(2 * (t >> 4) + 1) * next]
+                                               : (at[4 * next] + at[5 * next]) + (at[6 * next] + at[7 * next]);
+          y[k >> 2][k & 3] = j <= t ? fmaf(m * pw_all[w][max(t - j, 0)], v, y[k >> 2][k & 3]) : y[k >> 2][k & 3];
+        }
+      }
   };
   // Two buffers: a chunk is staged while the one before it is computed, each wave at its own time, and two chunks ahead are on
-  // their way in registers. One barrier a chunk.
-  fetch(s0);
-  stage(0);
-  if (s0 + kCh < s1) fetch(s0 + kCh);
+  // their way in registers. One barrier a chunk. OWN: three of k and q, staged a chunk earlier, since q k^T of a chunk is formed during the one before.
+  int slot = 0;
+  if constexpr (OWN) {
+    auto rows = [&](int c0) __attribute__((always_inline)) {
+      if (c0 < s1) whole_or_not(c0, fetch_kq);
+    };
+    rows(s0);
+    stage_kq(0);
+    rows(s0 + kCh);
+    stage_kq(1);
+    rows(s0 + 2 * kCh);
+    whole_or_not(s0, fetch_rest);
+    stage_rest(0);
+    if (s0 + kCh < s1) whole_or_not(s0 + kCh, fetch_rest);
+    __syncthreads();
+    if constexpr (FULL) raw_parts(0, raw_all[0]);
+  } else {
+    fetch(s0);
+    stage(0);
+    if (s0 + kCh < s1) fetch(s0 + kCh);
+  }
   __syncthreads();
   int buf = 0;
   for (int c0 = s0; c0 < s1; c0 += kCh, buf ^= 1) {
     const int cn = min(kCh, s1 - c0);
-    const float *k_lds = k_all[buf], *q_lds = q_all[buf];
+    const int here = OWN ? slot : buf, next_slot = here == 2 ? 0 : here + 1, last_slot = here == 0 ? 2 : here - 1;
+    const float *k_lds = k_all[here], *q_lds = q_all[here];
     const auto& pt_lds = pt_all[buf];
     const auto& ge_lds = ge_all[buf];
     if constexpr (NORM) {
@@ -579,14 +701,26 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
       }
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
-        o[x] = scale4((qs[0][x] + qs[1][x]) + (qs[2][x] + qs[3][x]), rows4(ge_lds[hw], x));
+        o[x] = scale4((qs[0][x] + qs[1][x]) + (qs[2][x] + qs[3][x]), OWN ? g_fac[x] : rows4(ge_lds[hw], x));
         if constexpr (KIND == kChunkStep) o[x] += skip * U[x];
       }
-      triangle(o, pt_lds[hw], U);
+      if constexpr (OWN) own_triangle(o, raw_all[buf], U);
+      else triangle(o, pt_lds[hw], U);
     }
 #pragma unroll
-    for (int x = 0; x < 2; ++x) u2[x] = scale4(U[x], rows4(ge_lds[hw] + kCh, x));
-    const float g_last = ge_lds[hw][cn - 1];
+    for (int x = 0; x < 2; ++x) {
+      if constexpr (OWN) {
+        float4 e = e_fac[x];
+        if (cn < kCh) {                                // (tokens past the end are zeros)
+          const int at = cn - 1 - 16 * x - 4 * quad;
+          e = float4{pw_all[w][max(at, 0)], pw_all[w][max(at - 1, 0)], pw_all[w][max(at - 2, 0)], pw_all[w][max(at - 3, 0)]};
+        }
+        u2[x] = scale4(U[x], e);
+      } else {
+        u2[x] = scale4(U[x], rows4(ge_lds[hw] + kCh, x));
+      }
+    }
+    const float g_last = OWN ? pw_all[w][cn] : ge_lds[hw][cn - 1];
     bool odd = !CUT;
     if constexpr (CUT) {
       float z = 0.0f;
@@ -627,7 +761,13 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
         S[j] = add;
       }
     } else {
-      stage(buf ^ 1);
+      if constexpr (OWN) {
+        if constexpr (FULL) raw_parts(next_slot, raw_all[buf ^ 1]);
+        stage_kq(last_slot);
+        stage_rest(0);
+      } else {
+        stage(buf ^ 1);
+      }
 #pragma unroll
       for (int j = 0; j < DT; ++j) {
         // constant decays, slow as a rule: what the chunk adds in two sums of its own, for fewer roundings at the state's magnitude
@@ -643,7 +783,13 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
           S[j][i] = APART ? fmaf(S[j][i], g_last, fmaf(S[j][i], cn == kCh ? g_rest : 0.0f, add[0][i] + add[1][i])) : add[0][i];
       }
     }
-    if (c0 + 2 * kCh < s1) fetch(c0 + 2 * kCh);
+    if constexpr (OWN) {
+      if (c0 + 3 * kCh < s1) whole_or_not(c0 + 3 * kCh, fetch_kq);
+      if (c0 + 2 * kCh < s1) whole_or_not(c0 + 2 * kCh, fetch_rest);
+      slot = next_slot;
+    } else if (c0 + 2 * kCh < s1) {
+      fetch(c0 + 2 * kCh);
+    }
     if constexpr (NORM) {
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
@@ -997,12 +1143,12 @@ __global__ __launch_bounds__(256) void chunk_combine_kernel(ChunkParams p) {
   }
 }
 
-template <typename T, int KIND, int DT, int NW, int HPW>
+template <typename T, int KIND, int DT, int NW, int HPW, bool OWN = false>
 static void chunk_launch(const ChunkParams& p, int B, hipStream_t s) {
   dim3 grid(p.H / HPW * (p.Dv / 16 / (NW / HPW)), p.segs, B), block(NW * 64);
   auto scan = [&](auto mode) {
     if constexpr (KIND == kChunkStep) chunk_step_kernel<DT, NW, HPW, decltype(mode)::value><<<grid, block, 0, s>>>(p);
-    else chunk_scan_kernel<T, KIND, DT, NW, HPW, decltype(mode)::value><<<grid, block, 0, s>>>(p);
+    else chunk_scan_kernel<T, KIND, DT, NW, HPW, decltype(mode)::value, false, OWN><<<grid, block, 0, s>>>(p);
   };
   if (p.segs <= 1) {
     scan(std::integral_constant<int, 0>{});
@@ -1020,19 +1166,27 @@ static void chunk_launch(const ChunkParams& p, int B, hipStream_t s) {
 // and k are staged twice); beyond that the halves only take each other's place. us, 8 / 4 waves, 16 heads of 128 x 128, prompts of 1000: delta
 // rule 1 prompt 268 / 186, 8 284 / 207, 10 294 / 384; constant decays 228 / 168, 253 / 194, 259 / 294; heads of 64 x 64, delta rule, 12
 // prompts 204 / 150. Step sizes are bound by a chunk's chain either way (one prompt of 4096, 32 heads of 128 x 64, 469 / 500).
+//
+// Constant decays on launches that are not of few workgroups form P in the scan (OWN), and have no launch in front of it: q k^T of a chunk is 5 % more of the
+// chain, and the powers of the decay are the same in every chunk. 16 x 1024 tokens, 16 heads of 128, the layer 810 -> 784 us (61 us in front, the silu
+// of q and k once more and 67 MB through memory); 8 x 1000, heads of 64, 240 -> 229; 32 x 500 814 -> 797. Few workgroups wait for the longer chain
+// (one prompt of 1000 138 -> 144) and keep the launch.
 template <typename T, int KIND, int DT>
 static void chunk_waves(const ChunkParams& p, int64_t tokens, int B, hipStream_t s) {
   const int64_t pieces = p.segs > 1 ? std::min<int64_t>(static_cast<int64_t>(B) * p.segs, tokens / p.seg_len + B) : B;
-  const bool few = KIND != kChunkStep && pieces * p.H * p.Dv / 128 <= 128;
+  const bool small = pieces * p.H * p.Dv / 128 <= 128, few = KIND != kChunkStep && small;
+  constexpr bool CONST = KIND == kChunkConst;
+  if (!CONST || small) chunk_prep_kernel<T, KIND, DT * 16><<<dim3(static_cast<unsigned>(tokens / kCh + B), p.G), dim3(256), 0, s>>>(p);
   if (p.Dv % 128 == 0 && !few) {
-    chunk_launch<T, KIND, DT, 8, 1>(p, B, s);
+    chunk_launch<T, KIND, DT, 8, 1, CONST>(p, B, s);
     return;
   }
   if (p.Dv % 128 != 0 && p.H / p.G % 2 == 0 && !few) {
-    chunk_launch<T, KIND, DT, 8, 2>(p, B, s);
+    chunk_launch<T, KIND, DT, 8, 2, CONST>(p, B, s);
     return;
   }
-  chunk_launch<T, KIND, DT, 4, 1>(p, B, s);
+  if (CONST && !few) chunk_launch<T, KIND, DT, 4, 1, CONST>(p, B, s);
+  else chunk_launch<T, KIND, DT, 4, 1>(p, B, s);
 }
 
 // The delta rule with norm and gate: heads of 64 or 128 values, on eight waves.
@@ -1055,14 +1209,8 @@ static void chunk_norm_dispatch(const ChunkParams& p, int64_t tokens, int B, hip
 
 template <typename T, int KIND>
 static void chunk_dispatch(const ChunkParams& p, int64_t tokens, int B, hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>(tokens / kCh + B), p.G), block(256);
-  if (p.D == 64) {
-    chunk_prep_kernel<T, KIND, 64><<<grid, block, 0, s>>>(p);
-    chunk_waves<T, KIND, 4>(p, tokens, B, s);
-  } else {
-    chunk_prep_kernel<T, KIND, 128><<<grid, block, 0, s>>>(p);
-    chunk_waves<T, KIND, 8>(p, tokens, B, s);
-  }
+  if (p.D == 64) chunk_waves<T, KIND, 4>(p, tokens, B, s);
+  else chunk_waves<T, KIND, 8>(p, tokens, B, s);
 }
 
 static int chunk_segments(int kind, int max_new, int seg_len) {

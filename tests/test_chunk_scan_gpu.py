@@ -313,3 +313,36 @@ def test_large_delta_launches_with_values_that_are_not_finite(bad):
         assert rel(x, y.to(F64)) < 2 * REL
     if bad == bad and abs(bad) > 3.4e38:
         assert not torch.isfinite(got[140, 8:12]).all() and not torch.isfinite(got[270, 9, 5])
+
+
+# constant decays on launches of more than 128 workgroups form P in the scan: whole and partial chunks, fewer chunks than are staged ahead, segments
+@pytest.mark.parametrize("H,D,Dv,new,ctx", [(32, 128, 128, [33, 64, 1, 95, 32, 130, 161], [0, 4, 0, 9, 1, 0, 2]), (64, 64, 64, [40, 97, 129, 0, 31, 66], [3, 0, 0, 5, 1, 2]),
+                                            (8, 128, 128, [2100, 1500, 1700], [0, 3, 0])])
+def test_large_launches_of_constant_decays(H, D, Dv, new, ctx):
+    call, args, _ = case("const", new, H, H, D, Dv, seed=H + D)
+    step = make_step(new, ctx)
+    state = 0.3 * torch.randn(len(new), H, D, Dv, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    want_o, want_s = recurrence(*args, state, step)
+    o = call(state, step)
+    assert rel(o, want_o) < 2 * REL and rel(state, want_s) < 2 * REL
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_large_launches_of_constant_decays_with_values_that_are_not_finite(bad):
+    """q, k and v entries that are not finite reach their own tokens and those behind them in the same head, and no earlier or other one."""
+    H, D, Dv, new = 32, 128, 128, [100] * 6
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    proj = torch.randn(sum(new), 3 * H * D, device="cuda", generator=gen).bfloat16()
+    decay = torch.linspace(0.9, 0.999, H, device="cuda")
+    run = lambda x, st: mix_ops.lightning_attention(x, 0, H * D, 2 * H * D, decay, st, make_step(new, [0] * 6), H, D, Dv).view(-1, H, Dv)  # noqa: E731
+    s0, s1 = torch.zeros(6, H, D, Dv, device="cuda"), torch.zeros(6, H, D, Dv, device="cuda")
+    want = run(proj, s0)
+    proj[150, 3 * D + 7], proj[250, H * D + 9 * D + 4], proj[350, 2 * H * D + 5 * D + 100] = bad, bad, bad      # q of head 3, k of head 9, v of head 5
+    got = run(proj, s1)
+    assert not torch.isfinite(got[150, 3]).any() and not torch.isfinite(got[250, 9]).any() and not torch.isfinite(got[350:400, 5, 100]).any()
+    ok = torch.ones(sum(new), H, Dv, dtype=torch.bool, device="cuda")
+    ok[150, 3] = ok[250:300, 9] = ok[350:400, 5, 100] = False
+    # a wave that sees such a value goes through its block of tokens one by one: another order of the same sums
+    assert rel(torch.where(ok, got, 0.0), torch.where(ok, want, 0.0).to(F64)) < 4 * REL
+    rest = [h for h in range(H) if h not in (5, 9)]
+    assert torch.equal(s1[:, rest], s0[:, rest])
