@@ -762,8 +762,8 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
       }
     } else {
       if constexpr (OWN) {
-        if constexpr (FULL) raw_parts(next_slot, raw_all[buf ^ 1]);
         stage_kq(last_slot);
+        if constexpr (FULL) raw_parts(next_slot, raw_all[buf ^ 1]);
         stage_rest(0);
       } else {
         stage(buf ^ 1);
@@ -1168,8 +1168,8 @@ static void chunk_launch(const ChunkParams& p, int B, hipStream_t s) {
 // prompts 204 / 150. Step sizes are bound by a chunk's chain either way (one prompt of 4096, 32 heads of 128 x 64, 469 / 500).
 //
 // Constant decays on launches that are not of few workgroups form P in the scan (OWN), and have no launch in front of it: q k^T of a chunk is 5 % more of the
-// chain, and the powers of the decay are the same in every chunk. 16 x 1024 tokens, 16 heads of 128, the layer 810 -> 784 us (61 us in front, the silu
-// of q and k once more and 67 MB through memory); 8 x 1000, heads of 64, 240 -> 229; 32 x 500 814 -> 797. Few workgroups wait for the longer chain
+// chain, and the powers of the decay are the same in every chunk. 16 x 1024 tokens, 16 heads of 128, the layer 803 -> 774 us (61 us in front, the silu
+// of q and k once more and 67 MB through memory; 781 with q k^T in front of the staging); 8 x 1000, heads of 64, 240 -> 229; 32 x 500 814 -> 797. Few workgroups wait for the longer chain
 // (one prompt of 1000 138 -> 144) and keep the launch.
 template <typename T, int KIND, int DT>
 static void chunk_waves(const ChunkParams& p, int64_t tokens, int B, hipStream_t s) {
