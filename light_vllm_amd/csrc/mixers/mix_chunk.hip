@@ -1161,32 +1161,57 @@ static void chunk_launch(const ChunkParams& p, int B, hipStream_t s) {
   }
 }
 
+// Sequences, or segments of them at most.
+static int64_t chunk_pieces(int64_t tokens, int B, int segs, int seg_len) {
+  return segs > 1 ? std::min<int64_t>(static_cast<int64_t>(B) * segs, tokens / seg_len + B) : B;
+}
+
+static bool chunk_few(int64_t pieces, int H, int Dv) { return pieces * H * Dv / 128 <= 128; }
+
+// Whether a launch of constant decays forms P in the scan (OWN), without a launch in front of it: q k^T of a chunk is 5 % more of the chain, and
+// the powers of the decay are the same in every chunk. 16 x 1024 tokens, 16 heads of 128, the layer 803 -> 774 us (61 us in front, the silu of q and
+// k once more and 67 MB through memory; 781 with q k^T in front of the staging). Scans by themselves, us, launch in front / OWN:
+//   few workgroups wait for the longer chain: one prompt of 1000 138 / 144.
+//   128 x 128, 16 heads: 16 x 1024 292 / 268, 64 x 250 304 / 287, 256 x 64 393 / 379; 16 of 290 to 1680 421 / 421; not where one sequence is what the
+//     others are waiting for (one of 4000 beside 12 of 300 871 / 949).
+//   128 x 64: three chunks of q and k in LDS leave a compute unit one workgroup of four waves instead of two: 256 x 64 231 / 301, 11 x 1500, 32 heads,
+//     503 / 555; one of 4096 in segments 164 / 169.
+//   keys of 64: two workgroups of four waves instead of three, and a chain of its own in front of the first chunk. Even lengths gain,
+//     64 x 64, 32 heads, 16 x 1024 249 / 208, 128 x 120 243 / 236; 64 x 128, 16 heads, 188 / 179, 213 / 214; so do launches of one round that is
+//     not mostly idle behind its longest (64 heads of 64 x 64, 8 of 20 to 220 45 / 39). In several rounds two chunks a sequence
+//     lose (256 x 64 259 / 266 and 246 / 256), and so do uneven lengths (24 of 30 to 509 145 / 152; one of 4000 beside 12 of 300 453 / 522).
+// Random steps that the rule takes, of 329 for each size: 1.04 times faster in the mean (128 x 128; the slowest 0.98), 1.07 (64 x 64; 0.98) and 1.03 (64 x 128; 0.98).
+static bool chunk_own(int kind, int64_t tokens, int B, int max_new, int H, int D, int Dv, int segs, int seg_len) {
+  const int64_t pieces = chunk_pieces(tokens, B, segs, seg_len), longest = segs > 1 ? seg_len : max_new, columns = static_cast<int64_t>(H) * Dv;
+  if (kind != kChunkConst || chunk_few(pieces, H, Dv)) return false;
+  if (D == 128) return Dv % 128 == 0 && longest * pieces <= 3 * tokens;
+  const bool one_round = pieces * columns <= 256 * 128 && 5 * tokens * columns >= 2 * 256 * 128 * longest;      // 256 workgroups of 128 columns, 0.4 of them at work
+  return one_round || (tokens >= 96 * pieces && 2 * longest * pieces <= 3 * tokens);
+}
+
 // Eight waves a workgroup: 128 columns of a head, or two heads of 64 that share q and k. Launches of few workgroups, which leave half of the
 // chip empty, cut them in two (the f32 scans: a compute unit then holds one wave a SIMD, and a chunk takes two thirds of the time, though q
 // and k are staged twice); beyond that the halves only take each other's place. us, 8 / 4 waves, 16 heads of 128 x 128, prompts of 1000: delta
 // rule 1 prompt 268 / 186, 8 284 / 207, 10 294 / 384; constant decays 228 / 168, 253 / 194, 259 / 294; heads of 64 x 64, delta rule, 12
 // prompts 204 / 150. Step sizes are bound by a chunk's chain either way (one prompt of 4096, 32 heads of 128 x 64, 469 / 500).
-//
-// Constant decays on launches that are not of few workgroups form P in the scan (OWN), and have no launch in front of it: q k^T of a chunk is 5 % more of the
-// chain, and the powers of the decay are the same in every chunk. 16 x 1024 tokens, 16 heads of 128, the layer 803 -> 774 us (61 us in front, the silu
-// of q and k once more and 67 MB through memory; 781 with q k^T in front of the staging); 8 x 1000, heads of 64, 240 -> 229; 32 x 500 814 -> 797. Few workgroups wait for the longer chain
-// (one prompt of 1000 138 -> 144) and keep the launch.
 template <typename T, int KIND, int DT>
-static void chunk_waves(const ChunkParams& p, int64_t tokens, int B, hipStream_t s) {
-  const int64_t pieces = p.segs > 1 ? std::min<int64_t>(static_cast<int64_t>(B) * p.segs, tokens / p.seg_len + B) : B;
-  const bool small = pieces * p.H * p.Dv / 128 <= 128, few = KIND != kChunkStep && small;
+static void chunk_waves(const ChunkParams& p, int64_t tokens, int B, bool own, hipStream_t s) {
   constexpr bool CONST = KIND == kChunkConst;
-  if (!CONST || small) chunk_prep_kernel<T, KIND, DT * 16><<<dim3(static_cast<unsigned>(tokens / kCh + B), p.G), dim3(256), 0, s>>>(p);
-  if (p.Dv % 128 == 0 && !few) {
-    chunk_launch<T, KIND, DT, 8, 1, CONST>(p, B, s);
-    return;
+  if constexpr (CONST) {
+    if (own) {
+      if constexpr (DT == 4) {
+        if (p.Dv == 64) return chunk_launch<T, KIND, DT, 4, 1, true>(p, B, s);
+      }
+      return chunk_launch<T, KIND, DT, 8, 1, true>(p, B, s);
+    }
   }
-  if (p.Dv % 128 != 0 && p.H / p.G % 2 == 0 && !few) {
-    chunk_launch<T, KIND, DT, 8, 2, CONST>(p, B, s);
-    return;
+  chunk_prep_kernel<T, KIND, DT * 16><<<dim3(static_cast<unsigned>(tokens / kCh + B), p.G), dim3(256), 0, s>>>(p);
+  const bool few = KIND != kChunkStep && chunk_few(chunk_pieces(tokens, B, p.segs, p.seg_len), p.H, p.Dv);
+  if (p.Dv % 128 == 0 && !few) return chunk_launch<T, KIND, DT, 8, 1>(p, B, s);
+  if constexpr (!CONST) {                              // (heads of the layers share no q and k; others take four waves)
+    if (p.Dv % 128 != 0 && p.H / p.G % 2 == 0 && !few) return chunk_launch<T, KIND, DT, 8, 2>(p, B, s);
   }
-  if (CONST && !few) chunk_launch<T, KIND, DT, 4, 1, CONST>(p, B, s);
-  else chunk_launch<T, KIND, DT, 4, 1>(p, B, s);
+  chunk_launch<T, KIND, DT, 4, 1>(p, B, s);
 }
 
 // The delta rule with norm and gate: heads of 64 or 128 values, on eight waves.
@@ -1208,9 +1233,9 @@ static void chunk_norm_dispatch(const ChunkParams& p, int64_t tokens, int B, hip
 }
 
 template <typename T, int KIND>
-static void chunk_dispatch(const ChunkParams& p, int64_t tokens, int B, hipStream_t s) {
-  if (p.D == 64) chunk_waves<T, KIND, 4>(p, tokens, B, s);
-  else chunk_waves<T, KIND, 8>(p, tokens, B, s);
+static void chunk_dispatch(const ChunkParams& p, int64_t tokens, int B, bool own, hipStream_t s) {
+  if (p.D == 64) chunk_waves<T, KIND, 4>(p, tokens, B, own, s);
+  else chunk_waves<T, KIND, 8>(p, tokens, B, own, s);
 }
 
 static int chunk_segments(int kind, int max_new, int seg_len) {
@@ -1283,9 +1308,9 @@ static int chunk_scan(int kind, const void* q, int64_t ldq, const void* k, int64
     p.eps = norm->eps;
     p.gate_silu = norm->gate_silu;
     chunk_norm_dispatch(p, T, B, s);
-  } else if (kind == kChunkDelta) chunk_dispatch<float, kChunkDelta>(p, T, B, s);
-  else if (kind == kChunkStep) chunk_dispatch<bf16_t, kChunkStep>(p, T, B, s);
-  else chunk_dispatch<bf16_t, kChunkConst>(p, T, B, s);
+  } else if (kind == kChunkDelta) chunk_dispatch<float, kChunkDelta>(p, T, B, false, s);
+  else if (kind == kChunkStep) chunk_dispatch<bf16_t, kChunkStep>(p, T, B, false, s);
+  else chunk_dispatch<bf16_t, kChunkConst>(p, T, B, chunk_own(kind, T, B, max_new, H, D, Dv, p.segs, seg_len), s);
   return launched("lv_chunk_scan");
 }
 

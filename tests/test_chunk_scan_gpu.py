@@ -346,3 +346,29 @@ def test_large_launches_of_constant_decays_with_values_that_are_not_finite(bad):
     assert rel(torch.where(ok, got, 0.0), torch.where(ok, want, 0.0).to(F64)) < 4 * REL
     rest = [h for h in range(H) if h not in (5, 9)]
     assert torch.equal(s1[:, rest], s0[:, rest])
+
+
+# key sizes, value sizes and lengths on either side of the rule, whole and in segments; head 0 decays at once
+@pytest.mark.parametrize("H,D,Dv,new,seg,own", [
+    (48, 128, 128, [33, 130, 95], 0, True), (48, 128, 128, [330, 40], 128, True), (24, 128, 128, [300] + [9] * 9, 0, False),
+    (32, 128, 64, [33, 64, 1, 95, 32, 130, 161, 70, 97], 0, False), (48, 128, 64, [230, 97, 33], 64, False),
+    (48, 64, 128, [200, 180, 150], 0, True), (48, 64, 128, [400, 33, 95], 0, False), (96, 64, 128, [130, 100, 120], 0, True),
+    (96, 64, 128, [64, 65, 63], 0, False), (48, 64, 128, [256, 250, 240], 128, True), (96, 64, 64, [200, 180, 150], 0, True),
+    (96, 64, 64, [64, 65, 63, 33, 40, 64], 0, False), (96, 64, 64, [256, 250, 240], 128, True), (96, 64, 64, [230, 97, 33], 64, False)])
+def test_where_constant_decays_form_their_products_in_the_scan(H, D, Dv, new, seg, own, monkeypatch):
+    """Launches of more than 128 workgroups have no launch in front where that is faster, and are the recurrence either way."""
+    from torch.profiler import ProfilerActivity, profile
+    call, args, _ = case("const", new, H, H, D, Dv, seed=H + D + Dv, zeros=True)
+    step = make_step(new, [i % 2 for i in range(len(new))])
+    monkeypatch.setattr(mix_ops, "_segment_length", lambda *a: seg)
+    state = 0.3 * torch.randn(len(new), H, D, Dv, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    want_o, want_s = recurrence(*args, state, step)
+    s = state.clone()
+    o = call(s, step)
+    assert rel(o, want_o) < 2 * REL and rel(s, want_s) < 2 * REL
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        call(state, step)
+        torch.cuda.synchronize()
+    names = " ".join(e.key for e in prof.key_averages())
+    assert "chunk_scan_kernel" in names and ("chunk_prep_kernel" in names) != own and ("chunk_combine_kernel" in names) == (seg > 0)
