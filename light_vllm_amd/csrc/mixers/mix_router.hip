@@ -2,8 +2,8 @@
 // v_mfma_f32_16x16x4_f32, without a widened copy of the activations.
 //
 // Tokens whose experts nearly tie take one or the other by the order of these sums, so the order is that of the f32 product this stands in
-// for: one chain over k in blocks of 16, product i of a block on its entries i, 4 + i, 8 + i and 12 + i (the same bits at 32 and 64 experts
-// from 4500 tokens on, widths of 512 to 4096).
+// for: one chain over k in blocks of 16, product i of a block on its entries i, 4 + i, 8 + i and 12 + i. The same bits at widths of 512, 1024, 2048 and 4096
+// for 32 experts and 4500 (4096: 6000) to 32768 tokens, 64 experts and 9000 to 16384; beyond 16384 tokens the product of 64 experts sums otherwise.
 //
 // Bound by the chain of f32 products (16 x 16 x 4: 32 clocks on a SIMD; 14 us at 16384 x 2048 x 32) and by reading h once (67 MB there, 12 us).
 // A workgroup of eight waves takes 64 rows: four waves' worth of 16 rows, by halves of the experts, so that a SIMD has two chains to

@@ -1054,8 +1054,8 @@ def router_logits(h, router_w):
 
 def router_product(h, router_w):
     """f32 [T, E] = h router_w^T. Tokens whose experts nearly tie take one or the other by the order of these sums, so the order stays that of
-    the vendor's f32 product on widened activations, which lv_router_tiles keeps to the bit where router_tiles_ok holds. (f32 sums in three
-    bf16 pieces were no further from float64 and moved such tokens to other experts.)"""
+    the vendor's f32 product on widened activations, which lv_router_tiles was seen to keep to the bit wherever router_tiles_ok holds. (f32 sums
+    in three bf16 pieces were no further from float64 and moved such tokens to other experts.)"""
     if not router_tiles_ok(h, router_w):
         return F.linear(h.float(), router_w)
     T, W = h.shape
@@ -1068,16 +1068,18 @@ def router_product(h, router_w):
 
 def router_tiles_ok(h, router_w) -> bool:
     """Whether router_product takes lv_router_tiles: bf16 activations in rows of whole 16-byte pieces, widths that are powers of two, 32 or 64
-    experts, and token counts at which the vendor's product sums in the kernel's order and takes longer. (It sums otherwise at 16 and 48
-    experts, at other widths now and then, up to 4096 tokens, and at 24001 tokens of 4096 x 64.) us in a graph, widening and vendor's
+    experts, and token counts at which the vendor's product sums in the kernel's order and takes longer. The order is the vendor's
+    choice for a size, so it was compared: 32 experts, every ninth token count of 4500 to 32768 (6000 at width 4096), 64 experts, every fifth of
+    9000 to 16384, at widths 512, 1024, 2048 and 4096; all 18300 products were equal to the bit. (Otherwise at 64 experts from 16385 tokens on,
+    at 16 and 48 experts, at other widths now and then, up to 4096 tokens.) us in a graph, widening and vendor's
     product / lv_router_tiles, warm:
       32 experts, width 512: 4500 tokens 15 / 8, 16384 25 / 9; 2048: 5000 29 / 24, 16384 53 / 26, 32768 117 / 43; 4096: 5000 44 / 45, 7001 52 / 45.
-      64 experts, width 2048: 7001 37 / 41, 9000 53 / 41, 16384 67 / 42; 4096: 9000 95 / 76."""
+      64 experts, width 2048: 7001 37 / 41, 9000 53 / 41, 16384 67 / 42; 4096: 9000 95 / 76; launch by launch 512: 16384 29 / 14, 1024: 39 / 23."""
     if (type(h) not in _PLAIN or type(router_w) not in _PLAIN or _compiling() or _tracing() or h.dim() != 2 or not h.is_cuda
             or h.dtype is not torch.bfloat16 or router_w.dim() != 2 or router_w.dtype is not torch.float32):
         return False
     (T, W), E = h.shape, router_w.size(0)
-    few, most = (4500 if W < 4096 else 6000, 32768) if E == 32 else (9000, 20000)
+    few, most = (4500 if W < 4096 else 6000, 32768) if E == 32 else (9000, 16384)
     return (E in (32, 64) and few <= T <= most and 512 <= W <= 4096 and W & (W - 1) == 0 and not _transformed() and router_w.size(1) == W
             and router_w.is_contiguous() and h.stride(1) == 1 and h.stride(0) % 8 == 0 and h.stride(0) >= W
             and (h.data_ptr() | router_w.data_ptr()) & 15 == 0 and router_w.get_device() == h.get_device() == torch.cuda.current_device()

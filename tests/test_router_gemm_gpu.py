@@ -84,3 +84,16 @@ def test_which_calls_take_the_tiles():
                  (h, w.t().contiguous().t()), (h.view(5, 1000, 1024), w), (h.clone().requires_grad_(), w), (h, w.clone().requires_grad_())]:
         assert not ok(a, b)
         assert torch.equal(mix_ops.router_product(a, b), F.linear(a.float(), b))
+
+
+# the corners of the ranges, and counts just beyond, where the vendor's product sums in another order: the product itself
+@torch.inference_mode()
+@pytest.mark.parametrize("T,E,K,taken", [(4500, 32, 1024, True), (32768, 32, 512, True), (32767, 32, 1024, True), (24001, 32, 2048, True), (32768, 32, 4096, True), (9000, 64, 512, True),
+                                         (16384, 64, 512, True), (16384, 64, 1024, True), (16383, 64, 2048, True), (16384, 64, 4096, True), (9000, 64, 4096, True),
+                                         (16385, 64, 4096, False), (16448, 64, 512, False), (16448, 64, 1024, False), (16448, 64, 2048, False), (18496, 64, 4096, False)])
+def test_bits_at_the_corners(T, E, K, taken):
+    gen = torch.Generator(device="cuda").manual_seed(T + K)
+    h = torch.randn(T, K, device="cuda", generator=gen).bfloat16()
+    w = torch.randn(E, K, device="cuda", generator=gen) * K ** -0.5
+    assert mix_ops.router_tiles_ok(h, w) == taken
+    assert torch.equal(mix_ops.router_product(h, w), F.linear(h.float(), w))
