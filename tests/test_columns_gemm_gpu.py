@@ -68,3 +68,14 @@ def test_which_calls_are_split():
     a, b = x.clone().requires_grad_(), w.clone().requires_grad_()
     for p, q in [(a, w), (x, b)]:
         assert mix_ops._split_sizes(p, q) is None and mix_ops.linear(p, q).requires_grad
+
+
+# rows whose last tile of 256 is a part (of one row, of all but one), in whole rounds all the same
+@torch.inference_mode()
+@pytest.mark.parametrize("M,N,K,lead", [(7937, 2064, 1024, 0), (8191, 2112, 1088, 8), (16129, 1040, 1024, 0), (16300, 1028, 1024, 0)])
+def test_in_two_launches_of_odd_rows(M, N, K, lead):
+    x, w = case(M, N, K, M + N, lead)
+    assert mix_ops._split_sizes(x, w) is not None and mix_ops._split_sizes(x[:M // 256 * 256 - 256], w) is None
+    y = mix_ops.linear(x, w)
+    ref, most = bound(x, w)
+    assert y.shape == (M, N) and y.is_contiguous() and bool(((y.double() - ref).abs() <= most).all())
