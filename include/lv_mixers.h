@@ -447,7 +447,7 @@ int lv_gated_scan(int kind, const void* q, int64_t ldq, const void* k, int64_t l
  *   LV_MIX_CHUNK_DELTA  f32 rows q, k, v; a = beta f32 [T, H], decay f32 [T, H]
  * q, k aligned to four entries, ldq and ldk multiples of 4. max_new >= every sequence's new tokens. seg_len > 0 (a multiple of
  * 32, not for the delta rule): sequences are cut into segments of that many tokens whose contributions are formed side by
- * side. workspace: lv_chunk_scan_workspace_bytes with the same numbers, aligned to 16 bytes. */
+ * side. workspace: lv_chunk_scan_workspace_bytes with the same numbers, aligned to 16 bytes (NULL will do where that is 0). */
 int lv_chunk_scan(int kind, const void* q, int64_t ldq, const void* k, int64_t ldk, const void* v, int64_t ldv, const void* a,
                   int64_t lda, const void* decay, const void* p0, const void* p1, const void* p2, void* state,
                   const int32_t* cu_q, const int32_t* ctx_lens, const int32_t* slots, void* o, void* workspace,

@@ -1248,8 +1248,8 @@ extern "C" {
 int64_t lv_chunk_scan_workspace_bytes(int kind, int64_t T, int B, int max_new, int H, int D, int Dv, int seg_len) {
   if (T < 0 || B < 0 || H <= 0 || D <= 0 || Dv <= 0 || max_new < 0) return fail(-1, "lv_chunk_scan_workspace_bytes: bad sizes");
   const int64_t rows = T * H;
-  int64_t floats = rows * kCh * (kind == kChunkDelta ? 2 : 1) + 2 * ((rows + 3) / 4 * 4);
   const int segs = chunk_segments(kind, max_new, seg_len);
+  int64_t floats = chunk_own(kind, T, B, max_new, H, D, Dv, segs, seg_len) ? 0 : rows * kCh * (kind == kChunkDelta ? 2 : 1) + 2 * ((rows + 3) / 4 * 4);
   if (segs > 1) floats += static_cast<int64_t>(B) * segs * H * (static_cast<int64_t>(D) * Dv + 1);
   return floats * static_cast<int64_t>(sizeof(float));
 }
@@ -1260,7 +1260,7 @@ static int chunk_scan(int kind, const void* q, int64_t ldq, const void* k, int64
                       int64_t workspace_bytes, int64_t T, int B, int max_new, int H, int G, int D, int Dv, int seg_len,
                       const ChunkParams* norm, void* stream) {
   if (B == 0 || T == 0) return 0;
-  if (!q || !k || !v || !state || !cu_q || !ctx_lens || !slots || !o || !workspace) return fail(-1, "lv_chunk_scan: null pointer");
+  if (!q || !k || !v || !state || !cu_q || !ctx_lens || !slots || !o) return fail(-1, "lv_chunk_scan: null pointer");
   if (kind != kChunkStep && kind != kChunkConst && kind != kChunkDelta) return fail(-1, "lv_chunk_scan: kind %d", kind);
   if (kind == kChunkStep && (!a || !p0 || !p1 || !p2)) return fail(-1, "lv_chunk_scan: step sizes without their parameters");
   if (kind != kChunkStep && (!decay || (kind == kChunkDelta && !a))) return fail(-1, "lv_chunk_scan: no decays");
@@ -1272,7 +1272,9 @@ static int chunk_scan(int kind, const void* q, int64_t ldq, const void* k, int64
       reinterpret_cast<uintptr_t>(q) % piece != 0 || reinterpret_cast<uintptr_t>(k) % piece != 0 ||
       reinterpret_cast<uintptr_t>(state) % 16 != 0 || reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
     return fail(-1, "lv_chunk_scan: strides or alignment");
-  if (workspace_bytes < lv_chunk_scan_workspace_bytes(kind, T, B, max_new, H, D, Dv, seg_len))
+  const int64_t need = lv_chunk_scan_workspace_bytes(kind, T, B, max_new, H, D, Dv, seg_len);
+  if (need > 0 && !workspace) return fail(-1, "lv_chunk_scan: null pointer");
+  if (workspace_bytes < need)
     return fail(-3, "lv_chunk_scan: workspace of %lld bytes", static_cast<long long>(workspace_bytes));
   const int64_t rows = T * H, rows4 = (rows + 3) / 4 * 4;
   float* ws = static_cast<float*>(workspace);
@@ -1280,15 +1282,18 @@ static int chunk_scan(int kind, const void* q, int64_t ldq, const void* k, int64
                 static_cast<const float*>(p1), static_cast<const float*>(p2), static_cast<float*>(state), cu_q, ctx_lens, slots,
                 static_cast<float*>(o), nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, B, H, G, D, Dv, seg_len,
                 chunk_segments(kind, max_new, seg_len)};
-  p.P = ws;
-  ws += rows * kCh;
-  if (kind == kChunkDelta) {
-    p.Tm = ws;
+  const bool own = chunk_own(kind, T, B, max_new, H, D, Dv, p.segs, seg_len);
+  if (!own) {
+    p.P = ws;
     ws += rows * kCh;
+    if (kind == kChunkDelta) {
+      p.Tm = ws;
+      ws += rows * kCh;
+    }
+    p.Gf = ws;
+    p.Ef = ws + rows4;
+    ws += 2 * rows4;
   }
-  p.Gf = ws;
-  p.Ef = ws + rows4;
-  ws += 2 * rows4;
   if (p.segs > 1) {
     p.seg_state = ws;
     p.seg_decay = ws + static_cast<int64_t>(B) * p.segs * H * D * Dv;
@@ -1303,7 +1308,7 @@ static int chunk_scan(int kind, const void* q, int64_t ldq, const void* k, int64
     chunk_norm_dispatch(p, T, B, s);
   } else if (kind == kChunkDelta) chunk_dispatch<float, kChunkDelta>(p, T, B, false, s);
   else if (kind == kChunkStep) chunk_dispatch<bf16_t, kChunkStep>(p, T, B, false, s);
-  else chunk_dispatch<bf16_t, kChunkConst>(p, T, B, chunk_own(kind, T, B, max_new, H, D, Dv, p.segs, seg_len), s);
+  else chunk_dispatch<bf16_t, kChunkConst>(p, T, B, own, s);
   return launched("lv_chunk_scan");
 }
 

@@ -125,3 +125,15 @@ def test_where_the_norm_rides_with_the_scan(lens, H, Dv, pays):
     ([700, 100, 350, 600] * 4, 32, 64, 128, False), ([1024] * 9, 16, 128, 128, False), ([64] * 9, 16, 128, 128, True)])
 def test_where_the_norm_rides_by_head_sizes(lens, H, Dv, D, pays):
     assert mix_ops._chunk_norm_pays(lens, H, Dv, D) == pays
+
+
+@pytest.mark.parametrize("lens,seg,H,D,Dv,front", [
+    ([1024] * 16, 0, 16, 128, 128, False), ([1000], 0, 16, 128, 128, True), ([4000] + [300] * 12, 0, 16, 128, 128, True), ([1024] * 16, 0, 32, 128, 64, True),
+    ([1024] * 16, 0, 32, 64, 64, False), ([64] * 256, 0, 32, 64, 64, True), ([120] * 128, 0, 32, 64, 64, False), ([4000] + [300] * 12, 0, 32, 64, 64, True),
+    ([4096], 256, 32, 64, 64, False), ([4096], 256, 16, 128, 64, True), ([64] * 128, 0, 16, 64, 128, True)])
+def test_workspace_of_constant_decays(lens, seg, H, D, Dv, front):
+    """Launches that form their products in the scan keep none in memory: only the segments' states are asked for."""
+    from light_vllm_amd import _mixlib
+    T, B, segs = sum(lens), len(lens), -(-max(lens) // seg) if seg else 1
+    got = _mixlib.load().lv_chunk_scan_workspace_bytes(1, T, B, max(lens), H, D, Dv, seg)
+    assert got == 4 * ((T * H * 32 + 2 * (-(-T * H // 4) * 4) if front else 0) + (B * segs * H * (D * Dv + 1) if segs > 1 else 0))
