@@ -328,8 +328,9 @@ __device__ __forceinline__ chunk_bf16x8 join8(uint2 lo, uint2 hi) {
 // heads of 128: 267 + 59 us in two launches, 307 in one (the layer 829 -> 814).
 // CUT (delta rule, 128 rows of the state, eight waves): K^T U on the bf16 instructions, K and U cut into three pieces each (K once, where it is
 // staged; the state's other products would have it cut in every chunk): 1024 clocks a wave and chunk for 2048 of the chain's 6900 at the f32 rate. Sixteen
-// prompts of 1024 tokens, the layer 818 -> 803 us; 32 of 500 904 -> 888. States are 5.4 to 5.6e-8 off 64 bits (5.6 to 6.0 on f32 products: fewer roundings at the
-// state's magnitude), outputs 0.866e-7 either way. Constant decays gain nothing (833 / 836: their time is the silu of q, k and v), nor
+// prompts of 1024 tokens, the layer 818 -> 803 us; 32 of 500 904 -> 888. States off 64 bits, pieces / f32 products: decays
+// about 0.999, 1000 tokens, 1.6e-7 / 3.3e-7 (fewer roundings at the state's magnitude); fast decays, over all remainders of the last chunk, 6.8e-8 / 7.1e-8
+// root mean square, 8.4 / 9.9 the largest (by the places of the last tokens in the sum 0.7 to 1.4 of the other's). Outputs 8.8e-8 either way there, 1.9e-7 / 3.1e-7. Constant decays gain nothing (833 / 836: their time is the silu of q, k and v), nor
 // do launches of four waves (one prompt of 1000 250 / 255). Chunks with a value that is not finite take the f32 products.
 template <typename T, int KIND, int DT, int NW, int HPW, int MODE, bool NORM = false, bool OWN = false>
 __global__ __launch_bounds__(NW * 64, 2) void chunk_scan_kernel(ChunkParams p) {
