@@ -88,7 +88,7 @@ __global__ __launch_bounds__(512, 2) void router_tile_kernel(RouterParams p) {
     __builtin_amdgcn_sched_barrier(0);
   };
   // Step s (s % 4 = K): its fragments are in registers. Those of step s + 1 are read, step s + 2 goes from registers to its slot, which
-  // everyone read two steps ago, and step s + 6 is asked for in its place.
+  // everyone read during step s - 3, in front of a barrier, and step s + 6 is asked for in its place.
   Frags f0, f1;
   auto step = [&](auto K, const Frags& f, Frags& next, int s) __attribute__((always_inline)) {
     constexpr int k = decltype(K)::value;

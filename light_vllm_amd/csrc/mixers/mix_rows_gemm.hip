@@ -32,7 +32,7 @@ struct RowsGemmParams {
 };
 
 // A workgroup: 16 MT rows x 16 NT columns. PF pieces of 64 steps of k are on their way in registers. MANY: any number of rows, row tiles side by
-// side on the grid, column tiles below them (the columns that a wide product leaves beside its tiles).
+// side on the grid, and all columns in each (those that a wide product leaves beside its tiles).
 template <int MT, int NT, int PF, bool MANY = false>
 __global__ __launch_bounds__(kRowsWaves * kWave) void rows_gemm_kernel(RowsGemmParams p) {
   constexpr int NW = kRowsWaves, RS = NT * 16 + 4;
@@ -40,7 +40,7 @@ __global__ __launch_bounds__(kRowsWaves * kWave) void rows_gemm_kernel(RowsGemmP
   __shared__ __attribute__((aligned(16))) unsigned char lds[NW * PER];
   const int row_parts = (p.M + 16 * MT - 1) / (16 * MT);
   const int grp = blockIdx.x / (8 * row_parts), rem = blockIdx.x % (8 * row_parts);
-  const int n0 = MANY ? blockIdx.y * NT * 16 : (grp * 8 + rem % 8) * NT * 16, m0 = MANY ? blockIdx.x * MT * 16 : rem / 8 * MT * 16;
+  const int n0 = MANY ? 0 : (grp * 8 + rem % 8) * NT * 16, m0 = MANY ? blockIdx.x * MT * 16 : rem / 8 * MT * 16;
   if (n0 >= p.N) return;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, quad = lane >> 4;
   const int lrow = lane >> 3, lch = lane & 7;
@@ -180,7 +180,7 @@ extern "C" int lv_rows_gemm(const void* x, int64_t ldx, const void* w, int64_t l
 
 // Few columns of many rows, bound by reading x once (16384 x 2048 in 12.8 us, 5.2 TB/s, for 32 columns, 13.4 for 16, 16.3 for 64, of which the
 // rows of w that every workgroup reads are the rest): 32 rows a workgroup, eight waves share k, and all the columns in one, so that x is not
-// read twice. The vendor's product of 5152 columns instead of 5120 takes 37 us more.
+// read twice. The vendor's product of 5152 columns instead of 5120 takes 42 us more (232 -> 274).
 extern "C" int lv_columns_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, int64_t ldy, int64_t M, int N, int K,
                                void* stream) {
   if (M == 0 || N == 0) return 0;
