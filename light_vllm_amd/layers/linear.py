@@ -26,7 +26,9 @@ def _linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) ->
         # mix_ops.linear's first looks, without a call: a prompt's step on few tokens is bound by the host, and goes on to torch's linear here
         if bias is None and type(x) is _Tensor and not _compiling() and not _tracing():
             shape = x.shape
-            if len(shape) == 2 and (shape[0] <= _FEW or shape[0] >= _MANY):
+            if len(shape) == 2 and shape[0] <= _FEW:
+                return mix_ops.rows_linear(x, weight)
+            if len(shape) == 2 and shape[0] >= _MANY:
                 return mix_ops.linear(x, weight)
     return F.linear(x, weight, bias)
 

@@ -1994,13 +1994,18 @@ def _split_linear(x, w, sizes):
     return y
 
 
-def linear(x, w):
-    """x [..., K] w [N, K]^T. Few rows of bf16 (decode steps) take lv_rows_gemm, many rows and a few columns more than whole tiles two launches
-    (_split_sizes), everything else torch's linear."""
+def rows_linear(x, w):
+    """linear for at most ROWS_GEMM_MAX rows: lv_rows_gemm or torch's linear, without a look at what only many rows can have."""
     sizes = _rows_gemm_sizes(x, w)
     if sizes is None:
-        sizes = _split_sizes(x, w)
-        return F.linear(x, w) if sizes is None else _split_linear(x, w, sizes)
+        return F.linear(x, w)
     if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
         return _RowsLinear.apply(x, w, sizes)
     return _rows_gemm(x, w, sizes)
+
+
+def linear(x, w):
+    """x [..., K] w [N, K]^T. Few rows of bf16 (decode steps) take lv_rows_gemm, many rows and a few columns more than whole tiles two launches
+    (_split_sizes), everything else torch's linear."""
+    sizes = _split_sizes(x, w)
+    return rows_linear(x, w) if sizes is None else _split_linear(x, w, sizes)

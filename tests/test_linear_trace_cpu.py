@@ -80,3 +80,15 @@ def test_operands_that_are_no_matrices(m):
         x = torch.randn(shape)
         assert torch.equal(m(x), F.linear(x, m.weight))
     assert torch.func.vmap(m)(torch.randn(2, 8, K)).shape == (2, 8, N)
+
+
+def test_few_rows_are_not_asked_what_only_many_can_have(monkeypatch):
+    """Eager steps of few tokens are bound by the host: a projection of theirs looks for the kernel of few rows only, one between for none."""
+    asked = []
+    for name in ("_split_sizes", "_rows_gemm_sizes"):
+        monkeypatch.setattr(mix_ops, name, lambda x, w, name=name: asked.append((name, len(x))))
+    m = layer(ReplicatedLinear)
+    with torch.no_grad():
+        for n in (8, 64, 65, 4095, 4096):
+            assert torch.equal(m(rows(n)), F.linear(rows(n), m.weight))
+    assert asked == [("_rows_gemm_sizes", 8), ("_rows_gemm_sizes", 64), ("_split_sizes", 4096), ("_rows_gemm_sizes", 4096)]
