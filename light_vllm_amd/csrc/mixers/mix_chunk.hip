@@ -10,7 +10,7 @@
 //   O = diag(G) Q S + P U,      P_tj = D_tj (q_t . k_j) w_j for j <= t   (w = 1 for the delta rule)
 //   S <- G_last S + K^T diag(E w) U
 //
-// chunk_prep_kernel      T, P, G and E w of every chunk, all of them side by side (large launches of constant decays form them in the scan)
+// chunk_prep_kernel      T, P, G and E w of every chunk, all of them side by side (constant decays may form them in the scan: chunk_own)
 // chunk_scan_kernel      the chain over a sequence's chunks; a wave owns all D rows of 16 columns of the state
 // chunk_step_kernel      the same for step sizes, on the bf16 matrix instructions
 // chunk_combine_kernel   starting states of a sequence's segments, where there are too few sequences for the chip

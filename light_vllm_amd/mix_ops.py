@@ -38,7 +38,8 @@ CHUNK_FROM = {CHUNK_STEP: 80, CHUNK_CONST: 80, CHUNK_DELTA: 32}
 # What _chunk_pays weighs from there on, in us, by kind and rows of the state: a token of the longest sequence in the token loop
 # (launches of fewer than 1024 workgroups, of more), 256 x 128 columns by a token in it; a chunk behind another one, 256 x 128
 # columns by a chunk; what two launches cost more than one. Fitted to 258 steps of 1 to 256 sequences, one portion beside decoded
-# tokens, equal portions and mixtures: of those that CHUNK_FROM lets through, the choice is within 7 % of the better one.
+# tokens, equal portions and mixtures: of those that CHUNK_FROM lets through, the choice is within 7 % of the better one. Large launches of
+# constant decays have one launch less since: 198 of 200 steps of theirs within 7 %, the others 8 and 14 (3 and 7 us).
 CHUNK_COSTS = {(CHUNK_STEP, 64): (0.29, 0.49, 0.28, 1.1, 5.6, 14.5), (CHUNK_STEP, 128): (0.34, 0.78, 0.47, 2.8, 7.2, 10.5),
                (CHUNK_CONST, 64): (0.19, 0.40, 0.46, 1.8, 5.3, 12.5), (CHUNK_CONST, 128): (0.32, 0.80, 0.62, 4.0, 7.2, 14.5),
                (CHUNK_DELTA, 64): (0.51, 0.59, 0.41, 5.3, 8.7, 11.0), (CHUNK_DELTA, 128): (0.76, 1.0, 0.83, 7.9, 8.2, 9.5)}
@@ -241,8 +242,10 @@ def _segment_length(lens, wgs, state_bytes) -> int:
     """Tokens of the segments that sequences are cut into, 0: none. A workgroup (one of `wgs` a sequence or segment) fills a
     compute unit, so a launch takes rounds of 256 of them, as long as their segment; segments cost 1.45 times the products (their
     contributions are formed first). 7 prompts of 900 to 3750 tokens, 32 heads of 128 x 64: 741 us whole, 445 / 463 / 615 us
-    in segments of 256 / 512 / 1024; one of 4096: 713, 119 / 173 / 303 us; 8 of 2048, 16 heads of 128 x 128: 471 us whole, 440 / 404 /
-    409 us. Segments whose states would take more than 256 MB are not considered."""
+    in segments of 256 / 512 / 1024; one of 4096: 713, 119 / 173 / 303 us. Constant decays, 16 heads of 128 x 128, 4 of 4096: 681
+    whole, 399 in segments of 1024. Of 50 steps of theirs it takes the best of five lengths, to 2 %, in 37, and one that is 4 to 22 %
+    behind in the others: 8 of 2048 374 whole, 455 / 416 / 399 in segments; 16 of 1024, heads of 128 x 64, 223 whole, 273 of 512;
+    one of 4000 beside 12 of 300 325 of 256, 286 of 512. Segments whose states would take more than 256 MB are not considered."""
     longest = max(lens)
     whole = len(lens) * wgs
     best, cost = 0, longest if whole <= 256 else max(longest, sum(lens) * wgs // 256 + longest // 2)
